@@ -52,6 +52,7 @@ class Frame(ctypes.Structure):
         ("tile_order", ctypes.c_void_p),
         ("depth_order", ctypes.c_void_p),
         ("n_instances", ctypes.c_uint64),
+        ("n_instances_live", ctypes.c_void_p),
         ("keys", ctypes.c_void_p * 2),
         ("vals", ctypes.c_void_p * 2),
         ("sort_tmp", ctypes.c_void_p),
@@ -80,8 +81,30 @@ class Frame(ctypes.Structure):
     ]
 
 
+class Workspace(ctypes.Structure):
+    """``struct htgs_workspace``."""
+    _fields_ = [
+        ("front", ctypes.c_void_p),
+        ("front_bytes", ctypes.c_uint64),
+        ("back", ctypes.c_void_p),
+        ("back_bytes", ctypes.c_uint64),
+        ("expected", ctypes.c_uint64),
+        ("max_weights", ctypes.c_void_p),
+        ("weight_threshold", ctypes.c_float),
+        ("what", ctypes.c_int32),
+        ("front_needed", ctypes.c_uint64),
+        ("back_needed", ctypes.c_uint64),
+        ("n_instances", ctypes.c_uint64),
+        ("selector", ctypes.c_int32),
+    ]
+
+
+WORKSPACE_TOO_SMALL = 4
+RUN_RENDER, RUN_FORWARD, RUN_MAX_WEIGHTS = 0, 1, 2
+
 # every symbol include/htgs_amd.h declares: name -> (restype, argtypes)
 _FRAME_P = ctypes.POINTER(Frame)
+_WORKSPACE_P = ctypes.POINTER(Workspace)
 SYMBOLS = {
     "htgs_last_error": (ctypes.c_char_p, []),
     "htgs_tile_size": (ctypes.c_int, [ctypes.c_int]),
@@ -120,6 +143,9 @@ SYMBOLS = {
     "htgs_update_3d_filter": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
                                              ctypes.c_int, ctypes.c_int, ctypes.c_float, ctypes.c_float, ctypes.c_float, ctypes.c_float,
                                              ctypes.c_float, ctypes.c_float, ctypes.c_float, ctypes.c_void_p]),
+    "htgs_run": (ctypes.c_int, [_FRAME_P, _WORKSPACE_P]),
+    "htgs_run_rest": (ctypes.c_int, [_FRAME_P, _WORKSPACE_P]),
+    "htgs_run_sizes": (ctypes.c_int, [_FRAME_P, _WORKSPACE_P]),
     "htgs_check_reciprocal": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p]),
     "htgs_check_tile_cull": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p]),
 }

@@ -168,13 +168,8 @@ __global__ void __launch_bounds__(256) check_tile_cull_16_kernel(
     }
 }
 
-// the least length of a part of a long list (0: lists are not split, there is no spare value buffer to leave the parts' results in)
-static uint32_t long_part_floor(const htgs_frame *f, int selector, uint32_t n_tiles)
-{
-    if (f->vals[selector ^ 1] == nullptr) return 0u;
-    const uint64_t floor = (f->n_instances + n_tiles - 1) / n_tiles;
-    return floor < 1u ? 1u : (uint32_t)floor;
-}
+// (lists are not split without a spare value buffer to leave the parts' results in)
+static PartFloor long_part_floor(const htgs_frame *f, int selector) { return PartFloor{ instance_count(f), f->vals[selector ^ 1] != nullptr ? 1u : 0u }; }
 
 template <int K, bool FAST>
 static void launch_hybrid(const htgs_frame *f, int selector, uint32_t grid_w, uint32_t n_tiles)
@@ -184,11 +179,11 @@ static void launch_hybrid(const htgs_frame *f, int selector, uint32_t grid_w, ui
     if (f->long_tiles != nullptr && threshold <= kPackedListMost)
         hipLaunchKernelGGL((blend_hybrid_kernel<K, FAST, true>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
-                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector, n_tiles), f->tile_order);
+                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
     else
         hipLaunchKernelGGL((blend_hybrid_kernel<K, FAST>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
-                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector, n_tiles), f->tile_order);
+                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
     if (f->long_tiles)      // (one workgroup per compute unit; they find an empty list on ordinary frames)
         hipLaunchKernelGGL((blend_hybrid_long_kernel<K, FAST, HTGS_PRIM_FLOATS / 4, HybridImage>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0,
                            (hipStream_t)f->stream, f->ranges, f->vals[selector], (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w,
@@ -202,11 +197,11 @@ static void launch_first_k(const htgs_frame *f, int selector, uint32_t grid_w, u
     if (!FAST && f->long_tiles != nullptr && threshold <= kPackedListMost)
         hipLaunchKernelGGL((blend_first_k_kernel<K, false, true>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
-                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector, n_tiles), f->tile_order);
+                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
     else
         hipLaunchKernelGGL((blend_first_k_kernel<K, FAST>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
-                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector, n_tiles), f->tile_order);
+                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
     if (f->long_tiles)
         hipLaunchKernelGGL((blend_first_k_long_kernel<K, FAST, HTGS_PRIM_FLOATS / 4, FirstKImage>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0,
                            (hipStream_t)f->stream, f->ranges, f->vals[selector], (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w,
@@ -250,7 +245,7 @@ static void launch_blend(const htgs_frame *f, int selector, uint32_t grid_w, uin
             const uint32_t threshold = f->long_list_threshold > 0 ? (uint32_t)f->long_list_threshold : kLongListDefault;
             hipLaunchKernelGGL(blend_oit_kernel<FAST>, dim3(n_tiles), dim3(64), 0, s, f->ranges, f->vals[selector], (const float4 *)f->prim,
                                f->image, depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw, f->long_tiles, threshold,
-                               long_part_floor(f, selector, n_tiles), f->tile_order);
+                               long_part_floor(f, selector), f->tile_order);
             if (f->long_tiles)
                 hipLaunchKernelGGL((blend_oit_long_kernel<FAST, HTGS_PRIM_FLOATS / 4, OitImage>), dim3(256), dim3(64 * kLongWaves), 0, s, f->ranges, f->vals[selector],
                                    (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->vals[selector ^ 1], threshold,

@@ -108,7 +108,7 @@ struct HybridRecords {
 template <int K>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 5 : 3))) blend_hybrid_forward_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
-    uint32_t *__restrict__ long_tiles, uint32_t long_threshold, uint32_t part_floor, const uint32_t *__restrict__ tile_order, const HybridRecords finish)
+    uint32_t *__restrict__ long_tiles, uint32_t long_threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, const HybridRecords finish)
 {
     __shared__ TileStageQ st;
     __shared__ QuadrantLists ql;
@@ -116,7 +116,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
     const uint32_t lane = threadIdx.x;
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
     if (long_tiles != nullptr && last - first > long_threshold) {
-        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, long_part_words<K>(), part_floor);
+        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, long_part_words<K>(), part_floor.get(gridDim.x));
         return;
     }
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
@@ -191,7 +191,7 @@ struct FirstKRecords {
 template <int K>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 5 : 2))) blend_first_k_forward_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
-    uint32_t *__restrict__ long_tiles, uint32_t long_threshold, uint32_t part_floor, const uint32_t *__restrict__ tile_order, const FirstKRecords finish)
+    uint32_t *__restrict__ long_tiles, uint32_t long_threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, const FirstKRecords finish)
 {
     __shared__ TileStageQ st;
     __shared__ QuadrantLists ql;
@@ -199,7 +199,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
     const uint32_t lane = threadIdx.x;
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
     if (long_tiles != nullptr && last - first > long_threshold) {
-        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, first_k_part_words<K>(), part_floor);
+        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, first_k_part_words<K>(), part_floor.get(gridDim.x));
         return;
     }
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
@@ -237,7 +237,7 @@ struct OitRecords {
 
 __global__ void __launch_bounds__(64) blend_oit_forward_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
-    uint32_t *__restrict__ long_tiles, uint32_t long_threshold, uint32_t part_floor, const uint32_t *__restrict__ tile_order, const OitRecords finish)
+    uint32_t *__restrict__ long_tiles, uint32_t long_threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, const OitRecords finish)
 {
     __shared__ TileStageQ st;
     __shared__ QuadrantLists ql;
@@ -245,7 +245,7 @@ __global__ void __launch_bounds__(64) blend_oit_forward_kernel(
     const uint32_t lane = threadIdx.x;
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
     if (long_tiles != nullptr && last - first > long_threshold) {
-        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, kOitPartWords, part_floor);
+        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, kOitPartWords, part_floor.get(gridDim.x));
         return;
     }
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
@@ -301,13 +301,8 @@ __global__ void __launch_bounds__(256) blend_global_forward_kernel(
     image[pix] = r; image[np + pix] = g; image[2 * np + pix] = b;
 }
 
-// the least length of a part of a long list (0: lists are not split, there is no spare value buffer to leave the parts' results in)
-static uint32_t forward_part_floor(const htgs_frame *f, int sel, uint32_t n_tiles)
-{
-    if (f->vals[sel ^ 1] == nullptr) return 0u;
-    const uint64_t floor = (f->n_instances + n_tiles - 1) / n_tiles;
-    return floor < 1u ? 1u : (uint32_t)floor;
-}
+// (lists are not split without a spare value buffer to leave the parts' results in)
+static PartFloor forward_part_floor(const htgs_frame *f, int sel) { return PartFloor{ instance_count(f), f->vals[sel ^ 1] != nullptr ? 1u : 0u }; }
 static uint32_t forward_threshold(const htgs_frame *f) { return f->long_list_threshold > 0 ? (uint32_t)f->long_list_threshold : kLongListDefault; }
 
 template <int K>
@@ -316,7 +311,7 @@ static void launch_hybrid_forward(const htgs_frame *f, int sel, uint32_t grid_w,
     constexpr int REC4 = HTGS_PRIM_FLOATS_TRAIN / 4;
     const HybridRecords finish = { f->image, f->core_idx, (float4 *)f->core_info, f->tail_info, (uint32_t)f->width, (uint32_t)f->height, (size_t)n_tiles * 64u };
     hipLaunchKernelGGL((blend_hybrid_forward_kernel<K>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim,
-                       (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, forward_threshold(f), forward_part_floor(f, sel, n_tiles), f->tile_order, finish);
+                       (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, forward_threshold(f), forward_part_floor(f, sel), f->tile_order, finish);
     if (f->long_tiles)
         hipLaunchKernelGGL((blend_hybrid_long_kernel<K, false, REC4, HybridRecords>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0,
                            (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w,
@@ -328,7 +323,7 @@ static void launch_first_k_forward(const htgs_frame *f, int sel, uint32_t grid_w
     constexpr int REC4 = HTGS_PRIM_FLOATS_TRAIN / 4;
     const FirstKRecords finish = { f->image, f->core_idx, (float4 *)f->core_info, (uint32_t)f->width, (uint32_t)f->height, (size_t)n_tiles * 64u };
     hipLaunchKernelGGL((blend_first_k_forward_kernel<K>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim,
-                       (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, forward_threshold(f), forward_part_floor(f, sel, n_tiles), f->tile_order, finish);
+                       (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, forward_threshold(f), forward_part_floor(f, sel), f->tile_order, finish);
     if (f->long_tiles)
         hipLaunchKernelGGL((blend_first_k_long_kernel<K, false, REC4, FirstKRecords>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0,
                            (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w,
@@ -339,7 +334,7 @@ static void launch_oit_forward(const htgs_frame *f, int sel, uint32_t grid_w, ui
     constexpr int REC4 = HTGS_PRIM_FLOATS_TRAIN / 4;
     const OitRecords finish = { f->image, f->tail_info, (uint32_t)f->width, (uint32_t)f->height, (size_t)n_tiles * 64u };
     hipLaunchKernelGGL(blend_oit_forward_kernel, dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim,
-                       (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, forward_threshold(f), forward_part_floor(f, sel, n_tiles), f->tile_order, finish);
+                       (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, forward_threshold(f), forward_part_floor(f, sel), f->tile_order, finish);
     if (f->long_tiles)
         hipLaunchKernelGGL((blend_oit_long_kernel<false, REC4, OitRecords, false>), dim3(256), dim3(64 * kLongWaves), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel],
                            (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->vals[sel ^ 1], forward_threshold(f), finish);

@@ -116,6 +116,33 @@ int sort_u32_pairs(void *stream, uint32_t *const keys[2], uint32_t *const vals[2
 int sort_u32_pairs_with_rectangles(void *stream, uint32_t *const keys[2], uint32_t *const vals[2], uint32_t *sort_tmp, uint64_t n, int bits,
                                    const uint16_t *rectangles_in, uint16_t *rectangles_out, uint32_t *counts_out, uint32_t culled);
 
+// The number of (tile, Gaussian) instances as a kernel sees it.  live = nullptr: `most` is the number, the host knows it
+// (the stage-by-stage entry points).  Otherwise the kernels were queued before the host knew: they read the number the scan
+// left on the device, and a number beyond `most`, which the buffers and the launches were sized for, counts as 0 -- every
+// list is empty and the host, which learns the number meanwhile, queues the stages again (htgs_run).
+struct InstanceCount {
+    const uint32_t *live;
+    uint32_t most;
+    __device__ __forceinline__ uint32_t get() const
+    {
+        if (live == nullptr) return most;
+        const uint32_t n = *live;
+        return n <= most ? n : 0u;
+    }
+};
+inline InstanceCount instance_count(const htgs_frame *f) { return InstanceCount{ f->n_instances_live, (uint32_t)f->n_instances }; }
+// The least length of a part of a very long list: the frame's average list, rounded up (0: lists are not split)
+struct PartFloor {
+    InstanceCount count;
+    uint32_t split;
+    __device__ __forceinline__ uint32_t get(uint32_t n_tiles) const
+    {
+        if (split == 0u) return 0u;
+        const uint32_t n = count.get(), floor = n / n_tiles + (n % n_tiles != 0u ? 1u : 0u);
+        return floor < 1u ? 1u : floor;
+    }
+};
+
 // host side error reporting (api.hip)
 int fail(int code, const char *fmt, ...);
 int check_launch(const char *what);

@@ -62,7 +62,8 @@ __global__ void __launch_bounds__(kScanBlock) scan_reduce_kernel(const uint32_t 
 // the reference; a frame whose counts add up to more than 2^32 - 2 publishes 0xffffffff, which no valid frame
 // produces, so that the host can refuse it instead of sizing its buffers from a wrapped sum.
 __global__ void __launch_bounds__(kScanBlock) scan_apply_kernel(const uint32_t *__restrict__ in, const uint32_t *__restrict__ tile_sums,
-                                                               uint32_t *__restrict__ out, uint32_t *__restrict__ total_out, int n)
+                                                               uint32_t *__restrict__ out, uint32_t *__restrict__ total_out, int n,
+                                                               unsigned long long *__restrict__ host_total, uint32_t tag)
 {
     __shared__ uint32_t wave_sums[kScanBlock / kWave];
     __shared__ unsigned long long s_wide[kScanBlock / kWave];
@@ -95,7 +96,11 @@ __global__ void __launch_bounds__(kScanBlock) scan_apply_kernel(const uint32_t *
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
         const unsigned long long sum = before + total;
-        *total_out = sum > 0xfffffffeull ? 0xffffffffu : (uint32_t)sum;
+        const uint32_t total32 = sum > 0xfffffffeull ? 0xffffffffu : (uint32_t)sum;
+        *total_out = total32;
+        // the same for the host, which waits for this word (its upper half says which frame it belongs to) and not for the stream
+        if (host_total != nullptr)
+            __hip_atomic_store(host_total, (unsigned long long)tag << 32 | total32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -193,8 +198,9 @@ __global__ void __launch_bounds__(256) gather_counts_kernel(const uint32_t *__re
 // A thread takes the keys of one 16-byte word (and the key before them) and writes a range boundary wherever two
 // neighbours differ.
 template <typename KeyT, int SHIFT>
-__global__ void __launch_bounds__(256) extract_ranges_kernel(const KeyT *__restrict__ keys, uint32_t *__restrict__ ranges, uint64_t n)
+__global__ void __launch_bounds__(256) extract_ranges_kernel(const KeyT *__restrict__ keys, uint32_t *__restrict__ ranges, InstanceCount count)
 {
+    const uint64_t n = count.get();
     constexpr int kPer = 16 / sizeof(KeyT);
     const uint64_t first = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * kPer;
     if (first >= n) return;
@@ -359,7 +365,7 @@ static uint32_t *static_scan_scratch()
     return g_scratch_ptr[dev];
 }
 
-static int launch_scan(const htgs_frame *f, uint32_t *tile_sums, const char *who)
+static int launch_scan(const htgs_frame *f, uint32_t *tile_sums, const char *who, unsigned long long *host_total = nullptr, uint32_t tag = 0)
 {
     hipStream_t s = (hipStream_t)f->stream;
     const int n = f->n_primitives;
@@ -389,7 +395,7 @@ static int launch_scan(const htgs_frame *f, uint32_t *tile_sums, const char *who
     }
     if (tiles > 0) {
         hipLaunchKernelGGL(scan_reduce_kernel, dim3(tiles), dim3(kScanBlock), 0, s, counts, tile_sums, n);
-        hipLaunchKernelGGL(scan_apply_kernel, dim3(tiles), dim3(kScanBlock), 0, s, counts, tile_sums, f->offsets, f->n_instances_dev, n);
+        hipLaunchKernelGGL(scan_apply_kernel, dim3(tiles), dim3(kScanBlock), 0, s, counts, tile_sums, f->offsets, f->n_instances_dev, n, host_total, tag);
     } else {
         hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(256), 0, s, f->n_instances_dev, (size_t)1, (uint32_t *)nullptr, (uint32_t *)nullptr);
     }
@@ -430,6 +436,14 @@ extern "C" int htgs_scan_offsets(const htgs_frame *f)
     if (!f->n_instances_dev || !f->scan_tmp) return fail(HTGS_ERR_ARGUMENT, "htgs_scan_offsets: null pointer");
     return launch_scan(f, f->scan_tmp, "htgs_scan_offsets");
 }
+
+namespace htgs {
+int scan_offsets_publish(const htgs_frame *f, unsigned long long *host_total, uint32_t tag)
+{
+    if (!f->n_instances_dev || !f->scan_tmp) return fail(HTGS_ERR_ARGUMENT, "htgs_scan_offsets: null pointer");
+    return launch_scan(f, f->scan_tmp, "htgs_scan_offsets", host_total, tag);
+}
+}  // namespace htgs
 
 extern "C" int htgs_scan_static_max_primitives(void) { return kStaticScanWords * kScanTile; }
 
@@ -508,11 +522,11 @@ extern "C" int htgs_extract_ranges(const htgs_frame *f, int selector)
         const uint64_t per_block = 256ull * (16 / kb);
         const dim3 grid((unsigned)((f->n_instances + per_block - 1) / per_block)), block(256);
         if (kb == 8)
-            hipLaunchKernelGGL((extract_ranges_kernel<uint64_t, 32>), grid, block, 0, s, (const uint64_t *)f->keys[selector], f->ranges, f->n_instances);
+            hipLaunchKernelGGL((extract_ranges_kernel<uint64_t, 32>), grid, block, 0, s, (const uint64_t *)f->keys[selector], f->ranges, instance_count(f));
         else if (kb == 4)
-            hipLaunchKernelGGL((extract_ranges_kernel<uint32_t, 0>), grid, block, 0, s, (const uint32_t *)f->keys[selector], f->ranges, f->n_instances);
+            hipLaunchKernelGGL((extract_ranges_kernel<uint32_t, 0>), grid, block, 0, s, (const uint32_t *)f->keys[selector], f->ranges, instance_count(f));
         else
-            hipLaunchKernelGGL((extract_ranges_kernel<uint16_t, 0>), grid, block, 0, s, (const uint16_t *)f->keys[selector], f->ranges, f->n_instances);
+            hipLaunchKernelGGL((extract_ranges_kernel<uint16_t, 0>), grid, block, 0, s, (const uint16_t *)f->keys[selector], f->ranges, instance_count(f));
     }
     if (f->tile_order) {
         const uint32_t grid_w = (uint32_t)div_up(f->width, tile), grid_h = (uint32_t)div_up(f->height, tile);

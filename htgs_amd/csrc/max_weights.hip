@@ -20,7 +20,7 @@ template <int K, int MODE>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 5 : 2))) max_weights_tile_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
     uint32_t *__restrict__ max_weights, uint32_t width, uint32_t height, uint32_t grid_w, float weight_threshold, const uint32_t *__restrict__ tile_order,
-    uint32_t *__restrict__ long_tiles, uint32_t long_threshold, uint32_t part_floor)
+    uint32_t *__restrict__ long_tiles, uint32_t long_threshold, PartFloor part_floor)
 {
     constexpr bool kCore = MODE != HTGS_MODE_OIT_BLEND;
     constexpr bool kTail = MODE != HTGS_MODE_ALPHA_BLEND_FIRST_K;
@@ -34,7 +34,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
         const uint32_t length = ranges[2 * tile + 1] - ranges[2 * tile];
         if (long_tiles != nullptr && length > long_threshold) {
             constexpr uint32_t part_words = MODE == HTGS_MODE_HYBRID_BLEND ? long_part_words<KS>() : MODE == HTGS_MODE_OIT_BLEND ? kOitPartWords : first_k_part_words<KS>();
-            if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, length, long_threshold, part_words, part_floor);
+            if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, length, long_threshold, part_words, part_floor.get(gridDim.x));
             return;
         }
     }
@@ -192,12 +192,12 @@ struct MaxWeightsOit {
 // After the kernels for very long lists have left the tail weights of such tiles: the tiles are entered on the list again,
 // in parts, for the second walk.
 __global__ void __launch_bounds__(256) max_weights_tail_enter_kernel(const uint32_t *__restrict__ ranges, uint32_t *__restrict__ long_tiles, uint32_t n_tiles,
-                                                                    uint32_t long_threshold, uint32_t part_floor)
+                                                                    uint32_t long_threshold, PartFloor part_floor)
 {
     const uint32_t tile = blockIdx.x * 256 + threadIdx.x;
     if (tile >= n_tiles) return;
     const uint32_t length = ranges[2 * tile + 1] - ranges[2 * tile];
-    if (length > long_threshold) long_tile_enter(long_tiles, tile, n_tiles, length, long_threshold / 4u, 0u, part_floor);   // (parts of one threshold's length)
+    if (length > long_threshold) long_tile_enter(long_tiles, tile, n_tiles, length, long_threshold / 4u, 0u, part_floor.get(n_tiles));   // (parts of one threshold's length)
 }
 // The second walk (alpha * tail weight for every fragment that passes the cut-off) over the parts of the very long lists:
 // a workgroup of four waves per part, every wave a share of it; the maximum is order independent, nothing to merge.
@@ -234,12 +234,10 @@ __global__ void __launch_bounds__(64 * kTailWaves) max_weights_tail_long_kernel(
     }
 }
 
-// the least length of a part of a long list; 0: lists are not split (there is no spare value buffer for what the parts leave behind)
-static uint32_t part_floor_of(const htgs_frame *f, int sel, uint32_t n_tiles, bool needs_spare)
+// (lists are not split when there is no spare value buffer for what the parts leave behind)
+static PartFloor part_floor_of(const htgs_frame *f, int sel, bool needs_spare)
 {
-    if (needs_spare && f->vals[sel ^ 1] == nullptr) return 0u;
-    const uint64_t floor = (f->n_instances + n_tiles - 1) / n_tiles;
-    return floor < 1u ? 1u : (uint32_t)floor;
+    return PartFloor{ instance_count(f), needs_spare && f->vals[sel ^ 1] == nullptr ? 0u : 1u };
 }
 // the tiles with very long lists are taken by the kernels that share a list only when the caller provided the list for such
 // tiles and, in the modes with a tail, the per-pixel scratch for the tail weights between the two walks
@@ -254,7 +252,7 @@ static void launch_tile(const htgs_frame *f, int sel, uint32_t *max_weights, flo
     const bool shared = shares_long_lists<MODE>(f);
     const uint32_t w = (uint32_t)f->width, h = (uint32_t)f->height;
     hipLaunchKernelGGL((max_weights_tile_kernel<K, MODE>), dim3(n_tiles), dim3(64), 0, s, f->ranges, f->vals[sel], (const float4 *)f->prim, max_weights, w, h, grid_w,
-                       thr, f->tile_order, shared ? f->long_tiles : nullptr, threshold, part_floor_of(f, sel, n_tiles, true));
+                       thr, f->tile_order, shared ? f->long_tiles : nullptr, threshold, part_floor_of(f, sel, true));
     if (!shared) return;
     constexpr int REC4 = HTGS_PRIM_FLOATS / 4;
     if constexpr (MODE == HTGS_MODE_HYBRID_BLEND)
@@ -269,7 +267,7 @@ static void launch_tile(const htgs_frame *f, int sel, uint32_t *max_weights, flo
                            (const float4 *)f->prim, f->long_tiles, w, h, grid_w, f->vals[sel ^ 1], threshold, MaxWeightsOit{ f->pixel_scratch, thr });
     if constexpr (MODE != HTGS_MODE_ALPHA_BLEND_FIRST_K) {
         hipLaunchKernelGGL(max_weights_tail_enter_kernel, dim3((n_tiles + 255) / 256), dim3(256), 0, s, f->ranges, f->long_tiles, n_tiles, threshold,
-                           part_floor_of(f, sel, n_tiles, false));
+                           part_floor_of(f, sel, false));
         hipLaunchKernelGGL(max_weights_tail_long_kernel<MODE>, dim3(1024), dim3(64 * kTailWaves), 0, s, f->ranges, f->vals[sel], (const float4 *)f->prim, f->long_tiles,
                            max_weights, f->pixel_scratch, w, h, grid_w, thr, threshold);
     }

@@ -32,16 +32,20 @@ __device__ __forceinline__ uint32_t digit_of(KeyT k, int shift, uint32_t mask) {
 constexpr uint32_t kXcds = 8;
 __device__ __forceinline__ uint32_t xcd_contiguous_block(uint32_t launched, uint32_t n_blocks)
 {
+    // (the launch may be larger than n_blocks asks for: its blocks beyond an XCD's share have nothing to do)
     const uint32_t per_xcd = (n_blocks + kXcds - 1) / kXcds;
-    return (launched % kXcds) * per_xcd + launched / kXcds;           // >= n_blocks: nothing to do
+    return launched / kXcds < per_xcd ? (launched % kXcds) * per_xcd + launched / kXcds : n_blocks;           // >= n_blocks: nothing to do
 }
+__device__ __forceinline__ uint32_t blocks_of(uint32_t n, uint32_t per_block) { return n / per_block + (n % per_block != 0u ? 1u : 0u); }
 inline uint32_t xcd_padded_grid(uint32_t n_blocks) { return (n_blocks + kXcds - 1) / kXcds * kXcds; }
 
 template <typename KeyT, int THREADS = SortShape<KeyT>::threads, int BITS = SortDigit<KeyT>::bits>
 __global__ void __launch_bounds__(THREADS) digit_histogram_kernel(const KeyT *__restrict__ keys, uint32_t *__restrict__ hist,
-                                                                uint64_t n, uint32_t n_blocks, int shift, uint32_t mask)
+                                                                InstanceCount count, int shift, uint32_t mask)
 {
     constexpr int kSortThreads = THREADS, kSortTile = kSortThreads * kSortItems, kRadix = 1 << BITS;
+    const uint64_t n = count.get();
+    const uint32_t n_blocks = blocks_of((uint32_t)n, kSortTile);
     static_assert(kRadix <= kSortThreads, "one thread per digit");
     __shared__ uint32_t counts[kRadix];
     const uint32_t block = xcd_contiguous_block(blockIdx.x, n_blocks);
@@ -73,8 +77,10 @@ __global__ void __launch_bounds__(THREADS) digit_histogram_kernel(const KeyT *__
 }
 
 // block d scans row d of hist in place (exclusive) and writes the row total to totals[d]
-__global__ void __launch_bounds__(kScanThreads) digit_row_scan_kernel(uint32_t *__restrict__ hist, uint32_t *__restrict__ totals, uint32_t n_blocks)
+__global__ void __launch_bounds__(kScanThreads) digit_row_scan_kernel(uint32_t *__restrict__ hist, uint32_t *__restrict__ totals, InstanceCount count,
+                                                                      uint32_t per_block)
 {
+    const uint32_t n_blocks = blocks_of(count.get(), per_block);
     constexpr int kSortThreads = kScanThreads, kSortWaves = kScanThreads / kWave;
     __shared__ uint32_t wave_sums[kSortWaves];
     uint32_t *row = hist + (size_t)blockIdx.x * n_blocks;
@@ -112,12 +118,14 @@ __global__ void __launch_bounds__(kScanThreads) digit_row_scan_kernel(uint32_t *
 template <typename KeyT, int THREADS = SortShape<KeyT>::threads, int BITS = SortDigit<KeyT>::bits, bool RECTANGLES = false>
 __global__ void __launch_bounds__(THREADS) digit_scatter_kernel(
     const KeyT *__restrict__ keys_in, const uint32_t *__restrict__ vals_in, KeyT *__restrict__ keys_out, uint32_t *__restrict__ vals_out,
-    const uint32_t *__restrict__ hist, const uint32_t *__restrict__ totals, uint64_t n, uint32_t n_blocks, int shift, uint32_t mask,
+    const uint32_t *__restrict__ hist, const uint32_t *__restrict__ totals, InstanceCount count, int shift, uint32_t mask,
     bool last_pass = false, const uint2 *__restrict__ rectangles_in = nullptr, uint2 *__restrict__ rectangles_out = nullptr,
     uint32_t *__restrict__ counts_out = nullptr, uint32_t culled = 0)
 {
     constexpr int kSortThreads = THREADS, kSortWaves = kSortThreads / kWave, kSortTile = kSortThreads * kSortItems;
     constexpr int kBits = BITS, kRadix = 1 << kBits, kDigitWaves = kRadix / kWave;
+    const uint64_t n = count.get();
+    const uint32_t n_blocks = blocks_of((uint32_t)n, kSortTile);
     // (16-bit counters: a block holds 8192 items; with 512 digits and 8-byte keys two blocks still fit a CU's LDS)
     __shared__ uint16_t counts[kSortWaves][kRadix];    // per wave: running digit count, later the wave's base inside the block
     __shared__ uint32_t digit_start[kRadix];           // first slot of each digit in the block-local order
@@ -288,9 +296,10 @@ __global__ void __launch_bounds__(THREADS) digit_scatter_kernel(
 
 // streaming_result: the sorted values leave the last pass as streaming stores (the instance lists, which the blend reads once)
 template <typename KeyT, int THREADS = SortShape<KeyT>::threads, int BITS = SortDigit<KeyT>::bits>
-static int sort_pairs(hipStream_t s, void *const keys[2], uint32_t *const vals[2], uint32_t *sort_tmp, uint64_t n, int end_bit, int *selector,
+static int sort_pairs(hipStream_t s, void *const keys[2], uint32_t *const vals[2], uint32_t *sort_tmp, InstanceCount count, int end_bit, int *selector,
                       bool streaming_result = false)
 {
+    const uint64_t n = count.most;
     constexpr int kSortThreads = THREADS, kSortTile = kSortThreads * kSortItems;
     const uint32_t n_blocks = (uint32_t)((n + kSortTile - 1) / kSortTile);
     constexpr int kBits = BITS, kRadix = 1 << kBits;
@@ -305,10 +314,10 @@ static int sort_pairs(hipStream_t s, void *const keys[2], uint32_t *const vals[2
         const uint32_t mask = (1u << bits) - 1u;
         const KeyT *kin = (const KeyT *)keys[cur];
         KeyT *kout = (KeyT *)keys[cur ^ 1];
-        hipLaunchKernelGGL((digit_histogram_kernel<KeyT, THREADS, BITS>), dim3(xcd_padded_grid(n_blocks)), dim3(kSortThreads), 0, s, kin, hist, n, n_blocks, shift, mask);
-        hipLaunchKernelGGL(digit_row_scan_kernel, dim3(kRadix), dim3(kScanThreads), 0, s, hist, totals, n_blocks);
+        hipLaunchKernelGGL((digit_histogram_kernel<KeyT, THREADS, BITS>), dim3(xcd_padded_grid(n_blocks)), dim3(kSortThreads), 0, s, kin, hist, count, shift, mask);
+        hipLaunchKernelGGL(digit_row_scan_kernel, dim3(kRadix), dim3(kScanThreads), 0, s, hist, totals, count, (uint32_t)kSortTile);
         hipLaunchKernelGGL((digit_scatter_kernel<KeyT, THREADS, BITS>), dim3(xcd_padded_grid(n_blocks)), dim3(kSortThreads), 0, s, kin, vals[cur], kout, vals[cur ^ 1],
-                           hist, totals, n, n_blocks, shift, mask, streaming_result && shift + step >= end_bit);
+                           hist, totals, count, shift, mask, streaming_result && shift + step >= end_bit);
         cur ^= 1;
     }
     *selector = cur;
@@ -325,11 +334,12 @@ int sort_u32_pairs_with_rectangles(void *stream, uint32_t *const keys[2], uint32
     hipStream_t s = (hipStream_t)stream;
     const uint32_t n_blocks = (uint32_t)((n + kTile - 1) / kTile);
     uint32_t *hist = sort_tmp, *totals = sort_tmp + (size_t)kRadix * n_blocks;
+    const InstanceCount count = { nullptr, (uint32_t)n };
     const uint32_t mask = (1u << bits) - 1u;
-    hipLaunchKernelGGL((digit_histogram_kernel<uint32_t, kThreads, kBits>), dim3(xcd_padded_grid(n_blocks)), dim3(kThreads), 0, s, keys[0], hist, n, n_blocks, 0, mask);
-    hipLaunchKernelGGL(digit_row_scan_kernel, dim3(kRadix), dim3(kScanThreads), 0, s, hist, totals, n_blocks);
+    hipLaunchKernelGGL((digit_histogram_kernel<uint32_t, kThreads, kBits>), dim3(xcd_padded_grid(n_blocks)), dim3(kThreads), 0, s, keys[0], hist, count, 0, mask);
+    hipLaunchKernelGGL(digit_row_scan_kernel, dim3(kRadix), dim3(kScanThreads), 0, s, hist, totals, count, (uint32_t)kTile);
     hipLaunchKernelGGL((digit_scatter_kernel<uint32_t, kThreads, kBits, true>), dim3(xcd_padded_grid(n_blocks)), dim3(kThreads), 0, s, keys[0], vals[0], keys[1],
-                       vals[1], hist, totals, n, n_blocks, 0, mask, false, reinterpret_cast<const uint2 *>(rectangles_in),
+                       vals[1], hist, totals, count, 0, mask, false, reinterpret_cast<const uint2 *>(rectangles_in),
                        reinterpret_cast<uint2 *>(rectangles_out), counts_out, culled);
     return check_launch("sort");
 }
@@ -340,10 +350,11 @@ int sort_u32_pairs(void *stream, uint32_t *const keys[2], uint32_t *const vals[2
     *selector = 0;
     if (n == 0) return HTGS_OK;
     void *const k[2] = { keys[0], keys[1] };
+    const InstanceCount count = { nullptr, (uint32_t)n };
     // a few million pairs: with 8-bit digits blocks of 4096 items, the smallest the kernels take, so that every compute
     // unit has several; 9-bit digits need a thread per digit (8192 items)
-    if (digit_bits == 9) return sort_pairs<uint32_t, 512, 9>((hipStream_t)stream, k, vals, sort_tmp, n, end_bit, selector);
-    return sort_pairs<uint32_t, kSortTileMin / kSortItems, 8>((hipStream_t)stream, k, vals, sort_tmp, n, end_bit, selector);
+    if (digit_bits == 9) return sort_pairs<uint32_t, 512, 9>((hipStream_t)stream, k, vals, sort_tmp, count, end_bit, selector);
+    return sort_pairs<uint32_t, kSortTileMin / kSortItems, 8>((hipStream_t)stream, k, vals, sort_tmp, count, end_bit, selector);
 }
 
 }  // namespace htgs
@@ -370,8 +381,8 @@ extern "C" int htgs_sort_instances(const htgs_frame *f, int *selector)
     const int end_bit = htgs_frame_end_bit(f);
     hipStream_t s = (hipStream_t)f->stream;
     switch (htgs_frame_key_bytes(f)) {
-        case 8: return sort_pairs<uint64_t>(s, f->keys, f->vals, f->sort_tmp, f->n_instances, end_bit, selector, true);
-        case 4: return sort_pairs<uint32_t>(s, f->keys, f->vals, f->sort_tmp, f->n_instances, end_bit, selector, true);
-        default: return sort_pairs<uint16_t>(s, f->keys, f->vals, f->sort_tmp, f->n_instances, end_bit, selector, true);
+        case 8: return sort_pairs<uint64_t>(s, f->keys, f->vals, f->sort_tmp, instance_count(f), end_bit, selector, true);
+        case 4: return sort_pairs<uint32_t>(s, f->keys, f->vals, f->sort_tmp, instance_count(f), end_bit, selector, true);
+        default: return sort_pairs<uint16_t>(s, f->keys, f->vals, f->sort_tmp, instance_count(f), end_bit, selector, true);
     }
 }

@@ -1,0 +1,264 @@
+// Whole passes in one call: the scratch carved out of two workspaces, every stage queued before the host knows the number of
+// instances, and a wait for that one word instead of for the stream.
+// Restates the drivers <mode>::inference / forward / update_max_weights (R/src/hybrid_blend/inference.cu:57-183,
+// forward.cu:57-189, update_max_weights.cu:30-165).
+//
+// The number of instances decides the size of the per-instance buffers, so the reference stops the host at it.  Stopped
+// there, the device runs dry until the host has read the number and queued the second half: 30 us of a frame, 100 us of a
+// training step whose buffers are allocated in between.  Here a caller that has rendered before says how many instances to
+// expect; both halves are queued, the kernels take the number from the device (InstanceCount), and the scan's last block
+// also writes it to host memory, where this thread picks it up while the device sorts.
+#include "common.h"
+#include <mutex>
+#include <vector>
+
+namespace htgs {
+
+int scan_offsets_publish(const htgs_frame *f, unsigned long long *host_total, uint32_t tag);   // instances.hip
+
+// ---------------------------------------------------------------------------------------------
+// Words in coherent host memory that a frame's scan writes and the host waits for.  One per call that is under way: taken
+// from a free list and given back, a page of them at a time; the pages stay until the process ends.
+// ---------------------------------------------------------------------------------------------
+struct HostWord {
+    unsigned long long value;              // tag << 32 | number of instances
+    uint32_t tag;                          // of the last frame it was used for
+    uint32_t pad[13];                      // a cache line each
+};
+static std::mutex g_words_mutex;
+static std::vector<HostWord *> g_free_words;
+constexpr size_t kWordsPerPage = 64;
+
+static HostWord *take_word()
+{
+    std::lock_guard<std::mutex> lock(g_words_mutex);
+    if (g_free_words.empty()) {
+        void *page = nullptr;
+        const hipError_t e = hipHostMalloc(&page, kWordsPerPage * sizeof(HostWord), hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent);
+        if (e != hipSuccess || !page) {
+            fail(HTGS_ERR_HIP, "htgs_run: hipHostMalloc: %s", hipGetErrorString(e));
+            return nullptr;
+        }
+        HostWord *w = static_cast<HostWord *>(page);
+        for (size_t i = 0; i < kWordsPerPage; ++i) {
+            w[i].value = 0;
+            w[i].tag = 0;
+            g_free_words.push_back(w + i);
+        }
+    }
+    HostWord *w = g_free_words.back();
+    g_free_words.pop_back();
+    w->tag = w->tag == 0xffffffffu ? 1u : w->tag + 1u;     // (never 0, which the fresh word holds)
+    return w;
+}
+static void give_back_word(HostWord *w)
+{
+    std::lock_guard<std::mutex> lock(g_words_mutex);
+    g_free_words.push_back(w);
+}
+
+// Waits for the word: a busy loop that ends when the scan has run, or when the stream has nothing left to run (a stream
+// that failed, say) and the word is still not there.
+static int wait_for_word(const HostWord *w, hipStream_t s, uint64_t *n)
+{
+    for (uint32_t spin = 0;; ++spin) {
+        const unsigned long long v = __atomic_load_n(&w->value, __ATOMIC_ACQUIRE);
+        if ((uint32_t)(v >> 32) == w->tag) { *n = (uint32_t)v; return HTGS_OK; }
+        if ((spin & 0xfffu) == 0xfffu) {
+            const hipError_t e = hipStreamQuery(s);
+            if (e == hipErrorNotReady) { (void)hipGetLastError(); continue; }
+            if (e != hipSuccess) return fail(HTGS_ERR_HIP, "htgs_run: %s", hipGetErrorString(e));
+            const unsigned long long last = __atomic_load_n(&w->value, __ATOMIC_ACQUIRE);
+            if ((uint32_t)(last >> 32) == w->tag) { *n = (uint32_t)last; return HTGS_OK; }
+            return fail(HTGS_ERR_HIP, "htgs_run: the number of instances did not arrive");
+        }
+        __builtin_ia32_pause();
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// workspaces
+// ---------------------------------------------------------------------------------------------
+struct Carver {
+    unsigned char *base;                   // nullptr: sizes only
+    uint64_t used;
+    template <typename T> T *take(uint64_t count)
+    {
+        T *p = base != nullptr && count > 0 ? reinterpret_cast<T *>(base + used) : nullptr;
+        used += (count * sizeof(T) + 255) & ~255ull;
+        return p;
+    }
+};
+
+static uint64_t carve_front(htgs_frame *f, int what, void *base)
+{
+    Carver c = { static_cast<unsigned char *>(base), 0 };
+    const uint64_t n = (uint64_t)f->n_primitives;
+    const int tile = tile_size(f->mode);
+    const uint64_t n_tiles = (uint64_t)div_up(f->width, tile) * div_up(f->height, tile);
+    const bool train = what == HTGS_RUN_FORWARD;
+    f->prim_floats = train ? HTGS_PRIM_FLOATS_TRAIN : HTGS_PRIM_FLOATS;
+    f->n_touched = c.take<uint32_t>(n);
+    f->offsets = c.take<uint32_t>(n);
+    f->bounds = c.take<uint16_t>(4 * n);
+    f->prim = c.take<float>((uint64_t)f->prim_floats * n);
+    f->clamp_info = train ? c.take<uint8_t>(3 * n) : nullptr;
+    f->scan_tmp = c.take<uint32_t>(htgs_scan_tmp_words((int)n));
+    f->n_instances_dev = c.take<uint32_t>(1);
+    f->ranges = c.take<uint32_t>(2 * n_tiles);
+    // (the modes that walk all of a list)
+    f->long_tiles = f->mode != HTGS_MODE_ALPHA_BLEND_GLOBAL_ORDERING ? c.take<uint32_t>(8 + 3 * n_tiles) : nullptr;
+    f->tile_order = c.take<uint32_t>(htgs_tile_order_words(f->mode, f->width, f->height));
+    // GLOBAL_ORDERING without a backward pass, and the image-only fast path of the two modes with a sorted core
+    const bool by_depth = !train && (f->mode == HTGS_MODE_ALPHA_BLEND_GLOBAL_ORDERING ||
+                                     (what == HTGS_RUN_RENDER && f->fast_math && f->mode != HTGS_MODE_OIT_BLEND));
+    f->depth_order = by_depth ? c.take<uint32_t>(htgs_depth_order_words((int)n)) : nullptr;
+    const bool has_core = f->mode == HTGS_MODE_HYBRID_BLEND || f->mode == HTGS_MODE_ALPHA_BLEND_FIRST_K;
+    const bool has_tail = f->mode == HTGS_MODE_HYBRID_BLEND || f->mode == HTGS_MODE_OIT_BLEND;
+    f->pixel_scratch = what == HTGS_RUN_MAX_WEIGHTS && has_tail ? c.take<float>(64 * n_tiles) : nullptr;
+    const uint64_t records = 64 * n_tiles, K = (uint64_t)htgs_effective_k(f->K);
+    f->core_idx = train && has_core ? c.take<uint32_t>(K * records) : nullptr;
+    f->core_info = train && has_core ? c.take<float>(4 * K * records) : nullptr;
+    f->tail_info = train && has_tail ? c.take<float>(6 * records) : nullptr;
+    return c.used;
+}
+// (after carve_front: whether the frame has depth_order decides the width of its keys)
+static uint64_t carve_back(htgs_frame *f, uint64_t n_instances, void *base)
+{
+    Carver c = { static_cast<unsigned char *>(base), 0 };
+    const uint64_t m = n_instances > 0 ? n_instances : 1, kb = (uint64_t)htgs_frame_key_bytes(f);
+    for (int i = 0; i < 2; ++i) f->keys[i] = c.take<unsigned char>(kb * m);
+    for (int i = 0; i < 2; ++i) f->vals[i] = c.take<uint32_t>(m);
+    f->sort_tmp = c.take<uint32_t>(htgs_sort_tmp_words(m));
+    return c.used;
+}
+constexpr uint64_t kMostInstances = 0xfffffffeull;
+// the number of instances that launches and buffers are sized for when `expected` are expected
+static uint64_t with_headroom(uint64_t expected)
+{
+    const uint64_t n = expected + expected / 8 + 4096;
+    return n < kMostInstances ? n : kMostInstances;
+}
+// the most instances, up to `wanted`, whose scratch fits into `bytes`
+static uint64_t fitting(htgs_frame *f, uint64_t wanted, uint64_t bytes)
+{
+    uint64_t n = wanted;
+    if (carve_back(f, n, nullptr) <= bytes) return n;
+    // (per instance: two keys, two values and the sort's share of a histogram row)
+    const uint64_t fixed = carve_back(f, 1, nullptr) + 4096, per16 = 32ull * (uint64_t)htgs_frame_key_bytes(f) + 128 + 4;
+    if (bytes <= fixed) return 0;
+    n = (bytes - fixed) * 16 / per16;
+    n = n < wanted ? n : wanted;
+    return carve_back(f, n, nullptr) <= bytes ? n : 0;
+}
+
+static int check_run(const htgs_frame *f, const htgs_workspace *w, const char *who)
+{
+    if (!f || !w) return fail(HTGS_ERR_ARGUMENT, "%s: null argument", who);
+    if (f->mode < 0 || f->mode > 3) return fail(HTGS_ERR_MODE, "unsupported rasterizer mode");
+    if (w->what < HTGS_RUN_RENDER || w->what > HTGS_RUN_MAX_WEIGHTS) return fail(HTGS_ERR_ARGUMENT, "%s: unknown pass", who);
+    if (f->n_primitives < 0 || f->width <= 0 || f->height <= 0 || f->total_sh_bases < 0) return fail(HTGS_ERR_ARGUMENT, "%s: bad sizes", who);
+    if (((uintptr_t)w->front | (uintptr_t)w->back) & 255) return fail(HTGS_ERR_ARGUMENT, "%s: workspaces must be 256-byte aligned", who);
+    return HTGS_OK;
+}
+
+static int queue_front(const htgs_frame *f, const htgs_workspace *w, HostWord *word)
+{
+    htgs_frame t = *f;
+    if (w->what != HTGS_RUN_RENDER) t.scale_modifier = 1.0f;       // as htgs_forward_front, htgs_max_weights_front
+    if (w->what == HTGS_RUN_MAX_WEIGHTS) {
+        t.sh_0 = t.sh_rest = nullptr;
+        t.active_sh_bases = 1;
+        t.total_sh_bases = 0;
+    }
+    const int rc = htgs_preprocess(&t);
+    return rc != HTGS_OK ? rc : scan_offsets_publish(&t, &word->value, word->tag);
+}
+static int queue_back(htgs_frame *f, htgs_workspace *w)
+{
+    int rc = htgs_create_instances(f);
+    if (rc == HTGS_OK) rc = htgs_sort_instances(f, &w->selector);
+    if (rc == HTGS_OK) rc = htgs_extract_ranges(f, w->selector);
+    if (rc != HTGS_OK) return rc;
+    switch (w->what) {
+        case HTGS_RUN_RENDER: return htgs_blend(f, w->selector);
+        case HTGS_RUN_FORWARD: return htgs_blend_forward(f, w->selector);
+        default: return htgs_max_weights_blend(f, w->selector, w->max_weights, w->weight_threshold);
+    }
+}
+
+}  // namespace htgs
+
+using namespace htgs;
+
+extern "C" int htgs_run_sizes(const htgs_frame *f, htgs_workspace *w)
+{
+    const int rc = check_run(f, w, "htgs_run_sizes");
+    if (rc != HTGS_OK) return rc;
+    htgs_frame t = *f;
+    w->front_needed = carve_front(&t, w->what, nullptr);
+    t.depth_order = t.mode == HTGS_MODE_ALPHA_BLEND_GLOBAL_ORDERING && w->what != HTGS_RUN_FORWARD ? (uint32_t *)256 : nullptr;
+    w->back_needed = carve_back(&t, with_headroom(w->expected), nullptr);
+    return HTGS_OK;
+}
+
+extern "C" int htgs_run(htgs_frame *f, htgs_workspace *w)
+{
+    int rc = check_run(f, w, "htgs_run");
+    if (rc != HTGS_OK) return rc;
+    w->selector = 0;
+    w->n_instances = 0;
+    w->front_needed = carve_front(f, w->what, w->front);
+    if (w->front == nullptr || w->front_bytes < w->front_needed) return HTGS_WORKSPACE;
+    hipStream_t s = (hipStream_t)f->stream;
+    f->n_instances_live = nullptr;
+    f->n_instances = 0;
+    if (f->n_primitives == 0) return htgs_run_rest(f, w);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone)
+        return fail(HTGS_ERR_ARGUMENT, "htgs_run: the host waits for the number of instances, which a stream under capture never gives");
+    HostWord *word = take_word();
+    if (!word) return HTGS_ERR_HIP;
+    rc = queue_front(f, w, word);
+    if (rc != HTGS_OK) {
+        // (a kernel that was queued may still write the word: it is not used again)
+        return rc;
+    }
+    uint64_t queued_for = 0;
+    if (w->expected > 0 && w->back != nullptr) {
+        queued_for = fitting(f, with_headroom(w->expected), w->back_bytes);
+        if (queued_for >= w->expected) {
+            carve_back(f, queued_for, w->back);
+            f->n_instances = queued_for;
+            f->n_instances_live = f->n_instances_dev;
+            rc = queue_back(f, w);
+            f->n_instances_live = nullptr;
+            if (rc != HTGS_OK) return rc;
+        } else queued_for = 0;
+    }
+    uint64_t n = 0;
+    rc = wait_for_word(word, s, &n);
+    if (rc != HTGS_OK) return rc;
+    give_back_word(word);
+    w->n_instances = n;
+    f->n_instances = n;
+    if (n > kMostInstances) return HTGS_OK;                  // (the caller refuses the frame)
+    if (queued_for > 0 && n <= queued_for) return HTGS_OK;
+    return htgs_run_rest(f, w);
+}
+
+extern "C" int htgs_run_rest(htgs_frame *f, htgs_workspace *w)
+{
+    int rc = check_run(f, w, "htgs_run_rest");
+    if (rc != HTGS_OK) return rc;
+    const uint64_t n = w->n_instances;
+    if (n > kMostInstances) return fail(HTGS_ERR_ARGUMENT, "htgs_run_rest: more than 2^32-2 instances");
+    f->n_instances = n;
+    f->n_instances_live = nullptr;
+    const uint64_t needed = carve_back(f, n, n > 0 ? w->back : nullptr);
+    if (n > 0 && (w->back == nullptr || w->back_bytes < needed)) {
+        w->back_needed = carve_back(f, with_headroom(n), nullptr);
+        return HTGS_WORKSPACE;
+    }
+    return queue_back(f, w);
+}

@@ -8,6 +8,7 @@ torch only owns the device memory and the stream, every kernel is hand-written H
 from __future__ import annotations
 
 import ctypes
+import struct
 import threading
 from enum import Enum
 from typing import NamedTuple, Optional
@@ -94,6 +95,9 @@ class ScratchPool:
     def __init__(self):
         self.buffers: dict = {}
         self.last_used = 0
+        self.expected: dict = {}              # instances that the last pass of a kind had, which sizes the launches of the next
+        self.frame = _native.Frame()          # filled in anew by every call of ``_run_pass``
+        self.workspace = _native.Workspace()
 
     def nbytes(self) -> int:
         return sum(b.numel() * b.element_size() for b in self.buffers.values())
@@ -356,38 +360,10 @@ class FrameBuffers:
     def run_backward(self, grad_image: torch.Tensor, densification_info: Optional[torch.Tensor] = None,
                      use_distance_scaling: bool = False):
         """``_C.backward`` of the reference: the six gradients; ``densification_info`` is updated in place."""
-        dev, n = self.device, self.n
-        grad_image = _dev_f32(grad_image, "grad_image", dev)
-        if tuple(grad_image.shape) != (3, self.height, self.width):
-            raise RuntimeError("grad_image must be [3,H,W]")
-        total_sh = int(self.sh_rest.shape[1])
-        f32 = dict(dtype=torch.float32, device=dev)
-        # one row per instance, every one written by the blend kernels: no initialisation needed
-        self.grad_rows = torch.empty((max(self.n_instances, 1), 16), **f32)
-        grads = [torch.empty((n, 3), **f32), torch.empty((n, 3), **f32), torch.empty((n, 4), **f32), torch.empty((n, 1), **f32),
-                 torch.empty((n, 1, 3), **f32), torch.empty((n, total_sh, 3), **f32)]
-        f = self.frame
-        f.stream = torch.cuda.current_stream(dev).cuda_stream
-        f.grad_image, f.grad_rows = _ptr(grad_image), _ptr(self.grad_rows)
-        (f.grad_positions, f.grad_scales, f.grad_rotations, f.grad_opacities, f.grad_sh_0, f.grad_sh_rest) = [_ptr(g) for g in grads]
-        rows = 0
-        helper = None
-        if densification_info is not None and densification_info.numel() > 0:
-            rows = int(densification_info.shape[0])
-            if rows not in (2, 3) or densification_info.numel() != rows * n or not densification_info.is_contiguous() \
-                    or densification_info.dtype != torch.float32 or densification_info.device != dev:
-                raise RuntimeError("densification_info must be a contiguous float32 [2,N] or [3,N] tensor on the GPU")
-            f.densification_info = densification_info.data_ptr()
-            if rows == 3:
-                helper = torch.empty(max(self.n_instances, 1), **f32)
-        else:
-            f.densification_info = 0
-        f.densification_rows = rows
-        f.dens_helper = _ptr(helper)
-        f.use_distance_scaling = int(bool(use_distance_scaling))
-        self.grads = grads           # keeps the bound outputs alive for blend_backward / preprocess_backward
-        _native.check(self.lib.htgs_backward(self._ref, self.selector))
-        return grads
+        # (kept alive for blend_backward / preprocess_backward)
+        self.grads, self._backward_buffers = _run_backward(self.frame, self.selector, self.device, grad_image, densification_info, use_distance_scaling)
+        self.grad_rows = self._backward_buffers[1]
+        return self.grads
 
     def blend_backward(self):
         """The blend half of the last ``run_backward`` again, into the same buffers (per-stage timing)."""
@@ -398,6 +374,151 @@ class FrameBuffers:
         _native.check(self.lib.htgs_preprocess_backward(self._ref))
 
 
+# positions ... cam_position, n_primitives ... height, near_plane, far_plane, scale_modifier: the head of ``htgs_frame``
+_FRAME_HEAD = struct.Struct("=9Q7i3f")
+_UINT8 = torch.uint8
+
+
+def _pass_inputs(frame: "_native.Frame", positions, scales, rotations, opacities, sh_0, sh_rest, settings: RasterizerSettings) -> bool:
+    """The head of ``frame`` from tensors that can be handed over as they are (float32, contiguous, on one GPU, shapes
+    that agree); False when one of them cannot, which the caller leaves to ``FrameBuffers`` and its messages."""
+    M, VPM, cam, mode, K, active, width, height, near, far, modifier = settings
+    mode = _mode_value(mode)
+    if not 0 <= mode <= 3 or not isinstance(positions, torch.Tensor) or not positions.is_cuda:
+        return False
+    dev, n = positions.device, positions.shape[0]
+    with_colour = sh_0 is not None
+    for t in (positions, scales, rotations, opacities, M, VPM, cam, sh_0, sh_rest) if with_colour else (positions, scales, rotations, opacities, M, VPM, cam):
+        if not isinstance(t, torch.Tensor) or t.dtype is not torch.float32 or not t.is_contiguous() or t.device != dev:
+            return False
+    if positions.shape != (n, 3) or scales.shape != (n, 3) or rotations.shape != (n, 4) or opacities.numel() != n or M.numel() != 16 \
+            or VPM.numel() != 16 or cam.numel() != 3:
+        return False
+    total = 0
+    if with_colour:
+        if sh_0.numel() != 3 * n or sh_rest.dim() != 3 or sh_rest.shape[0] != n or sh_rest.shape[2] != 3:
+            return False
+        total = sh_rest.shape[1]
+    _FRAME_HEAD.pack_into(frame, 0, positions.data_ptr(), scales.data_ptr(), rotations.data_ptr(), opacities.data_ptr(), sh_0.data_ptr() if with_colour else 0,
+                          sh_rest.data_ptr() if total and n else 0, M.data_ptr(), VPM.data_ptr(), cam.data_ptr(), n, total, int(active), mode, int(K),
+                          int(width), int(height), float(near), float(far), float(modifier))
+    return True
+
+
+def _run_pass(lib, frame, workspace, what: int, pool: "ScratchPool", dev: torch.device, stream: int, keep: Optional[list] = None) -> None:
+    """One ``htgs_run`` on workspaces of the pool; with ``keep`` (a training frame, whose scratch lives until its backward
+    pass) on fresh ones, which are appended to it."""
+    f, w = ctypes.byref(frame), ctypes.byref(workspace)
+    key = (what, frame.mode)
+    frame.stream = stream
+    workspace.what = what
+    workspace.expected = pool.expected.get(key, 0)
+
+    def provide(name: str, needed: int) -> torch.Tensor:
+        if keep is None:
+            return pool.get(name, needed, _UINT8, dev)
+        buf = torch.empty(needed, dtype=_UINT8, device=dev)
+        keep.append(buf)
+        return buf
+
+    if keep is not None:
+        _native.check(lib.htgs_run_sizes(f, w))
+        front = provide("front", workspace.front_needed)
+        back = provide("back", workspace.back_needed) if workspace.expected else None
+    else:
+        front, back = pool.buffers.get("front"), pool.buffers.get("back")
+    workspace.front, workspace.front_bytes = (front.data_ptr(), front.numel()) if front is not None else (0, 0)
+    workspace.back, workspace.back_bytes = (back.data_ptr(), back.numel()) if back is not None else (0, 0)
+    status = lib.htgs_run(f, w)
+    if status == _native.WORKSPACE_TOO_SMALL and workspace.front_bytes < workspace.front_needed:
+        front = provide("front", workspace.front_needed)
+        workspace.front, workspace.front_bytes = front.data_ptr(), front.numel()
+        status = lib.htgs_run(f, w)
+    if status == _native.WORKSPACE_TOO_SMALL:
+        back = provide("back", workspace.back_needed)
+        workspace.back, workspace.back_bytes = back.data_ptr(), back.numel()
+        status = lib.htgs_run_rest(f, w)
+    _native.check(status)
+    pool.expected[key] = checked_instance_count(workspace.n_instances)
+
+
+def _render(positions, scales, rotations, opacities, sh_0, sh_rest, settings, to_chw, use_median_depth, fast):
+    """``(image, depth)`` of one inference frame; ``depth`` is None on the image-only path."""
+    cuda = isinstance(positions, torch.Tensor) and positions.is_cuda
+    pool = ScratchPool.current(positions.device) if cuda else None
+    if pool is None or not _pass_inputs(pool.frame, positions, scales, rotations, opacities, sh_0, sh_rest, settings):
+        with torch.no_grad():
+            image, depth = FrameBuffers(positions, scales, rotations, opacities, sh_0, sh_rest, settings, to_chw, use_median_depth, pool=pool, fast=fast).run()
+        return image, None if fast else depth.unsqueeze(0) if to_chw else depth.unsqueeze(-1)
+    dev, frame = positions.device, pool.frame
+    w, h = frame.width, frame.height
+    image = torch.empty((3, h, w) if to_chw else (h, w, 3), dtype=torch.float32, device=dev)
+    depth = None if fast else torch.empty((1, h, w) if to_chw else (h, w, 1), dtype=torch.float32, device=dev)
+    frame.image, frame.depth = image.data_ptr(), 0 if fast else depth.data_ptr()
+    frame.to_chw, frame.use_median_depth, frame.fast_math = bool(to_chw), bool(use_median_depth), fast
+    _run_pass(_native.lib(), frame, pool.workspace, _native.RUN_RENDER, pool, dev, ScratchPool._stream_id(dev))
+    return image, depth
+
+
+class _TrainingFrame:
+    """One training frame: the filled-in ``htgs_frame`` and the tensors its pointers lead to, from the forward pass until the
+    last backward pass that uses it."""
+
+    def __init__(self, positions, scales, rotations, opacities, sh_0, sh_rest, settings: RasterizerSettings):
+        self.fallback = None
+        if not isinstance(positions, torch.Tensor) or not positions.is_cuda \
+                or not _pass_inputs(frame := _native.Frame(), positions, scales, rotations, opacities, sh_0, sh_rest, settings):
+            self.fallback = FrameBuffers(positions, scales, rotations, opacities, sh_0, sh_rest, settings, True, False, train=True)
+            self.image = self.fallback.run_forward()
+            self.fallback.image = self.image.detach()
+            return
+        dev = positions.device
+        self.frame, self.device = frame, dev
+        self.image = torch.empty((3, frame.height, frame.width), dtype=torch.float32, device=dev)
+        frame.image, frame.to_chw = self.image.data_ptr(), 1
+        workspace = _native.Workspace()
+        # (the image detached: the tensor that is returned leads to its graph node, which leads here)
+        self.keep = [positions, scales, rotations, opacities, sh_0, sh_rest, settings, self.image.detach()]
+        _run_pass(_native.lib(), frame, workspace, _native.RUN_FORWARD, ScratchPool.current(dev), dev, ScratchPool._stream_id(dev), self.keep)
+        self.selector = workspace.selector
+
+    def backward(self, grad_image, densification_info, use_distance_scaling):
+        if self.fallback is not None:
+            return self.fallback.run_backward(grad_image, densification_info, use_distance_scaling)
+        return _run_backward(self.frame, self.selector, self.device, grad_image, densification_info, use_distance_scaling)[0]
+
+
+def _run_backward(f: "_native.Frame", selector: int, dev: torch.device, grad_image: torch.Tensor, densification_info: Optional[torch.Tensor],
+                  use_distance_scaling: bool):
+    """The six gradients of the training frame ``f``, and the other buffers its pointers lead to afterwards."""
+    n, total_sh, n_instances = f.n_primitives, f.total_sh_bases, f.n_instances
+    grad_image = _dev_f32(grad_image, "grad_image", dev)
+    if tuple(grad_image.shape) != (3, f.height, f.width):
+        raise RuntimeError("grad_image must be [3,H,W]")
+    f32 = dict(dtype=torch.float32, device=dev)
+    # one row per instance, every one written by the blend kernels: no initialisation needed
+    grad_rows = torch.empty((max(n_instances, 1), 16), **f32)
+    grads = [torch.empty((n, 3), **f32), torch.empty((n, 3), **f32), torch.empty((n, 4), **f32), torch.empty((n, 1), **f32),
+             torch.empty((n, 1, 3), **f32), torch.empty((n, total_sh, 3), **f32)]
+    f.stream = ScratchPool._stream_id(dev)
+    f.grad_image, f.grad_rows = _ptr(grad_image), grad_rows.data_ptr()
+    (f.grad_positions, f.grad_scales, f.grad_rotations, f.grad_opacities, f.grad_sh_0, f.grad_sh_rest) = [_ptr(g) for g in grads]
+    rows, helper = 0, None
+    if densification_info is not None and densification_info.numel() > 0:
+        rows = int(densification_info.shape[0])
+        if rows not in (2, 3) or densification_info.numel() != rows * n or not densification_info.is_contiguous() \
+                or densification_info.dtype != torch.float32 or densification_info.device != dev:
+            raise RuntimeError("densification_info must be a contiguous float32 [2,N] or [3,N] tensor on the GPU")
+        if rows == 3:
+            helper = torch.empty(max(n_instances, 1), **f32)
+    f.densification_info = densification_info.data_ptr() if rows else 0
+    f.densification_rows = rows
+    f.dens_helper = _ptr(helper)
+    f.use_distance_scaling = int(bool(use_distance_scaling))
+    _native.check(_native.lib().htgs_backward(ctypes.byref(f), selector))
+    return grads, (grad_image, grad_rows, helper)
+
+
 class _Rasterize(torch.autograd.Function):
     """Differentiable render (reference: rasterization.py:45-113).  The frame object saved on ``ctx`` owns the
     scratch that the reference returns to Python as four byte blobs and keeps in ``ctx.save_for_backward``
@@ -406,9 +527,8 @@ class _Rasterize(torch.autograd.Function):
     @staticmethod
     def forward(ctx, positions, scales, rotations, opacities, sh_0, sh_rest, densification_info, rasterizer_settings,
                 use_distance_scaling):
-        fb = FrameBuffers(positions, scales, rotations, opacities, sh_0, sh_rest, rasterizer_settings, True, False, train=True)
-        image = fb.run_forward()
-        ctx.fb = fb
+        ctx.fb = _TrainingFrame(positions, scales, rotations, opacities, sh_0, sh_rest, rasterizer_settings)
+        image, ctx.fb.image = ctx.fb.image, None
         ctx.save_for_backward(positions, scales, rotations, opacities, sh_0, sh_rest)
         ctx.densification_info = densification_info
         ctx.mark_non_differentiable(densification_info)
@@ -419,7 +539,7 @@ class _Rasterize(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, grad_image):
         _ = ctx.saved_tensors      # raises if an input was modified in place since forward
-        grads = ctx.fb.run_backward(grad_image, ctx.densification_info, ctx.use_distance_scaling)
+        grads = ctx.fb.backward(grad_image, ctx.densification_info, ctx.use_distance_scaling)
         return (*grads, None, None, None)
 
 
@@ -452,16 +572,28 @@ def update_max_weights(
 ) -> None:
     """Raises ``max_weights`` ([N] or [N,1] float32, in place) to the largest blending weight each Gaussian reaches in
     this view; weights below ``weight_threshold`` are ignored (reference: rasterization.py:189-206)."""
-    run_max_weights(max_weights, positions, scales, rotations, opacities, settings, weight_threshold)
+    cuda = isinstance(positions, torch.Tensor) and positions.is_cuda
+    pool = ScratchPool.current(positions.device) if cuda else None
+    if pool is None or not _pass_inputs(pool.frame, positions, scales, rotations, opacities, None, None, settings):
+        run_max_weights(max_weights, positions, scales, rotations, opacities, settings, weight_threshold)
+        return
+    _check_max_weights(max_weights, positions.shape[0])
+    frame, w = pool.frame, pool.workspace
+    frame.image, frame.depth, frame.fast_math = 0, 0, 0
+    w.max_weights, w.weight_threshold = max_weights.data_ptr(), float(weight_threshold)
+    _run_pass(_native.lib(), frame, w, _native.RUN_MAX_WEIGHTS, pool, positions.device, ScratchPool._stream_id(positions.device))
+
+
+def _check_max_weights(max_weights, n: int) -> None:
+    if not (isinstance(max_weights, torch.Tensor) and max_weights.is_cuda and max_weights.dtype == torch.float32
+            and max_weights.is_contiguous() and max_weights.numel() == n):
+        raise RuntimeError("max_weights must be a contiguous float32 GPU tensor with one element per Gaussian")
 
 
 def run_max_weights(max_weights, positions, scales, rotations, opacities, settings, weight_threshold, long_list_threshold: int = 0) -> FrameBuffers:
     """``update_max_weights`` with the length beyond which a tile's list is shared between waves and workgroups made
     explicit (0: the library's default); returns the frame."""
-    n = positions.shape[0]
-    if not (isinstance(max_weights, torch.Tensor) and max_weights.is_cuda and max_weights.dtype == torch.float32
-            and max_weights.is_contiguous() and max_weights.numel() == n):
-        raise RuntimeError("max_weights must be a contiguous float32 GPU tensor with one element per Gaussian")
+    _check_max_weights(max_weights, positions.shape[0])
     with torch.no_grad():
         fb = FrameBuffers(positions, scales, rotations, opacities, None, None, settings, True, False,
                           pool=ScratchPool.current(positions.device), long_list_threshold=long_list_threshold)
@@ -493,12 +625,7 @@ def rasterize(
     fraction of 19 to 23 bits (image within 1e-6, depth within 1e-5 of the same walk with alphas kept as floats; every
     test of a fragment is taken on the float).  ``FrameBuffers(..., long_list_threshold=8193).run()`` is that other
     walk: any threshold above 8192 selects it, a tenth slower in the blend stage."""
-    with torch.no_grad():
-        pool = ScratchPool.current(positions.device) if isinstance(positions, torch.Tensor) and positions.is_cuda else None
-        image, depth = FrameBuffers(positions, scales, rotations, opacities, sh_0, sh_rest, settings,
-                                    to_chw, use_median_depth, pool=pool).run()
-    depth = depth.unsqueeze(0) if to_chw else depth.unsqueeze(-1)
-    return image, depth
+    return _render(positions, scales, rotations, opacities, sh_0, sh_rest, settings, to_chw, use_median_depth, False)
 
 
 def fast_rasterize(
@@ -516,7 +643,4 @@ def fast_rasterize(
     take the hardware's reciprocal and 2^x (one ulp each) instead of the exactly reproducible routines and skip the
     depth map.  The image agrees with ``rasterize`` to rounding, except at the few pixels where a fragment sits
     within an ulp of an alpha threshold."""
-    with torch.no_grad():
-        pool = ScratchPool.current(positions.device) if isinstance(positions, torch.Tensor) and positions.is_cuda else None
-        image, _ = FrameBuffers(positions, scales, rotations, opacities, sh_0, sh_rest, settings, to_chw, False, pool=pool, fast=True).run()
-    return image
+    return _render(positions, scales, rotations, opacities, sh_0, sh_rest, settings, to_chw, False, True)[0]

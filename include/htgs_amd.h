@@ -9,7 +9,7 @@
  * memory, and every launch goes to the stream named in the frame.
  *
  * All functions return HTGS_OK (0) or an error code; htgs_last_error() gives the text.
- * Nothing here synchronises the host with the device.
+ * Only htgs_run and htgs_run_rest wait for the device, for one word: the frame's number of instances.
  */
 #ifndef HTGS_AMD_H
 #define HTGS_AMD_H
@@ -112,6 +112,9 @@ typedef struct htgs_frame {
                                   into the sorted core.  Ignored in the other cases */
     /* ---- per-instance scratch (PerInstanceBuffers, buffer_utils.h:56-84) ---- */
     uint64_t n_instances;      /* host copy of *n_instances_dev, needed from htgs_create_instances on */
+    const uint32_t *n_instances_live; /* NULL, or n_instances_dev: htgs_create_instances and the stages after it are queued before
+                                  the host knows the number and take it from the device; n_instances then is the most that
+                                  the buffers hold, and a frame with more instances comes out empty (see htgs_run) */
     void *keys[2];             /* [n_instances] of htgs_frame_key_bytes() each, ping-pong, 16-byte aligned */
     uint32_t *vals[2];         /* [n_instances] primitive index, ping-pong */
     uint32_t *sort_tmp;        /* htgs_sort_tmp_words(n_instances) words */
@@ -265,6 +268,41 @@ int htgs_max_weights_blend(const htgs_frame *f, int selector, float *max_weights
 int htgs_update_3d_filter(const float *positions, const float *w2c, float *filter_3d, uint8_t *visibility_mask, int n_points,
                           int width, int height, float focal_x, float focal_y, float center_x, float center_y,
                           float near_plane, float clipping_tolerance, float distance2filter, void *stream);
+
+/*
+ * Whole passes in one call, on workspaces instead of single scratch buffers (no counterpart in the reference, whose drivers
+ * allocate inside and stop at cudaMemcpy for the number of instances, R/src/hybrid_blend/inference.cu:118-119).
+ * htgs_run carves the frame's scratch out of `front` (what depends on the number of Gaussians and pixels) and `back` (what
+ * depends on the number of instances), fills the frame's scratch pointers in, queues the pass and waits for one word that
+ * the scan writes to host memory: the number of instances.  With `expected` (the number a frame before had, 0 if there was
+ * none) everything is queued at once, launches and buffers sized for an eighth more than that, and the word arrives while the
+ * device goes on with the later stages; only a frame that needs more than `back` holds or more than was expected is queued
+ * again from the duplication on.  HTGS_WORKSPACE: a workspace is too small; front_needed / back_needed say what is asked
+ * for.  After a short `front` nothing was queued: call htgs_run again.  After a short `back` the first half is done: call
+ * htgs_run_rest.  Workspaces are 256-byte aligned and, for HTGS_RUN_FORWARD, belong to the frame until its backward pass.
+ * Not for a stream that is being captured.
+ */
+#define HTGS_WORKSPACE 4
+#define HTGS_RUN_RENDER 0       /* htgs_render_front + htgs_render_back */
+#define HTGS_RUN_FORWARD 1      /* htgs_forward_front + htgs_forward_back; front also holds clamp_info and the pixel records */
+#define HTGS_RUN_MAX_WEIGHTS 2  /* htgs_max_weights_front + htgs_max_weights_back */
+typedef struct htgs_workspace {
+    void *front;
+    uint64_t front_bytes;
+    void *back;
+    uint64_t back_bytes;
+    uint64_t expected;
+    float *max_weights;         /* HTGS_RUN_MAX_WEIGHTS */
+    float weight_threshold;
+    int32_t what;               /* HTGS_RUN_* */
+    uint64_t front_needed, back_needed;    /* out */
+    uint64_t n_instances;       /* out: the frame's number of instances; 0xffffffff: more than 2^32 - 2 (nothing was rendered) */
+    int32_t selector;           /* out, as in htgs_sort_instances */
+} htgs_workspace;
+int htgs_run(htgs_frame *f, htgs_workspace *w);
+int htgs_run_rest(htgs_frame *f, htgs_workspace *w);
+/* bytes of `front` (front_needed) and of `back` for w->expected instances (back_needed); nothing is queued */
+int htgs_run_sizes(const htgs_frame *f, htgs_workspace *w);
 
 /* Self-check, no counterpart in the reference.  The forward blend kernels take 1/|d|^2 as v_rcp_f32 plus one fused
  * Newton step wherever 2^-120 <= |d|^2 < 2^121 and as the IEEE division elsewhere; this call compares the two on
