@@ -41,6 +41,8 @@ class Frame(ctypes.Structure):
         ("n_touched", ctypes.c_void_p),
         ("offsets", ctypes.c_void_p),
         ("bounds", ctypes.c_void_p),
+        ("touch", ctypes.c_void_p),
+        ("touch_cutoff_only", ctypes.c_int32),
         ("prim", ctypes.c_void_p),
         ("prim_floats", ctypes.c_int32),
         ("clamp_info", ctypes.c_void_p),

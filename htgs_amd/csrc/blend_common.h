@@ -404,14 +404,6 @@ __device__ __forceinline__ uint32_t quadrant_next_hit(QuadrantHits &w)
                      : [a0] "s"(a0), [a1] "s"(a1), [a2] "s"(a2), [a3] "s"(a3));
     return addr;
 }
-// orders one wave's LDS writes before its later LDS reads (the LDS serves a wave's instructions in order; this only keeps
-// the compiler from moving them)
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 // The walk itself: turn(addr) is called, with the lanes of the quadrants that still have a hit, once per loop turn.
 template <bool BANKED = false, typename Turn>
 __device__ __forceinline__ void quadrant_walk(QuadrantHits &hits, uint32_t stage_base, Turn &&turn)

@@ -57,10 +57,11 @@ inline bool frame_depth_ordered(const htgs_frame *f)
 }
 // the parts of depth_order, n4 = N rounded up to a multiple of four words each: depth keys and Gaussian indices (two
 // buffers each for the sort, which leaves its result in the first ones after four passes; htgs_preprocess writes the
-// pairs), the counts and the tile rectangles in depth order, scratch of the sort
+// pairs), the counts and the tile rectangles (or touch entries) in depth order, scratch of the sort
 struct DepthOrder {
     uint32_t *keys[2], *vals[2], *counts;
     uint16_t *bounds;
+    uint32_t *touch;
     uint32_t *sort_tmp;
 };
 inline DepthOrder depth_order_parts(const htgs_frame *f)
@@ -69,7 +70,7 @@ inline DepthOrder depth_order_parts(const htgs_frame *f)
     DepthOrder d;
     d.keys[0] = f->depth_order; d.keys[1] = f->depth_order + n4;
     d.vals[0] = f->depth_order + 2 * n4; d.vals[1] = f->depth_order + 3 * n4;
-    d.counts = f->depth_order + 4 * n4; d.bounds = reinterpret_cast<uint16_t *>(f->depth_order + 5 * n4); d.sort_tmp = f->depth_order + 7 * n4;
+    d.counts = f->depth_order + 4 * n4; d.bounds = reinterpret_cast<uint16_t *>(f->depth_order + 5 * n4); d.touch = f->depth_order + 5 * n4; d.sort_tmp = f->depth_order + 9 * n4;
     return d;
 }
 // The keys that sort the Gaussians by depth: the bit pattern of the centre's camera-space depth (for positive depths the
@@ -112,9 +113,10 @@ int sort_u32_pairs(void *stream, uint32_t *const keys[2], uint32_t *const vals[2
                    int *selector);
 // the same in one pass over keys of at most eight bits whose values are 0 .. n - 1 in this order, from keys / vals[0] to
 // keys / vals[1]; the tile rectangles (four 16-bit bounds per value) are written in sorted order as well, with the number
-// of tiles each covers (0 for the key `culled`)
+// of tiles each covers (0 for the key `culled`); touch_in / touch_out in their place if they are given
 int sort_u32_pairs_with_rectangles(void *stream, uint32_t *const keys[2], uint32_t *const vals[2], uint32_t *sort_tmp, uint64_t n, int bits,
-                                   const uint16_t *rectangles_in, uint16_t *rectangles_out, uint32_t *counts_out, uint32_t culled);
+                                   const uint16_t *rectangles_in, uint16_t *rectangles_out, const uint32_t *touch_in, uint32_t *touch_out,
+                                   uint32_t *counts_out, uint32_t culled);
 
 // The number of (tile, Gaussian) instances as a kernel sees it.  live = nullptr: `most` is the number, the host knows it
 // (the stage-by-stage entry points).  Otherwise the kernels were queued before the host knew: they read the number the scan
@@ -210,6 +212,15 @@ __device__ __forceinline__ float rcp_exact(float x)
     float r = rcp_refined(x);
     if (__builtin_expect(__any(!rcp_in_range(x)), 0)) r = 1.0f / x;
     return r;
+}
+
+// orders one wave's LDS writes before its later LDS reads (the LDS serves a wave's instructions in order; this only keeps
+// the compiler from moving them)
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 __device__ __forceinline__ float clamp_pos(float v) { return v > 0.0f ? v : 0.0f; }

@@ -2,7 +2,7 @@
 // Restates preprocess_cu of the four modes (R/include/hybrid_blend/kernels/inference.cuh:10-76 and siblings,
 // forward.cuh:10-76 for the clamp flags) on top of transform_and_cull / convert_sh_to_rgb
 // (R/include/kernel_utils.cuh:63-188).  No fused operations in this file: operand order of the reference.
-#include "common.h"
+#include "tile_span.h"
 
 namespace htgs {
 
@@ -64,7 +64,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) p
     uint8_t *__restrict__ clamp_info,
     int n, uint32_t grid_w, uint32_t grid_h, float tile, float min_alpha_rcp,
     int active_sh, int total_sh, float near_plane, float far_plane, float scale_modifier, int rec4,
-    uint32_t *__restrict__ depth_keys, uint32_t *__restrict__ depth_vals, uint32_t depth_base, uint32_t depth_culled, int depth_shift)
+    uint32_t *__restrict__ depth_keys, uint32_t *__restrict__ depth_vals, uint32_t depth_base, uint32_t depth_culled, int depth_shift,
+    uint4 *__restrict__ touch, float rho_most, int cutoff_only)
 {
     // One LDS buffer, used twice: first the block's slice of sh_rest (contiguous in memory, loaded with coalesced
     // 16-byte reads and then read back per Gaussian at a stride of 3 * total_sh words), then the block's records
@@ -118,6 +119,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) p
     float u[3], v[3], w[3];
     Row V1, V2, V4;
     uint32_t b0 = 0, b1 = 0, b2 = 0, b3 = 0;
+    TileOutline outline;
+    outline.ellipse = false;
     if (visible) {
         const float sx = scales[3 * (size_t)i], sy = scales[3 * (size_t)i + 1], sz = scales[3 * (size_t)i + 2];
         const float4 q = *reinterpret_cast<const float4 *>(rotations + 4 * (size_t)i);
@@ -154,8 +157,51 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) p
                 b3 = tile_ceil(((cy + ey) + 0.5f) / tile, grid_h);                         // :132
                 touched = (b1 - b0) * (b3 - b2);                                           // :136
                 visible = touched != 0;
+                if (touch != nullptr && visible) {
+                    const float A[4] = { V1.x, V1.y, V1.z, V1.w }, B[4] = { V2.x, V2.y, V2.z, V2.w }, C[4] = { V4.x, V4.y, V4.z, V4.w };
+                    outline = tile_outline(A, B, C, outline_rho(rho, rho_most, cutoff_only != 0), tile, b0, b1, b2, b3);
+                }
             }
         }
+    }
+    // htgs_frame.touch: which tiles of the rectangle are listed.  A lane goes through the rows of a rectangle of up to
+    // kMaskTiles tiles; the wave takes the rows of a larger one together, a lane per row.  Training frames list all of
+    // a large rectangle, whose gradient rows the backward pass places by the tile's position in it.
+    if (touch != nullptr) {
+        const bool train = rec4 != HTGS_PRIM_FLOATS / 4;
+        TileTouch t = { b0 | b2 << 16, (b1 - b0) | (b3 - b2) << 16, 0u, 0u };
+        const bool large = visible && touched > kMaskTiles;
+        if (visible && !large) {
+            unsigned long long mask = 0;
+            const uint32_t w = b1 - b0;
+            for (uint32_t row = b2, at = 0; row < b3; ++row, at += w) {
+                uint32_t x;
+                const uint32_t len = outline_row(outline, row, b0, b1, x);
+                // (len tiles from x on; 64 only where the row is all of the rectangle)
+                if (len != 0u) mask |= (~0ull >> (64u - len)) << (at + (x - b0));
+            }
+            // (in the training pass a Gaussian with a rectangle is one the view sees, whether a pixel lies in its outline or not)
+            if (train && mask == 0) mask = 1ull;
+            t.lo = (uint32_t)mask; t.hi = (uint32_t)(mask >> 32);
+            touched = touch_count(t);
+        }
+        if (!train) {
+            for (unsigned long long pending = __ballot(large); pending != 0; pending &= pending - 1) {     // (wave-uniform)
+                const int owner = __builtin_ctzll(pending);
+                const TileOutline o = broadcast_outline(outline, owner);
+                const uint32_t x0 = (uint32_t)__builtin_amdgcn_readlane((int)b0, owner), x1 = (uint32_t)__builtin_amdgcn_readlane((int)b1, owner);
+                const uint32_t y0 = (uint32_t)__builtin_amdgcn_readlane((int)b2, owner), y1 = (uint32_t)__builtin_amdgcn_readlane((int)b3, owner);
+                const uint32_t lane = threadIdx.x & (kWave - 1);
+                uint32_t sum = 0, x;
+                for (uint32_t row = y0 + lane; row < y1; row += kWave) sum += outline_row(o, row, x0, x1, x);
+#pragma unroll
+                for (int d = kWave / 2; d > 0; d >>= 1) sum += (uint32_t)__shfl_xor((int)sum, d, kWave);
+                if ((int)lane == owner) touched = sum;
+            }
+        }
+        if (large) t.lo = touched;
+        visible = visible && touched != 0;
+        if (visible) touch[i] = make_uint4(t.corner, t.size, t.lo, t.hi);
     }
     if (in_range) n_touched[i] = touched;
     // htgs_frame.depth_order: the pairs that sort the Gaussians by depth (depth_key_range() in common.h)
@@ -167,7 +213,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) p
         depth_vals[i] = (uint32_t)i;
     }
     s_visible[threadIdx.x] = visible;
-    if (visible)
+    if (visible && bounds != nullptr)
         *reinterpret_cast<ushort4 *>(bounds + 4 * (size_t)i) = make_ushort4((uint16_t)b0, (uint16_t)b1, (uint16_t)b2, (uint16_t)b3);
 
     // stage the block's SH coefficients
@@ -262,7 +308,7 @@ extern "C" int htgs_preprocess(const htgs_frame *f)
         return fail(HTGS_ERR_ARGUMENT, "htgs_preprocess: bad sizes");
     if (f->n_primitives == 0) return HTGS_OK;
     if (!f->positions || !f->scales || !f->rotations || !f->opacities || !f->M || !f->VPM ||
-        !f->cam_position || !f->n_touched || !f->bounds || !f->prim)
+        !f->cam_position || !f->n_touched || (!f->bounds && !f->touch) || !f->prim)
         return fail(HTGS_ERR_ARGUMENT, "htgs_preprocess: null pointer");
     // the SH bands read from sh_rest must exist: 3, 8 and 15 coefficients for degrees 1, 2, 3
     const int need = f->active_sh_bases > 9 ? 15 : f->active_sh_bases > 4 ? 8 : f->active_sh_bases > 1 ? 3 : 0;
@@ -280,12 +326,15 @@ extern "C" int htgs_preprocess(const htgs_frame *f)
     if (lds_bytes > 64 * 1024) return fail(HTGS_ERR_ARGUMENT, "htgs_preprocess: sh_rest has more than 21 coefficients per Gaussian");
     const bool ordered = frame_depth_ordered(f);
     if (ordered && ((uintptr_t)f->depth_order & 15)) return fail(HTGS_ERR_ARGUMENT, "htgs_preprocess: depth_order must be 16-byte aligned");
+    if ((uintptr_t)f->touch & 15) return fail(HTGS_ERR_ARGUMENT, "htgs_preprocess: touch must be 16-byte aligned");
+    const float cutoff_sq = f->mode == HTGS_MODE_ALPHA_BLEND_FIRST_K ? ModeCfg<HTGS_MODE_ALPHA_BLEND_FIRST_K>::cutoff_sq : ModeCfg<HTGS_MODE_HYBRID_BLEND>::cutoff_sq;
     const DepthOrder order = depth_order_parts(f);
     const DepthKeys order_keys = depth_key_range(f);
     hipLaunchKernelGGL(preprocess_kernel, dim3(div_up(f->n_primitives, 256)), dim3(256), lds_bytes, (hipStream_t)f->stream,
                        f->positions, f->scales, f->rotations, f->opacities, f->sh_0, f->sh_rest, f->M, f->VPM, f->cam_position,
                        f->n_touched, f->bounds, f->prim, f->clamp_info, f->n_primitives, grid_w, grid_h, (float)tile,
                        min_alpha_rcp, f->active_sh_bases, f->total_sh_bases, f->near_plane, f->far_plane, f->scale_modifier, prim_floats / 4,
-                       ordered ? order.keys[0] : nullptr, ordered ? order.vals[0] : nullptr, order_keys.base, order_keys.culled, order_keys.shift);
+                       ordered ? order.keys[0] : nullptr, ordered ? order.vals[0] : nullptr, order_keys.base, order_keys.culled, order_keys.shift,
+                       (uint4 *)f->touch, cutoff_sq, f->touch_cutoff_only);
     return check_launch("preprocess");
 }

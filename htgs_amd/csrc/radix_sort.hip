@@ -9,7 +9,7 @@
 //   digit_scatter   : re-reads the block's items, ranks them stably with wave64 ballots, scatters
 // Item order inside a block is (wave, round, lane); every rank below is computed in that order,
 // which is what keeps equal keys in their input order.
-#include "common.h"
+#include "tile_span.h"
 
 namespace htgs {
 
@@ -114,13 +114,13 @@ __global__ void __launch_bounds__(kScanThreads) digit_row_scan_kernel(uint32_t *
 // RECTANGLES (a sort of one pass over the Gaussians, whose values are their indices in the order of the input): the
 // Gaussians' tile rectangles, four 16-bit bounds each, travel with the pairs -- read in the order of the input, which is
 // theirs, written in sorted order, with the number of tiles each covers beside them (none for the key `culled`, whose
-// rectangle was never written).
+// rectangle was never written).  With touch_in the touch entries travel instead (htgs_frame.touch), straight to their places.
 template <typename KeyT, int THREADS = SortShape<KeyT>::threads, int BITS = SortDigit<KeyT>::bits, bool RECTANGLES = false>
 __global__ void __launch_bounds__(THREADS) digit_scatter_kernel(
     const KeyT *__restrict__ keys_in, const uint32_t *__restrict__ vals_in, KeyT *__restrict__ keys_out, uint32_t *__restrict__ vals_out,
     const uint32_t *__restrict__ hist, const uint32_t *__restrict__ totals, InstanceCount count, int shift, uint32_t mask,
     bool last_pass = false, const uint2 *__restrict__ rectangles_in = nullptr, uint2 *__restrict__ rectangles_out = nullptr,
-    uint32_t *__restrict__ counts_out = nullptr, uint32_t culled = 0)
+    uint32_t *__restrict__ counts_out = nullptr, uint32_t culled = 0, const uint4 *__restrict__ touch_in = nullptr, uint4 *__restrict__ touch_out = nullptr)
 {
     constexpr int kSortThreads = THREADS, kSortWaves = kSortThreads / kWave, kSortTile = kSortThreads * kSortItems;
     constexpr int kBits = BITS, kRadix = 1 << kBits, kDigitWaves = kRadix / kWave;
@@ -253,6 +253,23 @@ __global__ void __launch_bounds__(THREADS) digit_scatter_kernel(
     }
     if constexpr (RECTANGLES) {
         static_assert(!kTwoRounds && sizeof(KeyT) == 4, "the rectangles take the room of the keys and the values");
+        if (touch_in != nullptr) {
+#pragma unroll
+            for (int r = 0; r < kSortItems; ++r) {
+                const uint64_t i = wave_base + (uint64_t)r * kWave + lane;
+                if (i < n) {
+                    const uint32_t d = digit_of(key[r], shift, mask), pos = global_base[d] + (rank[r] - digit_start[d]);
+                    uint32_t count = 0;
+                    if (key[r] != (KeyT)culled) {
+                        const uint4 v = touch_in[i];
+                        count = touch_count(TileTouch{ v.x, v.y, v.z, v.w });
+                        touch_out[pos] = v;
+                    }
+                    counts_out[pos] = count;
+                }
+            }
+            return;
+        }
         uint2 *local_rectangles = reinterpret_cast<uint2 *>(local_raw);
         __syncthreads();
 #pragma unroll
@@ -325,7 +342,7 @@ static int sort_pairs(hipStream_t s, void *const keys[2], uint32_t *const vals[2
 }
 
 int sort_u32_pairs_with_rectangles(void *stream, uint32_t *const keys[2], uint32_t *const vals[2], uint32_t *sort_tmp, uint64_t n, int bits,
-                                   const uint16_t *rectangles_in, uint16_t *rectangles_out, uint32_t *counts_out, uint32_t culled)
+                                   const uint16_t *rectangles_in, uint16_t *rectangles_out, const uint32_t *touch_in, uint32_t *touch_out, uint32_t *counts_out, uint32_t culled)
 {
     if (n == 0) return HTGS_OK;
     if (bits < 1 || bits > 8) return fail(HTGS_ERR_ARGUMENT, "sort: one pass takes at most eight bits");
@@ -340,7 +357,8 @@ int sort_u32_pairs_with_rectangles(void *stream, uint32_t *const keys[2], uint32
     hipLaunchKernelGGL(digit_row_scan_kernel, dim3(kRadix), dim3(kScanThreads), 0, s, hist, totals, count, (uint32_t)kTile);
     hipLaunchKernelGGL((digit_scatter_kernel<uint32_t, kThreads, kBits, true>), dim3(xcd_padded_grid(n_blocks)), dim3(kThreads), 0, s, keys[0], vals[0], keys[1],
                        vals[1], hist, totals, count, 0, mask, false, reinterpret_cast<const uint2 *>(rectangles_in),
-                       reinterpret_cast<uint2 *>(rectangles_out), counts_out, culled);
+                       reinterpret_cast<uint2 *>(rectangles_out), counts_out, culled, reinterpret_cast<const uint4 *>(touch_in),
+                       reinterpret_cast<uint4 *>(touch_out));
     return check_launch("sort");
 }
 

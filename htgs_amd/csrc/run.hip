@@ -100,7 +100,10 @@ static uint64_t carve_front(htgs_frame *f, int what, void *base)
     f->prim_floats = train ? HTGS_PRIM_FLOATS_TRAIN : HTGS_PRIM_FLOATS;
     f->n_touched = c.take<uint32_t>(n);
     f->offsets = c.take<uint32_t>(n);
-    f->bounds = c.take<uint16_t>(4 * n);
+    f->bounds = nullptr;
+    f->touch = c.take<uint32_t>(4 * n);
+    // (the tail's second walk of the weights takes fragments below the alpha threshold)
+    f->touch_cutoff_only = what == HTGS_RUN_MAX_WEIGHTS ? 1 : 0;
     f->prim = c.take<float>((uint64_t)f->prim_floats * n);
     f->clamp_info = train ? c.take<uint8_t>(3 * n) : nullptr;
     f->scan_tmp = c.take<uint32_t>(htgs_scan_tmp_words((int)n));

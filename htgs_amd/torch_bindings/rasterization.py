@@ -158,7 +158,7 @@ class FrameBuffers:
     def __init__(self, positions, scales, rotations, opacities, sh_0, sh_rest, settings: RasterizerSettings,
                  to_chw: bool = True, use_median_depth: bool = False, train: bool = False,
                  pool: Optional[ScratchPool] = None, fast: bool = False, long_list_threshold: int = 0, order_tiles: bool = True,
-                 order_gaussians: bool = True):
+                 order_gaussians: bool = True, tight_lists: bool = False):
         mode = _mode_value(settings.mode)
         if mode not in (0, 1, 2, 3):
             raise RuntimeError("unsupported rasterizer mode")
@@ -196,6 +196,8 @@ class FrameBuffers:
         self.n_touched = self._scratch("n_touched", n, torch.int32)[:n]
         self.offsets = self._scratch("offsets", n, torch.int32)[:n]
         self.bounds = self._scratch("bounds", 4 * n, torch.int16)[:4 * n].view(n, 4)
+        # the tiles that a Gaussian's outline meets instead of all tiles of its rectangle (what ``rasterize`` and the others do)
+        self.touch = self._scratch("touch", 4 * n, torch.int32)[:4 * n].view(n, 4) if tight_lists else None
         # (training frames use 128-byte records: the backward pass finds the slot of an instance's gradient row in them)
         self.prim_floats = _native.PRIM_FLOATS_TRAIN if train else _native.PRIM_FLOATS
         self.prim = self._scratch("prim", self.prim_floats * n, torch.float32)[:self.prim_floats * n].view(n, self.prim_floats)
@@ -237,6 +239,7 @@ class FrameBuffers:
         f.near_plane, f.far_plane = float(settings.near_plane), float(settings.far_plane)
         f.scale_modifier = float(settings.scale_modifier)
         f.n_touched, f.offsets, f.bounds, f.prim = _ptr(self.n_touched), _ptr(self.offsets), _ptr(self.bounds), _ptr(self.prim)
+        f.touch = _ptr(self.touch)
         f.prim_floats = self.prim_floats
         f.clamp_info = _ptr(self.clamp_info)
         f.scan_tmp, f.n_instances_dev = _ptr(self.scan_tmp), _ptr(self.n_instances_dev)

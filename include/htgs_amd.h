@@ -37,7 +37,8 @@ extern "C" {
 #define HTGS_PRIM_FLOATS 20
 /* the training entry points use records of 128 bytes (one cache line per gather): the twenty floats above, then four
  * words written by htgs_create_instances for the backward pass -- the Gaussian's first slot in the unsorted instance
- * list (offsets[g-1]), x_min | y_min << 16 and the width of its tile rectangle, 0 -- then padding */
+ * list (offsets[g-1]), the tile at the corner of its rectangle, the rectangle's width or the mask of its listed tiles --
+ * then padding */
 #define HTGS_PRIM_FLOATS_TRAIN 32
 
 /*
@@ -68,6 +69,14 @@ typedef struct htgs_frame {
     uint32_t *n_touched;       /* [N] tiles covered, 0 = culled */
     uint32_t *offsets;         /* [N] inclusive prefix sum of n_touched */
     uint16_t *bounds;          /* [N,4] tile rectangle x_min,x_max,y_min,y_max (exclusive max) */
+    uint32_t *touch;           /* [N,4] or NULL, 16-byte aligned; replaces bounds (which may then be NULL).  A Gaussian is listed in
+                                  the tiles of its rectangle that its outline meets instead of in all of them; n_touched
+                                  counts those.  What is left out contributes to no pixel.  Per visible Gaussian: x_min |
+                                  y_min << 16, width | height << 16 of the rectangle, then a mask of the listed tiles,
+                                  row-major (rectangles of up to 64 tiles), or their number (larger ones, which a training
+                                  frame lists in full).  NULL: every tile of the rectangle, the reference's lists */
+    int32_t touch_cutoff_only; /* touch: keep the tiles that the cut-off alone reaches (htgs_max_weights_blend, whose second
+                                  walk has no alpha threshold) */
     float *prim;               /* [N,prim_floats] */
     int32_t prim_floats;       /* 0 or HTGS_PRIM_FLOATS for the inference entry points and htgs_max_weights_*,
                                   HTGS_PRIM_FLOATS_TRAIN for the training entry points (htgs_forward_*, htgs_blend_forward,
