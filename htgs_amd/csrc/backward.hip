@@ -1006,7 +1006,7 @@ static void launch_tail_backward_kernels(const htgs_frame *f, int sel, uint32_t 
                        f->ranges, f->vals[sel], (const float4 *)f->prim, f->core_idx, (const float4 *)f->core_info, f->tail_info, f->grad_image,
                        f->VPM, (float4 *)f->grad_rows, f->dens_helper, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->tile_order, f->long_tiles, threshold,
                        floor < 1u ? 1u : (uint32_t)floor);
-    if (f->long_tiles)      // (four workgroups per compute unit; they find an empty list on ordinary frames)
+    if (may_have_long_lists(f, threshold))      // (four workgroups per compute unit; they find an empty list on ordinary frames)
         hipLaunchKernelGGL((blend_tail_backward_long_kernel<K, MODE, HELPER>), dim3(1024), dim3(64 * kBackwardWaves), 0, (hipStream_t)f->stream,
                            f->ranges, f->vals[sel], (const float4 *)f->prim, f->core_idx, (const float4 *)f->core_info, f->tail_info, f->grad_image,
                            f->VPM, (float4 *)f->grad_rows, f->dens_helper, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, threshold);

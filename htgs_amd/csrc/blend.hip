@@ -184,7 +184,7 @@ static void launch_hybrid(const htgs_frame *f, int selector, uint32_t grid_w, ui
         hipLaunchKernelGGL((blend_hybrid_kernel<K, FAST>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
                            f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
-    if (f->long_tiles)      // (one workgroup per compute unit; they find an empty list on ordinary frames)
+    if (may_have_long_lists(f, threshold))      // (one workgroup per compute unit; they find an empty list on ordinary frames)
         hipLaunchKernelGGL((blend_hybrid_long_kernel<K, FAST, HTGS_PRIM_FLOATS / 4, HybridImage>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0,
                            (hipStream_t)f->stream, f->ranges, f->vals[selector], (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w,
                            f->vals[selector ^ 1], threshold,
@@ -202,7 +202,7 @@ static void launch_first_k(const htgs_frame *f, int selector, uint32_t grid_w, u
         hipLaunchKernelGGL((blend_first_k_kernel<K, FAST>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
                            f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
-    if (f->long_tiles)
+    if (may_have_long_lists(f, threshold))
         hipLaunchKernelGGL((blend_first_k_long_kernel<K, FAST, HTGS_PRIM_FLOATS / 4, FirstKImage>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0,
                            (hipStream_t)f->stream, f->ranges, f->vals[selector], (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w,
                            f->vals[selector ^ 1], threshold,
@@ -246,7 +246,7 @@ static void launch_blend(const htgs_frame *f, int selector, uint32_t grid_w, uin
             hipLaunchKernelGGL(blend_oit_kernel<FAST>, dim3(n_tiles), dim3(64), 0, s, f->ranges, f->vals[selector], (const float4 *)f->prim,
                                f->image, depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw, f->long_tiles, threshold,
                                long_part_floor(f, selector), f->tile_order);
-            if (f->long_tiles)
+            if (may_have_long_lists(f, threshold))
                 hipLaunchKernelGGL((blend_oit_long_kernel<FAST, HTGS_PRIM_FLOATS / 4, OitImage>), dim3(256), dim3(64 * kLongWaves), 0, s, f->ranges, f->vals[selector],
                                    (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->vals[selector ^ 1], threshold,
                                    OitImage{ f->image, depth, (uint32_t)f->width, (uint32_t)f->height, f->to_chw });

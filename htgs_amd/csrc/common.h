@@ -145,6 +145,30 @@ struct PartFloor {
     }
 };
 
+// What htgs_run's first queueing of a frame spares the later stages: the per-Gaussian stage also leaves the sums of its
+// blocks' counts (scan_tmp) and clears the ranges, the tile order's bins and the header of long_tiles.  Nothing of it holds
+// for a frame whose second half is queued again.
+constexpr int kCountBlock = 256;                 // Gaussians per block sum
+struct FrameStart {
+    uint32_t *block_sums;                        // [ceil(N / kCountBlock)] or nullptr
+    uint32_t *clear[3];                          // ranges, order bins, long_tiles header
+    uint32_t clear_words[3];
+};
+int preprocess_and_start(const htgs_frame *f, const FrameStart &start);                 // preprocess.hip
+// The scan for htgs_run, which also writes tag << 32 | total to host memory.  with_sums: scan_tmp holds FrameStart's sums.
+// Returns in *fused whether the scan was left to create_instances_fused (few Gaussians).
+int scan_offsets_publish(const htgs_frame *f, unsigned long long *host_total, uint32_t tag, bool with_sums, bool *fused);    // instances.hip
+int create_instances_fused(const htgs_frame *f, unsigned long long *host_total, uint32_t tag);
+// (cleared: the ranges, bins and header are zero already; ranged: the sort has written the ranges)
+int extract_ranges_of(const htgs_frame *f, int selector, bool cleared, bool ranged);
+int sort_instances_of(const htgs_frame *f, int *selector, bool *ranged);                // radix_sort.hip
+// words of scan_tmp for N Gaussians' block sums
+inline size_t block_sum_words(int n) { return (size_t)div_up(n > 0 ? n : 1, kCountBlock); }
+
+// Whether a list of the frame can be longer than `threshold` (a Gaussian is in a tile's list once): otherwise the kernels for
+// such lists, which would find nothing to do, are not launched.
+inline bool may_have_long_lists(const htgs_frame *f, uint32_t threshold) { return f->long_tiles != nullptr && (uint32_t)f->n_primitives > threshold; }
+
 // host side error reporting (api.hip)
 int fail(int code, const char *fmt, ...);
 int check_launch(const char *what);

@@ -253,7 +253,7 @@ static void launch_tile(const htgs_frame *f, int sel, uint32_t *max_weights, flo
     const uint32_t w = (uint32_t)f->width, h = (uint32_t)f->height;
     hipLaunchKernelGGL((max_weights_tile_kernel<K, MODE>), dim3(n_tiles), dim3(64), 0, s, f->ranges, f->vals[sel], (const float4 *)f->prim, max_weights, w, h, grid_w,
                        thr, f->tile_order, shared ? f->long_tiles : nullptr, threshold, part_floor_of(f, sel, true));
-    if (!shared) return;
+    if (!shared || !may_have_long_lists(f, threshold)) return;
     constexpr int REC4 = HTGS_PRIM_FLOATS / 4;
     if constexpr (MODE == HTGS_MODE_HYBRID_BLEND)
         hipLaunchKernelGGL((blend_hybrid_long_kernel<K, false, REC4, MaxWeightsHybrid>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0, s,

@@ -56,7 +56,23 @@ __device__ __forceinline__ void axis_extent(const float f[4], const Row &Vi, con
     extent = __builtin_sqrtf(clamp_pos(center * center - q));
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) preprocess_kernel(
+// sum over the wave, in its last lane (each step one addition whose operand comes from the lanes before)
+__device__ __forceinline__ uint32_t wave_sum_last(uint32_t v)
+{
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);     // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);     // row_shr:2
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);     // row_shr:4
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);     // row_shr:8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);     // row_bcast:15
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);     // row_bcast:31
+    return v;
+}
+
+// SH_REGS: 16-byte words of SH coefficients a thread holds while the bounds are computed (ceil(3 total_sh / 4): 12 for degree
+// 3, 16 for the most the kernel takes).  0: no bands beyond the constant one are active, and without those registers twice
+// as many waves fit.
+template <int SH_REGS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SH_REGS > 0 ? 3 : 6))) preprocess_kernel(
     const float *__restrict__ positions, const float *__restrict__ scales, const float *__restrict__ rotations,
     const float *__restrict__ opacities, const float *__restrict__ sh_0, const float *__restrict__ sh_rest,
     const float *__restrict__ M, const float *__restrict__ VPM_in, const float *__restrict__ cam_position,
@@ -65,7 +81,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) p
     int n, uint32_t grid_w, uint32_t grid_h, float tile, float min_alpha_rcp,
     int active_sh, int total_sh, float near_plane, float far_plane, float scale_modifier, int rec4,
     uint32_t *__restrict__ depth_keys, uint32_t *__restrict__ depth_vals, uint32_t depth_base, uint32_t depth_culled, int depth_shift,
-    uint4 *__restrict__ touch, float rho_most, int cutoff_only)
+    uint4 *__restrict__ touch, float rho_most, int cutoff_only, FrameStart start)
 {
     // One LDS buffer, used twice: first the block's slice of sh_rest (contiguous in memory, loaded with coalesced
     // 16-byte reads and then read back per Gaussian at a stride of 3 * total_sh words), then the block's records
@@ -74,6 +90,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) p
     extern __shared__ float4 lds4[];
     float *lds = reinterpret_cast<float *>(lds4);
     __shared__ uint8_t s_visible[256];
+    __shared__ uint32_t s_counts[256 / kWave];
     const int first = blockIdx.x * 256;
     const int i = first + threadIdx.x;
     const bool in_range = i < n;
@@ -89,13 +106,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) p
 
     // The block's slice of sh_rest is three quarters of everything this kernel reads.  Its loads are issued first,
     // into registers, so that they are in flight while the bounds are computed; they reach LDS further down.
-    constexpr int kShRegs = 16;                                    // 16-byte words per thread: 256 x 3 x 21 / 4 / 256
+    constexpr int kShRegs = SH_REGS;
     const int per = 3 * total_sh;                                  // words per Gaussian
     const int n_block = n - first < 256 ? n - first : 256;
     const size_t base_word = (size_t)first * per;                 // multiple of 256 words: 16-byte aligned
     const int words = active_sh > 1 ? n_block * per : 0;
     const float4 *src4 = reinterpret_cast<const float4 *>(sh_rest + base_word);
-    float sh_regs[kShRegs][4];
+    float sh_regs[kShRegs > 0 ? kShRegs : 1][4];
 #pragma unroll
     for (int k = 0; k < kShRegs; ++k) {
         const int q = k * 256 + threadIdx.x;
@@ -204,6 +221,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) p
         if (visible) touch[i] = make_uint4(t.corner, t.size, t.lo, t.hi);
     }
     if (in_range) n_touched[i] = touched;
+    if (start.block_sums != nullptr) {
+        const uint32_t sum = wave_sum_last(in_range ? touched : 0u);
+        if ((threadIdx.x & (kWave - 1)) == kWave - 1) s_counts[threadIdx.x / kWave] = sum;
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            for (uint32_t w = blockIdx.x * 256u + threadIdx.x; w < start.clear_words[k]; w += gridDim.x * 256u) start.clear[k][w] = 0u;
+    }
     // htgs_frame.depth_order: the pairs that sort the Gaussians by depth (depth_key_range() in common.h)
     if (depth_keys != nullptr && in_range) {
         // (a depth that is not a number passes the cull above, as in the reference, where its bit pattern sorts behind every
@@ -224,6 +248,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) p
     }
     for (int q = (words & ~3) + threadIdx.x; q < words; q += 256) lds[q] = sh_rest[base_word + q];
     __syncthreads();
+    if (start.block_sums != nullptr && threadIdx.x == 0) start.block_sums[blockIdx.x] = (s_counts[0] + s_counts[1]) + (s_counts[2] + s_counts[3]);
 
     // view-dependent colour, kernel_utils.cuh:152-187
     float res[3] = { 0.0f, 0.0f, 0.0f };
@@ -297,11 +322,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) p
     }
 }
 
-}  // namespace htgs
-
-extern "C" int htgs_preprocess(const htgs_frame *f)
+int preprocess_and_start(const htgs_frame *f, const FrameStart &start)
 {
-    using namespace htgs;
     if (!f) return fail(HTGS_ERR_ARGUMENT, "htgs_preprocess: null frame");
     if (f->mode < 0 || f->mode > 3) return fail(HTGS_ERR_MODE, "unsupported rasterizer mode");
     if (f->n_primitives < 0 || f->width <= 0 || f->height <= 0 || f->total_sh_bases < 0)
@@ -330,11 +352,16 @@ extern "C" int htgs_preprocess(const htgs_frame *f)
     const float cutoff_sq = f->mode == HTGS_MODE_ALPHA_BLEND_FIRST_K ? ModeCfg<HTGS_MODE_ALPHA_BLEND_FIRST_K>::cutoff_sq : ModeCfg<HTGS_MODE_HYBRID_BLEND>::cutoff_sq;
     const DepthOrder order = depth_order_parts(f);
     const DepthKeys order_keys = depth_key_range(f);
-    hipLaunchKernelGGL(preprocess_kernel, dim3(div_up(f->n_primitives, 256)), dim3(256), lds_bytes, (hipStream_t)f->stream,
+    const auto kernel = f->active_sh_bases <= 1 ? preprocess_kernel<0> : f->total_sh_bases <= 15 ? preprocess_kernel<12> : preprocess_kernel<16>;
+    hipLaunchKernelGGL(kernel, dim3(div_up(f->n_primitives, 256)), dim3(256), lds_bytes, (hipStream_t)f->stream,
                        f->positions, f->scales, f->rotations, f->opacities, f->sh_0, f->sh_rest, f->M, f->VPM, f->cam_position,
                        f->n_touched, f->bounds, f->prim, f->clamp_info, f->n_primitives, grid_w, grid_h, (float)tile,
                        min_alpha_rcp, f->active_sh_bases, f->total_sh_bases, f->near_plane, f->far_plane, f->scale_modifier, prim_floats / 4,
                        ordered ? order.keys[0] : nullptr, ordered ? order.vals[0] : nullptr, order_keys.base, order_keys.culled, order_keys.shift,
-                       (uint4 *)f->touch, cutoff_sq, f->touch_cutoff_only);
+                       (uint4 *)f->touch, cutoff_sq, f->touch_cutoff_only, start);
     return check_launch("preprocess");
 }
+
+}  // namespace htgs
+
+extern "C" int htgs_preprocess(const htgs_frame *f) { return htgs::preprocess_and_start(f, htgs::FrameStart{}); }

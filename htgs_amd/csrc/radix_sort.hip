@@ -14,6 +14,10 @@
 namespace htgs {
 
 constexpr int kSortItems = 16;                              // rounds per wave
+// A sort of up to kSmallSort items takes blocks of a quarter of the items: with 8192 to a block a million items occupy half of
+// the compute units, each for the 14 us that sixteen rounds of ranking take one after the other.
+constexpr int kSmallItems = 4;
+constexpr uint64_t kSmallSort = 2u << 20;
 // digit width per key type; kRadix digits, the first kRadix threads of a block own one digit each
 template <typename KeyT> struct SortDigit { static constexpr int bits = sizeof(KeyT) == 8 ? 9 : 8; };
 constexpr int kMaxRadix = 512;
@@ -39,11 +43,11 @@ __device__ __forceinline__ uint32_t xcd_contiguous_block(uint32_t launched, uint
 __device__ __forceinline__ uint32_t blocks_of(uint32_t n, uint32_t per_block) { return n / per_block + (n % per_block != 0u ? 1u : 0u); }
 inline uint32_t xcd_padded_grid(uint32_t n_blocks) { return (n_blocks + kXcds - 1) / kXcds * kXcds; }
 
-template <typename KeyT, int THREADS = SortShape<KeyT>::threads, int BITS = SortDigit<KeyT>::bits>
+template <typename KeyT, int THREADS = SortShape<KeyT>::threads, int BITS = SortDigit<KeyT>::bits, int ITEMS = kSortItems>
 __global__ void __launch_bounds__(THREADS) digit_histogram_kernel(const KeyT *__restrict__ keys, uint32_t *__restrict__ hist,
                                                                 InstanceCount count, int shift, uint32_t mask)
 {
-    constexpr int kSortThreads = THREADS, kSortTile = kSortThreads * kSortItems, kRadix = 1 << BITS;
+    constexpr int kSortThreads = THREADS, kSortTile = kSortThreads * ITEMS, kRadix = 1 << BITS;
     const uint64_t n = count.get();
     const uint32_t n_blocks = blocks_of((uint32_t)n, kSortTile);
     static_assert(kRadix <= kSortThreads, "one thread per digit");
@@ -58,8 +62,10 @@ __global__ void __launch_bounds__(THREADS) digit_histogram_kernel(const KeyT *__
     if (base + kSortTile <= n) {
         const uint4 *words = reinterpret_cast<const uint4 *>(keys + base);      // kSortTile keys are a multiple of 16 bytes
 #pragma unroll
-        for (int r = 0; r < kSortItems / kPer; ++r) {
-            const uint4 word = words[r * kSortThreads + threadIdx.x];
+        for (int r = 0; r < (ITEMS + kPer - 1) / kPer; ++r) {
+            const int at = r * kSortThreads + threadIdx.x;
+            if (ITEMS % kPer != 0 && at >= kSortTile / kPer) break;
+            const uint4 word = words[at];
             KeyT k[kPer];
             __builtin_memcpy(k, &word, 16);
 #pragma unroll
@@ -67,7 +73,7 @@ __global__ void __launch_bounds__(THREADS) digit_histogram_kernel(const KeyT *__
         }
     } else {
 #pragma unroll
-        for (int r = 0; r < kSortItems; ++r) {
+        for (int r = 0; r < ITEMS; ++r) {
             const uint64_t i = base + (uint64_t)r * kSortThreads + threadIdx.x;
             if (i < n) atomicAdd(&counts[digit_of(keys[i], shift, mask)], 1u);
         }
@@ -115,14 +121,15 @@ __global__ void __launch_bounds__(kScanThreads) digit_row_scan_kernel(uint32_t *
 // Gaussians' tile rectangles, four 16-bit bounds each, travel with the pairs -- read in the order of the input, which is
 // theirs, written in sorted order, with the number of tiles each covers beside them (none for the key `culled`, whose
 // rectangle was never written).  With touch_in the touch entries travel instead (htgs_frame.touch), straight to their places.
-template <typename KeyT, int THREADS = SortShape<KeyT>::threads, int BITS = SortDigit<KeyT>::bits, bool RECTANGLES = false>
+template <typename KeyT, int THREADS = SortShape<KeyT>::threads, int BITS = SortDigit<KeyT>::bits, bool RECTANGLES = false,
+          int ITEMS = kSortItems>
 __global__ void __launch_bounds__(THREADS) digit_scatter_kernel(
     const KeyT *__restrict__ keys_in, const uint32_t *__restrict__ vals_in, KeyT *__restrict__ keys_out, uint32_t *__restrict__ vals_out,
     const uint32_t *__restrict__ hist, const uint32_t *__restrict__ totals, InstanceCount count, int shift, uint32_t mask,
     bool last_pass = false, const uint2 *__restrict__ rectangles_in = nullptr, uint2 *__restrict__ rectangles_out = nullptr,
     uint32_t *__restrict__ counts_out = nullptr, uint32_t culled = 0, const uint4 *__restrict__ touch_in = nullptr, uint4 *__restrict__ touch_out = nullptr)
 {
-    constexpr int kSortThreads = THREADS, kSortWaves = kSortThreads / kWave, kSortTile = kSortThreads * kSortItems;
+    constexpr int kSortThreads = THREADS, kSortWaves = kSortThreads / kWave, kSortTile = kSortThreads * ITEMS;
     constexpr int kBits = BITS, kRadix = 1 << kBits, kDigitWaves = kRadix / kWave;
     const uint64_t n = count.get();
     const uint32_t n_blocks = blocks_of((uint32_t)n, kSortTile);
@@ -146,12 +153,12 @@ __global__ void __launch_bounds__(THREADS) digit_scatter_kernel(
     __syncthreads();
 
     const uint64_t block_base = (uint64_t)block * kSortTile;
-    const uint64_t wave_base = block_base + (uint64_t)wave * (kWave * kSortItems);
-    KeyT key[kSortItems];
-    uint32_t val[kSortItems];
-    uint32_t rank[kSortItems];
+    const uint64_t wave_base = block_base + (uint64_t)wave * (kWave * ITEMS);
+    KeyT key[ITEMS];
+    uint32_t val[ITEMS];
+    uint32_t rank[ITEMS];
 #pragma unroll
-    for (int r = 0; r < kSortItems; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
         const uint64_t i = wave_base + (uint64_t)r * kWave + lane;
         const bool valid = i < n;
         // (the last reads of these buffers before they are written again: streaming, nothing to keep in the caches)
@@ -220,7 +227,7 @@ __global__ void __launch_bounds__(THREADS) digit_scatter_kernel(
 
     // group the block's items by digit in LDS (stable), ...
 #pragma unroll
-    for (int r = 0; r < kSortItems; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
         const uint64_t i = wave_base + (uint64_t)r * kWave + lane;
         rank[r] += counts[wave][digit_of(key[r], shift, mask)];          // now the item's slot in the block-local order
         if (i < n) {
@@ -231,11 +238,11 @@ __global__ void __launch_bounds__(THREADS) digit_scatter_kernel(
     __syncthreads();
     // ... then stream them out: neighbouring threads write neighbouring addresses inside each digit's run
     const uint32_t n_local = n - block_base < (uint64_t)kSortTile ? (uint32_t)(n - block_base) : (uint32_t)kSortTile;
-    uint32_t digits[kSortItems / 2];           // two rounds: the digits, two to a register, for the values' turn
+    uint32_t digits[ITEMS / 2];           // two rounds: the digits, two to a register, for the values' turn
 #pragma unroll
-    for (int r = 0; r < kSortItems / 2; ++r) digits[r] = 0u;
+    for (int r = 0; r < ITEMS / 2; ++r) digits[r] = 0u;
 #pragma unroll
-    for (int r = 0; r < kSortItems; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
         const uint32_t i = (uint32_t)r * kSortThreads + threadIdx.x;
         if (i < n_local) {
             const KeyT k = local_keys[i];
@@ -255,7 +262,7 @@ __global__ void __launch_bounds__(THREADS) digit_scatter_kernel(
         static_assert(!kTwoRounds && sizeof(KeyT) == 4, "the rectangles take the room of the keys and the values");
         if (touch_in != nullptr) {
 #pragma unroll
-            for (int r = 0; r < kSortItems; ++r) {
+            for (int r = 0; r < ITEMS; ++r) {
                 const uint64_t i = wave_base + (uint64_t)r * kWave + lane;
                 if (i < n) {
                     const uint32_t d = digit_of(key[r], shift, mask), pos = global_base[d] + (rank[r] - digit_start[d]);
@@ -273,13 +280,13 @@ __global__ void __launch_bounds__(THREADS) digit_scatter_kernel(
         uint2 *local_rectangles = reinterpret_cast<uint2 *>(local_raw);
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < kSortItems; ++r) {
+        for (int r = 0; r < ITEMS; ++r) {
             const uint64_t i = wave_base + (uint64_t)r * kWave + lane;
             if (i < n) local_rectangles[rank[r]] = key[r] == (KeyT)culled ? make_uint2(0u, 0u) : rectangles_in[i];
         }
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < kSortItems; ++r) {
+        for (int r = 0; r < ITEMS; ++r) {
             const uint32_t i = (uint32_t)r * kSortThreads + threadIdx.x;
             if (i < n_local) {
                 const uint32_t d = digits[r / 2] >> (16 * (r % 2)) & 0xffffu;
@@ -293,13 +300,13 @@ __global__ void __launch_bounds__(THREADS) digit_scatter_kernel(
     if (kTwoRounds) {
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < kSortItems; ++r) {
+        for (int r = 0; r < ITEMS; ++r) {
             const uint64_t i = wave_base + (uint64_t)r * kWave + lane;
             if (i < n) local_vals[rank[r]] = val[r];
         }
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < kSortItems; ++r) {
+        for (int r = 0; r < ITEMS; ++r) {
             const uint32_t i = (uint32_t)r * kSortThreads + threadIdx.x;
             if (i < n_local) {
                 const uint32_t d = digits[r / 2] >> (16 * (r % 2)) & 0xffffu;
@@ -312,12 +319,12 @@ __global__ void __launch_bounds__(THREADS) digit_scatter_kernel(
 }
 
 // streaming_result: the sorted values leave the last pass as streaming stores (the instance lists, which the blend reads once)
-template <typename KeyT, int THREADS = SortShape<KeyT>::threads, int BITS = SortDigit<KeyT>::bits>
+template <typename KeyT, int THREADS = SortShape<KeyT>::threads, int BITS = SortDigit<KeyT>::bits, int ITEMS = kSortItems>
 static int sort_pairs(hipStream_t s, void *const keys[2], uint32_t *const vals[2], uint32_t *sort_tmp, InstanceCount count, int end_bit, int *selector,
                       bool streaming_result = false)
 {
     const uint64_t n = count.most;
-    constexpr int kSortThreads = THREADS, kSortTile = kSortThreads * kSortItems;
+    constexpr int kSortThreads = THREADS, kSortTile = kSortThreads * ITEMS;
     const uint32_t n_blocks = (uint32_t)((n + kSortTile - 1) / kSortTile);
     constexpr int kBits = BITS, kRadix = 1 << kBits;
     uint32_t *hist = sort_tmp;
@@ -331,9 +338,9 @@ static int sort_pairs(hipStream_t s, void *const keys[2], uint32_t *const vals[2
         const uint32_t mask = (1u << bits) - 1u;
         const KeyT *kin = (const KeyT *)keys[cur];
         KeyT *kout = (KeyT *)keys[cur ^ 1];
-        hipLaunchKernelGGL((digit_histogram_kernel<KeyT, THREADS, BITS>), dim3(xcd_padded_grid(n_blocks)), dim3(kSortThreads), 0, s, kin, hist, count, shift, mask);
+        hipLaunchKernelGGL((digit_histogram_kernel<KeyT, THREADS, BITS, ITEMS>), dim3(xcd_padded_grid(n_blocks)), dim3(kSortThreads), 0, s, kin, hist, count, shift, mask);
         hipLaunchKernelGGL(digit_row_scan_kernel, dim3(kRadix), dim3(kScanThreads), 0, s, hist, totals, count, (uint32_t)kSortTile);
-        hipLaunchKernelGGL((digit_scatter_kernel<KeyT, THREADS, BITS>), dim3(xcd_padded_grid(n_blocks)), dim3(kSortThreads), 0, s, kin, vals[cur], kout, vals[cur ^ 1],
+        hipLaunchKernelGGL((digit_scatter_kernel<KeyT, THREADS, BITS, false, ITEMS>), dim3(xcd_padded_grid(n_blocks)), dim3(kSortThreads), 0, s, kin, vals[cur], kout, vals[cur ^ 1],
                            hist, totals, count, shift, mask, streaming_result && shift + step >= end_bit);
         cur ^= 1;
     }
@@ -371,8 +378,172 @@ int sort_u32_pairs(void *stream, uint32_t *const keys[2], uint32_t *const vals[2
     const InstanceCount count = { nullptr, (uint32_t)n };
     // a few million pairs: with 8-bit digits blocks of 4096 items, the smallest the kernels take, so that every compute
     // unit has several; 9-bit digits need a thread per digit (8192 items)
+    if (digit_bits == 9 && n <= kSmallSort) return sort_pairs<uint32_t, 512, 9, kSmallItems>((hipStream_t)stream, k, vals, sort_tmp, count, end_bit, selector);
     if (digit_bits == 9) return sort_pairs<uint32_t, 512, 9>((hipStream_t)stream, k, vals, sort_tmp, count, end_bit, selector);
+    if (n <= kSmallSort / 2) return sort_pairs<uint32_t, kSortTileMin / kSortItems, 8, kSmallItems>((hipStream_t)stream, k, vals, sort_tmp, count, end_bit, selector);
     return sort_pairs<uint32_t, kSortTileMin / kSortItems, 8>((hipStream_t)stream, k, vals, sort_tmp, count, end_bit, selector);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Few instances over few tiles: one pass with the tile itself as the digit.  Three launches (counts per block, rows of
+// counts, scatter) instead of the six of two digit passes and the ranges' own: a tile's range is where its digit starts
+// and how many there are.  A block's items scatter over most of the tiles, so nothing is regrouped in LDS first; the
+// whole list fits the last-level cache.
+// ---------------------------------------------------------------------------------------------
+constexpr int kTileSortThreads = 512, kTileSortWaves = kTileSortThreads / kWave, kTileSortBlock = kTileSortThreads * kSmallItems;
+constexpr uint64_t kTileSortMost = 512u << 10;             // instances
+constexpr uint32_t kTileSortTiles = 4096;                  // (16-bit counts of twelve-bit digits for eight waves: 64 KB of LDS)
+
+template <int BITS>
+__global__ void __launch_bounds__(kTileSortThreads) tile_histogram_kernel(const uint16_t *__restrict__ keys, uint32_t *__restrict__ hist, InstanceCount count,
+                                                                         uint32_t n_tiles)
+{
+    __shared__ uint32_t counts[1 << BITS];
+    const uint32_t n = count.get(), n_blocks = blocks_of(n, kTileSortBlock);
+    if (blockIdx.x >= n_blocks) return;
+    for (uint32_t d = threadIdx.x; d < (1u << BITS); d += kTileSortThreads) counts[d] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSmallItems; ++r) {
+        const uint32_t i = blockIdx.x * kTileSortBlock + (uint32_t)r * kTileSortThreads + threadIdx.x;
+        if (i < n) atomicAdd(&counts[keys[i]], 1u);
+    }
+    __syncthreads();
+    for (uint32_t d = threadIdx.x; d < n_tiles; d += kTileSortThreads) hist[(size_t)d * n_blocks + blockIdx.x] = counts[d];
+}
+// a wave per tile: exclusive scan of its row in place, the row's total to totals
+__global__ void __launch_bounds__(256) tile_row_scan_kernel(uint32_t *__restrict__ hist, uint32_t *__restrict__ totals, InstanceCount count, uint32_t n_tiles)
+{
+    const uint32_t n_blocks = blocks_of(count.get(), kTileSortBlock);
+    const uint32_t d = blockIdx.x * (256 / kWave) + threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    if (d >= n_tiles) return;
+    uint32_t *row = hist + (size_t)d * n_blocks;
+    uint32_t carry = 0;
+    for (uint32_t start = 0; start < n_blocks; start += kWave) {
+        const uint32_t i = start + lane, v = i < n_blocks ? row[i] : 0u;
+        uint32_t inc = v;
+#pragma unroll
+        for (uint32_t s = 1; s < kWave; s <<= 1) {
+            const uint32_t t = (uint32_t)__shfl_up((int)inc, s, kWave);
+            if (lane >= s) inc += t;
+        }
+        if (i < n_blocks) row[i] = carry + inc - v;
+        carry += (uint32_t)__builtin_amdgcn_readlane((int)inc, kWave - 1);
+    }
+    if (lane == 0) totals[d] = carry;
+}
+template <int BITS>
+__global__ void __launch_bounds__(kTileSortThreads) tile_scatter_kernel(const uint16_t *__restrict__ keys, const uint32_t *__restrict__ vals_in,
+                                                                       uint32_t *__restrict__ vals_out, const uint32_t *__restrict__ hist,
+                                                                       const uint32_t *__restrict__ totals, uint32_t *__restrict__ ranges, InstanceCount count,
+                                                                       uint32_t n_tiles)
+{
+    constexpr uint32_t kRadix = 1u << BITS, kPer = kRadix / kTileSortThreads;
+    static_assert(kPer >= 1, "a thread owns whole digits");
+    __shared__ uint16_t counts[kTileSortWaves][kRadix];    // per wave: running count of each tile, later the wave's base inside the block
+    __shared__ uint32_t base[kRadix];                      // where the block's items of each tile start in the output
+    __shared__ uint32_t wave_sums[kTileSortWaves];
+    const uint32_t n = count.get(), n_blocks = blocks_of(n, kTileSortBlock);
+    // (without instances the first block still writes the ranges)
+    if (blockIdx.x >= n_blocks && blockIdx.x != 0) return;
+    const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    for (uint32_t c = threadIdx.x; c < kTileSortWaves * kRadix / 2; c += kTileSortThreads) reinterpret_cast<uint32_t *>(&counts[0][0])[c] = 0;
+    __syncthreads();
+    uint32_t key[kSmallItems], val[kSmallItems], rank[kSmallItems];
+#pragma unroll
+    for (int r = 0; r < kSmallItems; ++r) {
+        const uint32_t i = blockIdx.x * kTileSortBlock + wave * (kWave * kSmallItems) + (uint32_t)r * kWave + lane;
+        key[r] = i < n ? keys[i] : 0u;
+        val[r] = i < n ? vals_in[i] : 0u;
+    }
+#pragma unroll
+    for (int r = 0; r < kSmallItems; ++r) {
+        const bool valid = blockIdx.x * kTileSortBlock + wave * (kWave * kSmallItems) + (uint32_t)r * kWave + lane < n;
+        // lanes of this wave with the same tile (digit_scatter_kernel)
+        const uint64_t present = __ballot(valid);
+        uint32_t peers_lo = (uint32_t)present, peers_hi = (uint32_t)(present >> 32);
+#pragma unroll
+        for (int b = 0; b < BITS; ++b) {
+            const uint32_t bit = (uint32_t)__builtin_amdgcn_sbfe((int)key[r], b, 1);
+            const uint64_t vote = __ballot(bit != 0u);
+            peers_lo &= ~((uint32_t)vote ^ bit);
+            peers_hi &= ~((uint32_t)(vote >> 32) ^ bit);
+        }
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi(peers_hi, __builtin_amdgcn_mbcnt_lo(peers_lo, 0u));
+        uint32_t seen = 0;
+        if (valid) {
+            seen = counts[wave][key[r]];
+            if (below == 0) counts[wave][key[r]] = (uint16_t)(seen + (uint32_t)(__builtin_popcount(peers_lo) + __builtin_popcount(peers_hi)));
+        }
+        rank[r] = seen + below;
+    }
+    // where each tile starts: a thread owns kPer neighbouring tiles
+    uint32_t total[kPer], sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+        const uint32_t d = threadIdx.x * kPer + k;
+        total[k] = n != 0u && d < n_tiles ? totals[d] : 0u;
+        sum += total[k];
+    }
+    uint32_t inc = sum;
+#pragma unroll
+    for (uint32_t s = 1; s < kWave; s <<= 1) {
+        const uint32_t t = (uint32_t)__shfl_up((int)inc, s, kWave);
+        if (lane >= s) inc += t;
+    }
+    if (lane == kWave - 1) wave_sums[wave] = inc;
+    __syncthreads();
+    uint32_t start = inc - sum;
+#pragma unroll
+    for (int w = 0; w < kTileSortWaves; ++w) start += (uint32_t)w < wave ? wave_sums[w] : 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+        const uint32_t d = threadIdx.x * kPer + k;
+        if (blockIdx.x == 0 && d < n_tiles) *reinterpret_cast<uint2 *>(ranges + 2 * (size_t)d) = make_uint2(start, start + total[k]);
+        base[d] = start;
+        start += total[k];
+        uint32_t run = 0;
+#pragma unroll
+        for (int w = 0; w < kTileSortWaves; ++w) {
+            const uint32_t c = counts[w][d];
+            counts[w][d] = (uint16_t)run;
+            run += c;
+        }
+    }
+    if (blockIdx.x >= n_blocks) return;                    // (no instances)
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSmallItems; ++r) {
+        const uint32_t i = blockIdx.x * kTileSortBlock + wave * (kWave * kSmallItems) + (uint32_t)r * kWave + lane;
+        if (i < n) vals_out[base[key[r]] + hist[(size_t)key[r] * n_blocks + blockIdx.x] + counts[wave][key[r]] + rank[r]] = val[r];
+    }
+}
+template <int BITS>
+static int sort_by_tile(const htgs_frame *f, uint32_t n_tiles)
+{
+    hipStream_t s = (hipStream_t)f->stream;
+    const InstanceCount count = instance_count(f);
+    const uint32_t n_blocks = (uint32_t)((f->n_instances + kTileSortBlock - 1) / kTileSortBlock);
+    uint32_t *hist = f->sort_tmp, *totals = hist + (size_t)n_blocks * n_tiles;
+    const uint16_t *keys = (const uint16_t *)f->keys[0];
+    hipLaunchKernelGGL(tile_histogram_kernel<BITS>, dim3(n_blocks), dim3(kTileSortThreads), 0, s, keys, hist, count, n_tiles);
+    hipLaunchKernelGGL(tile_row_scan_kernel, dim3((n_tiles + 3) / 4), dim3(256), 0, s, hist, totals, count, n_tiles);
+    hipLaunchKernelGGL(tile_scatter_kernel<BITS>, dim3(n_blocks), dim3(kTileSortThreads), 0, s, keys, f->vals[0], f->vals[1], hist, totals, f->ranges, count, n_tiles);
+    return check_launch("sort");
+}
+
+// htgs_sort_instances for htgs_run: where the one pass by tile applies it also writes the ranges (*ranged)
+int sort_instances_of(const htgs_frame *f, int *selector, bool *ranged)
+{
+    *ranged = false;
+    const int tile = tile_size(f->mode);
+    const uint64_t n_tiles = (uint64_t)div_up(f->width, tile) * div_up(f->height, tile);
+    if (htgs_frame_key_bytes(f) != 2 || n_tiles > kTileSortTiles || f->n_instances == 0 || f->n_instances > kTileSortMost || !f->ranges)
+        return htgs_sort_instances(f, selector);
+    *ranged = true;
+    *selector = 1;
+    return n_tiles <= 512 ? sort_by_tile<9>(f, (uint32_t)n_tiles) : n_tiles <= 1024 ? sort_by_tile<10>(f, (uint32_t)n_tiles)
+         : n_tiles <= 2048 ? sort_by_tile<11>(f, (uint32_t)n_tiles) : sort_by_tile<12>(f, (uint32_t)n_tiles);
 }
 
 }  // namespace htgs
@@ -383,7 +554,12 @@ extern "C" size_t htgs_sort_tmp_words(uint64_t n_instances)
 {
     const uint64_t n_blocks = (n_instances + kSortTileMin - 1) / kSortTileMin;
     // (256 digits x blocks of half the real size = 512 digits x real blocks: either digit width fits)
-    return (size_t)(256 * (n_blocks > 0 ? n_blocks : 1) + 2 * kMaxRadix);
+    uint64_t words = 256 * (n_blocks > 0 ? n_blocks : 1) + 2 * kMaxRadix;
+    // smaller blocks of the small sorts, the same way; rows of a count per tile where one pass by tile may be taken
+    const uint64_t n_small = n_instances < kSmallSort ? n_instances : kSmallSort, small = 512 * (n_small / (256 * kSmallItems) + 1) + 2 * kMaxRadix;
+    const uint64_t n_tile = n_instances < kTileSortMost ? n_instances : kTileSortMost, by_tile = kTileSortTiles * (n_tile / kTileSortBlock + 2);
+    words = words > small ? words : small;
+    return (size_t)(words > by_tile ? words : by_tile);
 }
 
 extern "C" int htgs_sort_instances(const htgs_frame *f, int *selector)
@@ -398,6 +574,12 @@ extern "C" int htgs_sort_instances(const htgs_frame *f, int *selector)
     if (((uintptr_t)f->keys[0] | (uintptr_t)f->keys[1]) & 15) return fail(HTGS_ERR_ARGUMENT, "htgs_sort_instances: keys must be 16-byte aligned");
     const int end_bit = htgs_frame_end_bit(f);
     hipStream_t s = (hipStream_t)f->stream;
+    if (f->n_instances <= kSmallSort)
+        switch (htgs_frame_key_bytes(f)) {
+            case 8: return sort_pairs<uint64_t, 512, 9, kSmallItems>(s, f->keys, f->vals, f->sort_tmp, instance_count(f), end_bit, selector, true);
+            case 4: return sort_pairs<uint32_t, 512, 8, kSmallItems>(s, f->keys, f->vals, f->sort_tmp, instance_count(f), end_bit, selector, true);
+            default: return sort_pairs<uint16_t, 512, 8, kSmallItems>(s, f->keys, f->vals, f->sort_tmp, instance_count(f), end_bit, selector, true);
+        }
     switch (htgs_frame_key_bytes(f)) {
         case 8: return sort_pairs<uint64_t>(s, f->keys, f->vals, f->sort_tmp, instance_count(f), end_bit, selector, true);
         case 4: return sort_pairs<uint32_t>(s, f->keys, f->vals, f->sort_tmp, instance_count(f), end_bit, selector, true);

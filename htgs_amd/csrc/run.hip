@@ -14,8 +14,6 @@
 
 namespace htgs {
 
-int scan_offsets_publish(const htgs_frame *f, unsigned long long *host_total, uint32_t tag);   // instances.hip
-
 // ---------------------------------------------------------------------------------------------
 // Words in coherent host memory that a frame's scan writes and the host waits for.  One per call that is under way: taken
 // from a free list and given back, a page of them at a time; the pages stay until the process ends.
@@ -90,6 +88,7 @@ struct Carver {
     }
 };
 
+constexpr uint64_t kUnorderedTiles = 4096;      // of a wave each; a quarter as many of four waves
 static uint64_t carve_front(htgs_frame *f, int what, void *base)
 {
     Carver c = { static_cast<unsigned char *>(base), 0 };
@@ -111,7 +110,8 @@ static uint64_t carve_front(htgs_frame *f, int what, void *base)
     f->ranges = c.take<uint32_t>(2 * n_tiles);
     // (the modes that walk all of a list)
     f->long_tiles = f->mode != HTGS_MODE_ALPHA_BLEND_GLOBAL_ORDERING ? c.take<uint32_t>(8 + 3 * n_tiles) : nullptr;
-    f->tile_order = c.take<uint32_t>(htgs_tile_order_words(f->mode, f->width, f->height));
+    // (a grid whose workgroups are all on the device at once is taken in any order)
+    f->tile_order = n_tiles > (tile == 8 ? kUnorderedTiles : kUnorderedTiles / 4) ? c.take<uint32_t>(htgs_tile_order_words(f->mode, f->width, f->height)) : nullptr;
     // GLOBAL_ORDERING without a backward pass, and the image-only fast path of the two modes with a sorted core
     const bool by_depth = !train && (f->mode == HTGS_MODE_ALPHA_BLEND_GLOBAL_ORDERING ||
                                      (what == HTGS_RUN_RENDER && f->fast_math && f->mode != HTGS_MODE_OIT_BLEND));
@@ -142,17 +142,17 @@ static uint64_t with_headroom(uint64_t expected)
     const uint64_t n = expected + expected / 8 + 4096;
     return n < kMostInstances ? n : kMostInstances;
 }
-// the most instances, up to `wanted`, whose scratch fits into `bytes`
-static uint64_t fitting(htgs_frame *f, uint64_t wanted, uint64_t bytes)
+// the most instances from `least` to with_headroom(least) whose scratch fits into `bytes`, 0 if not even `least` do
+static uint64_t fitting(htgs_frame *f, uint64_t least, uint64_t bytes)
 {
-    uint64_t n = wanted;
-    if (carve_back(f, n, nullptr) <= bytes) return n;
-    // (per instance: two keys, two values and the sort's share of a histogram row)
-    const uint64_t fixed = carve_back(f, 1, nullptr) + 4096, per16 = 32ull * (uint64_t)htgs_frame_key_bytes(f) + 128 + 4;
-    if (bytes <= fixed) return 0;
-    n = (bytes - fixed) * 16 / per16;
-    n = n < wanted ? n : wanted;
-    return carve_back(f, n, nullptr) <= bytes ? n : 0;
+    uint64_t lo = least, hi = with_headroom(least);
+    if (carve_back(f, hi, nullptr) <= bytes) return hi;
+    if (carve_back(f, lo, nullptr) > bytes) return 0;
+    for (int step = 0; step < 5; ++step) {                 // (lo fits, hi does not)
+        const uint64_t mid = lo + (hi - lo) / 2;
+        if (carve_back(f, mid, nullptr) <= bytes) lo = mid; else hi = mid;
+    }
+    return lo;
 }
 
 static int check_run(const htgs_frame *f, const htgs_workspace *w, const char *who)
@@ -165,7 +165,8 @@ static int check_run(const htgs_frame *f, const htgs_workspace *w, const char *w
     return HTGS_OK;
 }
 
-static int queue_front(const htgs_frame *f, const htgs_workspace *w, HostWord *word)
+// The first half.  starts: the second half follows at once (FrameStart); *fused as in scan_offsets_publish.
+static int queue_front(const htgs_frame *f, const htgs_workspace *w, HostWord *word, bool starts, bool *fused)
 {
     htgs_frame t = *f;
     if (w->what != HTGS_RUN_RENDER) t.scale_modifier = 1.0f;       // as htgs_forward_front, htgs_max_weights_front
@@ -174,14 +175,28 @@ static int queue_front(const htgs_frame *f, const htgs_workspace *w, HostWord *w
         t.active_sh_bases = 1;
         t.total_sh_bases = 0;
     }
-    const int rc = htgs_preprocess(&t);
-    return rc != HTGS_OK ? rc : scan_offsets_publish(&t, &word->value, word->tag);
+    FrameStart start = {};
+    if (starts) {
+        const int tile = tile_size(f->mode);
+        const uint32_t n_tiles = (uint32_t)div_up(f->width, tile) * (uint32_t)div_up(f->height, tile);
+        start.block_sums = f->scan_tmp;
+        start.clear[0] = f->ranges; start.clear_words[0] = 2 * n_tiles;
+        if (f->tile_order) {
+            start.clear[1] = f->tile_order + n_tiles;
+            start.clear_words[1] = (uint32_t)htgs_tile_order_words(f->mode, f->width, f->height) - n_tiles;
+        }
+        if (f->long_tiles) { start.clear[2] = f->long_tiles; start.clear_words[2] = 8; }
+    }
+    const int rc = preprocess_and_start(&t, start);
+    return rc != HTGS_OK ? rc : scan_offsets_publish(&t, &word->value, word->tag, starts, fused);
 }
-static int queue_back(htgs_frame *f, htgs_workspace *w)
+// The second half; cleared: with what FrameStart left, fused: with the scan.
+static int queue_back(htgs_frame *f, htgs_workspace *w, bool cleared, HostWord *fused)
 {
-    int rc = htgs_create_instances(f);
-    if (rc == HTGS_OK) rc = htgs_sort_instances(f, &w->selector);
-    if (rc == HTGS_OK) rc = htgs_extract_ranges(f, w->selector);
+    bool ranged = false;
+    int rc = fused ? create_instances_fused(f, &fused->value, fused->tag) : htgs_create_instances(f);
+    if (rc == HTGS_OK) rc = sort_instances_of(f, &w->selector, &ranged);
+    if (rc == HTGS_OK) rc = extract_ranges_of(f, w->selector, cleared, ranged);
     if (rc != HTGS_OK) return rc;
     switch (w->what) {
         case HTGS_RUN_RENDER: return htgs_blend(f, w->selector);
@@ -222,22 +237,18 @@ extern "C" int htgs_run(htgs_frame *f, htgs_workspace *w)
         return fail(HTGS_ERR_ARGUMENT, "htgs_run: the host waits for the number of instances, which a stream under capture never gives");
     HostWord *word = take_word();
     if (!word) return HTGS_ERR_HIP;
-    rc = queue_front(f, w, word);
-    if (rc != HTGS_OK) {
-        // (a kernel that was queued may still write the word: it is not used again)
-        return rc;
-    }
-    uint64_t queued_for = 0;
-    if (w->expected > 0 && w->back != nullptr) {
-        queued_for = fitting(f, with_headroom(w->expected), w->back_bytes);
-        if (queued_for >= w->expected) {
-            carve_back(f, queued_for, w->back);
-            f->n_instances = queued_for;
-            f->n_instances_live = f->n_instances_dev;
-            rc = queue_back(f, w);
-            f->n_instances_live = nullptr;
-            if (rc != HTGS_OK) return rc;
-        } else queued_for = 0;
+    const uint64_t queued_for = w->expected > 0 && w->back != nullptr ? fitting(f, w->expected, w->back_bytes) : 0;
+    bool fused = false;
+    // (after a failure a kernel that was queued may still write the word: it is not used again)
+    rc = queue_front(f, w, word, queued_for > 0, &fused);
+    if (rc != HTGS_OK) return rc;
+    if (queued_for > 0) {
+        carve_back(f, queued_for, w->back);
+        f->n_instances = queued_for;
+        f->n_instances_live = f->n_instances_dev;
+        rc = queue_back(f, w, true, fused ? word : nullptr);
+        f->n_instances_live = nullptr;
+        if (rc != HTGS_OK) return rc;
     }
     uint64_t n = 0;
     rc = wait_for_word(word, s, &n);
@@ -263,5 +274,5 @@ extern "C" int htgs_run_rest(htgs_frame *f, htgs_workspace *w)
         w->back_needed = carve_back(f, with_headroom(n), nullptr);
         return HTGS_WORKSPACE;
     }
-    return queue_back(f, w);
+    return queue_back(f, w, false, nullptr);
 }
