@@ -241,7 +241,8 @@ __device__ __forceinline__ void banked_quadrant_pixel(uint32_t lane, uint32_t &l
 
 // kCullPixels: a slot counts for a quadrant when the instance passes the cut-off -- with the walk's own arithmetic -- at
 // one of the pixels named by pixel_lanes (a wave-uniform mask over the lanes of the quadrant walk) that lie in it.
-enum { kCullNone = 0, kCullAlpha = 1, kCullCutoff = 2, kCullPixels = 3 };
+// kCullScaled: kCullAlpha for a least alpha of the walk's own, as opacity times cull_scale = the mode's least alpha over it.
+enum { kCullNone = 0, kCullAlpha = 1, kCullCutoff = 2, kCullPixels = 3, kCullScaled = 4 };
 
 // With QUADRANTS the result has one bit per 4x4 quadrant of the tile (tile_quadrant_hits) instead of one for the tile.
 // REC4: 16-byte words per record of prim (five; eight in training frames).
@@ -251,12 +252,12 @@ enum { kCullNone = 0, kCullAlpha = 1, kCullCutoff = 2, kCullPixels = 3 };
 template <int MODE, int N, bool DEPTH, int CULL = kCullNone, bool QUADRANTS = false, int REC4 = HTGS_PRIM_FLOATS / 4, bool UNIT = false, bool POS = false,
           bool GIVEN = false>
 __device__ __forceinline__ uint32_t tile_stage_load(TileStage<N> &st, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst,
-                                                    uint32_t fetch, uint32_t last, int slot, float cx, float cy, uint64_t pixel_lanes = 0, uint32_t given = 0);
+                                                    uint32_t fetch, uint32_t last, int slot, float cx, float cy, uint64_t pixel_lanes = 0, uint32_t given = 0, float cull_scale = 1.0f);
 
 // (PixelTerms is complete by the time the template is instantiated)
 template <int MODE, int N, bool DEPTH, int CULL, bool QUADRANTS, int REC4, bool UNIT, bool POS, bool GIVEN>
 __device__ __forceinline__ uint32_t tile_stage_load(TileStage<N> &st, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst,
-                                                    uint32_t fetch, uint32_t last, int slot, float cx, float cy, uint64_t pixel_lanes, uint32_t given)
+                                                    uint32_t fetch, uint32_t last, int slot, float cx, float cy, uint64_t pixel_lanes, uint32_t given, float cull_scale)
 {
     if (fetch >= last) return 0;
     const uint32_t g = GIVEN ? given : inst[fetch];
@@ -324,7 +325,7 @@ __device__ __forceinline__ uint32_t tile_stage_load(TileStage<N> &st, const floa
         return bits;
     }
     else if constexpr (QUADRANTS && ModeCfg<MODE>::tile == 16) return tile_quadrant_hits16<MODE>(n, d, CULL == kCullCutoff ? 1.0f : col.w);
-    else if constexpr (QUADRANTS) return tile_quadrant_hits<MODE>(n, d, CULL == kCullCutoff ? 1.0f : col.w);
+    else if constexpr (QUADRANTS) return tile_quadrant_hits<MODE>(n, d, CULL == kCullCutoff ? 1.0f : CULL == kCullScaled ? col.w * cull_scale : col.w);
     else return (uint32_t)!tile_misses<MODE>(n, d, CULL == kCullCutoff ? 1.0f : col.w);
 }
 
@@ -485,7 +486,8 @@ __device__ __forceinline__ void quadrant_list_walk(const QuadrantLists &ql, uint
 // entry is then there when the batch is staged, and the records' fetch does not wait for it).
 template <int MODE, bool DEPTH, int CULL, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, bool UNIT = false, bool POS = false, bool AHEAD = false, typename Turn>
 __device__ __forceinline__ void tile_list_walk(TileStageQ &st, QuadrantLists &ql, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst,
-                                               uint32_t first, uint32_t last, uint32_t lane, float cx, float cy, Turn &&turn, uint64_t pixel_lanes = 0)
+                                               uint32_t first, uint32_t last, uint32_t lane, float cx, float cy, Turn &&turn, uint64_t pixel_lanes = 0,
+                                               float cull_scale = 1.0f)
 {
     stage_dummy_init(st, lane);
     uint32_t listed = 0;
@@ -493,7 +495,7 @@ __device__ __forceinline__ void tile_list_walk(TileStageQ &st, QuadrantLists &ql
     for (uint32_t base = first; base < last; base += 64) {
         if (SOLO) __syncthreads(); else wave_lds_sync();
         const uint32_t bits = tile_stage_load<MODE, kStageSlots, DEPTH, CULL, true, REC4, UNIT, POS, AHEAD>(st, prim, inst, base + lane, last, lane + 1, cx, cy, pixel_lanes,
-                                                                                                           listed);
+                                                                                                           listed, cull_scale);
         if (AHEAD) listed = base + 64u + lane < last ? inst[base + 64u + lane] : 0u;
         const uint32_t n_turns = quadrant_lists_build(ql, bits, lane, st);
         if (SOLO) __syncthreads(); else wave_lds_sync();

@@ -101,8 +101,7 @@ static uint64_t carve_front(htgs_frame *f, int what, void *base)
     f->offsets = c.take<uint32_t>(n);
     f->bounds = nullptr;
     f->touch = c.take<uint32_t>(4 * n);
-    // (the tail's second walk of the weights takes fragments below the alpha threshold)
-    f->touch_cutoff_only = what == HTGS_RUN_MAX_WEIGHTS ? 1 : 0;
+    f->touch_cutoff_only = 0;
     f->prim = c.take<float>((uint64_t)f->prim_floats * n);
     f->clamp_info = train ? c.take<uint8_t>(3 * n) : nullptr;
     f->scan_tmp = c.take<uint32_t>(htgs_scan_tmp_words((int)n));
@@ -228,6 +227,9 @@ extern "C" int htgs_run(htgs_frame *f, htgs_workspace *w)
     w->n_instances = 0;
     w->front_needed = carve_front(f, w->what, w->front);
     if (w->front == nullptr || w->front_bytes < w->front_needed) return HTGS_WORKSPACE;
+    // (the tail's second walk of the weights takes fragments below the alpha threshold of 1/255; a tail's weight is at most
+    // one per unit of alpha, so a weight threshold above leaves none of those)
+    f->touch_cutoff_only = w->what == HTGS_RUN_MAX_WEIGHTS && !(w->weight_threshold > 0.004f) ? 1 : 0;
     hipStream_t s = (hipStream_t)f->stream;
     f->n_instances_live = nullptr;
     f->n_instances = 0;
