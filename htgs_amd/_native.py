@@ -51,6 +51,7 @@ class Frame(ctypes.Structure):
         ("ranges", ctypes.c_void_p),
         ("long_tiles", ctypes.c_void_p),
         ("long_list_threshold", ctypes.c_int32),
+        ("waves_per_tile", ctypes.c_int32),
         ("tile_order", ctypes.c_void_p),
         ("depth_order", ctypes.c_void_p),
         ("n_instances", ctypes.c_uint64),

@@ -444,7 +444,7 @@ __global__ void __launch_bounds__(64 * kBackwardWaves) __attribute__((amdgpu_wav
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
     const uint32_t *__restrict__ core_idx, const float4 *__restrict__ core_info, const float *__restrict__ tail_info,
     const float *__restrict__ grad_image, const float *__restrict__ VPM, float4 *__restrict__ grad_rows, float *__restrict__ helper_rows,
-    uint32_t width, uint32_t height, uint32_t grid_w, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ long_tiles, uint32_t long_threshold,
+    uint32_t width, uint32_t height, uint32_t grid_w, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ long_tiles, ListThreshold threshold,
     uint32_t part_floor)
 {
     __shared__ BackwardTileTerms<K, HELPER> lds;
@@ -452,6 +452,7 @@ __global__ void __launch_bounds__(64 * kBackwardWaves) __attribute__((amdgpu_wav
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
     if (first == last) return;               // nothing was drawn into this tile (whole workgroup)
     // a very long list is left to blend_tail_backward_long_kernel, in parts (no part leaves anything behind for the others)
+    const uint32_t long_threshold = threshold.get(long_tiles);
     if (long_tiles != nullptr && last - first > long_threshold) {
         // (parts of one threshold's length: nothing is merged afterwards, so the finer the parts the better they spread)
         if (threadIdx.x == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold / 4u, 0u, part_floor);
@@ -467,11 +468,12 @@ __global__ void __launch_bounds__(64 * kBackwardWaves) __attribute__((amdgpu_wav
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
     const uint32_t *__restrict__ core_idx, const float4 *__restrict__ core_info, const float *__restrict__ tail_info,
     const float *__restrict__ grad_image, const float *__restrict__ VPM, float4 *__restrict__ grad_rows, float *__restrict__ helper_rows,
-    uint32_t width, uint32_t height, uint32_t grid_w, const uint32_t *long_tiles, uint32_t long_threshold)
+    uint32_t width, uint32_t height, uint32_t grid_w, const uint32_t *long_tiles, ListThreshold threshold)
 {
     __shared__ BackwardTileTerms<K, HELPER> lds;
     __shared__ uint32_t s_next;
     if (long_tiles[0] == 0) return;                   // (the ordinary frame)
+    const uint32_t long_threshold = threshold.get(long_tiles);
     const uint32_t n_tiles = grid_w * ((height + 7u) / 8u);
     uint32_t round = 0;
     LongEntry e;
@@ -999,14 +1001,14 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
 template <int K, int MODE, bool HELPER>
 static void launch_tail_backward_kernels(const htgs_frame *f, int sel, uint32_t grid_w, uint32_t n_tiles)
 {
-    const uint32_t threshold = f->long_list_threshold > 0 ? (uint32_t)f->long_list_threshold : kLongListDefault;
+    const ListThreshold threshold = list_threshold(f);
     // the least length of a part of a long list: the frame's average list, so that the parts of all tiles fit the list of entries
     const uint64_t floor = (f->n_instances + n_tiles - 1) / n_tiles;
     hipLaunchKernelGGL((blend_tail_backward_moments_kernel<K, MODE, HELPER>), dim3(n_tiles), dim3(64 * kBackwardWaves), 0, (hipStream_t)f->stream,
                        f->ranges, f->vals[sel], (const float4 *)f->prim, f->core_idx, (const float4 *)f->core_info, f->tail_info, f->grad_image,
                        f->VPM, (float4 *)f->grad_rows, f->dens_helper, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->tile_order, f->long_tiles, threshold,
                        floor < 1u ? 1u : (uint32_t)floor);
-    if (may_have_long_lists(f, threshold))      // (four workgroups per compute unit; they find an empty list on ordinary frames)
+    if (may_have_long_lists(f))      // (four workgroups per compute unit; they find an empty list on ordinary frames)
         hipLaunchKernelGGL((blend_tail_backward_long_kernel<K, MODE, HELPER>), dim3(1024), dim3(64 * kBackwardWaves), 0, (hipStream_t)f->stream,
                            f->ranges, f->vals[sel], (const float4 *)f->prim, f->core_idx, (const float4 *)f->core_info, f->tail_info, f->grad_image,
                            f->VPM, (float4 *)f->grad_rows, f->dens_helper, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, threshold);

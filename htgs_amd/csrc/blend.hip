@@ -174,9 +174,9 @@ static PartFloor long_part_floor(const htgs_frame *f, int selector) { return Par
 template <int K, bool FAST>
 static void launch_hybrid(const htgs_frame *f, int selector, uint32_t grid_w, uint32_t n_tiles)
 {
-    const uint32_t threshold = f->long_list_threshold > 0 ? (uint32_t)f->long_list_threshold : kLongListDefault;
+    const ListThreshold threshold = list_threshold(f);
     // (the fast path packs a core entry's place in its list into 13 bits where no list of the launch can be longer)
-    if (f->long_tiles != nullptr && threshold <= kPackedListMost)
+    if (f->long_tiles != nullptr && most_threshold(f) <= kPackedListMost)
         hipLaunchKernelGGL((blend_hybrid_kernel<K, FAST, true>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
                            f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
@@ -184,7 +184,7 @@ static void launch_hybrid(const htgs_frame *f, int selector, uint32_t grid_w, ui
         hipLaunchKernelGGL((blend_hybrid_kernel<K, FAST>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
                            f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
-    if (may_have_long_lists(f, threshold))      // (one workgroup per compute unit; they find an empty list on ordinary frames)
+    if (may_have_long_lists(f))      // (one workgroup per compute unit; they find an empty list on ordinary frames)
         hipLaunchKernelGGL((blend_hybrid_long_kernel<K, FAST, HTGS_PRIM_FLOATS / 4, HybridImage>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0,
                            (hipStream_t)f->stream, f->ranges, f->vals[selector], (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w,
                            f->vals[selector ^ 1], threshold,
@@ -193,8 +193,8 @@ static void launch_hybrid(const htgs_frame *f, int selector, uint32_t grid_w, ui
 template <int K, bool FAST>
 static void launch_first_k(const htgs_frame *f, int selector, uint32_t grid_w, uint32_t n_tiles)
 {
-    const uint32_t threshold = f->long_list_threshold > 0 ? (uint32_t)f->long_list_threshold : kLongListDefault;
-    if (!FAST && f->long_tiles != nullptr && threshold <= kPackedListMost)
+    const ListThreshold threshold = list_threshold(f);
+    if (!FAST && f->long_tiles != nullptr && most_threshold(f) <= kPackedListMost)
         hipLaunchKernelGGL((blend_first_k_kernel<K, false, true>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
                            f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
@@ -202,7 +202,7 @@ static void launch_first_k(const htgs_frame *f, int selector, uint32_t grid_w, u
         hipLaunchKernelGGL((blend_first_k_kernel<K, FAST>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
                            f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
-    if (may_have_long_lists(f, threshold))
+    if (may_have_long_lists(f))
         hipLaunchKernelGGL((blend_first_k_long_kernel<K, FAST, HTGS_PRIM_FLOATS / 4, FirstKImage>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0,
                            (hipStream_t)f->stream, f->ranges, f->vals[selector], (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w,
                            f->vals[selector ^ 1], threshold,
@@ -242,11 +242,11 @@ static void launch_blend(const htgs_frame *f, int selector, uint32_t grid_w, uin
             break;
         default:
         {
-            const uint32_t threshold = f->long_list_threshold > 0 ? (uint32_t)f->long_list_threshold : kLongListDefault;
+            const ListThreshold threshold = list_threshold(f);
             hipLaunchKernelGGL(blend_oit_kernel<FAST>, dim3(n_tiles), dim3(64), 0, s, f->ranges, f->vals[selector], (const float4 *)f->prim,
                                f->image, depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw, f->long_tiles, threshold,
                                long_part_floor(f, selector), f->tile_order);
-            if (may_have_long_lists(f, threshold))
+            if (may_have_long_lists(f))
                 hipLaunchKernelGGL((blend_oit_long_kernel<FAST, HTGS_PRIM_FLOATS / 4, OitImage>), dim3(256), dim3(64 * kLongWaves), 0, s, f->ranges, f->vals[selector],
                                    (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->vals[selector ^ 1], threshold,
                                    OitImage{ f->image, depth, (uint32_t)f->width, (uint32_t)f->height, f->to_chw });
@@ -277,6 +277,7 @@ extern "C" int htgs_blend(const htgs_frame *f, int selector)
     const uint32_t n_tiles = grid_w * grid_h;
     // (an entry of the list of long tiles holds the tile in 20 bits; htgs_scan_offsets refuses larger grids as well)
     if ((uint64_t)grid_w * grid_h > (1ull << 20)) return fail(HTGS_ERR_ARGUMENT, "htgs_blend: more than 2^20 tiles");
+    if (blend_waves(f, selector, grid_w, n_tiles)) return check_launch("blend");
     if (f->fast_math) launch_blend<true>(f, selector, grid_w, n_tiles);
     else launch_blend<false>(f, selector, grid_w, n_tiles);
     return check_launch("blend");

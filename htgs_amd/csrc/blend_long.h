@@ -158,7 +158,7 @@ __device__ __forceinline__ void core_key_walk(CoreKey &carried, CoreKey (&core)[
 template <int K, bool FAST, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, bool AHEAD = false>
 __device__ __forceinline__ void hybrid_key_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                 uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy,
-                                                CoreKey (&core)[K], HybridTail &tail, float &tie, const KeyFormat &fmt)
+                                                CoreKey (&core)[K], HybridTail &tail, float &tie, const KeyFormat &fmt, uint32_t list_first)
 {
     constexpr int MODE = HTGS_MODE_HYBRID_BLEND;
     constexpr int N = kStageSlots;
@@ -181,7 +181,7 @@ __device__ __forceinline__ void hybrid_key_walk(TileStageQ &st, QuadrantLists &q
             // (the fast path's alpha is opacity * 2^t with the opacity held to 1 and t <= 0 up to the rounding of the staged
             // quadratic: held to 1 here, the fraction has no room for more; the exact path's is held to 1 when it is evaluated)
             if constexpr (FAST) p3 = p3 < 1.0f ? p3 : 1.0f;
-            const uint32_t low = key_pack(p3, float_to_bits(col.w) - first, fmt);
+            const uint32_t low = key_pack(p3, float_to_bits(col.w) - list_first, fmt);
             p3 = key_alpha(low, fmt);
             tail.c0 = __builtin_fmaf(p3, col.x, tail.c0);
             tail.c1 = __builtin_fmaf(p3, col.y, tail.c1);
@@ -302,7 +302,7 @@ __device__ __forceinline__ void hybrid_tile_by_keys(TileStageQ &st, QuadrantList
     }
     float tie = __FLT_MAX__;
     const KeyFormat fmt = key_format(last > first ? last - first : 1u);
-    hybrid_key_walk<K, FAST, true, REC4, true>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, core, tail, tie, fmt);
+    hybrid_key_walk<K, FAST, true, REC4, true>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, core, tail, tie, fmt, first);
     if constexpr (FAST) {
         if (!px.inside) return;
         key_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
@@ -327,14 +327,135 @@ __device__ __forceinline__ void hybrid_tile_by_keys(TileStageQ &st, QuadrantList
 }
 
 // ---------------------------------------------------------------------------------------------
+// Several waves share a list: what each has walked is merged pairwise, in list order.  Two sorted cores are merged without
+// insertions: the nearer of entry i of one and entry K - 1 - i of the other are the K nearest of both (what is farther
+// joins the tail), in an order that log2 K rounds of compare and exchange sort -- K = 16: 48 exchanges of 28 cycles (8 for
+// keys), where inserting sixteen entries one by one takes 9000 cycles.  Which entry of exactly equal depth stays is not the
+// reference's choice then: tie receives the least depth at which that can matter, as in the walks.
+// ---------------------------------------------------------------------------------------------
+// LDS of a workgroup whose waves walk shares and then hand them on, ROWS rows of 64 lanes a share: the merge buffers, one
+// per pair of waves, lie over the stages.
+template <int WAVES, uint32_t ROWS> constexpr size_t shared_walk_lds()
+{
+    constexpr size_t stages = WAVES * (sizeof(TileStageQ) + ((sizeof(QuadrantLists) + 15) & ~(size_t)15)), buffers = (WAVES / 2) * (size_t)ROWS * 64 * 4;
+    return stages > buffers ? stages : buffers;
+}
+__device__ __forceinline__ TileStageQ &wave_stage(unsigned char *lds, uint32_t wave) { return reinterpret_cast<TileStageQ *>(lds)[wave]; }
+template <int WAVES>
+__device__ __forceinline__ QuadrantLists &wave_lists(unsigned char *lds, uint32_t wave)
+{
+    return *reinterpret_cast<QuadrantLists *>(lds + WAVES * sizeof(TileStageQ) + wave * ((sizeof(QuadrantLists) + 15) & ~(size_t)15));
+}
+
+// sorts a bitonic sequence of K keys
+template <int K>
+__device__ __forceinline__ void sort_bitonic(CoreKey (&core)[K])
+{
+#pragma unroll
+    for (int half = K / 2; half > 0; half /= 2) {
+#pragma unroll
+        for (int i = 0; i < K; ++i)
+            if ((i & half) == 0) {
+                CoreKey lo, hi;
+                asm("v_min_f64 %0, %2, %3\n\tv_max_f64 %1, %2, %3" : "=&v"(lo), "=&v"(hi) : "v"(core[i]), "v"(core[i + half]));
+                core[i] = lo;
+                core[i + half] = hi;
+            }
+    }
+}
+// A core of keys joins the running one; pushed(key) is called with every entry that is in neither's K nearest.  tie: see above.
+template <int K, bool TIES, typename Pushed>
+__device__ __forceinline__ void merge_key_cores(const float *from, CoreKey (&core)[K], float &tie, const KeyFormat &fmt, Pushed &&pushed)
+{
+    float least = __FLT_MAX__;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const CoreKey other = __hiloint2double((int)float_to_bits(from[(2 * (K - 1 - i)) * 64]), (int)float_to_bits(from[(2 * (K - 1 - i) + 1) * 64]));
+        CoreKey lo, hi;
+        asm("v_min_f64 %0, %2, %3\n\tv_max_f64 %1, %2, %3" : "=&v"(lo), "=&v"(hi) : "v"(core[i]), "v"(other));
+        core[i] = lo;
+        if (TIES) least = key_low(hi) >> fmt.shift != 0u && key_depth(hi) < least ? key_depth(hi) : least;
+        pushed(hi);
+    }
+    sort_bitonic<K>(core);
+    if (TIES) tie = least == key_depth(core[K - 1]) && least < tie ? least : tie;
+}
+// the same for cores of three registers a slot (an empty slot has alpha 0 and the largest depth)
+template <typename IndexT>
+__device__ __forceinline__ void order_entries(float &d0, float &a0, IndexT &i0, float &d1, float &a1, IndexT &i1)
+{
+    const bool swap = d1 < d0;
+    const float d = swap ? d1 : d0, a = swap ? a1 : a0;
+    const IndexT x = swap ? i1 : i0;
+    d1 = swap ? d0 : d1; a1 = swap ? a0 : a1; i1 = swap ? i0 : i1;
+    d0 = d; a0 = a; i0 = x;
+}
+template <int K, bool TIES, typename IndexT, typename Pushed>
+__device__ __forceinline__ void merge_cores(const float *from, float (&cd)[K], float (&ca)[K], IndexT (&ci)[K], float &tie, Pushed &&pushed)
+{
+    float least = __FLT_MAX__;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        float d = from[(3 * (K - 1 - i)) * 64], a = from[(3 * (K - 1 - i) + 1) * 64];
+        IndexT x;
+        const float bits = from[(3 * (K - 1 - i) + 2) * 64];
+        __builtin_memcpy(&x, &bits, 4);
+        order_entries(cd[i], ca[i], ci[i], d, a, x);
+        if (TIES) least = a > 0.0f && d < least ? d : least;
+        pushed(d, a);
+        asm volatile("" : "+v"(cd[i]), "+v"(ca[i]), "+v"(ci[i]));
+    }
+#pragma unroll
+    for (int half = K / 2; half > 0; half /= 2) {
+#pragma unroll
+        for (int i = 0; i < K; ++i)
+            if ((i & half) == 0) order_entries(cd[i], ca[i], ci[i], cd[i + half], ca[i + half], ci[i + half]);
+    }
+    if (TIES) tie = least == cd[K - 1] && least < tie ? least : tie;
+}
+template <int K, typename IndexT>
+__device__ __forceinline__ void give_core(float *to, const float (&cd)[K], const float (&ca)[K], const IndexT (&ci)[K])
+{
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        float bits;
+        __builtin_memcpy(&bits, &ci[i], 4);
+        to[(3 * i) * 64] = cd[i]; to[(3 * i + 1) * 64] = ca[i]; to[(3 * i + 2) * 64] = bits;
+    }
+}
+template <int K>
+__device__ __forceinline__ void give_key_core(float *to, const CoreKey (&core)[K])
+{
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        to[(2 * i) * 64] = key_depth(core[i]);
+        to[(2 * i + 1) * 64] = bits_to_float(key_low(core[i]));
+    }
+}
+template <int ROW>
+__device__ __forceinline__ void give_tail(float *to, const HybridTail &t, float tie)
+{
+    to[ROW * 64] = t.T; to[(ROW + 1) * 64] = t.c0; to[(ROW + 2) * 64] = t.c1; to[(ROW + 3) * 64] = t.c2; to[(ROW + 4) * 64] = t.alpha; to[(ROW + 5) * 64] = t.depth;
+    to[(ROW + 6) * 64] = tie;
+}
+template <int ROW>
+__device__ __forceinline__ void take_tail(const float *from, HybridTail &t, float &tie)
+{
+    t.T *= from[ROW * 64];
+    t.c0 += from[(ROW + 1) * 64]; t.c1 += from[(ROW + 2) * 64]; t.c2 += from[(ROW + 3) * 64]; t.alpha += from[(ROW + 4) * 64]; t.depth += from[(ROW + 5) * 64];
+    const float other = from[(ROW + 6) * 64];
+    tie = other < tie ? other : tie;
+}
+// ---------------------------------------------------------------------------------------------
 // Tiles with very long lists (HYBRID_BLEND, ALPHA_BLEND_FIRST_K and OIT_BLEND, which walk all of a list): the kernel
 // with one wave per tile puts a tile whose list is longer than long_threshold on a list instead of walking it, if the
 // caller provided that list, and a second launch of workgroups of kLongWaves waves takes those: one wave walks one tile at some
 // 200 ns per instance once it has a SIMD to itself, so a single list of 300 000 instances would otherwise hold the
 // launch for 70 ms.
-// long_tiles[0] = entries on the list, [1..3] = work counters, [4] = workgroups done, [5] = unused -- all zeroed with the
-// ranges and again by the last workgroup of the second launch; [6], [7] = tiles with pixels settled by a second look / walked again in one piece (upper half: of these, after a second look that ran out of
-// room) since the ranges were made (for the tests); then 2 n_tiles words for the entries (tile | part << 20 |
+// long_tiles[0] = entries on the list, [1..3] = work counters, [4] = workgroups done, all zeroed with the
+// ranges and again by the last workgroup of the second launch; [5] = the threshold, if it was chosen on the device
+// (ListThreshold); [6], [7] = tiles with pixels settled by a second look / walked again in one piece (upper half: of these,
+// after a second look that ran out of room) since the ranges were made (for the tests); then 2 n_tiles words for the entries (tile | part << 20 |
 // (parts - 1) << 25: a tile is on the list once per part, and the parts beyond the first of all tiles together are held
 // to n_tiles, so the list cannot overflow) and n_tiles words that count a tile's finished parts.
 // ---------------------------------------------------------------------------------------------
@@ -343,7 +464,6 @@ constexpr int kLongWaves = 16;
 // waves of a workgroup of the K-buffer kernels: sixteen share a compute unit's registers at 128 a lane, which a K-buffer of
 // 32 slots (96 registers) leaves too few of; eight have 256
 template <int K> constexpr int long_waves() { return K > 16 ? 8 : kLongWaves; }
-constexpr uint32_t kLongListDefault = 8192;
 // What a workgroup leaves of its part of a list, in 64-lane rows: HYBRID's core, tail and the depth of a tie.
 template <int K> constexpr uint32_t long_part_words() { return (3u * K + 7u) * 64u; }
 // The parts a list of this length is walked in by separate workgroups (1: by one).  A part is at least four times the
@@ -394,7 +514,7 @@ __device__ __forceinline__ bool long_tile_take(const uint32_t *long_tiles, const
                 __threadfence();
                 if (atomicAdd(header + 4, 1u) == gridDim.x - 1) {
 #pragma unroll
-                    for (uint32_t k = 0; k < 6; ++k) header[k] = 0u;
+                    for (uint32_t k = 0; k < 5; ++k) header[k] = 0u;
                 }
             }
             return false;
@@ -437,13 +557,14 @@ template <int K, bool FAST, bool KEYS = false>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 5 : KEYS ? 4 : 3))) blend_hybrid_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
     float *__restrict__ image, float *__restrict__ depths, uint32_t width, uint32_t height, uint32_t grid_w, int chw, int median,
-    uint32_t *__restrict__ long_tiles, uint32_t long_threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order)
 {
     __shared__ TileStageQ st;
     __shared__ QuadrantLists ql;
     const uint32_t tile = block_tile(tile_order);
     const uint32_t lane = threadIdx.x;
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
+    const uint32_t long_threshold = threshold.get(long_tiles);
     if (long_tiles != nullptr && last - first > long_threshold) {
         if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, long_part_words<K>(), part_floor.get(gridDim.x));
         return;
@@ -565,25 +686,28 @@ template <int K, bool FAST>
 __device__ __forceinline__ void hybrid_merge(const float *from, uint32_t lane, float (&cd)[K], float (&ca)[K], float (&ci)[K], HybridTail &tail,
                                              float &tie)
 {
-    constexpr bool kTies = !FAST;
-    from += lane;
-#pragma unroll
-    for (int i = 0; i < K; ++i) {
-        float depth = from[(3 * i) * 64], alpha = from[(3 * i + 1) * 64], index = from[(3 * i + 2) * 64];
-        if (alpha > 0.0f) {                    // a filled slot
-            if (kTies && depth == cd[K - 1]) tie = depth < tie ? depth : tie;
-            if (depth < cd[K - 1]) {
-                core_exchange_walk<K>(depth, alpha, index, cd, ca, ci);
-                if (kTies && alpha > 0.0f && depth == cd[K - 1]) tie = depth < tie ? depth : tie;
-            }
-            hybrid_tail_add<FAST>(tail, depth, alpha);
-        }
+    merge_cores<K, !FAST>(from + lane, cd, ca, ci, tie, [&](float depth, float alpha) { hybrid_tail_add<FAST>(tail, depth, alpha); });
+    take_tail<3 * K>(from + lane, tail, tie);
+}
+template <int K>
+__device__ __forceinline__ void hybrid_put(float *to, uint32_t lane, const float (&cd)[K], const float (&ca)[K], const float (&ci)[K], const HybridTail &tail, float tie)
+{
+    give_core<K>(to + lane, cd, ca, ci);
+    give_tail<3 * K>(to + lane, tail, tie);
+}
+// The waves' shares, merged pairwise into the first wave's: put(buffer) by the wave that hands its share on, merge(buffer) by
+// the one that takes it (all threads of the workgroup call this).
+template <int WAVES, uint32_t ROWS, typename Put, typename Merge>
+__device__ __forceinline__ void merge_all_shares(unsigned char *lds, uint32_t wave, Put &&put, Merge &&merge)
+{
+    for (uint32_t step = 1; step < (uint32_t)WAVES; step *= 2) {
+        float *buffer = reinterpret_cast<float *>(lds) + (size_t)(wave / (2u * step)) * ROWS * 64u;
+        __syncthreads();
+        if ((wave & (2u * step - 1u)) == step) put(buffer);
+        __syncthreads();
+        if ((wave & (2u * step - 1u)) == 0u) merge(buffer);
     }
-    tail.T *= from[(3 * K) * 64];
-    tail.c0 += from[(3 * K + 1) * 64]; tail.c1 += from[(3 * K + 2) * 64]; tail.c2 += from[(3 * K + 3) * 64];
-    tail.alpha += from[(3 * K + 4) * 64]; tail.depth += from[(3 * K + 5) * 64];
-    const float other = from[(3 * K + 6) * 64];
-    tie = other < tie ? other : tie;
+    __syncthreads();                                       // (the stages are free again)
 }
 // The long tiles: a workgroup of kLongWaves waves takes a tile, every wave walks a contiguous share of the list (whole
 // batches of 64) into a core and a tail of its own, and the shares are then merged into the first wave's, in list
@@ -596,12 +720,11 @@ __device__ __forceinline__ void hybrid_merge(const float *from, uint32_t lane, f
 template <int K, bool FAST, int REC4, typename Finish>
 __global__ void __launch_bounds__(64 * long_waves<K>()) blend_hybrid_long_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, const uint32_t *long_tiles,
-    uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ shortlist, uint32_t long_threshold, const Finish finish)
+    uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ shortlist, ListThreshold threshold, const Finish finish)
 {
     constexpr int kWaves = long_waves<K>();
-    __shared__ TileStageQ st[kWaves];
-    __shared__ QuadrantLists ql[kWaves];
-    __shared__ float s_merge[3 * K + 7][64];          // one wave's core, tail and least depth of a tie, lane-minor
+    constexpr uint32_t kRows = 3 * K + 7;             // a wave's core, tail and least depth of a tie
+    __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<kWaves, kRows>()];
     __shared__ uint32_t s_next;
     __shared__ uint32_t s_redo[2];                    // the pixels (lanes) to walk again
     __shared__ uint32_t s_short[kWaves];          // how many instances of each share reach one of them
@@ -610,6 +733,7 @@ __global__ void __launch_bounds__(64 * long_waves<K>()) blend_hybrid_long_kernel
     __shared__ float s_sums[kWaves][kAgainPixels][6], s_tails[64][6];   // tails of the pixels looked at again: per wave, whole
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     if (long_tiles[0] == 0) return;                   // (the ordinary frame)
+    const uint32_t long_threshold = threshold.get(long_tiles);
     const uint32_t n_tiles = grid_w * ((height + 7u) / 8u);
     uint32_t round = 0;
     LongEntry entry;
@@ -629,31 +753,16 @@ __global__ void __launch_bounds__(64 * long_waves<K>()) blend_hybrid_long_kernel
         float cd[K], ca[K], ci[K];
         hybrid_core_init<K>(cd, ca, ci);
         float tie = __FLT_MAX__;                        // least depth at which two fragments of equal depth met at the end of a core
-        hybrid_walk<K, FAST, false, kTies, false, REC4>(st[wave], ql[wave], inst, prim, seg_first, seg_last, lane, px.pt, px.cx, px.cy, cd, ca, ci, tail, &tie);
-        for (uint32_t s = 1; s < (uint32_t)kWaves; ++s) {
-            __syncthreads();                               // the buffer is free
-            if (wave == s) {
-#pragma unroll
-                for (int i = 0; i < K; ++i) { s_merge[3 * i][lane] = cd[i]; s_merge[3 * i + 1][lane] = ca[i]; s_merge[3 * i + 2][lane] = ci[i]; }
-                s_merge[3 * K][lane] = tail.T; s_merge[3 * K + 1][lane] = tail.c0; s_merge[3 * K + 2][lane] = tail.c1;
-                s_merge[3 * K + 3][lane] = tail.c2; s_merge[3 * K + 4][lane] = tail.alpha; s_merge[3 * K + 5][lane] = tail.depth;
-                s_merge[3 * K + 6][lane] = tie;
-            }
-            __syncthreads();
-            if (wave == 0) hybrid_merge<K, FAST>(&s_merge[0][0], lane, cd, ca, ci, tail, tie);
-        }
+        hybrid_walk<K, FAST, false, kTies, false, REC4>(wave_stage(lds, wave), wave_lists<kWaves>(lds, wave), inst, prim, seg_first, seg_last, lane, px.pt, px.cx, px.cy, cd, ca, ci, tail, &tie);
+        merge_all_shares<kWaves, kRows>(lds, wave, [&](float *to) { hybrid_put<K>(to, lane, cd, ca, ci, tail, tie); },
+                                        [&](const float *from) { hybrid_merge<K, FAST>(from, lane, cd, ca, ci, tail, tie); });
         if (parts > 1u) {
             // One of several parts: what it came to goes to the tile's stretch of the spare value buffer (which is as long as the
             // list and unused until pixels are walked again), and the workgroup that finds the other parts there already
             // merges them all, in list order, and goes on with the whole tile.
             float *const left = reinterpret_cast<float *>(shortlist + tile_first);
             if (wave == 0) {
-                float *mine = left + (size_t)part * long_part_words<K>() + lane;
-#pragma unroll
-                for (int i = 0; i < K; ++i) { mine[(3 * i) * 64] = cd[i]; mine[(3 * i + 1) * 64] = ca[i]; mine[(3 * i + 2) * 64] = ci[i]; }
-                mine[(3 * K) * 64] = tail.T; mine[(3 * K + 1) * 64] = tail.c0; mine[(3 * K + 2) * 64] = tail.c1;
-                mine[(3 * K + 3) * 64] = tail.c2; mine[(3 * K + 4) * 64] = tail.alpha; mine[(3 * K + 5) * 64] = tail.depth;
-                mine[(3 * K + 6) * 64] = tie;
+                hybrid_put<K>(left + (size_t)part * long_part_words<K>(), lane, cd, ca, ci, tail, tie);
                 __threadfence();
             }
             if (!long_part_done(long_tiles, n_tiles, entry, &s_whole)) continue;
@@ -679,7 +788,9 @@ __global__ void __launch_bounds__(64 * long_waves<K>()) blend_hybrid_long_kernel
             // shortlist, in list order), since the walk of one wave alone is bound by the latency of staging.
             bool redo = false;
             if (wave == 0) {
-                redo = tie <= cd[K - 1];
+                // (nothing was pushed out of a core that is not full; with a threshold of the caller's own such pixels get the
+                // second look all the same, which is how small scenes reach it)
+                redo = tie <= cd[K - 1] && (tie < __FLT_MAX__ || threshold.fixed != 0u);
 #pragma unroll
                 for (int i = 0; i + 1 < K; ++i) redo = redo || (ca[i + 1] > 0.0f && cd[i] == cd[i + 1]);
                 const uint64_t lanes = __ballot(redo);
@@ -701,7 +812,7 @@ __global__ void __launch_bounds__(64 * long_waves<K>()) blend_hybrid_long_kernel
                     }
                     __syncthreads();
                     const uint32_t listed = pixels_again<HTGS_MODE_HYBRID_BLEND, false, REC4>(
-                        reinterpret_cast<TileStage<64> &>(st[wave]), inst, prim, seg_first, seg_last, lane, px.cx, px.cy, redo_lanes, s_last_depth, s_sums[wave], shortlist + seg_first,
+                        reinterpret_cast<TileStage<64> &>(wave_stage(lds, wave)), inst, prim, seg_first, seg_last, lane, px.cx, px.cy, redo_lanes, s_last_depth, s_sums[wave], shortlist + seg_first,
                         (seg_last - seg_first) / 4u, [&](const uint32_t (&pixel)[kAgainPixels]) {
                             __syncthreads();
                             if (wave == 0 && lane < (uint32_t)kAgainPixels) {      // the waves' sums of a pixel, in list order
@@ -755,7 +866,7 @@ __global__ void __launch_bounds__(64 * long_waves<K>()) blend_hybrid_long_kernel
                     uint32_t kept = 0;
                     for (uint32_t base = seg_first; base < seg_last; base += 64) {
                         const uint32_t fetch = base + lane;
-                        const bool reaches = tile_stage_load<HTGS_MODE_HYBRID_BLEND, 64, true, kCullPixels, true, REC4>(reinterpret_cast<TileStage<64> &>(st[wave]), prim, inst, fetch, seg_last, lane,
+                        const bool reaches = tile_stage_load<HTGS_MODE_HYBRID_BLEND, 64, true, kCullPixels, true, REC4>(reinterpret_cast<TileStage<64> &>(wave_stage(lds, wave)), prim, inst, fetch, seg_last, lane,
                                                                                                                px.cx, px.cy, redo_lanes) != 0;
                         const uint64_t keep = __ballot(reaches);
                         if (reaches) shortlist[seg_first + kept + (uint32_t)__popcll(keep & ((1ull << lane) - 1ull))] = inst[fetch];
@@ -772,11 +883,11 @@ __global__ void __launch_bounds__(64 * long_waves<K>()) blend_hybrid_long_kernel
                     if (shortlist != nullptr) {
                         for (uint32_t s = 0; s < (uint32_t)kWaves; ++s) {
                             const uint32_t from = first + 64u * (uint32_t)((uint64_t)n_batches * s / kWaves);
-                            hybrid_walk<K, FAST, false, false, true, REC4>(st[0], ql[0], shortlist, prim, from, from + s_short[s], lane, px.pt, px.cx, px.cy, cd, ca, ci,
+                            hybrid_walk<K, FAST, false, false, true, REC4>(wave_stage(lds, 0), wave_lists<kWaves>(lds, 0), shortlist, prim, from, from + s_short[s], lane, px.pt, px.cx, px.cy, cd, ca, ci,
                                                                      tail, nullptr, redo_lanes);
                         }
                     } else {
-                        hybrid_walk<K, FAST, false, false, true, REC4>(st[0], ql[0], inst, prim, first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, tail, nullptr, redo_lanes);
+                        hybrid_walk<K, FAST, false, false, true, REC4>(wave_stage(lds, 0), wave_lists<kWaves>(lds, 0), inst, prim, first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, tail, nullptr, redo_lanes);
                     }
                     if (px.inside && redo) finish(prim, tile, px, cd, ca, ci, tail);
                 }
@@ -828,7 +939,7 @@ __device__ __forceinline__ void first_k_walk(TileStageQ &st, QuadrantLists &ql, 
 template <int K, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4>
 __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                  uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy,
-                                                 CoreKey (&core)[K], float &tie, const KeyFormat &fmt)
+                                                 CoreKey (&core)[K], float &tie, const KeyFormat &fmt, uint32_t list_first)
 {
     constexpr int MODE = HTGS_MODE_ALPHA_BLEND_FIRST_K;
     constexpr int N = kStageSlots;
@@ -839,7 +950,7 @@ __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &
         float depth = tile_frag_depth<N>(addr, pt, f);
         if (!(in_reach && depth < key_depth(core[K - 1]))) return;          // depth test before the exponential (:151)
         if (!tile_frag_alpha<MODE, false>(stage_opacity<N>(addr), f)) return;
-        CoreKey carried = make_key(depth, key_pack(f.alpha, stage_index<N>(addr) - first, fmt));      // (the slot's last word is the place in the list)
+        CoreKey carried = make_key(depth, key_pack(f.alpha, stage_index<N>(addr) - list_first, fmt));      // (the slot's last word is the place in the list)
         core_key_walk<K>(carried, core);
         depth = key_depth(carried);
         tie = key_low(carried) >> fmt.shift != 0u && depth == key_depth(core[K - 1]) && depth < tie ? depth : tie;
@@ -902,7 +1013,7 @@ template <int K, bool FAST, bool KEYS = false>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 5 : 2))) blend_first_k_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
     float *__restrict__ image, float *__restrict__ depths, uint32_t width, uint32_t height, uint32_t grid_w, int chw, int median,
-    uint32_t *__restrict__ long_tiles, uint32_t long_threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order)
 {
     static_assert(!(KEYS && FAST), "the keys of this mode are for the exact path");
     __shared__ TileStageQ st;
@@ -910,6 +1021,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
     const uint32_t tile = block_tile(tile_order);
     const uint32_t lane = threadIdx.x;
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
+    const uint32_t long_threshold = threshold.get(long_tiles);
     if (long_tiles != nullptr && last - first > long_threshold) {
         if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, first_k_part_words<K>(), part_floor.get(gridDim.x));
         return;
@@ -926,7 +1038,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
         }
         float tie = __FLT_MAX__;
         const KeyFormat fmt = key_format(last > first ? last - first : 1u);
-        first_k_key_walk<K, true>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, core, tie, fmt);
+        first_k_key_walk<K, true>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, core, tie, fmt, first);
         const bool again = px.inside && ((tie < __FLT_MAX__ && tie <= key_depth(core[K - 1])) || key_core_tied<K>(core, fmt));
         const uint64_t again_lanes = __ballot(again);
         first_k_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
@@ -951,33 +1063,18 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
 
 // A core and a tie depth (3K + 1 rows of 64 lanes at from[]) join the running ones: they cover the stretch of the list
 // that follows.
-template <int K, bool FAST>
+template <int K>
 __device__ __forceinline__ void first_k_merge(const float *from, uint32_t lane, float (&cd)[K], float (&ca)[K], uint32_t (&ci)[K], float &tie)
 {
-    constexpr bool kTies = true;
-    from += lane;
-#pragma unroll
-    for (int i = 0; i < K; ++i) {
-        float depth = from[(3 * i) * 64], alpha = from[(3 * i + 1) * 64];
-        uint32_t index = float_to_bits(from[(3 * i + 2) * 64]);
-        if (alpha > 0.0f) {                    // a filled slot
-            if (kTies && depth == cd[K - 1]) tie = depth < tie ? depth : tie;
-            if (depth < cd[K - 1]) {
-                core_exchange_walk<K>(depth, alpha, index, cd, ca, ci);
-                if (kTies && alpha > 0.0f && depth == cd[K - 1]) tie = depth < tie ? depth : tie;
-            }
-        }
-    }
-    const float other = from[(3 * K) * 64];
+    merge_cores<K, true>(from + lane, cd, ca, ci, tie, [](float, float) {});
+    const float other = from[(3 * K) * 64 + lane];
     tie = other < tie ? other : tie;
 }
 template <int K>
 __device__ __forceinline__ void first_k_put(float *to, uint32_t lane, const float (&cd)[K], const float (&ca)[K], const uint32_t (&ci)[K], float tie)
 {
-    to += lane;
-#pragma unroll
-    for (int i = 0; i < K; ++i) { to[(3 * i) * 64] = cd[i]; to[(3 * i + 1) * 64] = ca[i]; to[(3 * i + 2) * 64] = bits_to_float(ci[i]); }
-    to[(3 * K) * 64] = tie;
+    give_core<K>(to + lane, cd, ca, ci);
+    to[(3 * K) * 64 + lane] = tie;
 }
 
 // The tiles with very long lists, as in blend_hybrid_long_kernel: every wave of the workgroup walks a share of the list
@@ -990,16 +1087,16 @@ __device__ __forceinline__ void first_k_put(float *to, uint32_t lane, const floa
 template <int K, bool FAST, int REC4, typename Finish>
 __global__ void __launch_bounds__(64 * long_waves<K>()) blend_first_k_long_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, const uint32_t *long_tiles,
-    uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ spare, uint32_t long_threshold, const Finish finish)
+    uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ spare, ListThreshold threshold, const Finish finish)
 {
     constexpr int kWaves = long_waves<K>();
-    __shared__ TileStageQ st[kWaves];
-    __shared__ QuadrantLists ql[kWaves];
-    __shared__ float s_merge[3 * K + 1][64];
+    constexpr uint32_t kRows = 3 * K + 1;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<kWaves, kRows>()];
     __shared__ uint32_t s_next, s_whole, s_redo[2], s_listed[kWaves];
     __shared__ float s_last_depth[64];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     if (long_tiles[0] == 0) return;                   // (the ordinary frame)
+    const uint32_t long_threshold = threshold.get(long_tiles);
     const uint32_t n_tiles = grid_w * ((height + 7u) / 8u);
     constexpr bool kTies = true;                      // (the fast variant too: a tie decides which fragment a pixel shows)
     uint32_t round = 0;
@@ -1016,13 +1113,9 @@ __global__ void __launch_bounds__(64 * long_waves<K>()) blend_first_k_long_kerne
         uint32_t ci[K];
         first_k_core_init<K>(cd, ca, ci);
         float tie = __FLT_MAX__;
-        first_k_walk<K, FAST, false, kTies, REC4>(st[wave], ql[wave], inst, prim, share_first, share_last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie);
-        for (uint32_t s = 1; s < (uint32_t)kWaves; ++s) {
-            __syncthreads();                               // the buffer is free
-            if (wave == s) first_k_put<K>(&s_merge[0][0], lane, cd, ca, ci, tie);
-            __syncthreads();
-            if (wave == 0) first_k_merge<K, FAST>(&s_merge[0][0], lane, cd, ca, ci, tie);
-        }
+        first_k_walk<K, FAST, false, kTies, REC4>(wave_stage(lds, wave), wave_lists<kWaves>(lds, wave), inst, prim, share_first, share_last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie);
+        merge_all_shares<kWaves, kRows>(lds, wave, [&](float *to) { first_k_put<K>(to, lane, cd, ca, ci, tie); },
+                                        [&](const float *from) { first_k_merge<K>(from, lane, cd, ca, ci, tie); });
         if (e.parts > 1u) {
             float *const left = reinterpret_cast<float *>(spare + e.tile_first);
             if (wave == 0) {
@@ -1035,7 +1128,7 @@ __global__ void __launch_bounds__(64 * long_waves<K>()) blend_first_k_long_kerne
                 first_k_core_init<K>(cd, ca, ci);
                 tie = __FLT_MAX__;
                 for (uint32_t other = 0; other < e.parts; ++other)
-                    first_k_merge<K, FAST>(left + (size_t)other * first_k_part_words<K>(), lane, cd, ca, ci, tie);
+                    first_k_merge<K>(left + (size_t)other * first_k_part_words<K>(), lane, cd, ca, ci, tie);
             }
             long_wave_share(e.tile_first, e.tile_last, wave, share_first, share_last, kWaves);
             __syncthreads();                               // (the parts are read before the second look overwrites them)
@@ -1043,7 +1136,7 @@ __global__ void __launch_bounds__(64 * long_waves<K>()) blend_first_k_long_kerne
         if (kTies) {
             bool redo = false;
             if (wave == 0) {
-                redo = tie <= cd[K - 1];
+                redo = tie <= cd[K - 1] && (tie < __FLT_MAX__ || threshold.fixed != 0u);      // (as in blend_hybrid_long_kernel)
 #pragma unroll
                 for (int i = 0; i + 1 < K; ++i) redo = redo || (ca[i + 1] > 0.0f && cd[i] == cd[i + 1]);
                 const uint64_t lanes = __ballot(redo);
@@ -1058,7 +1151,7 @@ __global__ void __launch_bounds__(64 * long_waves<K>()) blend_first_k_long_kerne
                 if (spare != nullptr && __popcll(redo_lanes) <= kAgainMost) {
                     looked = true;
                     const uint32_t listed = pixels_again<HTGS_MODE_ALPHA_BLEND_FIRST_K, FAST, REC4>(
-                        reinterpret_cast<TileStage<64> &>(st[wave]), inst, prim, share_first, share_last, lane, px.cx, px.cy, redo_lanes, s_last_depth, nullptr, spare + share_first,
+                        reinterpret_cast<TileStage<64> &>(wave_stage(lds, wave)), inst, prim, share_first, share_last, lane, px.cx, px.cy, redo_lanes, s_last_depth, nullptr, spare + share_first,
                         (share_last - share_first) / 4u, [](const uint32_t (&)[kAgainPixels]) {});
                     if (lane == 0) s_listed[wave] = listed;
                     __syncthreads();
@@ -1080,7 +1173,7 @@ __global__ void __launch_bounds__(64 * long_waves<K>()) blend_first_k_long_kerne
                             }
                         }
                     } else {
-                        first_k_walk<K, FAST, false, false, REC4>(st[0], ql[0], inst, prim, e.tile_first, e.tile_last, lane, px.pt, px.cx, px.cy, cd, ca, ci);
+                        first_k_walk<K, FAST, false, false, REC4>(wave_stage(lds, 0), wave_lists<kWaves>(lds, 0), inst, prim, e.tile_first, e.tile_last, lane, px.pt, px.cx, px.cy, cd, ca, ci);
                     }
                     if (px.inside && redo) finish(prim, e.tile, px, cd, ca, ci);
                 }
@@ -1152,13 +1245,14 @@ template <bool FAST>
 __global__ void __launch_bounds__(64) blend_oit_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
     float *__restrict__ image, float *__restrict__ depths, uint32_t width, uint32_t height, uint32_t grid_w, int chw,
-    uint32_t *__restrict__ long_tiles, uint32_t long_threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order)
 {
     __shared__ TileStageQ st;
     __shared__ QuadrantLists ql;
     const uint32_t tile = block_tile(tile_order);
     const uint32_t lane = threadIdx.x;
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
+    const uint32_t long_threshold = threshold.get(long_tiles);
     if (long_tiles != nullptr && last - first > long_threshold) {
         if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, kOitPartWords, part_floor.get(gridDim.x));
         return;
@@ -1178,7 +1272,7 @@ __global__ void __launch_bounds__(64) blend_oit_kernel(
 template <bool FAST, int REC4, typename Finish, bool DEPTH = !FAST>
 __global__ void __launch_bounds__(64 * kLongWaves) blend_oit_long_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, const uint32_t *long_tiles,
-    uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ left, uint32_t long_threshold, const Finish finish)
+    uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ left, ListThreshold threshold, const Finish finish)
 {
     __shared__ TileStageQ st[kLongWaves];
     __shared__ QuadrantLists ql[kLongWaves];
@@ -1186,6 +1280,7 @@ __global__ void __launch_bounds__(64 * kLongWaves) blend_oit_long_kernel(
     __shared__ uint32_t s_next, s_whole;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     if (long_tiles[0] == 0) return;                   // (the ordinary frame)
+    const uint32_t long_threshold = threshold.get(long_tiles);
     const uint32_t n_tiles = grid_w * ((height + 7u) / 8u);
     uint32_t round = 0;
     LongEntry entry;

@@ -151,8 +151,8 @@ struct PartFloor {
 constexpr int kCountBlock = 256;                 // Gaussians per block sum
 struct FrameStart {
     uint32_t *block_sums;                        // [ceil(N / kCountBlock)] or nullptr
-    uint32_t *clear[3];                          // ranges, order bins, long_tiles header
-    uint32_t clear_words[3];
+    uint32_t *clear[4];                          // ranges, order bins, long_tiles header and the bins of its threshold
+    uint32_t clear_words[4];
 };
 int preprocess_and_start(const htgs_frame *f, const FrameStart &start);                 // preprocess.hip
 // The scan for htgs_run, which also writes tag << 32 | total to host memory.  with_sums: scan_tmp holds FrameStart's sums.
@@ -165,9 +165,46 @@ int sort_instances_of(const htgs_frame *f, int *selector, bool *ranged);        
 // words of scan_tmp for N Gaussians' block sums
 inline size_t block_sum_words(int n) { return (size_t)div_up(n > 0 ? n : 1, kCountBlock); }
 
-// Whether a list of the frame can be longer than `threshold` (a Gaussian is in a tile's list once): otherwise the kernels for
-// such lists, which would find nothing to do, are not launched.
-inline bool may_have_long_lists(const htgs_frame *f, uint32_t threshold) { return f->long_tiles != nullptr && (uint32_t)f->n_primitives > threshold; }
+// The length beyond which a list is shared between the waves and workgroups of the kernels for long lists.  One wave walks
+// such a list while the launch ends, so what a list may be long depends on the rest of the frame: a launch lasts some
+// (instances / waves that the device holds) turns per wave anyway, and a list of no more than that costs nothing.  The tile
+// order's stage knows the lists' lengths and leaves the longest that is within kThresholdShare times that, over the lists up
+// to it, in long_tiles[kChosenThreshold] (choose_threshold in instances.hip); without it the average of all lists is taken.
+// With the fixed threshold of 8192 the training pass of 600 k Gaussians of the stress scene at 1026x792, K = 32, took 3.0 ms
+// forward and 2.8 back, with 768 it takes 1.0 and 1.1; 6 M at 1600x1066 (chosen: 4096) 5.8 -> 4.7 ms.
+constexpr uint32_t kLongListDefault = 8192, kLeastThreshold = 512, kChosenThreshold = 5;
+constexpr float kThresholdShare = 1.5f, kWavesHeld = 5120.0f;         // (256 compute units, twenty waves each)
+struct ListThreshold {
+    uint32_t fixed;                        // 0: chosen on the device
+    InstanceCount count;
+    uint32_t waves;                        // per tile
+    __device__ __forceinline__ uint32_t get(const uint32_t *long_tiles) const
+    {
+        if (fixed != 0u || long_tiles == nullptr) return fixed;
+        const uint32_t chosen = long_tiles[kChosenThreshold];
+        if (chosen != 0u) return chosen;
+        const float t = kThresholdShare / kWavesHeld * (float)waves * (float)count.get();
+        return t < 2.0f * kLeastThreshold ? 2u * kLeastThreshold : t < (float)kLongListDefault ? (uint32_t)t : kLongListDefault;
+    }
+};
+inline bool chooses_threshold(const htgs_frame *f) { return f->long_list_threshold < 0 && f->long_tiles != nullptr; }
+inline ListThreshold list_threshold(const htgs_frame *f)
+{
+    const uint32_t fixed = f->long_list_threshold > 0 ? (uint32_t)f->long_list_threshold : chooses_threshold(f) ? 0u : kLongListDefault;
+    return ListThreshold{ fixed, instance_count(f), f->waves_per_tile > 1 ? (uint32_t)f->waves_per_tile : 1u };
+}
+// the longest list that the kernels with one workgroup per tile can meet
+inline uint32_t most_threshold(const htgs_frame *f) { return chooses_threshold(f) || f->long_list_threshold == 0 ? kLongListDefault : (uint32_t)f->long_list_threshold; }
+// Whether a list of the frame can be longer than the threshold (a Gaussian is in a tile's list once): otherwise the kernels
+// for such lists, which would find nothing to do, are not launched.
+inline bool may_have_long_lists(const htgs_frame *f)
+{
+    return f->long_tiles != nullptr && (uint32_t)f->n_primitives > (chooses_threshold(f) ? kLeastThreshold : most_threshold(f));
+}
+
+// Several waves walk a tile's list (blend_waves.h); false: the launch is left to the kernels with one
+bool blend_waves(const htgs_frame *f, int selector, uint32_t grid_w, uint32_t n_tiles);                 // blend_waves.hip
+bool blend_forward_waves(const htgs_frame *f, int selector, uint32_t grid_w, uint32_t n_tiles);         // blend_forward_waves.hip
 
 // host side error reporting (api.hip)
 int fail(int code, const char *fmt, ...);

@@ -409,12 +409,13 @@ __global__ void __launch_bounds__(256) extract_ranges_kernel(const KeyT *__restr
 // zeroes p[0, n) and, if given, the eight words at `also` and the kOrderWords words at `also_order`
 constexpr uint32_t kOrderBuckets = 132;                   // (130 in use)
 constexpr uint32_t kOrderWords = 2 * kOrderBuckets;       // bin totals, bin cursors
-__global__ void __launch_bounds__(256) fill_zero_kernel(uint32_t *p, size_t n, uint32_t *also, uint32_t *also_order)
+__global__ void __launch_bounds__(256) fill_zero_kernel(uint32_t *p, size_t n, uint32_t *also, uint32_t *also_order, uint32_t *also_bins)
 {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i < n) p[i] = 0;
     if (i < 8 && also) also[i] = 0;
     if (i < kOrderWords && also_order) also_order[i] = 0;
+    if (i < kOrderBuckets && also_bins) also_bins[i] = 0;
 }
 
 // The order in which the blend kernels take the tiles: longest lists first, in groups of neighbours.  One workgroup walks
@@ -471,23 +472,60 @@ __device__ __forceinline__ uint32_t order_place(uint32_t place, uint32_t t, uint
     const uint32_t interleaved = n_groups / kOrderDies * kOrderDies;
     return place < interleaved ? kOrderDies * (kOrderGroup * (place / kOrderDies) + t) + place % kOrderDies : kOrderGroup * place + t;
 }
-__global__ void __launch_bounds__(256) tile_order_count_kernel(const uint32_t *__restrict__ ranges, uint32_t *__restrict__ order, uint32_t grid_w,
-                                                               uint32_t grid_h)
+// ListThreshold: the lists by length, in the bins of the order (s_lists[b]: lists in bin b; 256 threads or more).  The launch
+// over the lists up to a bin's upper end is as long as their instances over the waves that the device holds; the largest
+// end that is within kThresholdShare times that is the threshold.
+__device__ __forceinline__ uint32_t bin_end(uint32_t bucket)           // the longest list of a bin (1 .. 128)
 {
-    __shared__ uint32_t count[kOrderBuckets];
-    if (threadIdx.x < kOrderBuckets) count[threadIdx.x] = 0;
+    const uint32_t q = 128u - bucket, p = q / 4u, sub = q % 4u;
+    return p >= 2u ? ((5u + sub) << (p - 2u)) - 1u : (1u << (p + 1u)) - 1u;
+}
+__device__ __forceinline__ void choose_threshold(const uint32_t *s_lists, float *s_sums, uint32_t *s_best, uint32_t waves, uint32_t *long_tiles)
+{
+    const uint32_t t = threadIdx.x, bucket = 128u - t;                  // (t = 0 .. 127: shortest first)
+    const float end = t < 128u ? (float)bin_end(bucket) : 0.0f;
+    if (t == 0) *s_best = kLeastThreshold;
+    if (t < 128u) s_sums[t] = (float)s_lists[bucket] * (0.9f * end);
+    for (uint32_t d = 1; d < 128u; d *= 2u) {
+        __syncthreads();
+        const float before = t >= d && t < 128u ? s_sums[t - d] : 0.0f;
+        __syncthreads();
+        if (t < 128u) s_sums[t] += before;
+    }
+    if (t < 128u && end <= (float)kLongListDefault && end <= kThresholdShare / kWavesHeld * (float)waves * s_sums[t]) atomicMax(s_best, (uint32_t)end);
     __syncthreads();
+    if (t == 0) long_tiles[kChosenThreshold] = *s_best;
+}
+__global__ void __launch_bounds__(256) tile_order_count_kernel(const uint32_t *__restrict__ ranges, uint32_t *__restrict__ order, uint32_t grid_w,
+                                                               uint32_t grid_h, uint32_t *__restrict__ list_bins)
+{
+    __shared__ uint32_t count[kOrderBuckets], lists[kOrderBuckets];
+    if (threadIdx.x < kOrderBuckets) count[threadIdx.x] = lists[threadIdx.x] = 0;
+    __syncthreads();
+    if (list_bins != nullptr) {
+        const uint32_t tile = blockIdx.x * 256 + threadIdx.x;
+        if (tile < grid_w * grid_h) atomicAdd(&lists[order_bucket(ranges[2 * tile + 1] - ranges[2 * tile])], 1u);
+    }
     const uint32_t n_tiles = grid_w * grid_h, i = blockIdx.x * 256 + threadIdx.x;
     uint32_t tile;
     const uint32_t length = order_group_length(ranges, i, n_tiles, grid_w, grid_h, tile);
     if (i % kOrderGroup == 0 && i / kOrderGroup < n_tiles / kOrderGroup) atomicAdd(&count[order_bucket(length)], 1u);
     __syncthreads();
     if (threadIdx.x < kOrderBuckets && count[threadIdx.x]) atomicAdd(order + n_tiles + threadIdx.x, count[threadIdx.x]);
+    if (list_bins != nullptr && threadIdx.x < kOrderBuckets && lists[threadIdx.x]) atomicAdd(list_bins + threadIdx.x, lists[threadIdx.x]);
 }
 __global__ void __launch_bounds__(256) tile_order_place_kernel(const uint32_t *__restrict__ ranges, uint32_t *__restrict__ order, uint32_t grid_w,
-                                                               uint32_t grid_h)
+                                                               uint32_t grid_h, const uint32_t *__restrict__ list_bins, uint32_t waves, uint32_t *__restrict__ long_tiles)
 {
     __shared__ uint32_t count[kOrderBuckets], total[kOrderBuckets], base[kOrderBuckets];
+    if (list_bins != nullptr && blockIdx.x == gridDim.x - 1) {          // (one block more than the tiles ask for)
+        __shared__ float sums[128];
+        __shared__ uint32_t best;
+        if (threadIdx.x < kOrderBuckets) total[threadIdx.x] = list_bins[threadIdx.x];
+        __syncthreads();
+        choose_threshold(total, sums, &best, waves, long_tiles);
+        return;
+    }
     const uint32_t n_tiles = grid_w * grid_h, n_groups = n_tiles / kOrderGroup;
     if (threadIdx.x < kOrderBuckets) { count[threadIdx.x] = 0; total[threadIdx.x] = order[n_tiles + threadIdx.x]; }
     __syncthreads();
@@ -511,6 +549,46 @@ __global__ void __launch_bounds__(256) tile_order_place_kernel(const uint32_t *_
     } else if (i < n_tiles) {
         order[i] = strip_order_tile(i, grid_w, grid_h);             // the tiles that fill no group, at the end
     }
+}
+
+// The two in one workgroup, for small grids.
+constexpr uint32_t kOneGroupTiles = 4096;
+__global__ void __launch_bounds__(1024) tile_order_one_group_kernel(const uint32_t *__restrict__ ranges, uint32_t *__restrict__ order, uint32_t grid_w,
+                                                                    uint32_t grid_h, uint32_t waves, uint32_t *__restrict__ long_tiles)
+{
+    __shared__ uint32_t count[kOrderBuckets], lists[kOrderBuckets], base[kOrderBuckets], best;
+    __shared__ float sums[128];
+    const uint32_t n_tiles = grid_w * grid_h, n_groups = n_tiles / kOrderGroup;
+    if (threadIdx.x < kOrderBuckets) count[threadIdx.x] = lists[threadIdx.x] = 0;
+    __syncthreads();
+    constexpr uint32_t kPer = kOneGroupTiles / 1024u;
+    uint32_t tiles[kPer], buckets[kPer];
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+        if (1024u * k >= n_tiles) break;                               // (the same for all threads)
+        const uint32_t i = 1024u * k + threadIdx.x;
+        buckets[k] = order_bucket(order_group_length(ranges, i, n_tiles, grid_w, grid_h, tiles[k]));
+        if (i % kOrderGroup == 0 && i / kOrderGroup < n_groups) atomicAdd(&count[buckets[k]], 1u);
+        if (long_tiles != nullptr && i < n_tiles) atomicAdd(&lists[order_bucket(ranges[2 * i + 1] - ranges[2 * i])], 1u);
+    }
+    __syncthreads();
+    if (threadIdx.x < kOrderBuckets) {
+        uint32_t start = 0;
+        for (uint32_t b = 0; b < threadIdx.x; ++b) start += count[b];
+        base[threadIdx.x] = start;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+        if (1024u * k >= n_tiles) break;
+        const uint32_t i = 1024u * k + threadIdx.x, group = i / kOrderGroup, t = i % kOrderGroup;
+        uint32_t place = 0;
+        if (t == 0 && group < n_groups) place = atomicAdd(&base[buckets[k]], 1u);
+        place = __shfl(place, (int)((threadIdx.x & (kWave - 1)) & ~(kOrderGroup - 1u)), kWave);
+        if (group < n_groups) order[order_place(place, t, n_groups)] = tiles[k];
+        else if (i < n_tiles) order[i] = strip_order_tile(i, grid_w, grid_h);
+    }
+    if (long_tiles != nullptr) choose_threshold(lists, sums, &best, waves, long_tiles);
 }
 
 // Scratch of htgs_scan_offsets_static: the per-block sums of the scan, held in the library's own device image so
@@ -588,7 +666,7 @@ static int launch_scan(const htgs_frame *f, uint32_t *tile_sums, const char *who
             hipLaunchKernelGGL(scan_reduce_kernel, dim3(tiles), dim3(kScanBlock), 0, s, counts, tile_sums, n);
         hipLaunchKernelGGL(scan_apply_kernel, dim3(tiles), dim3(kScanBlock), 0, s, counts, tile_sums, f->offsets, f->n_instances_dev, n, host_total, tag, sums_per_tile);
     } else {
-        hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(256), 0, s, f->n_instances_dev, (size_t)1, (uint32_t *)nullptr, (uint32_t *)nullptr);
+        hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(256), 0, s, f->n_instances_dev, (size_t)1, (uint32_t *)nullptr, (uint32_t *)nullptr, (uint32_t *)nullptr);
     }
     return check_launch("scan");
 }
@@ -736,10 +814,12 @@ int extract_ranges_of(const htgs_frame *f, int selector, bool cleared, bool rang
     hipStream_t s = (hipStream_t)f->stream;
     const int tile = tile_size(f->mode);
     const size_t n_tiles = (size_t)div_up(f->width, tile) * div_up(f->height, tile);
+    // (the words for the tiles' finished parts are free until the blend)
+    uint32_t *const list_bins = f->tile_order && chooses_threshold(f) && n_tiles >= kOrderBuckets ? f->long_tiles + 8 + 2 * n_tiles : nullptr;
     const size_t to_zero = 2 * n_tiles > kOrderWords ? 2 * n_tiles : kOrderWords;
     if (!cleared)
         hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((to_zero + 255) / 256)), dim3(256), 0, s, f->ranges, ranged ? (size_t)0 : 2 * n_tiles, f->long_tiles,
-                           f->tile_order ? f->tile_order + n_tiles : nullptr);
+                           f->tile_order ? f->tile_order + n_tiles : nullptr, list_bins);
     if (f->n_instances > 0 && !ranged) {
         if (!f->keys[selector]) return fail(HTGS_ERR_ARGUMENT, "htgs_extract_ranges: null pointer");
         if ((uintptr_t)f->keys[selector] & 15) return fail(HTGS_ERR_ARGUMENT, "htgs_extract_ranges: keys must be 16-byte aligned");
@@ -756,8 +836,13 @@ int extract_ranges_of(const htgs_frame *f, int selector, bool cleared, bool rang
     if (f->tile_order) {
         const uint32_t grid_w = (uint32_t)div_up(f->width, tile), grid_h = (uint32_t)div_up(f->height, tile);
         const dim3 grid((unsigned)((n_tiles + 255) / 256)), block(256);
-        hipLaunchKernelGGL(tile_order_count_kernel, grid, block, 0, s, f->ranges, f->tile_order, grid_w, grid_h);
-        hipLaunchKernelGGL(tile_order_place_kernel, grid, block, 0, s, f->ranges, f->tile_order, grid_w, grid_h);
+        const uint32_t waves = f->waves_per_tile > 1 ? (uint32_t)f->waves_per_tile : 1u;
+        if (n_tiles <= kOneGroupTiles) {
+            hipLaunchKernelGGL(tile_order_one_group_kernel, dim3(1), dim3(1024), 0, s, f->ranges, f->tile_order, grid_w, grid_h, waves, list_bins ? f->long_tiles : nullptr);
+            return check_launch("extract_ranges");
+        }
+        hipLaunchKernelGGL(tile_order_count_kernel, grid, block, 0, s, f->ranges, f->tile_order, grid_w, grid_h, list_bins);
+        hipLaunchKernelGGL(tile_order_place_kernel, dim3(grid.x + (list_bins ? 1u : 0u)), block, 0, s, f->ranges, f->tile_order, grid_w, grid_h, list_bins, waves, f->long_tiles);
     }
     return check_launch("extract_ranges");
 }

@@ -33,7 +33,7 @@ template <int K, int MODE>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 5 : 2))) max_weights_tile_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
     uint32_t *__restrict__ max_weights, uint32_t width, uint32_t height, uint32_t grid_w, float weight_threshold, const uint32_t *__restrict__ tile_order,
-    uint32_t *__restrict__ long_tiles, uint32_t long_threshold, PartFloor part_floor)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor)
 {
     constexpr bool kCore = MODE != HTGS_MODE_OIT_BLEND;
     constexpr bool kTail = MODE != HTGS_MODE_ALPHA_BLEND_FIRST_K;
@@ -45,6 +45,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
     {
         // a tile with a very long list is left to the kernels that share a list between waves and workgroups
         const uint32_t length = ranges[2 * tile + 1] - ranges[2 * tile];
+        const uint32_t long_threshold = threshold.get(long_tiles);
         if (long_tiles != nullptr && length > long_threshold) {
             constexpr uint32_t part_words = MODE == HTGS_MODE_HYBRID_BLEND ? long_part_words<KS>() : MODE == HTGS_MODE_OIT_BLEND ? kOitPartWords : first_k_part_words<KS>();
             if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, length, long_threshold, part_words, part_floor.get(gridDim.x));
@@ -205,11 +206,12 @@ struct MaxWeightsOit {
 // After the kernels for very long lists have left the tail weights of such tiles: the tiles are entered on the list again,
 // in parts, for the second walk.
 __global__ void __launch_bounds__(256) max_weights_tail_enter_kernel(const uint32_t *__restrict__ ranges, uint32_t *__restrict__ long_tiles, uint32_t n_tiles,
-                                                                    uint32_t long_threshold, PartFloor part_floor)
+                                                                    ListThreshold threshold, PartFloor part_floor)
 {
     const uint32_t tile = blockIdx.x * 256 + threadIdx.x;
     if (tile >= n_tiles) return;
     const uint32_t length = ranges[2 * tile + 1] - ranges[2 * tile];
+    const uint32_t long_threshold = threshold.get(long_tiles);
     if (length > long_threshold) long_tile_enter(long_tiles, tile, n_tiles, length, long_threshold / 4u, 0u, part_floor.get(n_tiles));   // (parts of one threshold's length)
 }
 // The second walk (alpha * tail weight for every fragment that passes the cut-off) over the parts of the very long lists:
@@ -219,13 +221,14 @@ template <int MODE>
 __global__ void __launch_bounds__(64 * kTailWaves) max_weights_tail_long_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, const uint32_t *long_tiles,
     uint32_t *__restrict__ max_weights, const float *__restrict__ tail_weights, uint32_t width, uint32_t height, uint32_t grid_w, float weight_threshold,
-    uint32_t long_threshold)
+    ListThreshold threshold)
 {
     __shared__ TileStageQ st[kTailWaves];
     __shared__ QuadrantLists ql[kTailWaves];
     __shared__ uint32_t s_next;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     if (long_tiles[0] == 0) return;                   // (the ordinary frame)
+    const uint32_t long_threshold = threshold.get(long_tiles);
     uint32_t round = 0;
     LongEntry e;
     while (long_tile_take(long_tiles, ranges, long_threshold, round, &s_next, e)) {
@@ -261,12 +264,12 @@ template <int K, int MODE>
 static void launch_tile(const htgs_frame *f, int sel, uint32_t *max_weights, float thr, uint32_t grid_w, uint32_t n_tiles)
 {
     hipStream_t s = (hipStream_t)f->stream;
-    const uint32_t threshold = f->long_list_threshold > 0 ? (uint32_t)f->long_list_threshold : kLongListDefault;
+    const ListThreshold threshold = list_threshold(f);
     const bool shared = shares_long_lists<MODE>(f);
     const uint32_t w = (uint32_t)f->width, h = (uint32_t)f->height;
     hipLaunchKernelGGL((max_weights_tile_kernel<K, MODE>), dim3(n_tiles), dim3(64), 0, s, f->ranges, f->vals[sel], (const float4 *)f->prim, max_weights, w, h, grid_w,
                        thr, f->tile_order, shared ? f->long_tiles : nullptr, threshold, part_floor_of(f, sel, true));
-    if (!shared || !may_have_long_lists(f, threshold)) return;
+    if (!shared || !may_have_long_lists(f)) return;
     constexpr int REC4 = HTGS_PRIM_FLOATS / 4;
     if constexpr (MODE == HTGS_MODE_HYBRID_BLEND)
         hipLaunchKernelGGL((blend_hybrid_long_kernel<K, false, REC4, MaxWeightsHybrid>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0, s,

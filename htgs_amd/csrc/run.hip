@@ -88,7 +88,15 @@ struct Carver {
     }
 };
 
-constexpr uint64_t kUnorderedTiles = 4096;      // of a wave each; a quarter as many of four waves
+// The waves that a tile gets (the lines: blend_waves.h).  The sums of OIT_BLEND leave a wave more to gain than cores, which have
+// to be merged and finished.
+static int waves_of(const htgs_frame *f, int what, uint64_t n_tiles)
+{
+    if (f->mode == HTGS_MODE_ALPHA_BLEND_GLOBAL_ORDERING || what == HTGS_RUN_MAX_WEIGHTS) return 1;
+    const uint64_t two = f->mode == HTGS_MODE_OIT_BLEND ? 16384 : what == HTGS_RUN_FORWARD ? 12288 : 15360;
+    return n_tiles <= 6144 ? 4 : n_tiles <= two ? 2 : 1;
+}
+constexpr uint64_t kUnorderedTiles = 1280;      // workgroups of four waves
 static uint64_t carve_front(htgs_frame *f, int what, void *base)
 {
     Carver c = { static_cast<unsigned char *>(base), 0 };
@@ -109,8 +117,10 @@ static uint64_t carve_front(htgs_frame *f, int what, void *base)
     f->ranges = c.take<uint32_t>(2 * n_tiles);
     // (the modes that walk all of a list)
     f->long_tiles = f->mode != HTGS_MODE_ALPHA_BLEND_GLOBAL_ORDERING ? c.take<uint32_t>(8 + 3 * n_tiles) : nullptr;
+    f->waves_per_tile = waves_of(f, what, n_tiles);
+    f->long_list_threshold = -1;                           // (ListThreshold)
     // (a grid whose workgroups are all on the device at once is taken in any order)
-    f->tile_order = n_tiles > (tile == 8 ? kUnorderedTiles : kUnorderedTiles / 4) ? c.take<uint32_t>(htgs_tile_order_words(f->mode, f->width, f->height)) : nullptr;
+    f->tile_order = n_tiles > kUnorderedTiles ? c.take<uint32_t>(htgs_tile_order_words(f->mode, f->width, f->height)) : nullptr;
     // GLOBAL_ORDERING without a backward pass, and the image-only fast path of the two modes with a sorted core
     const bool by_depth = !train && (f->mode == HTGS_MODE_ALPHA_BLEND_GLOBAL_ORDERING ||
                                      (what == HTGS_RUN_RENDER && f->fast_math && f->mode != HTGS_MODE_OIT_BLEND));
@@ -184,7 +194,10 @@ static int queue_front(const htgs_frame *f, const htgs_workspace *w, HostWord *w
             start.clear[1] = f->tile_order + n_tiles;
             start.clear_words[1] = (uint32_t)htgs_tile_order_words(f->mode, f->width, f->height) - n_tiles;
         }
-        if (f->long_tiles) { start.clear[2] = f->long_tiles; start.clear_words[2] = 8; }
+        if (f->long_tiles) {
+            start.clear[2] = f->long_tiles; start.clear_words[2] = 8;
+            if (f->tile_order) { start.clear[3] = f->long_tiles + 8 + 2 * (size_t)n_tiles; start.clear_words[3] = n_tiles < 132 ? n_tiles : 132; }
+        }
     }
     const int rc = preprocess_and_start(&t, start);
     return rc != HTGS_OK ? rc : scan_offsets_publish(&t, &word->value, word->tag, starts, fused);

@@ -158,7 +158,7 @@ class FrameBuffers:
     def __init__(self, positions, scales, rotations, opacities, sh_0, sh_rest, settings: RasterizerSettings,
                  to_chw: bool = True, use_median_depth: bool = False, train: bool = False,
                  pool: Optional[ScratchPool] = None, fast: bool = False, long_list_threshold: int = 0, order_tiles: bool = True,
-                 order_gaussians: bool = True, tight_lists: bool = False):
+                 order_gaussians: bool = True, tight_lists: bool = False, waves_per_tile: int = 1):
         mode = _mode_value(settings.mode)
         if mode not in (0, 1, 2, 3):
             raise RuntimeError("unsupported rasterizer mode")
@@ -245,6 +245,7 @@ class FrameBuffers:
         f.scan_tmp, f.n_instances_dev = _ptr(self.scan_tmp), _ptr(self.n_instances_dev)
         f.ranges = _ptr(self.ranges)
         f.long_tiles = _ptr(self.long_tiles)
+        f.waves_per_tile = int(waves_per_tile)
         f.tile_order = _ptr(self.tile_order)
         f.depth_order = _ptr(self.depth_order)
         f.long_list_threshold = int(long_list_threshold)      # 0: the library's default

@@ -89,16 +89,23 @@ typedef struct htgs_frame {
     uint32_t *long_tiles;      /* [8 + 3 n_tiles] or NULL.  HYBRID_BLEND, ALPHA_BLEND_FIRST_K and OIT_BLEND (the modes that
                                   walk all of a list), every blend stage: htgs_blend, htgs_blend_forward,
                                   htgs_blend_backward, htgs_max_weights_blend.  Tiles whose list is longer than
-                                  long_list_threshold are collected here (word 0: entries on the list, words 1-5: work
-                                  counters, words 6-7: how the tiles with fragments of equal depth were settled, for
-                                  tests; the eight header words are zeroed by htgs_extract_ranges, words 0-5 again by
+                                  long_list_threshold are collected here (word 0: entries on the list, words 1-4: work
+                                  counters, word 5: see long_list_threshold, words 6-7: how the tiles with fragments of
+                                  equal depth were settled, for tests; the eight header words are zeroed by
+                                  htgs_extract_ranges, words 0-4 again by
                                   every stage when it is done with the list; then 2 n_tiles words of entries -- a list
                                   of several times the threshold is entered in up to 32 parts -- and a counter per
                                   tile) and walked by several waves or workgroups each, the longest first; the forward
                                   stages then also overwrite vals[1 - selector], see htgs_blend.
                                   NULL: every tile is walked by one wave (no counterpart in the reference, which
                                   does that) */
-    int32_t long_list_threshold; /* 0 = the default (8192 instances) */
+    int32_t long_list_threshold; /* 0 = the default (8192 instances); negative: htgs_extract_ranges chooses one of 512 to 8192 from
+                                  the lengths of the frame's lists (word 5 of long_tiles) if it makes tile_order, else the
+                                  blend takes a multiple of their average */
+    int32_t waves_per_tile;    /* 0 or 1: one wave walks a tile of 8x8 pixels (the modes but GLOBAL_ORDERING); 2, 4: htgs_blend
+                                  and htgs_blend_forward give it as many, which walk a share of its list each and merge
+                                  what they have -- for grids of few tiles.  Needs long_tiles and a threshold of no more than
+                                  8192 (ignored otherwise).  Results agree up to the order of sums */
     uint32_t *tile_order;      /* htgs_tile_order_words() words or NULL.  Written by htgs_extract_ranges: the n_tiles tiles
                                   in groups of sixteen neighbours (a 4x4 patch), the groups with the longest lists first
                                   (binned by total length, four bins per power of two) and a group's tiles at the

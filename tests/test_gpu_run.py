@@ -25,7 +25,7 @@ def test_render_equals_the_stages(cuda, mode):
         print(f"case mode={mode} frame={i}", flush=True)
         s = scene.settings(RasterizerMode(mode), 4)
         image, depth = rasterize(*scene.gaussians(), s, i % 2 == 0, False)
-        want, want_depth = FrameBuffers(*scene.gaussians(), s, i % 2 == 0, False, tight_lists=True).run()
+        want, want_depth = FrameBuffers(*scene.gaussians(), s, i % 2 == 0, False, tight_lists=True, waves_per_tile=4).run()
         assert torch.equal(image, want) and torch.equal(depth.reshape(want_depth.shape), want_depth)
 
 
@@ -39,7 +39,7 @@ def test_training_and_max_weights_equal_the_stages(cuda, mode):
         leaves = [t.clone().requires_grad_() for t in scene.gaussians()]
         image = diff_rasterize(*leaves, torch.empty(0, device=cuda), s, False)
         grads = torch.autograd.grad(image, leaves, up)
-        fb = FrameBuffers(*scene.gaussians(), s, True, False, train=True, tight_lists=True)
+        fb = FrameBuffers(*scene.gaussians(), s, True, False, train=True, tight_lists=True, waves_per_tile=4)
         assert torch.equal(image.detach(), fb.run_forward())
         for got, want in zip(grads, fb.run_backward(up)):
             assert torch.equal(got, want)
