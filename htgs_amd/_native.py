@@ -52,6 +52,7 @@ class Frame(ctypes.Structure):
         ("long_tiles", ctypes.c_void_p),
         ("long_list_threshold", ctypes.c_int32),
         ("waves_per_tile", ctypes.c_int32),
+        ("long_counters", ctypes.c_void_p),
         ("tile_order", ctypes.c_void_p),
         ("depth_order", ctypes.c_void_p),
         ("n_instances", ctypes.c_uint64),

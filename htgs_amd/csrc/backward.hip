@@ -454,8 +454,8 @@ __global__ void __launch_bounds__(64 * kBackwardWaves) __attribute__((amdgpu_wav
     // a very long list is left to blend_tail_backward_long_kernel, in parts (no part leaves anything behind for the others)
     const uint32_t long_threshold = threshold.get(long_tiles);
     if (long_tiles != nullptr && last - first > long_threshold) {
-        // (parts of one threshold's length: nothing is merged afterwards, so the finer the parts the better they spread)
-        if (threadIdx.x == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold / 4u, 0u, part_floor);
+        // (nothing is merged afterwards)
+        if (threadIdx.x == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, threshold.least_backward_part(long_threshold), 0u, part_floor, long_threshold, threshold.counters);
         return;
     }
     backward_tile<K, MODE, HELPER>(lds, tile, first, last, gridDim.x, inst, prim, core_idx, core_info, tail_info, grad_image, VPM, grad_rows, helper_rows, width,
@@ -477,7 +477,7 @@ __global__ void __launch_bounds__(64 * kBackwardWaves) __attribute__((amdgpu_wav
     const uint32_t n_tiles = grid_w * ((height + 7u) / 8u);
     uint32_t round = 0;
     LongEntry e;
-    while (long_tile_take(long_tiles, ranges, long_threshold, round, &s_next, e))
+    while (long_tile_take(long_tiles, ranges, long_threshold, threshold.counters, round, &s_next, e))
         backward_tile<K, MODE, HELPER>(lds, e.tile, e.first, e.last, n_tiles, inst, prim, core_idx, core_info, tail_info, grad_image, VPM, grad_rows, helper_rows,
                                        width, height, grid_w);
 }

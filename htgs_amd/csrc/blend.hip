@@ -184,11 +184,8 @@ static void launch_hybrid(const htgs_frame *f, int selector, uint32_t grid_w, ui
         hipLaunchKernelGGL((blend_hybrid_kernel<K, FAST>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
                            f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
-    if (may_have_long_lists(f))      // (one workgroup per compute unit; they find an empty list on ordinary frames)
-        hipLaunchKernelGGL((blend_hybrid_long_kernel<K, FAST, HTGS_PRIM_FLOATS / 4, HybridImage>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0,
-                           (hipStream_t)f->stream, f->ranges, f->vals[selector], (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w,
-                           f->vals[selector ^ 1], threshold,
-                           HybridImage{ f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, f->to_chw, f->use_median_depth });
+    // (its workgroups find an empty list on ordinary frames)
+    launch_hybrid_long<K, FAST, HTGS_PRIM_FLOATS / 4>(f, selector, grid_w, HybridImage{ f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, f->to_chw, f->use_median_depth });
 }
 template <int K, bool FAST>
 static void launch_first_k(const htgs_frame *f, int selector, uint32_t grid_w, uint32_t n_tiles)
@@ -202,11 +199,7 @@ static void launch_first_k(const htgs_frame *f, int selector, uint32_t grid_w, u
         hipLaunchKernelGGL((blend_first_k_kernel<K, FAST>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
                            f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
-    if (may_have_long_lists(f))
-        hipLaunchKernelGGL((blend_first_k_long_kernel<K, FAST, HTGS_PRIM_FLOATS / 4, FirstKImage>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0,
-                           (hipStream_t)f->stream, f->ranges, f->vals[selector], (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w,
-                           f->vals[selector ^ 1], threshold,
-                           FirstKImage{ f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, f->to_chw, f->use_median_depth });
+    launch_first_k_long<K, FAST, HTGS_PRIM_FLOATS / 4>(f, selector, grid_w, FirstKImage{ f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, f->to_chw, f->use_median_depth });
 }
 
 template <bool FAST>
@@ -246,10 +239,7 @@ static void launch_blend(const htgs_frame *f, int selector, uint32_t grid_w, uin
             hipLaunchKernelGGL(blend_oit_kernel<FAST>, dim3(n_tiles), dim3(64), 0, s, f->ranges, f->vals[selector], (const float4 *)f->prim,
                                f->image, depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw, f->long_tiles, threshold,
                                long_part_floor(f, selector), f->tile_order);
-            if (may_have_long_lists(f))
-                hipLaunchKernelGGL((blend_oit_long_kernel<FAST, HTGS_PRIM_FLOATS / 4, OitImage>), dim3(256), dim3(64 * kLongWaves), 0, s, f->ranges, f->vals[selector],
-                                   (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->vals[selector ^ 1], threshold,
-                                   OitImage{ f->image, depth, (uint32_t)f->width, (uint32_t)f->height, f->to_chw });
+            launch_oit_long<FAST, HTGS_PRIM_FLOATS / 4, !FAST>(f, selector, grid_w, OitImage{ f->image, depth, (uint32_t)f->width, (uint32_t)f->height, f->to_chw });
             break;
         }
     }

@@ -26,7 +26,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
     const uint32_t long_threshold = threshold.get(long_tiles);
     if (long_tiles != nullptr && last - first > long_threshold) {
-        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, long_part_words<K>(), part_floor.get(gridDim.x));
+        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, threshold.least_part(long_threshold), long_part_words<K>(), part_floor.get(gridDim.x), long_threshold, threshold.counters);
         return;
     }
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
     const uint32_t long_threshold = threshold.get(long_tiles);
     if (long_tiles != nullptr && last - first > long_threshold) {
-        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, first_k_part_words<K>(), part_floor.get(gridDim.x));
+        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, threshold.least_part(long_threshold), first_k_part_words<K>(), part_floor.get(gridDim.x), long_threshold, threshold.counters);
         return;
     }
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
@@ -74,7 +74,7 @@ __global__ void __launch_bounds__(64) blend_oit_forward_kernel(
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
     const uint32_t long_threshold = threshold.get(long_tiles);
     if (long_tiles != nullptr && last - first > long_threshold) {
-        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, kOitPartWords, part_floor.get(gridDim.x));
+        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, threshold.least_part(long_threshold), kOitPartWords, part_floor.get(gridDim.x), long_threshold, threshold.counters);
         return;
     }
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
@@ -140,10 +140,7 @@ static void launch_hybrid_forward(const htgs_frame *f, int sel, uint32_t grid_w,
     const HybridRecords finish = { f->image, f->core_idx, (float4 *)f->core_info, f->tail_info, (uint32_t)f->width, (uint32_t)f->height, (size_t)n_tiles * 64u };
     hipLaunchKernelGGL((blend_hybrid_forward_kernel<K>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim,
                        (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, list_threshold(f), forward_part_floor(f, sel), f->tile_order, finish);
-    if (may_have_long_lists(f))
-        hipLaunchKernelGGL((blend_hybrid_long_kernel<K, false, REC4, HybridRecords>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0,
-                           (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w,
-                           f->vals[sel ^ 1], list_threshold(f), finish);
+    launch_hybrid_long<K, false, REC4>(f, sel, grid_w, finish);
 }
 template <int K>
 static void launch_first_k_forward(const htgs_frame *f, int sel, uint32_t grid_w, uint32_t n_tiles)
@@ -152,10 +149,7 @@ static void launch_first_k_forward(const htgs_frame *f, int sel, uint32_t grid_w
     const FirstKRecords finish = { f->image, f->core_idx, (float4 *)f->core_info, (uint32_t)f->width, (uint32_t)f->height, (size_t)n_tiles * 64u };
     hipLaunchKernelGGL((blend_first_k_forward_kernel<K>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim,
                        (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, list_threshold(f), forward_part_floor(f, sel), f->tile_order, finish);
-    if (may_have_long_lists(f))
-        hipLaunchKernelGGL((blend_first_k_long_kernel<K, false, REC4, FirstKRecords>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0,
-                           (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w,
-                           f->vals[sel ^ 1], list_threshold(f), finish);
+    launch_first_k_long<K, false, REC4>(f, sel, grid_w, finish);
 }
 static void launch_oit_forward(const htgs_frame *f, int sel, uint32_t grid_w, uint32_t n_tiles)
 {
@@ -163,9 +157,7 @@ static void launch_oit_forward(const htgs_frame *f, int sel, uint32_t grid_w, ui
     const OitRecords finish = { f->image, f->tail_info, (uint32_t)f->width, (uint32_t)f->height, (size_t)n_tiles * 64u };
     hipLaunchKernelGGL(blend_oit_forward_kernel, dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim,
                        (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, list_threshold(f), forward_part_floor(f, sel), f->tile_order, finish);
-    if (may_have_long_lists(f))
-        hipLaunchKernelGGL((blend_oit_long_kernel<false, REC4, OitRecords, false>), dim3(256), dim3(64 * kLongWaves), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel],
-                           (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->vals[sel ^ 1], list_threshold(f), finish);
+    launch_oit_long<false, REC4, false>(f, sel, grid_w, finish);
 }
 
 }  // namespace htgs

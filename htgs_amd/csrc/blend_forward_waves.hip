@@ -4,30 +4,28 @@
 
 namespace htgs {
 
-template <int WAVES, typename Main, typename Long, typename Finish>
-static void launch_waves(const htgs_frame *f, int sel, uint32_t grid_w, uint32_t n_tiles, Main main, Long long_kernel, unsigned long_blocks,
-                         unsigned long_threads, const Finish &finish)
+template <int WAVES, typename Main, typename Finish>
+static void launch_waves(const htgs_frame *f, int sel, uint32_t grid_w, uint32_t n_tiles, Main main, const Finish &finish)
 {
     hipStream_t s = (hipStream_t)f->stream;
     const PartFloor floor = { instance_count(f), f->vals[sel ^ 1] != nullptr ? 1u : 0u };
     hipLaunchKernelGGL(main, dim3(n_tiles), dim3(64 * WAVES), 0, s, f->ranges, f->vals[sel], (const float4 *)f->prim, (uint32_t)f->width, (uint32_t)f->height, grid_w,
                        f->long_tiles, list_threshold(f), floor, f->tile_order, finish);
-    if (may_have_long_lists(f))
-        hipLaunchKernelGGL(long_kernel, dim3(long_blocks), dim3(long_threads), 0, s, f->ranges, f->vals[sel], (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width,
-                           (uint32_t)f->height, grid_w, f->vals[sel ^ 1], list_threshold(f), finish);
 }
 template <int WAVES, int K>
 static void launch_k(const htgs_frame *f, int sel, uint32_t grid_w, uint32_t n_tiles)
 {
     constexpr int REC4 = HTGS_PRIM_FLOATS_TRAIN / 4;
-    constexpr unsigned blocks = 256 * kLongWaves / long_waves<K>(), threads = 64 * long_waves<K>();
     const uint32_t w = (uint32_t)f->width, h = (uint32_t)f->height;
-    if (f->mode == HTGS_MODE_HYBRID_BLEND)
-        launch_waves<WAVES>(f, sel, grid_w, n_tiles, blend_hybrid_waves_exact_kernel<WAVES, K, REC4, HybridRecords>, blend_hybrid_long_kernel<K, false, REC4, HybridRecords>, blocks, threads,
-                     HybridRecords{ f->image, f->core_idx, (float4 *)f->core_info, f->tail_info, w, h, (size_t)n_tiles * 64u });
-    else
-        launch_waves<WAVES>(f, sel, grid_w, n_tiles, blend_first_k_waves_exact_kernel<WAVES, K, false, REC4, FirstKRecords>, blend_first_k_long_kernel<K, false, REC4, FirstKRecords>, blocks,
-                     threads, FirstKRecords{ f->image, f->core_idx, (float4 *)f->core_info, w, h, (size_t)n_tiles * 64u });
+    if (f->mode == HTGS_MODE_HYBRID_BLEND) {
+        const HybridRecords finish = { f->image, f->core_idx, (float4 *)f->core_info, f->tail_info, w, h, (size_t)n_tiles * 64u };
+        launch_waves<WAVES>(f, sel, grid_w, n_tiles, blend_hybrid_waves_exact_kernel<WAVES, K, REC4, HybridRecords>, finish);
+        launch_hybrid_long<K, false, REC4>(f, sel, grid_w, finish);
+    } else {
+        const FirstKRecords finish = { f->image, f->core_idx, (float4 *)f->core_info, w, h, (size_t)n_tiles * 64u };
+        launch_waves<WAVES>(f, sel, grid_w, n_tiles, blend_first_k_waves_exact_kernel<WAVES, K, false, REC4, FirstKRecords>, finish);
+        launch_first_k_long<K, false, REC4>(f, sel, grid_w, finish);
+    }
 }
 
 template <int WAVES>
@@ -35,8 +33,9 @@ static void launch_mode(const htgs_frame *f, int sel, uint32_t grid_w, uint32_t 
 {
     if (f->mode == HTGS_MODE_OIT_BLEND) {
         constexpr int REC4 = HTGS_PRIM_FLOATS_TRAIN / 4;
-        launch_waves<WAVES>(f, sel, grid_w, n_tiles, blend_oit_waves_kernel<WAVES, false, REC4, OitRecords, false>, blend_oit_long_kernel<false, REC4, OitRecords, false>, 256u, 64u * kLongWaves,
-                     OitRecords{ f->image, f->tail_info, (uint32_t)f->width, (uint32_t)f->height, (size_t)n_tiles * 64u });
+        const OitRecords finish = { f->image, f->tail_info, (uint32_t)f->width, (uint32_t)f->height, (size_t)n_tiles * 64u };
+        launch_waves<WAVES>(f, sel, grid_w, n_tiles, blend_oit_waves_kernel<WAVES, false, REC4, OitRecords, false>, finish);
+        launch_oit_long<false, REC4, false>(f, sel, grid_w, finish);
         return;
     }
     switch (htgs_effective_k(f->K)) {

@@ -6,6 +6,8 @@
 // R/include/alpha_blend_first_k/kernels/inference.cuh:78-206 and R/include/oit_blend/kernels/inference.cuh:78-177.
 #pragma once
 
+#include <type_traits>
+
 #include "blend_common.h"
 
 namespace htgs {
@@ -449,7 +451,7 @@ __device__ __forceinline__ void take_tail(const float *from, HybridTail &t, floa
 // ---------------------------------------------------------------------------------------------
 // Tiles with very long lists (HYBRID_BLEND, ALPHA_BLEND_FIRST_K and OIT_BLEND, which walk all of a list): the kernel
 // with one wave per tile puts a tile whose list is longer than long_threshold on a list instead of walking it, if the
-// caller provided that list, and a second launch of workgroups of kLongWaves waves takes those: one wave walks one tile at some
+// caller provided that list, and a second launch of workgroups of several waves takes those: one wave walks one tile at some
 // 200 ns per instance once it has a SIMD to itself, so a single list of 300 000 instances would otherwise hold the
 // launch for 70 ms.
 // long_tiles[0] = entries on the list, [1..3] = work counters, [4] = workgroups done, all zeroed with the
@@ -460,31 +462,48 @@ __device__ __forceinline__ void take_tail(const float *from, HybridTail &t, floa
 // to n_tiles, so the list cannot overflow) and n_tiles words that count a tile's finished parts.
 // ---------------------------------------------------------------------------------------------
 constexpr uint32_t kLongHeader = 8, kLongRounds = 3, kLongParts = 32;
-constexpr int kLongWaves = 16;
-// waves of a workgroup of the K-buffer kernels: sixteen share a compute unit's registers at 128 a lane, which a K-buffer of
-// 32 slots (96 registers) leaves too few of; eight have 256
-template <int K> constexpr int long_waves() { return K > 16 ? 8 : kLongWaves; }
+constexpr int kLongWavesHeld = 16;        // waves that a compute unit holds of these kernels
+// calls launch(std::integral_constant<int, long_waves_of(f)>) for a core of K entries
+template <int K, typename Launch>
+inline void with_long_waves(const htgs_frame *f, Launch &&launch)
+{
+    if constexpr (K <= 16) {
+        if (long_waves_of(f) == 16u) { launch(std::integral_constant<int, 16>{}); return; }
+    }
+    launch(std::integral_constant<int, 8>{});
+}
+constexpr unsigned long_grid(int waves) { return 256u * (unsigned)(kLongWavesHeld / waves); }
+
 // What a workgroup leaves of its part of a list, in 64-lane rows: HYBRID's core, tail and the depth of a tie.
 template <int K> constexpr uint32_t long_part_words() { return (3u * K + 7u) * 64u; }
-// The parts a list of this length is walked in by separate workgroups (1: by one).  A part is at least four times the
-// threshold long, long enough that what the parts leave behind (part_words each) fits into the list's own stretch of
+// The parts a list of this length is walked in by separate workgroups (1: by one).  A part is at least part_least
+// long (least_part), long enough that what the parts leave behind (part_words each) fits into the list's own stretch of
 // the spare value buffer, and at least as long as the frame's average list (part_floor = instances / tiles, rounded
 // up): the parts beyond the first of all tiles together then cannot exceed the number of tiles, which is what the list
 // of entries has room for, and how a list is split is a function of its length and of the frame alone -- no budget
 // shared between workgroups, nothing that depends on the order in which they run.
-__device__ __forceinline__ uint32_t long_parts(uint32_t length, uint32_t long_threshold, uint32_t part_words, uint32_t part_floor)
+__device__ __forceinline__ uint32_t long_parts(uint32_t length, uint32_t part_least, uint32_t part_words, uint32_t part_floor)
 {
-    uint32_t least = 4u * long_threshold > part_words ? 4u * long_threshold : part_words;
+    uint32_t least = part_least > part_words ? part_least : part_words;
     least = least > part_floor ? least : part_floor;
     const uint32_t parts = length / least;
     return parts < 1u ? 1u : parts > kLongParts ? kLongParts : parts;
 }
+// With htgs_frame.long_counters every die has work counters of its own.  An atomic on a line that another die's cache holds
+// takes 0.1 us and the next one waits for it: with one counter for all, a list of 2000 entries cost three rounds of 2000 such
+// atomics (weights of 2.9 M Gaussians at 1416x701, OIT: 1430 us of a kernel that has next to nothing to walk; now 270).
 // (one lane of the tile's wave) enters the tile; part_floor = 0: in one part
 __device__ __forceinline__ void long_tile_enter(uint32_t *__restrict__ long_tiles, uint32_t tile, uint32_t n_tiles, uint32_t length,
-                                                uint32_t long_threshold, uint32_t part_words, uint32_t part_floor)
+                                                uint32_t part_least, uint32_t part_words, uint32_t part_floor, uint32_t long_threshold, uint32_t *counters)
 {
-    const uint32_t parts = part_floor != 0u ? long_parts(length, long_threshold, part_words, part_floor) : 1u;
+    const uint32_t parts = part_floor != 0u ? long_parts(length, part_least, part_words, part_floor) : 1u;
     if (parts > 1u) long_tiles[kLongHeader + 2u * n_tiles + tile] = 0u;
+    if (counters != nullptr) {
+        // (no part is longer than this; its class and the ones below it, which the other parts may be of)
+        const uint32_t longest = length / parts + 128u;
+        if (longest > 16u * long_threshold) counters[kDieRounds] = 1u;
+        if (longest > 4u * long_threshold) counters[kDieRounds + 1u] = 1u;
+    }
     const uint32_t at = kLongHeader + atomicAdd(long_tiles, parts);
     for (uint32_t part = 0; part < parts; ++part) long_tiles[at + part] = tile | part << 20 | (parts - 1u) << 25;
 }
@@ -495,26 +514,38 @@ struct LongEntry {
 // The workgroups take the entries off the list one by one, the longest first: the list is gone through kLongRounds times
 // (a counter per round, `round` starts at 0), and a round takes the entries of its length class only -- more than 16, more
 // than 4 and up to 4 times the threshold.  The lists differ in length by orders of magnitude, and the launch ends when the
-// workgroup with the longest one does.  Called by all threads of the workgroup (barriers inside); false: the list is
-// through.  The last workgroup to find that clears the list's header, so that the list is empty again for the next blend of
-// this frame (htgs_blend called again without htgs_extract_ranges).
+// workgroup with the longest one does.  With counters every die's workgroups go through every eighth entry, and a round
+// whose class no entry is of is left out.  Called by all threads of the workgroup (barriers inside); false: the list is
+// through.  The last workgroup to find that clears the list's header and the counters, so that the list is empty again for
+// the next blend of this frame (htgs_blend called again without htgs_extract_ranges).
 __device__ __forceinline__ bool long_tile_take(const uint32_t *long_tiles, const uint32_t *__restrict__ ranges, uint32_t long_threshold,
-                                               uint32_t &round, uint32_t *s_next, LongEntry &e)
+                                               uint32_t *counters, uint32_t &round, uint32_t *s_next, LongEntry &e)
 {
     const uint32_t n_long = long_tiles[0];
+    // (a launch of fewer workgroups than dies: as many shares of the list as workgroups)
+    const uint32_t shares = counters == nullptr ? 1u : gridDim.x < kDies ? gridDim.x : kDies, share = blockIdx.x % shares;
+    uint32_t *const line = counters != nullptr ? counters + kDieLine * share : const_cast<uint32_t *>(long_tiles) + 1;
     for (;;) {
+        if (counters != nullptr)
+            while (round + 1u < kLongRounds && counters[kDieRounds + round] == 0u) ++round;
         __syncthreads();
-        if (threadIdx.x == 0) *s_next = atomicAdd(const_cast<uint32_t *>(long_tiles) + 1 + round, 1u);
+        if (threadIdx.x == 0) *s_next = atomicAdd(line + round, 1u);
         __syncthreads();
-        const uint32_t j = (uint32_t)__builtin_amdgcn_readfirstlane((int)*s_next);     // (the same in every lane: what follows stays in scalar registers)
+        const uint32_t j = shares * (uint32_t)__builtin_amdgcn_readfirstlane((int)*s_next) + share;     // (the same in every lane: what follows stays in scalar registers)
         if (j >= n_long) {
             if (++round < kLongRounds) continue;
             if (threadIdx.x == 0) {
                 uint32_t *header = const_cast<uint32_t *>(long_tiles);
                 __threadfence();
-                if (atomicAdd(header + 4, 1u) == gridDim.x - 1) {
+                bool last = atomicAdd(line + kLongRounds, 1u) == (gridDim.x - share + shares - 1u) / shares - 1u;
+                if (last && counters != nullptr) last = atomicAdd(counters + kDieRounds + kLongRounds, 1u) == shares - 1u;
+                if (last) {
 #pragma unroll
                     for (uint32_t k = 0; k < 5; ++k) header[k] = 0u;
+                    if (counters != nullptr)
+                        for (uint32_t d = 0; d <= kDies; ++d)
+#pragma unroll
+                            for (uint32_t k = 0; k <= kLongRounds; ++k) counters[kDieLine * d + k] = 0u;
                 }
             }
             return false;
@@ -533,7 +564,7 @@ __device__ __forceinline__ bool long_tile_take(const uint32_t *long_tiles, const
 }
 // share of wave `wave` of [first, last): whole batches of 64
 __device__ __forceinline__ void long_wave_share(uint32_t first, uint32_t last, uint32_t wave, uint32_t &share_first, uint32_t &share_last,
-                                                uint32_t waves = kLongWaves)
+                                                uint32_t waves)
 {
     const uint32_t n_batches = (last - first + 63u) / 64u;
     share_first = first + 64u * (uint32_t)((uint64_t)n_batches * wave / waves);
@@ -566,7 +597,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
     const uint32_t long_threshold = threshold.get(long_tiles);
     if (long_tiles != nullptr && last - first > long_threshold) {
-        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, long_part_words<K>(), part_floor.get(gridDim.x));
+        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, threshold.least_part(long_threshold), long_part_words<K>(), part_floor.get(gridDim.x), long_threshold, threshold.counters);
         return;
     }
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
@@ -709,7 +740,7 @@ __device__ __forceinline__ void merge_all_shares(unsigned char *lds, uint32_t wa
     }
     __syncthreads();                                       // (the stages are free again)
 }
-// The long tiles: a workgroup of kLongWaves waves takes a tile, every wave walks a contiguous share of the list (whole
+// The long tiles: a workgroup of WAVES waves takes a tile, every wave walks a contiguous share of the list (whole
 // batches of 64) into a core and a tail of its own, and the shares are then merged into the first wave's, in list
 // order, through LDS: the entries of the incoming core enter the running core like fragments (what does not stay in
 // the core, of either, joins the tail), the tails add up.  The pixel gets the K nearest fragments of the whole list and
@@ -717,12 +748,12 @@ __device__ __forceinline__ void merge_all_shares(unsigned char *lds, uint32_t wa
 // sums are added (rounding) and which of two stored fragments of exactly equal depth is kept when a nearer one arrives.
 // finish(prim, tile, px, cd, ca, ci, tail) is called by the lanes of the first wave whose pixels lie inside the image, once
 // per pixel, with the pixel's finished core and tail.
-template <int K, bool FAST, int REC4, typename Finish>
-__global__ void __launch_bounds__(64 * long_waves<K>()) blend_hybrid_long_kernel(
+template <int K, int WAVES, bool FAST, int REC4, typename Finish>
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(K > 16 ? 2 : kLongWavesHeld / 4))) blend_hybrid_long_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, const uint32_t *long_tiles,
     uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ shortlist, ListThreshold threshold, const Finish finish)
 {
-    constexpr int kWaves = long_waves<K>();
+    constexpr int kWaves = WAVES;
     constexpr uint32_t kRows = 3 * K + 7;             // a wave's core, tail and least depth of a tie
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<kWaves, kRows>()];
     __shared__ uint32_t s_next;
@@ -737,7 +768,7 @@ __global__ void __launch_bounds__(64 * long_waves<K>()) blend_hybrid_long_kernel
     const uint32_t n_tiles = grid_w * ((height + 7u) / 8u);
     uint32_t round = 0;
     LongEntry entry;
-    while (long_tile_take(long_tiles, ranges, long_threshold, round, &s_next, entry)) {
+    while (long_tile_take(long_tiles, ranges, long_threshold, threshold.counters, round, &s_next, entry)) {
         // (the same in every lane; said so, they live in scalar registers through the walks that follow)
         const auto uniform = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
         const uint32_t tile = uniform(entry.tile), part = uniform(entry.part), parts = uniform(entry.parts), tile_first = uniform(entry.tile_first),
@@ -1023,7 +1054,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
     const uint32_t long_threshold = threshold.get(long_tiles);
     if (long_tiles != nullptr && last - first > long_threshold) {
-        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, first_k_part_words<K>(), part_floor.get(gridDim.x));
+        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, threshold.least_part(long_threshold), first_k_part_words<K>(), part_floor.get(gridDim.x), long_threshold, threshold.counters);
         return;
     }
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
@@ -1084,12 +1115,12 @@ __device__ __forceinline__ void first_k_put(float *to, uint32_t lane, const floa
 // replayed on the fragments that are not farther than the merged core's last entry -- or, when they are many or the room
 // for those fragments does not do, the first wave walks the whole list again for them.
 // finish(prim, tile, px, cd, ca, ci): as for blend_hybrid_long_kernel, with the pixel's finished core.
-template <int K, bool FAST, int REC4, typename Finish>
-__global__ void __launch_bounds__(64 * long_waves<K>()) blend_first_k_long_kernel(
+template <int K, int WAVES, bool FAST, int REC4, typename Finish>
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(K > 16 ? 2 : kLongWavesHeld / 4))) blend_first_k_long_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, const uint32_t *long_tiles,
     uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ spare, ListThreshold threshold, const Finish finish)
 {
-    constexpr int kWaves = long_waves<K>();
+    constexpr int kWaves = WAVES;
     constexpr uint32_t kRows = 3 * K + 1;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<kWaves, kRows>()];
     __shared__ uint32_t s_next, s_whole, s_redo[2], s_listed[kWaves];
@@ -1101,7 +1132,7 @@ __global__ void __launch_bounds__(64 * long_waves<K>()) blend_first_k_long_kerne
     constexpr bool kTies = true;                      // (the fast variant too: a tie decides which fragment a pixel shows)
     uint32_t round = 0;
     LongEntry entry;
-    while (long_tile_take(long_tiles, ranges, long_threshold, round, &s_next, entry)) {
+    while (long_tile_take(long_tiles, ranges, long_threshold, threshold.counters, round, &s_next, entry)) {
         // (the same in every lane; said so, they live in scalar registers through the walks that follow)
         const auto uniform = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
         const LongEntry e = { uniform(entry.tile), uniform(entry.part), uniform(entry.parts), uniform(entry.tile_first), uniform(entry.tile_last),
@@ -1254,7 +1285,7 @@ __global__ void __launch_bounds__(64) blend_oit_kernel(
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
     const uint32_t long_threshold = threshold.get(long_tiles);
     if (long_tiles != nullptr && last - first > long_threshold) {
-        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, kOitPartWords, part_floor.get(gridDim.x));
+        if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, threshold.least_part(long_threshold), kOitPartWords, part_floor.get(gridDim.x), long_threshold, threshold.counters);
         return;
     }
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
@@ -1270,13 +1301,13 @@ __global__ void __launch_bounds__(64) blend_oit_kernel(
 // result is that of the single walk up to the order of its sums.
 // finish(tile, px, sum): as for blend_hybrid_long_kernel, with the pixel's finished sums.
 template <bool FAST, int REC4, typename Finish, bool DEPTH = !FAST>
-__global__ void __launch_bounds__(64 * kLongWaves) blend_oit_long_kernel(
+__global__ void __launch_bounds__(64 * kOitLongWaves) blend_oit_long_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, const uint32_t *long_tiles,
     uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ left, ListThreshold threshold, const Finish finish)
 {
-    __shared__ TileStageQ st[kLongWaves];
-    __shared__ QuadrantLists ql[kLongWaves];
-    __shared__ float s_sums[kLongWaves][6][64];
+    __shared__ TileStageQ st[kOitLongWaves];
+    __shared__ QuadrantLists ql[kOitLongWaves];
+    __shared__ float s_sums[kOitLongWaves][6][64];
     __shared__ uint32_t s_next, s_whole;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     if (long_tiles[0] == 0) return;                   // (the ordinary frame)
@@ -1284,17 +1315,17 @@ __global__ void __launch_bounds__(64 * kLongWaves) blend_oit_long_kernel(
     const uint32_t n_tiles = grid_w * ((height + 7u) / 8u);
     uint32_t round = 0;
     LongEntry entry;
-    while (long_tile_take(long_tiles, ranges, long_threshold, round, &s_next, entry)) {
+    while (long_tile_take(long_tiles, ranges, long_threshold, threshold.counters, round, &s_next, entry)) {
         const TilePixel px = quadrant_tile_pixel(entry.tile, grid_w, lane, width, height);
         uint32_t share_first, share_last;
-        long_wave_share(entry.first, entry.last, wave, share_first, share_last);
+        long_wave_share(entry.first, entry.last, wave, share_first, share_last, kOitLongWaves);
         OitSums sum = { 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 1.0f };
         oit_walk<FAST, false, REC4, DEPTH>(st[wave], ql[wave], inst, prim, share_first, share_last, lane, px.pt, px.cx, px.cy, sum);
         s_sums[wave][0][lane] = sum.a0; s_sums[wave][1][lane] = sum.a1; s_sums[wave][2][lane] = sum.a2; s_sums[wave][3][lane] = sum.a3;
         s_sums[wave][4][lane] = sum.alpha; s_sums[wave][5][lane] = sum.T;
         __syncthreads();
         if (wave == 0) {
-            for (int w = 1; w < kLongWaves; ++w) {
+            for (int w = 1; w < kOitLongWaves; ++w) {
                 sum.a0 += s_sums[w][0][lane]; sum.a1 += s_sums[w][1][lane]; sum.a2 += s_sums[w][2][lane]; sum.a3 += s_sums[w][3][lane];
                 sum.alpha += s_sums[w][4][lane]; sum.T *= s_sums[w][5][lane];
             }
@@ -1318,6 +1349,36 @@ __global__ void __launch_bounds__(64 * kLongWaves) blend_oit_long_kernel(
         }
         if (wave == 0 && px.inside) finish(entry.tile, px, sum);
     }
+}
+
+
+// The launches of the kernels for very long lists, after the one that has put the tiles on the list
+template <int K, bool FAST, int REC4, typename Finish>
+static void launch_hybrid_long(const htgs_frame *f, int sel, uint32_t grid_w, const Finish &finish)
+{
+    if (!may_have_long_lists(f)) return;
+    with_long_waves<K>(f, [&](auto waves) {
+        constexpr int WAVES = decltype(waves)::value;
+        hipLaunchKernelGGL((blend_hybrid_long_kernel<K, WAVES, FAST, REC4, Finish>), dim3(long_grid(WAVES)), dim3(64 * WAVES), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel],
+                           (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->vals[sel ^ 1], list_threshold(f), finish);
+    });
+}
+template <int K, bool FAST, int REC4, typename Finish>
+static void launch_first_k_long(const htgs_frame *f, int sel, uint32_t grid_w, const Finish &finish)
+{
+    if (!may_have_long_lists(f)) return;
+    with_long_waves<K>(f, [&](auto waves) {
+        constexpr int WAVES = decltype(waves)::value;
+        hipLaunchKernelGGL((blend_first_k_long_kernel<K, WAVES, FAST, REC4, Finish>), dim3(long_grid(WAVES)), dim3(64 * WAVES), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel],
+                           (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->vals[sel ^ 1], list_threshold(f), finish);
+    });
+}
+template <bool FAST, int REC4, bool DEPTH, typename Finish>
+static void launch_oit_long(const htgs_frame *f, int sel, uint32_t grid_w, const Finish &finish)
+{
+    if (!may_have_long_lists(f)) return;
+    hipLaunchKernelGGL((blend_oit_long_kernel<FAST, REC4, Finish, DEPTH>), dim3(long_grid(kOitLongWaves)), dim3(64 * kOitLongWaves), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel],
+                       (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->vals[sel ^ 1], list_threshold(f), finish);
 }
 
 }  // namespace htgs

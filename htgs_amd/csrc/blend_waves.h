@@ -77,7 +77,8 @@ __device__ __forceinline__ bool tile_of_waves(const uint32_t *__restrict__ range
     first = ranges[2 * tile]; last = ranges[2 * tile + 1];
     const uint32_t long_threshold = threshold.get(long_tiles);
     if (long_tiles == nullptr || last - first <= long_threshold) return true;
-    if (threadIdx.x == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, long_threshold, part_words, part_floor.get(gridDim.x));
+    if (threadIdx.x == 0) long_tile_enter(long_tiles, tile, gridDim.x, last - first, threshold.least_part(long_threshold), part_words, part_floor.get(gridDim.x),
+                                          long_threshold, threshold.counters);
     return false;
 }
 

@@ -151,8 +151,8 @@ struct PartFloor {
 constexpr int kCountBlock = 256;                 // Gaussians per block sum
 struct FrameStart {
     uint32_t *block_sums;                        // [ceil(N / kCountBlock)] or nullptr
-    uint32_t *clear[4];                          // ranges, order bins, long_tiles header and the bins of its threshold
-    uint32_t clear_words[4];
+    uint32_t *clear[5];                          // ranges, order bins, long_tiles header and the bins of its threshold, long_counters
+    uint32_t clear_words[5];
 };
 int preprocess_and_start(const htgs_frame *f, const FrameStart &start);                 // preprocess.hip
 // The scan for htgs_run, which also writes tag << 32 | total to host memory.  with_sums: scan_tmp holds FrameStart's sums.
@@ -174,10 +174,23 @@ inline size_t block_sum_words(int n) { return (size_t)div_up(n > 0 ? n : 1, kCou
 // forward and 2.8 back, with 768 it takes 1.0 and 1.1; 6 M at 1600x1066 (chosen: 4096) 5.8 -> 4.7 ms.
 constexpr uint32_t kLongListDefault = 8192, kLeastThreshold = 512, kChosenThreshold = 5;
 constexpr float kThresholdShare = 1.5f, kWavesHeld = 5120.0f;         // (256 compute units, twenty waves each)
+// words of htgs_frame.long_counters: a line for each of the eight dies that the workgroups' indices go round (a work counter for
+// each of the long-list kernels' rounds and the workgroups that are done), then, for all of them, a word per round but the
+// last, set if the list may hold an entry for it, the dies that are done, and the share of a long list that a wave should get
+// (0: not chosen)
+constexpr uint32_t kDies = 8, kDieLine = 32, kDieRounds = kDies * kDieLine, kChosenShare = kDieRounds + 8;
+static_assert(HTGS_LONG_COUNTERS == kDieRounds + kDieLine, "a line per die and one for all");
+// What a wave of the long-list kernels gets of a list at least: half of what it would walk of all long lists if they were
+// shared evenly (longer shares spread badly, shorter ones cost more merges: 6 M Gaussians of the stress scene 5000 us with a
+// half, 5060 with all of it, 5560 with a quarter of the threshold), between two batches and the threshold.
+constexpr float kPartShare = 0.5f, kLongWavesOnDevice = 4096.0f;
+constexpr uint32_t kLeastShare = 128;
 struct ListThreshold {
     uint32_t fixed;                        // 0: chosen on the device
     InstanceCount count;
     uint32_t waves;                        // per tile
+    uint32_t part_waves;                   // of a workgroup that walks a part of a long list
+    uint32_t *counters;                    // htgs_frame.long_counters
     __device__ __forceinline__ uint32_t get(const uint32_t *long_tiles) const
     {
         if (fixed != 0u || long_tiles == nullptr) return fixed;
@@ -186,12 +199,38 @@ struct ListThreshold {
         const float t = kThresholdShare / kWavesHeld * (float)waves * (float)count.get();
         return t < 2.0f * kLeastThreshold ? 2u * kLeastThreshold : t < (float)kLongListDefault ? (uint32_t)t : kLongListDefault;
     }
+    // the least length of such a part
+    __device__ __forceinline__ uint32_t least_part(uint32_t long_threshold) const
+    {
+        const uint32_t share = fixed == 0u && counters != nullptr ? counters[kChosenShare] : 0u;
+        return share != 0u ? share * part_waves : part_waves / 4u * long_threshold;
+    }
+    // The backward pass's parts, which one workgroup walks each: of a threshold's length, and shorter where the long lists are
+    // few (20 k Gaussians of the stress scene at 400x300: a quarter of it 331 us a training step, all of it 370; 600 k at
+    // 700x500, OIT: 692 and 670).
+    __device__ __forceinline__ uint32_t least_backward_part(uint32_t long_threshold) const
+    {
+        const uint32_t share = fixed == 0u && counters != nullptr ? 2u * counters[kChosenShare] : 0u;
+        return share == 0u || share > long_threshold ? long_threshold : share > long_threshold / 4u ? share : long_threshold / 4u;
+    }
 };
 inline bool chooses_threshold(const htgs_frame *f) { return f->long_list_threshold < 0 && f->long_tiles != nullptr; }
+// The waves of a workgroup of the long-list kernels, of which a compute unit holds sixteen.  Sixteen to a workgroup shorten a
+// list most, but then a compute unit stands still while a workgroup merges its shares and takes its next part; two
+// workgroups of eight fill in for each other.  Where the lists are few the first counts, where they are many the
+// second: stress scene, K = 16, 16 waves -> 8: 300 k Gaussians at 1600x1000 602 -> 640 us, at 1024x768 425 -> 465, 600 k at
+// 1600x1000 932 -> 825, 1 M at 700x500 644 -> 588, 6 M at 1600x1066 5600 -> 5000.  The sums of OIT_BLEND are merged at once
+// (2.6 M Gaussians at 640x403: 796 -> 713 us) and a core of 32 leaves registers for eight waves only.
+constexpr int kOitLongWaves = 8, kManyGaussians = 1 << 19;
+inline uint32_t long_waves_of(const htgs_frame *f)
+{
+    if (f->mode == HTGS_MODE_OIT_BLEND) return kOitLongWaves;
+    return htgs_effective_k(f->K) > 16 || f->n_primitives > kManyGaussians ? 8u : 16u;
+}
 inline ListThreshold list_threshold(const htgs_frame *f)
 {
     const uint32_t fixed = f->long_list_threshold > 0 ? (uint32_t)f->long_list_threshold : chooses_threshold(f) ? 0u : kLongListDefault;
-    return ListThreshold{ fixed, instance_count(f), f->waves_per_tile > 1 ? (uint32_t)f->waves_per_tile : 1u };
+    return ListThreshold{ fixed, instance_count(f), f->waves_per_tile > 1 ? (uint32_t)f->waves_per_tile : 1u, long_waves_of(f), f->long_counters };
 }
 // the longest list that the kernels with one workgroup per tile can meet
 inline uint32_t most_threshold(const htgs_frame *f) { return chooses_threshold(f) || f->long_list_threshold == 0 ? kLongListDefault : (uint32_t)f->long_list_threshold; }

@@ -409,13 +409,15 @@ __global__ void __launch_bounds__(256) extract_ranges_kernel(const KeyT *__restr
 // zeroes p[0, n) and, if given, the eight words at `also` and the kOrderWords words at `also_order`
 constexpr uint32_t kOrderBuckets = 132;                   // (130 in use)
 constexpr uint32_t kOrderWords = 2 * kOrderBuckets;       // bin totals, bin cursors
-__global__ void __launch_bounds__(256) fill_zero_kernel(uint32_t *p, size_t n, uint32_t *also, uint32_t *also_order, uint32_t *also_bins)
+__global__ void __launch_bounds__(256) fill_zero_kernel(uint32_t *p, size_t n, uint32_t *also, uint32_t *also_order, uint32_t *also_bins,
+                                                       uint32_t *also_counters)
 {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i < n) p[i] = 0;
     if (i < 8 && also) also[i] = 0;
     if (i < kOrderWords && also_order) also_order[i] = 0;
     if (i < kOrderBuckets && also_bins) also_bins[i] = 0;
+    if (i < HTGS_LONG_COUNTERS && also_counters) also_counters[i] = 0;
 }
 
 // The order in which the blend kernels take the tiles: longest lists first, in groups of neighbours.  One workgroup walks
@@ -474,13 +476,14 @@ __device__ __forceinline__ uint32_t order_place(uint32_t place, uint32_t t, uint
 }
 // ListThreshold: the lists by length, in the bins of the order (s_lists[b]: lists in bin b; 256 threads or more).  The launch
 // over the lists up to a bin's upper end is as long as their instances over the waves that the device holds; the largest
-// end that is within kThresholdShare times that is the threshold.
+// end that is within kThresholdShare times that is the threshold.  What is in the lists beyond it, over the waves of the kernels
+// for those, gives the shares that they cut such lists into (kPartShare).
 __device__ __forceinline__ uint32_t bin_end(uint32_t bucket)           // the longest list of a bin (1 .. 128)
 {
     const uint32_t q = 128u - bucket, p = q / 4u, sub = q % 4u;
     return p >= 2u ? ((5u + sub) << (p - 2u)) - 1u : (1u << (p + 1u)) - 1u;
 }
-__device__ __forceinline__ void choose_threshold(const uint32_t *s_lists, float *s_sums, uint32_t *s_best, uint32_t waves, uint32_t *long_tiles)
+__device__ __forceinline__ void choose_threshold(const uint32_t *s_lists, float *s_sums, uint32_t *s_best, uint32_t waves, uint32_t *long_tiles, uint32_t *counters)
 {
     const uint32_t t = threadIdx.x, bucket = 128u - t;                  // (t = 0 .. 127: shortest first)
     const float end = t < 128u ? (float)bin_end(bucket) : 0.0f;
@@ -494,7 +497,13 @@ __device__ __forceinline__ void choose_threshold(const uint32_t *s_lists, float 
     }
     if (t < 128u && end <= (float)kLongListDefault && end <= kThresholdShare / kWavesHeld * (float)waves * s_sums[t]) atomicMax(s_best, (uint32_t)end);
     __syncthreads();
+    const float best = (float)*s_best;
     if (t == 0) long_tiles[kChosenThreshold] = *s_best;
+    // (the last bin whose lists are not long)
+    if (counters != nullptr && t < 127u && end <= best && (float)bin_end(bucket - 1u) > best) {
+        const float share = kPartShare / kLongWavesOnDevice * (s_sums[127] - s_sums[t]);
+        counters[kChosenShare] = share < (float)kLeastShare ? kLeastShare : share < best ? (uint32_t)share : *s_best;
+    }
 }
 __global__ void __launch_bounds__(256) tile_order_count_kernel(const uint32_t *__restrict__ ranges, uint32_t *__restrict__ order, uint32_t grid_w,
                                                                uint32_t grid_h, uint32_t *__restrict__ list_bins)
@@ -515,7 +524,8 @@ __global__ void __launch_bounds__(256) tile_order_count_kernel(const uint32_t *_
     if (list_bins != nullptr && threadIdx.x < kOrderBuckets && lists[threadIdx.x]) atomicAdd(list_bins + threadIdx.x, lists[threadIdx.x]);
 }
 __global__ void __launch_bounds__(256) tile_order_place_kernel(const uint32_t *__restrict__ ranges, uint32_t *__restrict__ order, uint32_t grid_w,
-                                                               uint32_t grid_h, const uint32_t *__restrict__ list_bins, uint32_t waves, uint32_t *__restrict__ long_tiles)
+                                                               uint32_t grid_h, const uint32_t *__restrict__ list_bins, uint32_t waves, uint32_t *__restrict__ long_tiles,
+                                                               uint32_t *__restrict__ long_counters)
 {
     __shared__ uint32_t count[kOrderBuckets], total[kOrderBuckets], base[kOrderBuckets];
     if (list_bins != nullptr && blockIdx.x == gridDim.x - 1) {          // (one block more than the tiles ask for)
@@ -523,7 +533,7 @@ __global__ void __launch_bounds__(256) tile_order_place_kernel(const uint32_t *_
         __shared__ uint32_t best;
         if (threadIdx.x < kOrderBuckets) total[threadIdx.x] = list_bins[threadIdx.x];
         __syncthreads();
-        choose_threshold(total, sums, &best, waves, long_tiles);
+        choose_threshold(total, sums, &best, waves, long_tiles, long_counters);
         return;
     }
     const uint32_t n_tiles = grid_w * grid_h, n_groups = n_tiles / kOrderGroup;
@@ -554,7 +564,8 @@ __global__ void __launch_bounds__(256) tile_order_place_kernel(const uint32_t *_
 // The two in one workgroup, for small grids.
 constexpr uint32_t kOneGroupTiles = 4096;
 __global__ void __launch_bounds__(1024) tile_order_one_group_kernel(const uint32_t *__restrict__ ranges, uint32_t *__restrict__ order, uint32_t grid_w,
-                                                                    uint32_t grid_h, uint32_t waves, uint32_t *__restrict__ long_tiles)
+                                                                    uint32_t grid_h, uint32_t waves, uint32_t *__restrict__ long_tiles,
+                                                               uint32_t *__restrict__ long_counters)
 {
     __shared__ uint32_t count[kOrderBuckets], lists[kOrderBuckets], base[kOrderBuckets], best;
     __shared__ float sums[128];
@@ -588,7 +599,7 @@ __global__ void __launch_bounds__(1024) tile_order_one_group_kernel(const uint32
         if (group < n_groups) order[order_place(place, t, n_groups)] = tiles[k];
         else if (i < n_tiles) order[i] = strip_order_tile(i, grid_w, grid_h);
     }
-    if (long_tiles != nullptr) choose_threshold(lists, sums, &best, waves, long_tiles);
+    if (long_tiles != nullptr) choose_threshold(lists, sums, &best, waves, long_tiles, long_counters);
 }
 
 // Scratch of htgs_scan_offsets_static: the per-block sums of the scan, held in the library's own device image so
@@ -666,7 +677,8 @@ static int launch_scan(const htgs_frame *f, uint32_t *tile_sums, const char *who
             hipLaunchKernelGGL(scan_reduce_kernel, dim3(tiles), dim3(kScanBlock), 0, s, counts, tile_sums, n);
         hipLaunchKernelGGL(scan_apply_kernel, dim3(tiles), dim3(kScanBlock), 0, s, counts, tile_sums, f->offsets, f->n_instances_dev, n, host_total, tag, sums_per_tile);
     } else {
-        hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(256), 0, s, f->n_instances_dev, (size_t)1, (uint32_t *)nullptr, (uint32_t *)nullptr, (uint32_t *)nullptr);
+        hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(256), 0, s, f->n_instances_dev, (size_t)1, (uint32_t *)nullptr, (uint32_t *)nullptr, (uint32_t *)nullptr,
+                           (uint32_t *)nullptr);
     }
     return check_launch("scan");
 }
@@ -816,10 +828,11 @@ int extract_ranges_of(const htgs_frame *f, int selector, bool cleared, bool rang
     const size_t n_tiles = (size_t)div_up(f->width, tile) * div_up(f->height, tile);
     // (the words for the tiles' finished parts are free until the blend)
     uint32_t *const list_bins = f->tile_order && chooses_threshold(f) && n_tiles >= kOrderBuckets ? f->long_tiles + 8 + 2 * n_tiles : nullptr;
-    const size_t to_zero = 2 * n_tiles > kOrderWords ? 2 * n_tiles : kOrderWords;
+    constexpr size_t kMostWords = kOrderWords > HTGS_LONG_COUNTERS ? kOrderWords : HTGS_LONG_COUNTERS;
+    const size_t to_zero = 2 * n_tiles > kMostWords ? 2 * n_tiles : kMostWords;
     if (!cleared)
         hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((to_zero + 255) / 256)), dim3(256), 0, s, f->ranges, ranged ? (size_t)0 : 2 * n_tiles, f->long_tiles,
-                           f->tile_order ? f->tile_order + n_tiles : nullptr, list_bins);
+                           f->tile_order ? f->tile_order + n_tiles : nullptr, list_bins, f->long_tiles ? f->long_counters : nullptr);
     if (f->n_instances > 0 && !ranged) {
         if (!f->keys[selector]) return fail(HTGS_ERR_ARGUMENT, "htgs_extract_ranges: null pointer");
         if ((uintptr_t)f->keys[selector] & 15) return fail(HTGS_ERR_ARGUMENT, "htgs_extract_ranges: keys must be 16-byte aligned");
@@ -838,11 +851,12 @@ int extract_ranges_of(const htgs_frame *f, int selector, bool cleared, bool rang
         const dim3 grid((unsigned)((n_tiles + 255) / 256)), block(256);
         const uint32_t waves = f->waves_per_tile > 1 ? (uint32_t)f->waves_per_tile : 1u;
         if (n_tiles <= kOneGroupTiles) {
-            hipLaunchKernelGGL(tile_order_one_group_kernel, dim3(1), dim3(1024), 0, s, f->ranges, f->tile_order, grid_w, grid_h, waves, list_bins ? f->long_tiles : nullptr);
+            hipLaunchKernelGGL(tile_order_one_group_kernel, dim3(1), dim3(1024), 0, s, f->ranges, f->tile_order, grid_w, grid_h, waves, list_bins ? f->long_tiles : nullptr,
+                               f->long_counters);
             return check_launch("extract_ranges");
         }
         hipLaunchKernelGGL(tile_order_count_kernel, grid, block, 0, s, f->ranges, f->tile_order, grid_w, grid_h, list_bins);
-        hipLaunchKernelGGL(tile_order_place_kernel, dim3(grid.x + (list_bins ? 1u : 0u)), block, 0, s, f->ranges, f->tile_order, grid_w, grid_h, list_bins, waves, f->long_tiles);
+        hipLaunchKernelGGL(tile_order_place_kernel, dim3(grid.x + (list_bins ? 1u : 0u)), block, 0, s, f->ranges, f->tile_order, grid_w, grid_h, list_bins, waves, f->long_tiles, f->long_counters);
     }
     return check_launch("extract_ranges");
 }

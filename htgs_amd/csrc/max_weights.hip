@@ -48,7 +48,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
         const uint32_t long_threshold = threshold.get(long_tiles);
         if (long_tiles != nullptr && length > long_threshold) {
             constexpr uint32_t part_words = MODE == HTGS_MODE_HYBRID_BLEND ? long_part_words<KS>() : MODE == HTGS_MODE_OIT_BLEND ? kOitPartWords : first_k_part_words<KS>();
-            if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, length, long_threshold, part_words, part_floor.get(gridDim.x));
+            if (lane == 0) long_tile_enter(long_tiles, tile, gridDim.x, length, threshold.least_part(long_threshold), part_words, part_floor.get(gridDim.x), long_threshold, threshold.counters);
             return;
         }
     }
@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(256) max_weights_tail_enter_kernel(const uint3
     if (tile >= n_tiles) return;
     const uint32_t length = ranges[2 * tile + 1] - ranges[2 * tile];
     const uint32_t long_threshold = threshold.get(long_tiles);
-    if (length > long_threshold) long_tile_enter(long_tiles, tile, n_tiles, length, long_threshold / 4u, 0u, part_floor.get(n_tiles));   // (parts of one threshold's length)
+    if (length > long_threshold) long_tile_enter(long_tiles, tile, n_tiles, length, long_threshold, 0u, part_floor.get(n_tiles), long_threshold, threshold.counters);   // (parts of one threshold's length)
 }
 // The second walk (alpha * tail weight for every fragment that passes the cut-off) over the parts of the very long lists:
 // a workgroup of four waves per part, every wave a share of it; the maximum is order independent, nothing to merge.
@@ -231,7 +231,7 @@ __global__ void __launch_bounds__(64 * kTailWaves) max_weights_tail_long_kernel(
     const uint32_t long_threshold = threshold.get(long_tiles);
     uint32_t round = 0;
     LongEntry e;
-    while (long_tile_take(long_tiles, ranges, long_threshold, round, &s_next, e)) {
+    while (long_tile_take(long_tiles, ranges, long_threshold, threshold.counters, round, &s_next, e)) {
         const TilePixel px = quadrant_tile_pixel(e.tile, grid_w, lane, width, height);
         const PixelTerms pt = px.pt;
         const float tail_weight = px.inside ? tail_weights[64u * (size_t)e.tile + lane] : 0.0f;
@@ -272,15 +272,11 @@ static void launch_tile(const htgs_frame *f, int sel, uint32_t *max_weights, flo
     if (!shared || !may_have_long_lists(f)) return;
     constexpr int REC4 = HTGS_PRIM_FLOATS / 4;
     if constexpr (MODE == HTGS_MODE_HYBRID_BLEND)
-        hipLaunchKernelGGL((blend_hybrid_long_kernel<K, false, REC4, MaxWeightsHybrid>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0, s,
-                           f->ranges, f->vals[sel], (const float4 *)f->prim, f->long_tiles, w, h, grid_w, f->vals[sel ^ 1], threshold,
-                           MaxWeightsHybrid{ max_weights, f->pixel_scratch, thr });
+        launch_hybrid_long<K, false, REC4>(f, sel, grid_w, MaxWeightsHybrid{ max_weights, f->pixel_scratch, thr });
     else if constexpr (MODE == HTGS_MODE_ALPHA_BLEND_FIRST_K)
-        hipLaunchKernelGGL((blend_first_k_long_kernel<K, false, REC4, MaxWeightsFirstK>), dim3(256 * kLongWaves / long_waves<K>()), dim3(64 * long_waves<K>()), 0, s,
-                           f->ranges, f->vals[sel], (const float4 *)f->prim, f->long_tiles, w, h, grid_w, f->vals[sel ^ 1], threshold, MaxWeightsFirstK{ max_weights, thr });
+        launch_first_k_long<K, false, REC4>(f, sel, grid_w, MaxWeightsFirstK{ max_weights, thr });
     else
-        hipLaunchKernelGGL((blend_oit_long_kernel<false, REC4, MaxWeightsOit, false>), dim3(256), dim3(64 * kLongWaves), 0, s, f->ranges, f->vals[sel],
-                           (const float4 *)f->prim, f->long_tiles, w, h, grid_w, f->vals[sel ^ 1], threshold, MaxWeightsOit{ f->pixel_scratch, thr });
+        launch_oit_long<false, REC4, false>(f, sel, grid_w, MaxWeightsOit{ f->pixel_scratch, thr });
     if constexpr (MODE != HTGS_MODE_ALPHA_BLEND_FIRST_K) {
         hipLaunchKernelGGL(max_weights_tail_enter_kernel, dim3((n_tiles + 255) / 256), dim3(256), 0, s, f->ranges, f->long_tiles, n_tiles, threshold,
                            part_floor_of(f, sel, false));

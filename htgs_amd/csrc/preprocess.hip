@@ -225,7 +225,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SH_REG
         const uint32_t sum = wave_sum_last(in_range ? touched : 0u);
         if ((threadIdx.x & (kWave - 1)) == kWave - 1) s_counts[threadIdx.x / kWave] = sum;
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < 5; ++k)
             for (uint32_t w = blockIdx.x * 256u + threadIdx.x; w < start.clear_words[k]; w += gridDim.x * 256u) start.clear[k][w] = 0u;
     }
     // htgs_frame.depth_order: the pairs that sort the Gaussians by depth (depth_key_range() in common.h)

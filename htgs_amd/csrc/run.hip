@@ -117,6 +117,7 @@ static uint64_t carve_front(htgs_frame *f, int what, void *base)
     f->ranges = c.take<uint32_t>(2 * n_tiles);
     // (the modes that walk all of a list)
     f->long_tiles = f->mode != HTGS_MODE_ALPHA_BLEND_GLOBAL_ORDERING ? c.take<uint32_t>(8 + 3 * n_tiles) : nullptr;
+    f->long_counters = f->mode != HTGS_MODE_ALPHA_BLEND_GLOBAL_ORDERING ? c.take<uint32_t>(HTGS_LONG_COUNTERS) : nullptr;
     f->waves_per_tile = waves_of(f, what, n_tiles);
     f->long_list_threshold = -1;                           // (ListThreshold)
     // (a grid whose workgroups are all on the device at once is taken in any order)
@@ -196,6 +197,7 @@ static int queue_front(const htgs_frame *f, const htgs_workspace *w, HostWord *w
         }
         if (f->long_tiles) {
             start.clear[2] = f->long_tiles; start.clear_words[2] = 8;
+            start.clear[4] = f->long_counters; start.clear_words[4] = HTGS_LONG_COUNTERS;
             if (f->tile_order) { start.clear[3] = f->long_tiles + 8 + 2 * (size_t)n_tiles; start.clear_words[3] = n_tiles < 132 ? n_tiles : 132; }
         }
     }

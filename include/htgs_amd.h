@@ -40,6 +40,7 @@ extern "C" {
  * list (offsets[g-1]), the tile at the corner of its rectangle, the rectangle's width or the mask of its listed tiles --
  * then padding */
 #define HTGS_PRIM_FLOATS_TRAIN 32
+#define HTGS_LONG_COUNTERS 288
 
 /*
  * One frame: inputs, caller-owned scratch and outputs.  Mirrors the argument list of
@@ -106,6 +107,10 @@ typedef struct htgs_frame {
                                   and htgs_blend_forward give it as many, which walk a share of its list each and merge
                                   what they have -- for grids of few tiles.  Needs long_tiles and a threshold of no more than
                                   8192 (ignored otherwise).  Results agree up to the order of sums */
+    uint32_t *long_counters;   /* [HTGS_LONG_COUNTERS] or NULL: work counters of long_tiles, a cache line for each accelerator die, in
+                                  place of words 1-4 of its header, which all dies otherwise contend for.  Zeroed and left
+                                  zero as those are; a frame has it for all of its stages or for none.  Ignored without
+                                  long_tiles */
     uint32_t *tile_order;      /* htgs_tile_order_words() words or NULL.  Written by htgs_extract_ranges: the n_tiles tiles
                                   in groups of sixteen neighbours (a 4x4 patch), the groups with the longest lists first
                                   (binned by total length, four bins per power of two) and a group's tiles at the
