@@ -173,7 +173,9 @@ inline size_t block_sum_words(int n) { return (size_t)div_up(n > 0 ? n : 1, kCou
 // With the fixed threshold of 8192 the training pass of 600 k Gaussians of the stress scene at 1026x792, K = 32, took 3.0 ms
 // forward and 2.8 back, with 768 it takes 1.0 and 1.1; 6 M at 1600x1066 (chosen: 4096) 5.8 -> 4.7 ms.
 constexpr uint32_t kLongListDefault = 8192, kLeastThreshold = 512, kChosenThreshold = 5;
-constexpr float kThresholdShare = 1.5f, kWavesHeld = 5120.0f;         // (256 compute units, twenty waves each)
+// Weights of a tail take two walks, of which most tiles with long lists are spared the second: there the length is 2.5 times as
+// much (weights of 2.9 M at 1416x701, OIT: 1150 -> 735 us; images and training lose 2 to 20 per cent with 2.5).
+constexpr float kThresholdShare = 1.5f, kWeightsShare = 2.5f, kWavesHeld = 5120.0f;         // (256 compute units, twenty waves each)
 // words of htgs_frame.long_counters: a line for each of the eight dies that the workgroups' indices go round (a work counter for
 // each of the long-list kernels' rounds and the workgroups that are done), then, for all of them, a word per round but the
 // last, set if the list may hold an entry for it, the dies that are done, and the share of a long list that a wave should get
@@ -188,7 +190,7 @@ constexpr uint32_t kLeastShare = 128;
 struct ListThreshold {
     uint32_t fixed;                        // 0: chosen on the device
     InstanceCount count;
-    uint32_t waves;                        // per tile
+    float share;                           // threshold_share
     uint32_t part_waves;                   // of a workgroup that walks a part of a long list
     uint32_t *counters;                    // htgs_frame.long_counters
     __device__ __forceinline__ uint32_t get(const uint32_t *long_tiles) const
@@ -196,7 +198,7 @@ struct ListThreshold {
         if (fixed != 0u || long_tiles == nullptr) return fixed;
         const uint32_t chosen = long_tiles[kChosenThreshold];
         if (chosen != 0u) return chosen;
-        const float t = kThresholdShare / kWavesHeld * (float)waves * (float)count.get();
+        const float t = share / kWavesHeld * (float)count.get();
         return t < 2.0f * kLeastThreshold ? 2u * kLeastThreshold : t < (float)kLongListDefault ? (uint32_t)t : kLongListDefault;
     }
     // the least length of such a part
@@ -227,10 +229,15 @@ inline uint32_t long_waves_of(const htgs_frame *f)
     if (f->mode == HTGS_MODE_OIT_BLEND) return kOitLongWaves;
     return htgs_effective_k(f->K) > 16 || f->n_primitives > kManyGaussians ? 8u : 16u;
 }
+// kThresholdShare times the waves that a tile has (pixel_scratch: max weights)
+inline float threshold_share(const htgs_frame *f)
+{
+    return f->pixel_scratch != nullptr ? kWeightsShare : kThresholdShare * (f->waves_per_tile > 1 ? (float)f->waves_per_tile : 1.0f);
+}
 inline ListThreshold list_threshold(const htgs_frame *f)
 {
     const uint32_t fixed = f->long_list_threshold > 0 ? (uint32_t)f->long_list_threshold : chooses_threshold(f) ? 0u : kLongListDefault;
-    return ListThreshold{ fixed, instance_count(f), f->waves_per_tile > 1 ? (uint32_t)f->waves_per_tile : 1u, long_waves_of(f), f->long_counters };
+    return ListThreshold{ fixed, instance_count(f), threshold_share(f), long_waves_of(f), f->long_counters };
 }
 // the longest list that the kernels with one workgroup per tile can meet
 inline uint32_t most_threshold(const htgs_frame *f) { return chooses_threshold(f) || f->long_list_threshold == 0 ? kLongListDefault : (uint32_t)f->long_list_threshold; }

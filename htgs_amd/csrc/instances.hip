@@ -483,7 +483,7 @@ __device__ __forceinline__ uint32_t bin_end(uint32_t bucket)           // the lo
     const uint32_t q = 128u - bucket, p = q / 4u, sub = q % 4u;
     return p >= 2u ? ((5u + sub) << (p - 2u)) - 1u : (1u << (p + 1u)) - 1u;
 }
-__device__ __forceinline__ void choose_threshold(const uint32_t *s_lists, float *s_sums, uint32_t *s_best, uint32_t waves, uint32_t *long_tiles, uint32_t *counters)
+__device__ __forceinline__ void choose_threshold(const uint32_t *s_lists, float *s_sums, uint32_t *s_best, float launch_share, uint32_t *long_tiles, uint32_t *counters)
 {
     const uint32_t t = threadIdx.x, bucket = 128u - t;                  // (t = 0 .. 127: shortest first)
     const float end = t < 128u ? (float)bin_end(bucket) : 0.0f;
@@ -495,7 +495,7 @@ __device__ __forceinline__ void choose_threshold(const uint32_t *s_lists, float 
         __syncthreads();
         if (t < 128u) s_sums[t] += before;
     }
-    if (t < 128u && end <= (float)kLongListDefault && end <= kThresholdShare / kWavesHeld * (float)waves * s_sums[t]) atomicMax(s_best, (uint32_t)end);
+    if (t < 128u && end <= (float)kLongListDefault && end <= launch_share / kWavesHeld * s_sums[t]) atomicMax(s_best, (uint32_t)end);
     __syncthreads();
     const float best = (float)*s_best;
     if (t == 0) long_tiles[kChosenThreshold] = *s_best;
@@ -524,7 +524,7 @@ __global__ void __launch_bounds__(256) tile_order_count_kernel(const uint32_t *_
     if (list_bins != nullptr && threadIdx.x < kOrderBuckets && lists[threadIdx.x]) atomicAdd(list_bins + threadIdx.x, lists[threadIdx.x]);
 }
 __global__ void __launch_bounds__(256) tile_order_place_kernel(const uint32_t *__restrict__ ranges, uint32_t *__restrict__ order, uint32_t grid_w,
-                                                               uint32_t grid_h, const uint32_t *__restrict__ list_bins, uint32_t waves, uint32_t *__restrict__ long_tiles,
+                                                               uint32_t grid_h, const uint32_t *__restrict__ list_bins, float share, uint32_t *__restrict__ long_tiles,
                                                                uint32_t *__restrict__ long_counters)
 {
     __shared__ uint32_t count[kOrderBuckets], total[kOrderBuckets], base[kOrderBuckets];
@@ -533,7 +533,7 @@ __global__ void __launch_bounds__(256) tile_order_place_kernel(const uint32_t *_
         __shared__ uint32_t best;
         if (threadIdx.x < kOrderBuckets) total[threadIdx.x] = list_bins[threadIdx.x];
         __syncthreads();
-        choose_threshold(total, sums, &best, waves, long_tiles, long_counters);
+        choose_threshold(total, sums, &best, share, long_tiles, long_counters);
         return;
     }
     const uint32_t n_tiles = grid_w * grid_h, n_groups = n_tiles / kOrderGroup;
@@ -564,7 +564,7 @@ __global__ void __launch_bounds__(256) tile_order_place_kernel(const uint32_t *_
 // The two in one workgroup, for small grids.
 constexpr uint32_t kOneGroupTiles = 4096;
 __global__ void __launch_bounds__(1024) tile_order_one_group_kernel(const uint32_t *__restrict__ ranges, uint32_t *__restrict__ order, uint32_t grid_w,
-                                                                    uint32_t grid_h, uint32_t waves, uint32_t *__restrict__ long_tiles,
+                                                                    uint32_t grid_h, float share, uint32_t *__restrict__ long_tiles,
                                                                uint32_t *__restrict__ long_counters)
 {
     __shared__ uint32_t count[kOrderBuckets], lists[kOrderBuckets], base[kOrderBuckets], best;
@@ -599,7 +599,7 @@ __global__ void __launch_bounds__(1024) tile_order_one_group_kernel(const uint32
         if (group < n_groups) order[order_place(place, t, n_groups)] = tiles[k];
         else if (i < n_tiles) order[i] = strip_order_tile(i, grid_w, grid_h);
     }
-    if (long_tiles != nullptr) choose_threshold(lists, sums, &best, waves, long_tiles, long_counters);
+    if (long_tiles != nullptr) choose_threshold(lists, sums, &best, share, long_tiles, long_counters);
 }
 
 // Scratch of htgs_scan_offsets_static: the per-block sums of the scan, held in the library's own device image so
@@ -849,14 +849,14 @@ int extract_ranges_of(const htgs_frame *f, int selector, bool cleared, bool rang
     if (f->tile_order) {
         const uint32_t grid_w = (uint32_t)div_up(f->width, tile), grid_h = (uint32_t)div_up(f->height, tile);
         const dim3 grid((unsigned)((n_tiles + 255) / 256)), block(256);
-        const uint32_t waves = f->waves_per_tile > 1 ? (uint32_t)f->waves_per_tile : 1u;
+        const float share = threshold_share(f);
         if (n_tiles <= kOneGroupTiles) {
-            hipLaunchKernelGGL(tile_order_one_group_kernel, dim3(1), dim3(1024), 0, s, f->ranges, f->tile_order, grid_w, grid_h, waves, list_bins ? f->long_tiles : nullptr,
+            hipLaunchKernelGGL(tile_order_one_group_kernel, dim3(1), dim3(1024), 0, s, f->ranges, f->tile_order, grid_w, grid_h, share, list_bins ? f->long_tiles : nullptr,
                                f->long_counters);
             return check_launch("extract_ranges");
         }
         hipLaunchKernelGGL(tile_order_count_kernel, grid, block, 0, s, f->ranges, f->tile_order, grid_w, grid_h, list_bins);
-        hipLaunchKernelGGL(tile_order_place_kernel, dim3(grid.x + (list_bins ? 1u : 0u)), block, 0, s, f->ranges, f->tile_order, grid_w, grid_h, list_bins, waves, f->long_tiles, f->long_counters);
+        hipLaunchKernelGGL(tile_order_place_kernel, dim3(grid.x + (list_bins ? 1u : 0u)), block, 0, s, f->ranges, f->tile_order, grid_w, grid_h, list_bins, share, f->long_tiles, f->long_counters);
     }
     return check_launch("extract_ranges");
 }
