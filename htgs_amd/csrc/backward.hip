@@ -677,24 +677,28 @@ __global__ void __launch_bounds__(256) blend_global_backward_kernel(
             });
         }
         __syncthreads();
-        // one thread per Gaussian of the batch: the quadrants' sums in a fixed order, the chain to the VPMT rows, the row
-        if (t < (uint32_t)nb) {
+        // Four lanes per Gaussian of the batch: each adds up its four of the sixteen sums over the quadrants, in their order
+        // (neighbouring lanes read neighbouring words of LDS, all of them at once), the four share them, and each writes a
+        // quarter of the row.
+        if (t < 4u * (uint32_t)nb) {
+            const uint32_t g = t >> 2, c = t & 3u;
+            const uint32_t reach = s_reach[g], walked = s_walked;
+            float own[4] = { 0.0f, 0.0f, 0.0f, 0.0f }, help = 0.0f;
+            bool any = false;
+#pragma unroll
+            for (uint32_t qd = 0; qd < 16; ++qd) {
+                const bool counts = ((reach >> qd) & 1u) && ((walked >> (qd >> 2)) & 1u);
+                const float4 p = s_part[qd][g][c];
+                own[0] += counts ? p.x : 0.0f; own[1] += counts ? p.y : 0.0f; own[2] += counts ? p.z : 0.0f; own[3] += counts ? p.w : 0.0f;
+                if (HELPER) { const float h = s_help[qd][g]; help += counts ? h : 0.0f; }
+                any = any || counts;
+            }
+            // (quad_perm: sums 4 r .. 4 r + 3 from lane r of the four)
             float m[16];
 #pragma unroll
-            for (int k = 0; k < 16; ++k) m[k] = 0.0f;
-            float help = 0.0f;
-            bool any = false;
-            const uint32_t reach = s_reach[t], walked = s_walked;
-            for (uint32_t qd = 0; qd < 16; ++qd) {
-                if (((reach >> qd) & 1u) && ((walked >> (qd >> 2)) & 1u)) {
-                    any = true;
-                    const float4 p0 = s_part[qd][t][0], p1 = s_part[qd][t][1], p2 = s_part[qd][t][2], p3 = s_part[qd][t][3];
-                    m[0] += p0.x; m[1] += p0.y; m[2] += p0.z; m[3] += p0.w;
-                    m[4] += p1.x; m[5] += p1.y; m[6] += p1.z; m[7] += p1.w;
-                    m[8] += p2.x; m[9] += p2.y; m[10] += p2.z; m[11] += p2.w;
-                    m[12] += p3.x; m[13] += p3.y; m[14] += p3.z; m[15] += p3.w;
-                    if (HELPER) help += s_help[qd][t];
-                }
+            for (int k = 0; k < 4; ++k) {
+                m[k] = dpp_take<0x00, 0xf>(own[k]); m[4 + k] = dpp_take<0x55, 0xf>(own[k]);
+                m[8 + k] = dpp_take<0xAA, 0xf>(own[k]); m[12 + k] = dpp_take<0xFF, 0xf>(own[k]);
             }
             RowGrads rg;
 #pragma unroll
@@ -704,15 +708,15 @@ __global__ void __launch_bounds__(256) blend_global_backward_kernel(
             for (int k = 0; k < 4; ++k) rg.e4[k] = 0.0f;
             if (any) {
                 const float S[6] = { m[4], m[5], m[6], m[7], m[8], m[9] }, Tm[6] = { m[10], m[11], m[12], m[13], m[14], m[15] };
-                moments_to_rows(s_rows[0][t], s_rows[1][t], s_rows[2][t], cx, cy, 2.0f * ModeCfg<MODE>::cutoff_rcp, S, Tm, rg);
+                moments_to_rows(s_rows[0][g], s_rows[1][g], s_rows[2][g], cx, cy, 2.0f * ModeCfg<MODE>::cutoff_rcp, S, Tm, rg);
             }
-            const uint32_t slot = instance_slot(s_rows[3][t], tile, grid_w);
-            float4 *row = grad_rows + 4 * (size_t)slot;
-            row[0] = make_float4(m[0], m[1], m[2], m[3]);
-            row[1] = make_float4(rg.da[0], rg.da[1], rg.da[2], rg.daw);
-            row[2] = make_float4(rg.db[0], rg.db[1], rg.db[2], rg.dbw);
-            row[3] = make_float4(rg.e4[0], rg.e4[1], rg.e4[2], rg.e4[3]);
-            if (HELPER) helper_rows[slot] = help;
+            const uint32_t slot = instance_slot(s_rows[3][g], tile, grid_w);
+            float4 out = make_float4(m[0], m[1], m[2], m[3]);
+            if (c == 1u) out = make_float4(rg.da[0], rg.da[1], rg.da[2], rg.daw);
+            if (c == 2u) out = make_float4(rg.db[0], rg.db[1], rg.db[2], rg.dbw);
+            if (c == 3u) out = make_float4(rg.e4[0], rg.e4[1], rg.e4[2], rg.e4[3]);
+            grad_rows[4 * (size_t)slot + c] = out;
+            if (HELPER && c == 0u) helper_rows[slot] = help;
         }
     }
     // instances behind the point where every pixel of the tile is saturated: rows of zeros
