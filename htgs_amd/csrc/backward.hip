@@ -602,23 +602,43 @@ __global__ void __launch_bounds__(256) blend_global_backward_kernel(
         if (__ballot(!done) != 0) {                                              // wave-uniform
             if (lane == 0) atomicOr(&s_walked, 1u << wave);
             QuadrantHits hits = quadrant_ballot(lane < (uint32_t)kGlobalBatch ? ((uint32_t)s_reach[lane] >> (4u * wave)) & 0xfu : 0u);
-            quadrant_walk<true>(hits, stage_base, [&](uint32_t addr) {
+            // Two turns at a time: what a fragment is without the transmittance, its alpha, is worked out for both together, two
+            // chains of some forty dependent instructions side by side (training step of 411 k Gaussians at 1297x839: 810 -> 774 us,
+            // of 51 k at 269x922: 826 -> 763).
+            struct Fragment {
+                uint32_t addr;
+                bool passes;
+                float G, alpha, opacity;
+                TileFrag f;
+            };
+            const auto evaluate = [&](uint32_t at) {
+                Fragment x;
+                // the forward pass's own arithmetic (blend_global_forward_kernel): same accept / reject decisions, same alpha
+                // (a quadrant without a hit left evaluates the batch's first slot, for nothing)
+                x.addr = at != kNoHit ? at + stage_base : stage_base;
+                const bool reached = tile_frag_cutoff<kGlobalBatch>(x.addr, pt, x.f);
+                x.f.den_rcp = rcp_exact(x.f.den);
+                x.G = d_exp2((x.f.num * ModeCfg<MODE>::exp2_scale) * x.f.den_rcp);
+                x.opacity = stage_opacity<kGlobalBatch>(x.addr);
+                const float ag = x.opacity * x.G;
+                x.alpha = ag < kMaxFragmentAlpha ? ag : kMaxFragmentAlpha;
+                x.passes = at != kNoHit && reached && !(x.alpha < ModeCfg<MODE>::min_alpha);
+                return x;
+            };
+            const auto turn = [&](const Fragment &x, bool listed) {
+                if (!listed) return;
+                const uint32_t addr = x.addr;
                 const uint32_t j = (addr - stage_base) >> 4;                     // the staged slot, the same in the quadrant's lanes
                 float acc[16];
 #pragma unroll
                 for (int k = 0; k < 16; ++k) acc[k] = 0.0f;
                 float help = 0.0f;
                 bool hit = false;
-                TileFrag f;
-                // the forward pass's own arithmetic (blend_global_forward_kernel): same accept / reject decisions, same alpha
-                if (!done && tile_frag_cutoff<kGlobalBatch>(addr, pt, f)) {
-                    f.den_rcp = rcp_exact(f.den);
-                    const float G = d_exp2((f.num * ModeCfg<MODE>::exp2_scale) * f.den_rcp);
-                    const float4 col = stage_row<kGlobalBatch, 5>(addr);
-                    const float opacity = stage_opacity<kGlobalBatch>(addr);
-                    const float ag = opacity * G;
-                    const float alpha = ag < kMaxFragmentAlpha ? ag : kMaxFragmentAlpha;
-                    if (!(alpha < ModeCfg<MODE>::min_alpha)) {
+                const TileFrag &f = x.f;
+                const float G = x.G, alpha = x.alpha, opacity = x.opacity;
+                if (!done && x.passes) {
+                    {
+                        const float4 col = stage_row<kGlobalBatch, 5>(addr);
                         hit = true;
                         const float bw = T * alpha;
                         acc[0] = bw * g0; acc[1] = bw * g1; acc[2] = bw * g2;                        // :171-174
@@ -674,7 +694,13 @@ __global__ void __launch_bounds__(256) blend_global_backward_kernel(
                     s_part[quadrant][j][lane >> 4] = make_float4(acc[0], acc[1], acc[2], acc[3]);
                     if (HELPER && lane < 16u) s_help[quadrant][j] = help;
                 }
-            });
+            };
+            while (quadrant_pending(hits)) {
+                const uint32_t one = quadrant_next_hit<true>(hits), two = quadrant_next_hit<true>(hits);
+                const Fragment x = evaluate(one), y = evaluate(two);
+                turn(x, one != kNoHit);
+                turn(y, two != kNoHit);
+            }
         }
         __syncthreads();
         // Four lanes per Gaussian of the batch: each adds up its four of the sixteen sums over the quadrants, in their order
