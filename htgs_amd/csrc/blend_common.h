@@ -425,11 +425,12 @@ __device__ __forceinline__ void quadrant_walk(QuadrantHits &hits, uint32_t stage
 // dummy slot, which fails the walk's own test, instead of being masked off: one exec level less.
 constexpr int kStageSlots = 65;
 typedef TileStage<kStageSlots> TileStageQ;
-struct QuadrantLists {
+struct __attribute__((aligned(8))) QuadrantLists {
     uint32_t a[4][64];
-    uint32_t beyond;            // (the walk reads one entry ahead)
+    uint32_t beyond[2];         // (the walks read one entry or one pair of entries ahead)
 };
 typedef __attribute__((address_space(3))) const uint32_t lds_u32;
+typedef __attribute__((address_space(3))) const uint64_t lds_u64;
 // (one lane) the slot that fails every test: |m|^2 / cut-off = 1 everywhere, |d|^2 = 1/2, opacity 0
 __device__ __forceinline__ void stage_dummy_init(TileStageQ &st, uint32_t lane)
 {
@@ -479,12 +480,33 @@ __device__ __forceinline__ void quadrant_list_walk(const QuadrantLists &ql, uint
     }
     if (t < n_turns) turn(addr);
 }
+// The same walk two turns at a time: turns(one, two) with the addresses of two turns in a row.  What the two fragments are is
+// worked out side by side, so that the waits of one -- for LDS, for a compare that a branch depends on -- are filled by the
+// other.  An odd number of turns ends with a turn of dummy slots (every list has 64 entries, the dummy's behind the hits).
+// A wave that runs alone issues an instruction every 2.5 ns, waits 24 ns for a row from LDS and 14 ns between a compare and
+// the branch on it; five waves a SIMD cover most of that but not all.  One turn -> two at a time, whole passes: HYBRID K = 16, 3 M
+// Gaussians at 1920x1080 1373 -> 1306 us, FIRST_K 1 M at 1280x720 351 -> 334, OIT 334 k at 1237x821 163.8 -> 159.8.  Cores of 32 have
+// no registers left for a second fragment and keep the walk above, like the walks with three registers a slot.
+template <typename Turns>
+__device__ __forceinline__ void quadrant_list_walk_pairs(const QuadrantLists &ql, uint32_t n_turns, uint32_t lane, Turns &&turns)
+{
+    uint32_t p = (uint32_t)(uintptr_t)(lds_u32 *)&ql.a[lane >> 4][0];
+    uint64_t at = *(lds_u64 *)(uintptr_t)p;
+    for (uint32_t t = 0; t < n_turns; t += 2) {
+        asm volatile("v_add_u32 %0, 8, %0" : "+v"(p));
+        const uint64_t next = *(lds_u64 *)(uintptr_t)p;
+        turns((uint32_t)at, (uint32_t)(at >> 32));
+        at = next;
+    }
+}
 // The walk over instances [first, last) of a tile's list (whole batches of 64 from `first` on) by one wave, lanes =
 // pixels by quadrants: every batch is staged (tile_stage_load with the CULL asked for), its quadrant lists are built and
 // turn(addr) is called for every turn.  SOLO: the wave is the whole workgroup (its barriers are the workgroup's).
 // AHEAD: a lane reads the list entry of the next batch before it walks this one (one register more through the walk; the
 // entry is then there when the batch is staged, and the records' fetch does not wait for it).
-template <int MODE, bool DEPTH, int CULL, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, bool UNIT = false, bool POS = false, bool AHEAD = false, typename Turn>
+// PAIRS: two turns at a time, turn(one, two).
+template <int MODE, bool DEPTH, int CULL, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, bool UNIT = false, bool POS = false, bool AHEAD = false, bool PAIRS = false,
+          typename Turn>
 __device__ __forceinline__ void tile_list_walk(TileStageQ &st, QuadrantLists &ql, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst,
                                                uint32_t first, uint32_t last, uint32_t lane, float cx, float cy, Turn &&turn, uint64_t pixel_lanes = 0,
                                                float cull_scale = 1.0f)
@@ -500,7 +522,8 @@ __device__ __forceinline__ void tile_list_walk(TileStageQ &st, QuadrantLists &ql
         const uint32_t n_turns = quadrant_lists_build(ql, bits, lane, st);
         if (SOLO) __syncthreads(); else wave_lds_sync();
         // lanes outside the image run along (their results are never stored): the loop stays wave-uniform
-        quadrant_list_walk(ql, n_turns, lane, turn);
+        if constexpr (PAIRS) quadrant_list_walk_pairs(ql, n_turns, lane, turn);
+        else quadrant_list_walk(ql, n_turns, lane, turn);
     }
 }
 // The per-pixel records of the training pass are kept tile by tile: the 64 pixels of an 8x8 tile, row-major, are
@@ -560,6 +583,44 @@ __device__ __forceinline__ bool tile_frag_alpha(float opacity, TileFrag &o)
     const float a = opacity * G;
     o.alpha = a < kMaxFragmentAlpha ? a : kMaxFragmentAlpha;
     return !(o.alpha < ModeCfg<MODE>::min_alpha);
+}
+
+// The exact fragment in one piece: whether it passes the cut-off and the alpha threshold; o is complete.  1 / |d|^2 is the refined
+// reciprocal, and the alpha is worked out with it before anything asks whether a lane's |d|^2 is outside that form's range
+// (rcp_exact's test): the branch then does not wait for its compare.
+template <int MODE, int N>
+__device__ __forceinline__ bool tile_frag_exact(uint32_t addr, const PixelTerms &p, TileFrag &o)
+{
+    const bool in_reach = tile_frag_cutoff<N>(addr, p, o);
+    const float opacity = stage_opacity<N>(addr);
+    const uint64_t leaves = __ballot(!rcp_in_range(o.den));
+    o.den_rcp = rcp_refined(o.den);
+    bool passes = tile_frag_alpha<MODE, false>(opacity, o);
+    if (__builtin_expect(leaves != 0, 0)) {
+        o.den_rcp = 1.0f / o.den;
+        passes = tile_frag_alpha<MODE, false>(opacity, o);
+    }
+    return passes && in_reach;
+}
+// two of them (quadrant_list_walk_pairs)
+template <int MODE, int N>
+__device__ __forceinline__ void tile_frag_exact_pair(uint32_t one, uint32_t two, const PixelTerms &p, TileFrag &o, TileFrag &t, bool &one_passes, bool &two_passes)
+{
+    const bool o_reach = tile_frag_cutoff<N>(one, p, o), t_reach = tile_frag_cutoff<N>(two, p, t);
+    const float o_opacity = stage_opacity<N>(one), t_opacity = stage_opacity<N>(two);
+    const uint64_t leaves = __ballot(!rcp_in_range(o.den)) | __ballot(!rcp_in_range(t.den));
+    o.den_rcp = rcp_refined(o.den);
+    t.den_rcp = rcp_refined(t.den);
+    one_passes = tile_frag_alpha<MODE, false>(o_opacity, o);
+    two_passes = tile_frag_alpha<MODE, false>(t_opacity, t);
+    if (__builtin_expect(leaves != 0, 0)) {
+        o.den_rcp = 1.0f / o.den;
+        t.den_rcp = 1.0f / t.den;
+        one_passes = tile_frag_alpha<MODE, false>(o_opacity, o);
+        two_passes = tile_frag_alpha<MODE, false>(t_opacity, t);
+    }
+    one_passes = one_passes && o_reach;
+    two_passes = two_passes && t_reach;
 }
 
 // The image-only fast path's fragment: with the opacity staged at no more than 1 (UNIT) alpha = opacity * G needs no clamp, and a

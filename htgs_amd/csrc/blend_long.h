@@ -75,11 +75,7 @@ __device__ __forceinline__ void hybrid_walk(TileStageQ &st, QuadrantLists &ql, c
         TileFrag f;
         bool fragment;
         if constexpr (FAST) fragment = tile_frag_fast<MODE, N>(addr, pt, f);
-        else {
-            const bool in_reach = tile_frag_cutoff<N>(addr, pt, f);
-            f.den_rcp = frag_rcp<FAST>(f.den);
-            fragment = tile_frag_alpha<MODE, FAST>(stage_opacity<N>(addr), f) && in_reach;
-        }
+        else fragment = tile_frag_exact<MODE, N>(addr, pt, f);
         const float4 col = stage_row<N, 5>(addr);
         if (!fragment) return;
         float depth = tile_frag_depth<N>(addr, pt, f);
@@ -131,10 +127,8 @@ __device__ __forceinline__ KeyFormat key_format(uint32_t list_length)      // 1 
 __device__ __forceinline__ float key_depth(CoreKey k) { return bits_to_float((uint32_t)__double2hiint(k)); }
 __device__ __forceinline__ uint32_t key_low(CoreKey k) { return (uint32_t)__double2loint(k); }
 __device__ __forceinline__ CoreKey make_key(float depth, uint32_t low) { return __hiloint2double((int)float_to_bits(depth), (int)low); }
-__device__ __forceinline__ uint32_t key_pack(float alpha, uint32_t place, const KeyFormat &f)      // alpha in [0, 1]
-{
-    return (uint32_t)__builtin_fmaf(alpha, f.one, 0.5f) << f.shift | place;
-}
+__device__ __forceinline__ uint32_t key_fraction(float alpha, const KeyFormat &f) { return (uint32_t)__builtin_fmaf(alpha, f.one, 0.5f); }      // alpha in [0, 1]
+__device__ __forceinline__ uint32_t key_pack(float alpha, uint32_t place, const KeyFormat &f) { return key_fraction(alpha, f) << f.shift | place; }
 __device__ __forceinline__ float key_alpha(uint32_t low, const KeyFormat &f) { return (float)(low >> f.shift) * f.one_rcp; }
 __device__ __forceinline__ void key_step(CoreKey &carried, CoreKey &slot)
 {
@@ -164,42 +158,52 @@ __device__ __forceinline__ void hybrid_key_walk(TileStageQ &st, QuadrantLists &q
 {
     constexpr int MODE = HTGS_MODE_HYBRID_BLEND;
     constexpr int N = kStageSlots;
-    tile_list_walk<MODE, true, kCullAlpha, SOLO, REC4, FAST, true, AHEAD>(st, ql, prim, inst, first, last, lane, cx, cy, [&](uint32_t addr) {
-        TileFrag f;
-        bool fragment;
-        if constexpr (FAST) fragment = tile_frag_fast<MODE, N>(addr, pt, f);
-        else {
-            const bool in_reach = tile_frag_cutoff<N>(addr, pt, f);
-            f.den_rcp = frag_rcp<FAST>(f.den);
-            fragment = tile_frag_alpha<MODE, FAST>(stage_opacity<N>(addr), f) && in_reach;
-        }
-        const float4 col = stage_row<N, 5>(addr);
-        if (!fragment) return;
-        float depth = tile_frag_depth<N>(addr, pt, f);
-        float p3 = f.alpha;
-        if (depth < key_depth(core[K - 1]) && f.alpha >= kMinAlphaCore) {
+    constexpr bool PAIRS = K <= 16;
+    // a fragment that passes the tests joins the pixel
+    const auto joins = [&](const TileFrag &f, float depth, const float4 &col) {
+        float p3 = f.alpha, leaving = p3;
+        if (depth < key_depth(core[K - 1]) && p3 >= kMinAlphaCore) {
             // (a fragment that enters the core has the alpha that its key holds from here on: what the colour sums
             // receive now is what is taken out of them again for the entries of the finished core)
             // (the fast path's alpha is opacity * 2^t with the opacity held to 1 and t <= 0 up to the rounding of the staged
             // quadratic: held to 1 here, the fraction has no room for more; the exact path's is held to 1 when it is evaluated)
             if constexpr (FAST) p3 = p3 < 1.0f ? p3 : 1.0f;
-            const uint32_t low = key_pack(p3, float_to_bits(col.w) - list_first, fmt);
-            p3 = key_alpha(low, fmt);
-            tail.c0 = __builtin_fmaf(p3, col.x, tail.c0);
-            tail.c1 = __builtin_fmaf(p3, col.y, tail.c1);
-            tail.c2 = __builtin_fmaf(p3, col.z, tail.c2);
-            CoreKey carried = make_key(depth, low);
+            const uint32_t fraction = key_fraction(p3, fmt);
+            p3 = (float)fraction * fmt.one_rcp;
+            CoreKey carried = make_key(depth, fraction << fmt.shift | (float_to_bits(col.w) - list_first));
             core_key_walk<K>(carried, core);
             depth = key_depth(carried);
-            p3 = key_alpha(key_low(carried), fmt);
-            if constexpr (!FAST) tie = p3 > 0.0f && depth == key_depth(core[K - 1]) && depth < tie ? depth : tie;
-        } else {
-            tail.c0 = __builtin_fmaf(p3, col.x, tail.c0);
-            tail.c1 = __builtin_fmaf(p3, col.y, tail.c1);
-            tail.c2 = __builtin_fmaf(p3, col.z, tail.c2);
+            leaving = key_alpha(key_low(carried), fmt);
+            // (the core's last depth never grows, so the latest of these depths is the least; an empty slot's is the largest float)
+            if constexpr (!FAST) tie = depth == key_depth(core[K - 1]) ? depth : tie;
         }
-        hybrid_tail_add<FAST>(tail, depth, p3);
-    });
+        tail.c0 = __builtin_fmaf(p3, col.x, tail.c0);
+        tail.c1 = __builtin_fmaf(p3, col.y, tail.c1);
+        tail.c2 = __builtin_fmaf(p3, col.z, tail.c2);
+        hybrid_tail_add<FAST>(tail, depth, leaving);
+    };
+    if constexpr (PAIRS) {
+        tile_list_walk<MODE, true, kCullAlpha, SOLO, REC4, FAST, true, AHEAD, true>(st, ql, prim, inst, first, last, lane, cx, cy, [&](uint32_t one, uint32_t two) {
+            TileFrag f1, f2;
+            bool pass1, pass2;
+            if constexpr (FAST) {
+                pass1 = tile_frag_fast<MODE, N>(one, pt, f1);
+                pass2 = tile_frag_fast<MODE, N>(two, pt, f2);
+            } else tile_frag_exact_pair<MODE, N>(one, two, pt, f1, f2, pass1, pass2);
+            // (for all lanes: hardly a turn has none that passes)
+            const float depth1 = tile_frag_depth<N>(one, pt, f1), depth2 = tile_frag_depth<N>(two, pt, f2);
+            const float4 col1 = stage_row<N, 5>(one), col2 = stage_row<N, 5>(two);
+            if (pass1) joins(f1, depth1, col1);
+            if (pass2) joins(f2, depth2, col2);
+        });
+    } else {
+        tile_list_walk<MODE, true, kCullAlpha, SOLO, REC4, FAST, true, AHEAD>(st, ql, prim, inst, first, last, lane, cx, cy, [&](uint32_t addr) {
+            TileFrag f;
+            const bool fragment = FAST ? tile_frag_fast<MODE, N>(addr, pt, f) : tile_frag_exact<MODE, N>(addr, pt, f);
+            const float4 col = stage_row<N, 5>(addr);
+            if (fragment) joins(f, tile_frag_depth<N>(addr, pt, f), col);
+        });
+    }
 }
 // two entries of the finished core are exactly as deep as each other (their order is the reference's insertion's to choose)
 template <int K>
@@ -973,17 +977,29 @@ __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &
 {
     constexpr int MODE = HTGS_MODE_ALPHA_BLEND_FIRST_K;
     constexpr int N = kStageSlots;
-    tile_list_walk<MODE, true, kCullAlpha, SOLO, REC4, false, true, true>(st, ql, prim, inst, first, last, lane, cx, cy, [&](uint32_t addr) {
-        TileFrag f;
-        const bool in_reach = tile_frag_cutoff<N>(addr, pt, f);
-        f.den_rcp = frag_rcp<false>(f.den);
-        float depth = tile_frag_depth<N>(addr, pt, f);
-        if (!(in_reach && depth < key_depth(core[K - 1]))) return;          // depth test before the exponential (:151)
-        if (!tile_frag_alpha<MODE, false>(stage_opacity<N>(addr), f)) return;
-        CoreKey carried = make_key(depth, key_pack(f.alpha, stage_index<N>(addr) - list_first, fmt));      // (the slot's last word is the place in the list)
-        core_key_walk<K>(carried, core);
-        depth = key_depth(carried);
-        tie = key_low(carried) >> fmt.shift != 0u && depth == key_depth(core[K - 1]) && depth < tie ? depth : tie;
+    tile_list_walk<MODE, true, kCullAlpha, SOLO, REC4, false, true, true, true>(st, ql, prim, inst, first, last, lane, cx, cy, [&](uint32_t one, uint32_t two) {
+        TileFrag f1, f2;
+        const bool reach1 = tile_frag_cutoff<N>(one, pt, f1), reach2 = tile_frag_cutoff<N>(two, pt, f2);
+        const uint64_t leaves = __ballot(!rcp_in_range(f1.den)) | __ballot(!rcp_in_range(f2.den));      // (tile_frag_exact)
+        f1.den_rcp = rcp_refined(f1.den);
+        f2.den_rcp = rcp_refined(f2.den);
+        float depth1 = tile_frag_depth<N>(one, pt, f1), depth2 = tile_frag_depth<N>(two, pt, f2);
+        if (__builtin_expect(leaves != 0, 0)) {
+            f1.den_rcp = 1.0f / f1.den;
+            f2.den_rcp = 1.0f / f2.den;
+            depth1 = tile_frag_depth<N>(one, pt, f1);
+            depth2 = tile_frag_depth<N>(two, pt, f2);
+        }
+        const auto joins = [&](uint32_t addr, TileFrag &f, bool in_reach, float depth) {
+            if (!(in_reach && depth < key_depth(core[K - 1]))) return;          // depth test before the exponential (:151)
+            if (!tile_frag_alpha<MODE, false>(stage_opacity<N>(addr), f)) return;
+            CoreKey carried = make_key(depth, key_pack(f.alpha, stage_index<N>(addr) - list_first, fmt));      // (the slot's last word is the place in the list)
+            core_key_walk<K>(carried, core);
+            depth = key_depth(carried);
+            tie = depth == key_depth(core[K - 1]) ? depth : tie;                // (as in hybrid_key_walk)
+        };
+        joins(one, f1, reach1, depth1);
+        joins(two, f2, reach2, depth2);
     });
 }
 // the finished keys as the three arrays the composite takes (an empty slot has the index 0xffffffff)
@@ -1229,24 +1245,25 @@ __device__ __forceinline__ void oit_walk(TileStageQ &st, QuadrantLists &ql, cons
 {
     constexpr int MODE = HTGS_MODE_OIT_BLEND;
     constexpr int N = kStageSlots;
-    tile_list_walk<MODE, DEPTH, kCullAlpha, SOLO, REC4, FAST>(st, ql, prim, inst, first, last, lane, cx, cy, [&](uint32_t addr) {
-        TileFrag f;
-        bool fragment;
-        if constexpr (FAST) fragment = tile_frag_fast<MODE, N>(addr, pt, f);
-        else {
-            const bool in_reach = tile_frag_cutoff<N>(addr, pt, f);
-            f.den_rcp = frag_rcp<FAST>(f.den);
-            fragment = tile_frag_alpha<MODE, FAST>(stage_opacity<N>(addr), f) && in_reach;
-        }
-        const float4 col = stage_row<N, 5>(addr);
-        if (!fragment) return;
-        const float depth = DEPTH ? tile_frag_depth<N>(addr, pt, f) : 0.0f;
-        sum.a0 = __builtin_fmaf(f.alpha, col.x, sum.a0);
-        sum.a1 = __builtin_fmaf(f.alpha, col.y, sum.a1);
-        sum.a2 = __builtin_fmaf(f.alpha, col.z, sum.a2);
-        if (DEPTH) sum.a3 = __builtin_fmaf(f.alpha, depth, sum.a3);
-        sum.alpha += f.alpha;
-        sum.T *= 1.0f - f.alpha;
+    tile_list_walk<MODE, DEPTH, kCullAlpha, SOLO, REC4, FAST, false, false, true>(st, ql, prim, inst, first, last, lane, cx, cy, [&](uint32_t one, uint32_t two) {
+        TileFrag f1, f2;
+        bool pass1, pass2;
+        if constexpr (FAST) {
+            pass1 = tile_frag_fast<MODE, N>(one, pt, f1);
+            pass2 = tile_frag_fast<MODE, N>(two, pt, f2);
+        } else tile_frag_exact_pair<MODE, N>(one, two, pt, f1, f2, pass1, pass2);
+        const float4 col1 = stage_row<N, 5>(one), col2 = stage_row<N, 5>(two);
+        const float depth1 = DEPTH ? tile_frag_depth<N>(one, pt, f1) : 0.0f, depth2 = DEPTH ? tile_frag_depth<N>(two, pt, f2) : 0.0f;
+        const auto joins = [&](const TileFrag &f, float depth, const float4 &col) {
+            sum.a0 = __builtin_fmaf(f.alpha, col.x, sum.a0);
+            sum.a1 = __builtin_fmaf(f.alpha, col.y, sum.a1);
+            sum.a2 = __builtin_fmaf(f.alpha, col.z, sum.a2);
+            if (DEPTH) sum.a3 = __builtin_fmaf(f.alpha, depth, sum.a3);
+            sum.alpha += f.alpha;
+            sum.T *= 1.0f - f.alpha;
+        };
+        if (pass1) joins(f1, depth1, col1);
+        if (pass2) joins(f2, depth2, col2);
     });
 }
 __device__ __forceinline__ void oit_composite(const OitSums &sum, float *__restrict__ image, float *__restrict__ depths, uint32_t width, uint32_t height,
