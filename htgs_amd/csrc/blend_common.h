@@ -694,7 +694,7 @@ __device__ __forceinline__ void core_exchange_walk(float &depth, float &alpha, I
     }
 }
 
-// The image-only fast path inserts by shifting instead: the entry that moves down the core alternates between two register
+// The image-only fast path, and the shared walks of blend_hybrid_long_kernel, insert by shifting instead: the entry that moves down the core alternates between two register
 // triples, so that a slot costs two moves per register (slot -> the other triple, this triple -> slot) instead of an
 // exchange through a scratch register.  Both triples start out as the fragment; a lane joins at the first slot that is
 // not nearer than its fragment and from there on moves every slot down by one (<=: once it has joined, the entry it carries
