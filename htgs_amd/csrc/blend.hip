@@ -50,22 +50,30 @@ __global__ void __launch_bounds__(256) blend_global_kernel(
         const uint32_t stage_base = __builtin_amdgcn_readfirstlane(stage_address(st));
         subtile_walk(s_reach, stage_base, last - base < 256u ? last - base : 256u, wave, lane,
                      [&]() { return __ballot(!done) == 0; },       // every pixel of the sub-tile is opaque
-                     [&](uint32_t addr) {
-            TileFrag f;
-            if (done || !tile_frag_cutoff<256>(addr, pt, f)) return;
-            f.den_rcp = frag_rcp<FAST>(f.den);
-            const float4 q4 = stage_row<256, 4>(addr);
-            if (!tile_frag_alpha<MODE, FAST>(q4.w, f)) return;
-            const float4 col = stage_row<256, 5>(addr);
-            const float wgt = T * f.alpha;
-            r = __builtin_fmaf(wgt, col.x, r);
-            g = __builtin_fmaf(wgt, col.y, g);
-            b = __builtin_fmaf(wgt, col.z, b);
-            const float depth = q4.z;
-            if (median) depth_pixel = T > 0.5f ? depth : depth_pixel;
-            else depth_pixel = __builtin_fmaf(wgt, depth, depth_pixel);
-            T *= 1.0f - f.alpha;
-            if (T < kTransmittanceThreshold) done = true;
+                     [&](uint32_t one, bool one_listed, uint32_t two, bool two_listed) {
+            TileFrag f1, f2;
+            bool pass1, pass2;
+            if constexpr (FAST) {
+                pass1 = tile_frag_cutoff<256>(one, pt, f1);
+                pass2 = tile_frag_cutoff<256>(two, pt, f2);
+                f1.den_rcp = frag_rcp<true>(f1.den);
+                f2.den_rcp = frag_rcp<true>(f2.den);
+                pass1 = tile_frag_alpha<MODE, true>(stage_opacity<256>(one), f1) && pass1;
+                pass2 = tile_frag_alpha<MODE, true>(stage_opacity<256>(two), f2) && pass2;
+            } else tile_frag_exact_pair<MODE, 256>(one, two, pt, f1, f2, pass1, pass2);
+            const auto joins = [&](uint32_t addr, const TileFrag &f) {
+                const float4 q4 = stage_row<256, 4>(addr), col = stage_row<256, 5>(addr);
+                const float wgt = T * f.alpha;
+                r = __builtin_fmaf(wgt, col.x, r);
+                g = __builtin_fmaf(wgt, col.y, g);
+                b = __builtin_fmaf(wgt, col.z, b);
+                const float depth = q4.z;
+                if constexpr (!FAST) depth_pixel = median ? (T > 0.5f ? depth : depth_pixel) : __builtin_fmaf(wgt, depth, depth_pixel);
+                T *= 1.0f - f.alpha;
+                done = T < kTransmittanceThreshold;
+            };
+            if (pass1 && one_listed && !done) joins(one, f1);
+            if (pass2 && two_listed && !done) joins(two, f2);
         });
     }
     if (!inside) return;

@@ -405,17 +405,6 @@ __device__ __forceinline__ uint32_t quadrant_next_hit(QuadrantHits &w)
                      : [a0] "s"(a0), [a1] "s"(a1), [a2] "s"(a2), [a3] "s"(a3));
     return addr;
 }
-// The walk itself: turn(addr) is called, with the lanes of the quadrants that still have a hit, once per loop turn.
-template <bool BANKED = false, typename Turn>
-__device__ __forceinline__ void quadrant_walk(QuadrantHits &hits, uint32_t stage_base, Turn &&turn)
-{
-    // (the exit is taken from the scalar masks, not from the lanes' addresses: an exit test that the optimizer can fold
-    // into the per-lane test below makes the loop, and the masks it carries, divergent in the compiler's eyes)
-    while (quadrant_pending(hits)) {
-        const uint32_t addr = quadrant_next_hit<BANKED>(hits);
-        if (addr != kNoHit) turn(addr + stage_base);
-    }
-}
 // Quadrant lists: the same walk with the scalar bit scans taken out of the loop.  After a batch is staged, the slots that
 // reach quadrant q are written, in list order, to a short list in LDS (their LDS addresses), padded up to the length of
 // the longest of the four lists with the address of a slot that no fragment passes (entry 0 of every row of a stage with
@@ -764,15 +753,21 @@ __device__ __forceinline__ void subtile_pixel(uint32_t thread, uint32_t &local_x
     local_y += 8u * (thread >> 7);
 }
 // One batch of 256 staged instances (reach[slot]: the sixteen quadrant bits tile_stage_load returned for it): the wave
-// walks the hits of its own four quadrants, 64 slots at a time, and stops early once all_done() says so (wave-uniform).
-template <typename Done, typename Turn>
+// walks the hits of its own four quadrants, 64 slots at a time, and stops early once all_done() says so (wave-uniform).  Two turns
+// at a time, for the reason given at quadrant_list_walk_pairs: turns(one, one_listed, two, two_listed); a quadrant without a hit left
+// gets the part's first slot, not listed.
+template <typename Done, typename Turns>
 __device__ __forceinline__ void subtile_walk(const uint16_t *reach, uint32_t stage_base, uint32_t n_staged, uint32_t wave, uint32_t lane,
-                                             Done &&all_done, Turn &&turn)
+                                             Done &&all_done, Turns &&turns)
 {
     for (uint32_t part = 0; part < 4 && 64u * part < n_staged; ++part) {
         if (all_done()) break;
         QuadrantHits hits = quadrant_ballot(((uint32_t)reach[64u * part + lane] >> (4u * wave)) & 0xfu);
-        quadrant_walk(hits, stage_base + 64u * 16u * part, turn);
+        const uint32_t part_base = stage_base + 64u * 16u * part;
+        while (quadrant_pending(hits)) {
+            const uint32_t one = quadrant_next_hit(hits), two = quadrant_next_hit(hits);
+            turns(one != kNoHit ? one + part_base : part_base, one != kNoHit, two != kNoHit ? two + part_base : part_base, two != kNoHit);
+        }
     }
 }
 

@@ -111,18 +111,21 @@ __global__ void __launch_bounds__(256) blend_global_forward_kernel(
         const uint32_t stage_base = __builtin_amdgcn_readfirstlane(stage_address(st));
         subtile_walk(s_reach, stage_base, last - base < 256u ? last - base : 256u, wave, lane,
                      [&]() { return __ballot(!done) == 0; },
-                     [&](uint32_t addr) {
-            TileFrag f;
-            if (done || !tile_frag_cutoff<256>(addr, pt, f)) return;
-            f.den_rcp = rcp_exact(f.den);
-            const float4 col = stage_row<256, 5>(addr);
-            if (!tile_frag_alpha<MODE>(stage_opacity<256>(addr), f)) return;
-            const float bw = T * f.alpha;
-            r = __builtin_fmaf(bw, col.x, r);
-            g = __builtin_fmaf(bw, col.y, g);
-            b = __builtin_fmaf(bw, col.z, b);
-            T *= 1.0f - f.alpha;
-            if (T < kTransmittanceThreshold) done = true;
+                     [&](uint32_t one, bool one_listed, uint32_t two, bool two_listed) {
+            TileFrag f1, f2;
+            bool pass1, pass2;
+            tile_frag_exact_pair<MODE, 256>(one, two, pt, f1, f2, pass1, pass2);
+            const auto joins = [&](uint32_t addr, const TileFrag &f) {
+                const float4 col = stage_row<256, 5>(addr);
+                const float bw = T * f.alpha;
+                r = __builtin_fmaf(bw, col.x, r);
+                g = __builtin_fmaf(bw, col.y, g);
+                b = __builtin_fmaf(bw, col.z, b);
+                T *= 1.0f - f.alpha;
+                done = T < kTransmittanceThreshold;
+            };
+            if (pass1 && one_listed && !done) joins(one, f1);
+            if (pass2 && two_listed && !done) joins(two, f2);
         });
     }
     if (!inside) return;

@@ -138,15 +138,18 @@ __global__ void __launch_bounds__(256) max_weights_global_kernel(
         const uint32_t stage_base = __builtin_amdgcn_readfirstlane(stage_address(st));
         subtile_walk(s_reach, stage_base, last - base < 256u ? last - base : 256u, wave, lane,
                      [&]() { return __ballot(!done) == 0; },
-                     [&](uint32_t addr) {
-            TileFrag f;
-            if (done || !tile_frag_cutoff<256>(addr, pt, f)) return;
-            f.den_rcp = rcp_exact(f.den);
-            if (!tile_frag_alpha<MODE>(stage_opacity<256>(addr), f)) return;
-            const float w = T * f.alpha;
-            T *= 1.0f - f.alpha;
-            if (T < kTransmittanceThreshold) done = true;
-            if (!(w < weight_threshold)) raise_max(max_weights, stage_index<256>(addr), w);
+                     [&](uint32_t one, bool one_listed, uint32_t two, bool two_listed) {
+            TileFrag f1, f2;
+            bool pass1, pass2;
+            tile_frag_exact_pair<MODE, 256>(one, two, pt, f1, f2, pass1, pass2);
+            const auto joins = [&](uint32_t addr, const TileFrag &f) {
+                const float w = T * f.alpha;
+                T *= 1.0f - f.alpha;
+                done = T < kTransmittanceThreshold;
+                if (!(w < weight_threshold)) raise_max(max_weights, stage_index<256>(addr), w);
+            };
+            if (pass1 && one_listed && !done) joins(one, f1);
+            if (pass2 && two_listed && !done) joins(two, f2);
         });
     }
 }
