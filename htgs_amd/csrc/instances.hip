@@ -238,8 +238,8 @@ __global__ void __launch_bounds__(256) create_instances_kernel(
 }
 
 // The same for a frame with htgs_frame.touch (tile_span.h): the tiles of a Gaussian's mask, bit by bit, or the rows of a
-// rectangle too large for a mask, worked out again from its record.  The block's instances of the masks are written element
-// by element as above (a slot's bit is found by popcounts in halves); the large rectangles are the waves' own work, one
+// rectangle too large for a mask, worked out again from its record.  The block's instances of the masks go through LDS, from
+// where they are written element by element; the large rectangles are the waves' own work, one
 // after the other, the rows in the lanes and then the row's tiles element by element over a search in the rows' ends.
 // Which tile of a Gaussian comes first does not matter: the sort that follows is by tile.
 // SCAN: the offsets are not there yet.  Every block adds up the block sums before its own (few: kFusedScanMost Gaussians)
@@ -251,6 +251,8 @@ struct FusedScan {
     unsigned long long *host_total;
     uint32_t tag;
 };
+constexpr uint32_t kListWindow = 2048;           // (256 Gaussians have 1300 instances of masks on average: one window)
+constexpr uint32_t kListOwn = 12;                // tiles of a mask that a lane puts down by itself (15 M instances: 6 tiles 66 us, 8 54, 12 46, 16 48)
 template <typename KeyT, bool DEPTH, bool ORDERED, bool SCAN = false>
 __global__ void __launch_bounds__(256) create_listed_kernel(
     const uint32_t *__restrict__ counts, const uint32_t *__restrict__ offsets, const uint4 *__restrict__ touch,
@@ -259,9 +261,8 @@ __global__ void __launch_bounds__(256) create_listed_kernel(
     FusedScan scan)
 {
     static_assert(!(DEPTH && ORDERED), "keys of the tile alone");
-    __shared__ uint32_t s_end[256], s_base[256];     // ends of the masks' instances within the block's; what to add for their place in the list
-    __shared__ uint32_t s_corner[256], s_lo[256], s_hi[256], s_depth[DEPTH ? 256 : 1], s_gaussian[ORDERED ? 256 : 1];
-    __shared__ uint8_t s_width[256];
+    __shared__ uint32_t s_list[kListWindow], s_base[256];     // instances of the masks: tile (of 2^20 at most) | thread << 20; what to add for their place in the list
+    __shared__ uint32_t s_depth[DEPTH ? 256 : 1], s_gaussian[ORDERED ? 256 : 1];
     __shared__ uint32_t s_sums[kScanBlock / kWave];
     __shared__ uint32_t s_row_end[256 / kWave][kWave], s_row_tile[256 / kWave][kWave];
     const int first = blockIdx.x * 256;
@@ -317,27 +318,50 @@ __global__ void __launch_bounds__(256) create_listed_kernel(
     const uint32_t masked = large ? 0u : count;
     uint32_t total;
     const uint32_t inc = block_inclusive_scan(masked, s_sums, &total);
-    s_end[threadIdx.x] = inc;
     s_base[threadIdx.x] = (end - count) - (inc - masked);
-    s_corner[threadIdx.x] = (t.corner >> 16) * grid_w + (t.corner & 0xffffu);
-    s_lo[threadIdx.x] = t.lo; s_hi[threadIdx.x] = t.hi;
-    s_width[threadIdx.x] = (uint8_t)(t.size & 0xffffu);               // (at most kMaskTiles where it is read)
     if (ORDERED) s_gaussian[threadIdx.x] = gaussian;
     if (DEPTH) s_depth[threadIdx.x] = depth;
-    __syncthreads();
-    for (uint32_t e = threadIdx.x; e < total; e += 256) {
-        uint32_t lo = 0, hi = 255;                                    // smallest l with s_end[l] > e
-#pragma unroll
-        for (int step = 0; step < 8; ++step) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (s_end[mid] > e) hi = mid; else lo = mid + 1;
+    {
+        // Every thread puts its mask's tiles down in LDS, a window of the block's list at a time, and the block writes them out
+        // in order.  (Looking up an element's Gaussian and its bit of the mask element by element took 130 instructions and
+        // eight dependent reads of LDS for every 64 of them: 15 M instances of 3 M Gaussians 61 -> 47 us, whole frame 1304 -> 1296; the
+        // stress scene's, a third of whose Gaussians have more than twelve tiles, 170 -> 176.)
+        // A mask of many tiles would keep the other lanes waiting: the wave takes those one by one, a bit in each lane.
+        const uint32_t begin = inc - masked;
+        const bool many = masked > kListOwn;
+        uint32_t lo = large || many ? 0u : t.lo, hi = large || many ? 0u : t.hi, at = begin;
+        const uint32_t w = t.size & 0xffffu, corner = (t.corner >> 16) * grid_w + (t.corner & 0xffffu);
+        const float per_row = __builtin_amdgcn_rcpf((float)w);
+        for (uint32_t from = 0; from < total; from += kListWindow) {       // (the same for the whole block)
+            if (from != 0u) __syncthreads();                              // (the window before is read)
+            while ((lo | hi) != 0u && at < from + kListWindow) {
+                const bool low = lo != 0u;
+                const uint32_t word = low ? lo : hi, rest = word & (word - 1u), bit = (uint32_t)__builtin_ctz(word) + (low ? 0u : 32u);
+                lo = low ? rest : lo;
+                hi = low ? hi : rest;
+                // (bit < 64 and w <= 64: the quotient of bit + 1/2 is never within rounding of a whole number)
+                const uint32_t row = (uint32_t)(((float)bit + 0.5f) * per_row);
+                s_list[at - from] = (corner + __umul24(row, grid_w) + (bit - __umul24(row, w))) | threadIdx.x << 20;
+                ++at;
+            }
+            for (unsigned long long owners = __ballot(many && begin < from + kListWindow && inc > from); owners != 0; owners &= owners - 1) {     // (wave-uniform)
+                const int owner = __builtin_ctzll(owners);
+                const auto of = [owner](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, owner); };
+                const uint32_t olo = of(t.lo), ohi = of(t.hi), ow = of(w);
+                const uint32_t to = of(begin) + __builtin_amdgcn_mbcnt_hi(ohi, __builtin_amdgcn_mbcnt_lo(olo, 0u));
+                const uint32_t row = (uint32_t)(((float)lane + 0.5f) * bits_to_float(of(float_to_bits(per_row))));
+                const bool set = ((lane < 32u ? olo >> lane : ohi >> (lane - 32u)) & 1u) != 0u;
+                if (set && to >= from && to < from + kListWindow)
+                    s_list[to - from] = (of(corner) + __umul24(row, grid_w) + (lane - __umul24(row, ow))) | (wave * kWave + (uint32_t)owner) << 20;
+            }
+            __syncthreads();
+            const uint32_t here = total - from < kListWindow ? total - from : kListWindow;
+            for (uint32_t e = threadIdx.x; e < here; e += 256) {
+                const uint32_t listed = s_list[e], l = listed >> 20, tile = listed & 0xfffffu, to = s_base[l] + from + e;
+                keys[to] = DEPTH ? (KeyT)((uint64_t)tile << (DEPTH ? 32 : 0) | (uint64_t)s_depth[DEPTH ? l : 0]) : (KeyT)tile;
+                vals[to] = ORDERED ? s_gaussian[l] : (uint32_t)(first + l);
+            }
         }
-        const uint32_t l = lo, bit = nth_bit(s_lo[l], s_hi[l], e - (l == 0 ? 0u : s_end[l - 1])), w = s_width[l];
-        // (bit < 64 and w <= 64: the quotient of bit + 1/2 is never within rounding of a whole number)
-        const uint32_t row = (uint32_t)(((float)bit + 0.5f) * __builtin_amdgcn_rcpf((float)w));
-        const uint32_t tile = s_corner[l] + row * grid_w + (bit - row * w), at = s_base[l] + e;
-        keys[at] = DEPTH ? (KeyT)((uint64_t)tile << (DEPTH ? 32 : 0) | (uint64_t)s_depth[DEPTH ? l : 0]) : (KeyT)tile;
-        vals[at] = ORDERED ? s_gaussian[l] : (uint32_t)(first + l);
     }
     for (unsigned long long pending = __ballot(large); pending != 0; pending &= pending - 1) {      // (wave-uniform)
         const int owner = __builtin_ctzll(pending);

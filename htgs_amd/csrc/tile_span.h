@@ -114,21 +114,4 @@ __device__ __forceinline__ TileOutline broadcast_outline(const TileOutline &o, i
     return TileOutline{ from(o.lo), from(o.hi), from(o.cy), from(o.shear), from(o.rx2), from(o.iy2), from(o.yr), from(o.above), from(o.below),
                         __builtin_amdgcn_readlane((int)o.ellipse, owner) != 0 };
 }
-// the t-th set bit of a mask
-__device__ __forceinline__ uint32_t nth_bit(uint32_t lo, uint32_t hi, uint32_t t)
-{
-    const uint32_t below = (uint32_t)__builtin_popcount(lo);
-    uint32_t word = t < below ? lo : hi, at = t < below ? 0u : 32u;
-    t = t < below ? t : t - below;
-#pragma unroll
-    for (uint32_t half = 16; half > 0; half >>= 1) {
-        const uint32_t c = (uint32_t)__builtin_popcount(word & ((1u << half) - 1u));
-        const bool upper = t >= c;
-        t = upper ? t - c : t;
-        word = upper ? word >> half : word;
-        at = upper ? at + half : at;
-    }
-    return at;
-}
-
 }  // namespace htgs

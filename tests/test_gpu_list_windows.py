@@ -1,0 +1,54 @@
+"""The duplication of masks goes through a window of 2048 instances in LDS, masks of up to twelve tiles lane by lane and larger ones by the
+whole wave: blocks of 256 Gaussians with few and many instances, masks around twelve tiles and the largest, against the instances
+listed one rectangle at a time on the host."""
+import numpy as np
+import pytest
+import torch
+
+from htgs_amd.torch_bindings import FrameBuffers, RasterizerMode
+from util import tie_scene, u32
+
+pytestmark = pytest.mark.gpu
+
+
+def listed(fb):
+    """Per Gaussian the tiles of its touch entry, from the entry itself."""
+    touch = u32(fb.touch).reshape(-1, 4)
+    counts = u32(fb.n_touched)
+    pairs = []
+    for g in np.flatnonzero(counts):
+        corner, size, lo, hi = (int(v) for v in touch[g])
+        x0, y0, w, h = corner & 0xffff, corner >> 16, size & 0xffff, size >> 16
+        if w * h > 64:
+            return None
+        mask = lo | hi << 32
+        tiles = [(y0 + b // w) * fb.grid_w + x0 + b % w for b in range(64) if mask >> b & 1]
+        assert len(tiles) == counts[g]
+        pairs += [(t, g) for t in tiles]
+    return sorted(pairs)
+
+
+@pytest.mark.parametrize("mode", [0, 2, 3])
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 700])
+@pytest.mark.parametrize("spread", ["small", "around twelve", "largest"])
+def test_instances_of_masks(cuda, spread, n, mode):
+    print(f"case spread={spread} n={n} mode={mode}", flush=True)
+    rng = np.random.default_rng(n)
+    scene = tie_scene(rng.uniform(1.0, 9.0, n).tolist(), rng.uniform(0.3, 1.0, n).tolist(), rng.uniform(0.0, 1.0, (n, 3)).tolist())
+    scene.scales *= {"small": 0.2, "around twelve": 1.0, "largest": 2.0}[spread] * torch.from_numpy(rng.uniform(0.6, 1.0, (n, 1)).astype(np.float32))
+    scene.positions[:, :2] = torch.from_numpy(rng.uniform(-0.2, 0.2, (n, 2)).astype(np.float32)) * scene.positions[:, 2:3]
+    gpu = scene.to(cuda)
+    fb = FrameBuffers(*gpu.gaussians(), gpu.settings(RasterizerMode(mode), 4), True, False, tight_lists=True, order_gaussians=False)
+    fb.preprocess()
+    fb.scan()
+    count = fb.read_instance_count()
+    fb.alloc_instances(count)
+    fb.create_instances()
+    torch.cuda.synchronize()
+    want = listed(fb)
+    assert want is not None and len(want) == count            # (an 8x8 grid: every rectangle has a mask)
+    keys = u32(fb.keys[0])[:count].astype(np.uint64)
+    tiles = keys >> np.uint64(32) if mode == 2 else keys
+    got = list(zip(tiles.astype(np.int64).tolist(), u32(fb.vals[0])[:count].tolist()))
+    assert [g for _, g in got] == sorted(g for _, g in got)   # in the Gaussians' order, which the stable sort keeps
+    assert sorted(got) == want
