@@ -183,9 +183,10 @@ static uint64_t fitting(htgs_frame *f, uint64_t least, uint64_t bytes)
     return lo;
 }
 
-// Frames whose scan is fused (65536 Gaussians at most) on grids of no more tiles have their blend queued before the number is
+// Frames of at most kBlendAheadGaussians on grids of no more tiles have their blend queued before the number is
 // there: 20 k Gaussians at 400x304 in training 201 us a step so, 207 otherwise, and the records of 6144 tiles are written twice in 25 us.
 constexpr uint64_t kBlendAheadTiles = 6144;
+constexpr int kBlendAheadGaussians = 65536;
 static int check_run(const htgs_frame *f, const htgs_workspace *w, const char *who)
 {
     if (!f || !w) return fail(HTGS_ERR_ARGUMENT, "%s: null argument", who);
@@ -289,7 +290,7 @@ extern "C" int htgs_run(htgs_frame *f, htgs_workspace *w)
         f->n_instances_live = f->n_instances_dev;
         rc = queue_lists(f, w, true, fused ? word : nullptr);
         const int tile = tile_size(f->mode);
-        blended = fused && (uint64_t)div_up(f->width, tile) * div_up(f->height, tile) <= kBlendAheadTiles;
+        blended = fused && f->n_primitives <= kBlendAheadGaussians && (uint64_t)div_up(f->width, tile) * div_up(f->height, tile) <= kBlendAheadTiles;
         if (rc == HTGS_OK && blended) rc = queue_blend(f, w);
         f->n_instances_live = nullptr;
         if (rc != HTGS_OK) return rc;
