@@ -197,7 +197,7 @@ constexpr uint32_t kTurnPairs = 61;
 // quadratics num(dx, dy) = |m|^2 / cut-off and den(dx, dy) = |d|^2, and m = Am + dy Bm + dx Cm, d = A + dy B + dx C, so
 //     dL/dAm = 2 kc (S00 Am + S01 Bm + S10 Cm),  dL/dBm = 2 kc (S01 Am + S02 Bm + S11 Cm),  dL/dCm = 2 kc (S10 Am + S11 Bm + S20 Cm)
 // with the moments S_ij = sum over the tile's pixels of dL/dnum dx^i dy^j (and the same with dL/dden for A, B, C).
-// A fragment therefore costs twelve fused multiply-adds with scalar monomials instead of the reference's chain to
+// A fragment therefore costs six sums of its pixel row (QuadrantMoments) instead of the reference's chain to
 // the three VPMT rows (backward.cuh:260-289), which is applied once per (Gaussian, tile) at the end.  The third
 // densification row (HELPER) is a sum of absolute values per fragment and cannot go through the moments: it takes
 // the fourth components of the fragment's dL/dVPMT rows, which need m and the two plane normals at the pixel.
