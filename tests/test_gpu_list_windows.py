@@ -52,3 +52,33 @@ def test_instances_of_masks(cuda, spread, n, mode):
     got = list(zip(tiles.astype(np.int64).tolist(), u32(fb.vals[0])[:count].tolist()))
     assert [g for _, g in got] == sorted(g for _, g in got)   # in the Gaussians' order, which the stable sort keeps
     assert sorted(got) == want
+
+
+@pytest.mark.parametrize("mode", [0, 2, 3])
+def test_instances_on_a_grid_beyond_two_to_the_twenty_tiles(cuda, mode):
+    """The duplication on its own, with offsets from elsewhere (the scan stops at 2^20 tiles): an entry of the window has room for 2^24."""
+    print(f"case mode={mode}", flush=True)
+    n = 1000
+    rng = np.random.default_rng(3)
+    scene = tie_scene(rng.uniform(1.0, 9.0, n).tolist(), rng.uniform(0.3, 1.0, n).tolist(), rng.uniform(0.0, 1.0, (n, 3)).tolist())
+    scene.positions[:, :2] = torch.from_numpy(rng.uniform(-0.3, 0.3, (n, 2)).astype(np.float32)) * scene.positions[:, 2:3]
+    by = 512.0 if mode == 2 else 256.0
+    scene.width, scene.height = int(64 * by) + 16, int(32 * by) + 16
+    scene.VPM[0] *= by
+    scene.VPM[1] *= by / 2.0
+    scene.scales *= 1.0 / by
+    gpu = scene.to(cuda)
+    fb = FrameBuffers(*gpu.gaussians(), gpu.settings(RasterizerMode(mode), 4), True, False, tight_lists=True, order_gaussians=False)
+    assert 1 << 20 < fb.n_tiles < 1 << 24
+    fb.preprocess()
+    offsets = torch.cumsum(fb.n_touched, 0).to(torch.int32)
+    fb.offsets.copy_(offsets)
+    count = int(offsets[-1])
+    fb.alloc_instances(count)
+    fb.create_instances()
+    torch.cuda.synchronize()
+    want = listed(fb)
+    assert want is not None and len(want) == count and max(t for t, _ in want) > 1 << 20
+    keys = u32(fb.keys[0])[:count].astype(np.uint64)
+    tiles = keys >> np.uint64(32) if mode == 2 else keys
+    assert sorted(zip(tiles.astype(np.int64).tolist(), u32(fb.vals[0])[:count].tolist())) == want
