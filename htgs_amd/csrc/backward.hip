@@ -830,6 +830,7 @@ __global__ void __launch_bounds__(256) blend_global_backward_kernel(
 // per-Gaussian part: grad_rows -> gradients of the parameters; SH backward; densification statistics
 // (R/include/hybrid_blend/kernels/backward.cuh:10-102, R/include/kernel_utils.cuh:44-61,190-281)
 // ---------------------------------------------------------------------------------------------
+constexpr int kShRegs = 16;                  // 16-byte words of sh_rest a thread holds: 64 words, 21 coefficients, a Gaussian
 __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     const float *__restrict__ positions, const float *__restrict__ scales, const float *__restrict__ rotations,
     const float *__restrict__ sh_rest, const uint32_t *__restrict__ n_touched, const uint8_t *__restrict__ clamp_info,
@@ -852,7 +853,6 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     const int n_block = n - first < 256 ? n - first : 256;
     const size_t base_word = (size_t)first * per;                 // multiple of 256 words: 16-byte aligned
     const int words = n_block * per;
-    constexpr int kShRegs = 16;
     float sh_regs[kShRegs][4];
     if (active_sh > 1) {
         const float4 *src4 = reinterpret_cast<const float4 *>(sh_rest + base_word);
@@ -1217,8 +1217,9 @@ extern "C" int htgs_preprocess_backward(const htgs_frame *f)
     const float *helper = (f->densification_info && f->densification_rows == 3) ? f->dens_helper : nullptr;
     if (f->densification_info && f->densification_rows == 3 && !helper && f->n_instances > 0)
         return fail(HTGS_ERR_ARGUMENT, "htgs_preprocess_backward: 3-row densification_info needs dens_helper");
+    // (with 21 coefficients the kernel has 67 KB of LDS, 63 of them here and 4 for the row sums; a workgroup can have 160)
     const size_t lds_bytes = (size_t)256 * 3 * f->total_sh_bases * sizeof(float);
-    if (lds_bytes > 64 * 1024) return fail(HTGS_ERR_ARGUMENT, "htgs_preprocess_backward: sh_rest has more than 21 coefficients per Gaussian");
+    if (lds_bytes > 256 * 4 * kShRegs * sizeof(float)) return fail(HTGS_ERR_ARGUMENT, "htgs_preprocess_backward: sh_rest has more than 21 coefficients per Gaussian");
     hipLaunchKernelGGL(preprocess_backward_kernel, dim3(div_up(f->n_primitives, 256)), dim3(256), lds_bytes, (hipStream_t)f->stream,
                        f->positions, f->scales, f->rotations, f->sh_rest, f->n_touched, f->clamp_info,
                        (const float4 *)f->grad_rows, f->offsets, helper, f->M, f->VPM,

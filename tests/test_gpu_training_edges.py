@@ -72,3 +72,26 @@ def test_gradients_are_deterministic(cuda, mode):
     _, _, _, second = run_both(scene, mode, 16, cuda)
     for name, a, b in zip(NAMES, first, second):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("mode", [0, 2])
+@pytest.mark.parametrize("total", [16, 20, 21])
+def test_more_coefficients_than_the_bands_need(cuda, total, mode):
+    """Up to 21 coefficients a Gaussian (63 KB of LDS for a block's, beside 4 KB for its row sums); the unused ones have no gradient."""
+    print(f"case total={total} mode={mode}", flush=True)
+    scene = make_scene(0, 3000)
+    rest = torch.randn(3000, total, 3, generator=torch.Generator().manual_seed(total)) * 0.1
+    scene = dataclasses.replace(scene, sh_rest=rest.contiguous(), active_sh_bases=16)
+    fwd, want, image, grads = run_both(scene, mode, 4, cuda)
+    assert np.abs(image.cpu().numpy() - fwd["image"]).max() <= 1e-4
+    for name, got in zip(NAMES, grads):
+        assert_grad_close(name, got.cpu().numpy(), want[name])
+    assert float(grads[5][:, 15:].abs().sum()) == 0.0
+
+
+def test_too_many_coefficients_are_refused(cuda):
+    scene = dataclasses.replace(make_scene(0, 100), sh_rest=torch.zeros(100, 22, 3)).to(cuda)
+    fb = FrameBuffers(*scene.gaussians(), scene.settings(RasterizerMode.HYBRID_BLEND, 4), True, False, train=True)
+    fb.run_forward()                                         # (one band active: the coefficients are not read)
+    with pytest.raises(RuntimeError, match="21 coefficients"):
+        fb.run_backward(torch.ones(3, scene.height, scene.width, device=cuda))
