@@ -255,7 +255,12 @@ struct FusedScan {
 };
 constexpr uint32_t kListWindow = 2048;           // (256 Gaussians have 1300 instances of masks on average: one window)
 constexpr uint32_t kListTileBits = 24;           // of an entry of the window, beside the eight of the thread
-constexpr uint32_t kListOwn = 12;                // tiles of a mask that a lane puts down by itself (15 M instances: 6 tiles 66 us, 8 54, 12 46, 16 48)
+// Tiles of a mask that a lane puts down by itself; twice as many in a wave in which more than kListBetween masks have one to two times that:
+// the wave takes those one by one otherwise.  (us; all by the lane up to 6, 8, 12, 16, 24 tiles: 15 M instances of 3 M Gaussians 66, 54,
+// 46, 48, 51.  With one line at twelve -> with the second, and the search element by element that this replaced: OIT 50 k Gaussians at
+// 1600x900 of 19 tiles each 22.1 -> 19.7, 20.0; 500 k at 1920x1080 of e^-3.6 52.8 -> 44.0, 48.8; 300 k of e^-3 85 -> 80.6, 80.7; the stress
+// scene's 6 M 178 -> 178, 175; the 3 M 46.9 -> 47.3, 59.3.)
+constexpr uint32_t kListOwn = 12, kListBetween = 12;
 template <typename KeyT, bool DEPTH, bool ORDERED, bool SCAN = false>
 __global__ void __launch_bounds__(256) create_listed_kernel(
     const uint32_t *__restrict__ counts, const uint32_t *__restrict__ offsets, const uint4 *__restrict__ touch,
@@ -327,11 +332,11 @@ __global__ void __launch_bounds__(256) create_listed_kernel(
     {
         // Every thread puts its mask's tiles down in LDS, a window of the block's list at a time, and the block writes them out
         // in order.  (Looking up an element's Gaussian and its bit of the mask element by element took 130 instructions and
-        // eight dependent reads of LDS for every 64 of them: 15 M instances of 3 M Gaussians 61 -> 47 us, whole frame 1304 -> 1296; the
-        // stress scene's, a third of whose Gaussians have more than twelve tiles, 170 -> 176.)
+        // eight dependent reads of LDS for every 64 of them: 15 M instances of 3 M Gaussians 61 -> 47 us, whole frame 1304 -> 1296.)
         // A mask of many tiles would keep the other lanes waiting: the wave takes those one by one, a bit in each lane.
         const uint32_t begin = inc - masked;
-        const bool many = masked > kListOwn;
+        const uint64_t between = __ballot(masked > kListOwn && masked <= 2u * kListOwn);
+        const bool many = masked > (__popcll(between) > (int)kListBetween ? 2u * kListOwn : kListOwn);
         uint32_t lo = large || many ? 0u : t.lo, hi = large || many ? 0u : t.hi, at = begin;
         const uint32_t w = t.size & 0xffffu, corner = (t.corner >> 16) * grid_w + (t.corner & 0xffffu);
         const float per_row = __builtin_amdgcn_rcpf((float)w);

@@ -1,6 +1,6 @@
 """The duplication of masks goes through a window of 2048 instances in LDS, masks of up to twelve tiles lane by lane and larger ones by the
-whole wave: blocks of 256 Gaussians with few and many instances, masks around twelve tiles and the largest, against the instances
-listed one rectangle at a time on the host."""
+whole wave, or up to twenty-four lane by lane in a wave with more than twelve masks between the two: blocks of 256 Gaussians with few and
+many instances, masks around twelve tiles, around twenty-four and the largest, against the instances listed one rectangle at a time on the host."""
 import numpy as np
 import pytest
 import torch
@@ -30,13 +30,15 @@ def listed(fb):
 
 @pytest.mark.parametrize("mode", [0, 2, 3])
 @pytest.mark.parametrize("n", [1, 255, 256, 257, 700])
-@pytest.mark.parametrize("spread", ["small", "around twelve", "largest"])
+@pytest.mark.parametrize("spread", ["small", "around twelve", "around twenty-four", "few large", "largest"])
 def test_instances_of_masks(cuda, spread, n, mode):
     print(f"case spread={spread} n={n} mode={mode}", flush=True)
     rng = np.random.default_rng(n)
     scene = tie_scene(rng.uniform(1.0, 9.0, n).tolist(), rng.uniform(0.3, 1.0, n).tolist(), rng.uniform(0.0, 1.0, (n, 3)).tolist())
-    scene.scales *= {"small": 0.2, "around twelve": 1.0, "largest": 2.0}[spread] * torch.from_numpy(rng.uniform(0.6, 1.0, (n, 1)).astype(np.float32))
+    scene.scales *= {"small": 0.2, "around twelve": 1.0, "around twenty-four": 1.4, "few large": 0.3, "largest": 2.0}[spread] * torch.from_numpy(rng.uniform(0.6, 1.0, (n, 1)).astype(np.float32))
     scene.positions[:, :2] = torch.from_numpy(rng.uniform(-0.2, 0.2, (n, 2)).astype(np.float32)) * scene.positions[:, 2:3]
+    if spread == "few large":
+        scene.scales[torch.from_numpy(rng.random(n) < 0.12)] *= 5.0
     gpu = scene.to(cuda)
     fb = FrameBuffers(*gpu.gaussians(), gpu.settings(RasterizerMode(mode), 4), True, False, tight_lists=True, order_gaussians=False)
     fb.preprocess()
@@ -47,6 +49,14 @@ def test_instances_of_masks(cuda, spread, n, mode):
     torch.cuda.synchronize()
     want = listed(fb)
     assert want is not None and len(want) == count            # (an 8x8 grid: every rectangle has a mask)
+    if mode != 2 and n >= 255 and spread not in ("small", "largest"):
+        sizes = np.pad(u32(fb.n_touched), (0, -n % 64)).reshape(-1, 64)
+        between, beyond = ((sizes > 12) & (sizes <= 24)).sum(1), (sizes > 24).sum(1)
+        print("between:", between.tolist(), "beyond:", beyond.tolist())
+        if spread == "few large":                            # the line at twelve, and masks on both sides of it
+            assert between.max() <= 12 and between.any() and beyond.any()
+        else:                                                # the line at twenty-four
+            assert between.max() > 12 and (beyond.any() or spread == "around twelve")
     keys = u32(fb.keys[0])[:count].astype(np.uint64)
     tiles = keys >> np.uint64(32) if mode == 2 else keys
     got = list(zip(tiles.astype(np.int64).tolist(), u32(fb.vals[0])[:count].tolist()))
