@@ -152,8 +152,8 @@ def views(scene, cuda):
 
 @pytest.mark.parametrize("n,mode", [(3000, 0), (3000, 2), (80_000, 0), (80_000, 1), (80_000, 2), (80_000, 3)])
 def test_changing_views(cuda, n, mode):
-    """More instances than the buffers hold or the launches were sized for, with the scan in the duplication (up to 65536 Gaussians), on
-    its own and behind the sort by depth: images, gradients and weights of a sequence of views against the stages; a training frame
+    """More instances than the buffers hold or the launches were sized for, with the blend queued ahead (3000 Gaussians) and behind the
+    number (80 000), with the scan in the duplication and, where the Gaussians are sorted by depth first, on its own: images, gradients and weights of a sequence of views against the stages; a training frame
     keeps the workspace that it was rendered with and no other."""
     scene = make_scene(0, n)
     todo, scene_gpu = [s._replace(mode=RasterizerMode(mode)) for s in views(scene, cuda)], scene.to(cuda)
