@@ -254,7 +254,8 @@ struct FusedScan {
     uint32_t tag;
 };
 constexpr uint32_t kListWindow = 2048;           // (256 Gaussians have 1300 instances of masks on average: one window)
-constexpr uint32_t kListTileBits = 24;           // of an entry of the window, beside the eight of the thread
+constexpr uint32_t kListTileBits = 24;           // of an entry of the window, beside the eight of the thread: the tile counted from its rectangle's corner, whatever
+                                                 // the grid (64 rows of 2^16 tiles at most; corner and place are one read of LDS)
 // Tiles of a mask that a lane puts down by itself; twice as many in a wave in which more than kListBetween masks have one to two times that:
 // the wave takes those one by one otherwise.  (us; all by the lane up to 6, 8, 12, 16, 24 tiles: 15 M instances of 3 M Gaussians 66, 54,
 // 46, 48, 51.  With one line at twelve -> with the second, and the search element by element that this replaced: OIT 50 k Gaussians at
@@ -269,7 +270,8 @@ __global__ void __launch_bounds__(256) create_listed_kernel(
     FusedScan scan)
 {
     static_assert(!(DEPTH && ORDERED), "keys of the tile alone");
-    __shared__ uint32_t s_list[kListWindow], s_base[256];     // instances of the masks: tile | thread << kListTileBits; what to add for their place in the list
+    __shared__ uint32_t s_list[kListWindow];                  // instances of the masks: tile from the corner | thread << kListTileBits
+    __shared__ uint2 s_from[256];                             // what to add for their place in the list, and the corner
     __shared__ uint32_t s_depth[DEPTH ? 256 : 1], s_gaussian[ORDERED ? 256 : 1];
     __shared__ uint32_t s_sums[kScanBlock / kWave];
     __shared__ uint32_t s_row_end[256 / kWave][kWave], s_row_tile[256 / kWave][kWave];
@@ -326,7 +328,7 @@ __global__ void __launch_bounds__(256) create_listed_kernel(
     const uint32_t masked = large ? 0u : count;
     uint32_t total;
     const uint32_t inc = block_inclusive_scan(masked, s_sums, &total);
-    s_base[threadIdx.x] = (end - count) - (inc - masked);
+    s_from[threadIdx.x] = make_uint2((end - count) - (inc - masked), (t.corner >> 16) * grid_w + (t.corner & 0xffffu));
     if (ORDERED) s_gaussian[threadIdx.x] = gaussian;
     if (DEPTH) s_depth[threadIdx.x] = depth;
     {
@@ -338,7 +340,7 @@ __global__ void __launch_bounds__(256) create_listed_kernel(
         const uint64_t between = __ballot(masked > kListOwn && masked <= 2u * kListOwn);
         const bool many = masked > (__popcll(between) > (int)kListBetween ? 2u * kListOwn : kListOwn);
         uint32_t lo = large || many ? 0u : t.lo, hi = large || many ? 0u : t.hi, at = begin;
-        const uint32_t w = t.size & 0xffffu, corner = (t.corner >> 16) * grid_w + (t.corner & 0xffffu);
+        const uint32_t w = t.size & 0xffffu;
         const float per_row = __builtin_amdgcn_rcpf((float)w);
         for (uint32_t from = 0; from < total; from += kListWindow) {       // (the same for the whole block)
             if (from != 0u) __syncthreads();                              // (the window before is read)
@@ -349,7 +351,7 @@ __global__ void __launch_bounds__(256) create_listed_kernel(
                 hi = low ? hi : rest;
                 // (bit < 64 and w <= 64: the quotient of bit + 1/2 is never within rounding of a whole number)
                 const uint32_t row = (uint32_t)(((float)bit + 0.5f) * per_row);
-                s_list[at - from] = (corner + __umul24(row, grid_w) + (bit - __umul24(row, w))) | threadIdx.x << kListTileBits;
+                s_list[at - from] = (__umul24(row, grid_w) + (bit - __umul24(row, w))) | threadIdx.x << kListTileBits;
                 ++at;
             }
             for (unsigned long long owners = __ballot(many && begin < from + kListWindow && inc > from); owners != 0; owners &= owners - 1) {     // (wave-uniform)
@@ -360,12 +362,14 @@ __global__ void __launch_bounds__(256) create_listed_kernel(
                 const uint32_t row = (uint32_t)(((float)lane + 0.5f) * bits_to_float(of(float_to_bits(per_row))));
                 const bool set = ((lane < 32u ? olo >> lane : ohi >> (lane - 32u)) & 1u) != 0u;
                 if (set && to >= from && to < from + kListWindow)
-                    s_list[to - from] = (of(corner) + __umul24(row, grid_w) + (lane - __umul24(row, ow))) | (wave * kWave + (uint32_t)owner) << kListTileBits;
+                    s_list[to - from] = (__umul24(row, grid_w) + (lane - __umul24(row, ow))) | (wave * kWave + (uint32_t)owner) << kListTileBits;
             }
             __syncthreads();
             const uint32_t here = total - from < kListWindow ? total - from : kListWindow;
             for (uint32_t e = threadIdx.x; e < here; e += 256) {
-                const uint32_t listed = s_list[e], l = listed >> kListTileBits, tile = listed & ((1u << kListTileBits) - 1u), to = s_base[l] + from + e;
+                const uint32_t listed = s_list[e], l = listed >> kListTileBits;
+                const uint2 base = s_from[l];
+                const uint32_t tile = base.y + (listed & ((1u << kListTileBits) - 1u)), to = base.x + from + e;
                 keys[to] = DEPTH ? (KeyT)((uint64_t)tile << (DEPTH ? 32 : 0) | (uint64_t)s_depth[DEPTH ? l : 0]) : (KeyT)tile;
                 vals[to] = ORDERED ? s_gaussian[l] : (uint32_t)(first + l);
             }
@@ -871,9 +875,6 @@ static int create_instances(const htgs_frame *f, const FusedScan *scan)
     const int prim_floats = frame_prim_floats(f);
     if (prim_floats < 0) return fail(HTGS_ERR_ARGUMENT, "htgs_create_instances: prim_floats must be 0, %d or %d", HTGS_PRIM_FLOATS, HTGS_PRIM_FLOATS_TRAIN);
     if (f->touch) {
-        // (htgs_scan_offsets and htgs_blend stop at 2^20 tiles; a caller with offsets of its own gets as far as an entry of the window holds)
-        if ((uint64_t)grid_w * (uint64_t)div_up(f->height, tile) > (1ull << kListTileBits))
-            return fail(HTGS_ERR_ARGUMENT, "htgs_create_instances: more than 2^24 tiles");
         const bool first_k = f->mode == HTGS_MODE_ALPHA_BLEND_FIRST_K;
         const float min_alpha_rcp = first_k ? 20.0f : 255.0f;
         const float cutoff_sq = first_k ? ModeCfg<HTGS_MODE_ALPHA_BLEND_FIRST_K>::cutoff_sq : ModeCfg<HTGS_MODE_HYBRID_BLEND>::cutoff_sq;

@@ -189,20 +189,6 @@ def test_instance_counts_beyond_32_bit_offsets_are_refused():
     assert lib.htgs_create_instances(ctypes.byref(f)) == 2 and b"null pointer" in lib.htgs_last_error()
 
 
-def test_duplication_refuses_grids_beyond_its_window():
-    """An entry of the duplication's window in LDS holds the tile in 24 bits beside the thread; a larger grid is refused before the launch.
-    (No pointer is followed.)"""
-    lib = _native.lib()
-    f = _native.Frame()
-    f.n_primitives = f.n_instances = 1
-    for name in ("n_touched", "offsets", "touch", "prim"):
-        setattr(f, name, 256)                                # any address that is not NULL
-    f.keys[0] = f.vals[0] = 256
-    for mode, tile in ((0, 8), (1, 8), (2, 16), (3, 8)):
-        f.mode, f.width, f.height = mode, 4097 * tile, 4096 * tile
-        assert lib.htgs_create_instances(ctypes.byref(f)) == 2 and b"2^24 tiles" in lib.htgs_last_error()
-
-
 def test_self_check_entry_points_reject_bad_arguments():
     lib = _native.lib()
     f = _native.Frame()

@@ -65,21 +65,25 @@ def test_instances_of_masks(cuda, spread, n, mode):
 
 
 @pytest.mark.parametrize("mode", [0, 2, 3])
-def test_instances_on_a_grid_beyond_two_to_the_twenty_tiles(cuda, mode):
-    """The duplication on its own, with offsets from elsewhere (the scan stops at 2^20 tiles): an entry of the window has room for 2^24."""
-    print(f"case mode={mode}", flush=True)
+@pytest.mark.parametrize("by", [256, 1024])
+def test_instances_on_a_grid_beyond_two_to_the_twenty_tiles(cuda, by, mode):
+    """The duplication on its own, with offsets from elsewhere (the scan stops at 2^20 tiles): an entry of the window counts its tile from
+    the mask's corner, whose number has 32 bits.  (Grids of 2^21 and 2^25 tiles; the stages in question have no image and no ranges.)"""
+    print(f"case by={by} mode={mode}", flush=True)
     n = 1000
     rng = np.random.default_rng(3)
     scene = tie_scene(rng.uniform(1.0, 9.0, n).tolist(), rng.uniform(0.3, 1.0, n).tolist(), rng.uniform(0.0, 1.0, (n, 3)).tolist())
     scene.positions[:, :2] = torch.from_numpy(rng.uniform(-0.3, 0.3, (n, 2)).astype(np.float32)) * scene.positions[:, 2:3]
-    by = 512.0 if mode == 2 else 256.0
-    scene.width, scene.height = int(64 * by) + 16, int(32 * by) + 16
+    by *= 2 if mode == 2 else 1                              # (tiles of twice the edge)
     scene.VPM[0] *= by
     scene.VPM[1] *= by / 2.0
     scene.scales *= 1.0 / by
     gpu = scene.to(cuda)
     fb = FrameBuffers(*gpu.gaussians(), gpu.settings(RasterizerMode(mode), 4), True, False, tight_lists=True, order_gaussians=False)
-    assert 1 << 20 < fb.n_tiles < 1 << 24
+    fb.frame.width, fb.frame.height = 64 * by + 16, 32 * by + 16
+    fb.grid_w = (fb.frame.width + fb.tile - 1) // fb.tile
+    fb.key_bytes = fb.lib.htgs_frame_key_bytes(fb._ref)
+    assert fb.key_bytes == (8 if mode == 2 else 4)
     fb.preprocess()
     offsets = torch.cumsum(fb.n_touched, 0).to(torch.int32)
     fb.offsets.copy_(offsets)
@@ -88,7 +92,8 @@ def test_instances_on_a_grid_beyond_two_to_the_twenty_tiles(cuda, mode):
     fb.create_instances()
     torch.cuda.synchronize()
     want = listed(fb)
-    assert want is not None and len(want) == count and max(t for t, _ in want) > 1 << 20
+    assert want is not None and len(want) == count
+    assert max(t for t, _ in want) > (1 << 20 if by <= 512 else 1 << 24)
     keys = u32(fb.keys[0])[:count].astype(np.uint64)
     tiles = keys >> np.uint64(32) if mode == 2 else keys
     assert sorted(zip(tiles.astype(np.int64).tolist(), u32(fb.vals[0])[:count].tolist())) == want
