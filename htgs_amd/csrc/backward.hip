@@ -45,14 +45,14 @@ __device__ __forceinline__ int find_core_slot(const uint32_t *__restrict__ keys,
 }
 
 // ---------------------------------------------------------------------------------------------
-// HYBRID_BLEND (K >= 1), OIT_BLEND (K == 0) and ALPHA_BLEND_FIRST_K (core only, no tail): one lane per Gaussian
-// of the staged batch, all lanes walk the 64 pixels of the tile together (per-pixel terms are LDS broadcasts).
+// HYBRID_BLEND (K >= 1), OIT_BLEND (K == 0) and ALPHA_BLEND_FIRST_K (core only, no tail): one lane per Gaussian of the
+// tile's list and 4x4 quadrant of the tile that it can reach, which walks the quadrant's sixteen pixels (backward_tile).
 // The reference's FIRST_K backward runs one thread per stored fragment with ~20 atomics each
 // (R/include/alpha_blend_first_k/kernels/backward.cuh:60-206); walking the tile's list and looking each
 // (Gaussian, pixel) up in the stored core visits the same fragments.
 // ---------------------------------------------------------------------------------------------
-// A workgroup is four waves sharing one tile's per-pixel terms in LDS (22 KB for K = 16); wave w takes the
-// batches w, w + 4, ... of the tile's list.
+// A workgroup is four waves sharing one tile's per-pixel terms and a chunk of 256 instances in LDS (25 KB for K = 16); the
+// waves take the turns of the chunk one after the other.
 constexpr int kBackwardWaves = 4;
 
 // Gradients of the three VPMT rows from the moments of dL/d|m|^2 (S, times kc2 / 2) and dL/d|d|^2 (T) over a tile,
@@ -108,7 +108,7 @@ __device__ __forceinline__ void moments_to_rows(const float4 &V1, const float4 &
 // stress scene at 1600x1066 2414 -> 2250 (of which the second look of the forward pass 35), 500 k at 1280x720 with K = 32
 // 1176 -> 1080.  What bounds it now: a vector instruction every 3.6 cycles, a hundred and thirty a pixel, of which the search for
 // the core's slot is thirty (110 us of the step).
-// A lane builds its Gaussian's quadratics again (a hundred instructions against three thousand of the walk; its record
+// A lane builds its Gaussian's quadratics again (a hundred instructions against the two thousand of its sixteen pixels; its record
 // is in the caches), walks the quadrant's 16 pixels row by row, and the two to four lanes of one Gaussian, neighbours, fold
 // their sixteen sums with two shifted additions; the first lane of each Gaussian applies the chain and writes the gradient row.
 // Where a pixel's terms sit in LDS.  The lanes of a turn read the terms of up to four pixels, one per quadrant, at the
@@ -129,7 +129,7 @@ constexpr int kTrainRec4 = HTGS_PRIM_FLOATS_TRAIN / 4;
 // plus the tile's place among those listed for it, both from the sixth word of the training record -- first slot, corner of
 // its rectangle (column_bits), then either the rectangle's width (all of it is listed, row-major) or, with bit 31 of the second
 // word set, the width in bits 24-30 there and the mask of the listed tiles in the last two.  Without branches
-// and divisions, since every lane of a batch works one out (blend backward, 1 M at 1080p, HYBRID K = 16: 929 -> 918 us on these
+// and divisions, since one is worked out for every instance (blend backward, 1 M at 1080p, HYBRID K = 16: 929 -> 918 us on these
 // lists, 908 -> 896 on whole rectangles against a division by the grid's width and a branch for each form).
 struct TilePlace {
     uint32_t column, row, shift;           // of the tile; column_bits
@@ -513,8 +513,9 @@ __global__ void __launch_bounds__(64 * kBackwardWaves) __attribute__((amdgpu_wav
 }
 
 // The tiles with very long lists (and their parts): the workgroups take them off the list the kernel above made, longest first.
-// (Four waves per SIMD: with the bookkeeping of the parts the 96 registers of five leave 128 bytes a lane in scratch memory, read inside
-// the pixel loop; training step of 600 k of the stress scene at 1600x1066 2210 -> 2160 us.)
+// (Four waves per SIMD: with the bookkeeping of the parts the 96 registers of five leave up to 128 bytes a lane in scratch memory, read inside
+// the pixel loop.  Training step of 600 k of the stress scene at 1600x1066, five -> four waves: HYBRID K = 1 1718 -> 1694 us, 4 1763 -> 1739,
+// 8 1870 -> 1835, 16 2170 -> 2111; FIRST_K K = 4 1184 -> 1175; OIT 1525 -> 1505.)
 template <int K, int MODE, bool HELPER>
 __global__ void __launch_bounds__(64 * kBackwardWaves) __attribute__((amdgpu_waves_per_eu(HELPER ? 3 : 4))) blend_tail_backward_long_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,

@@ -454,7 +454,8 @@ __device__ __forceinline__ void quadrant_list_walk(const QuadrantLists &ql, uint
 // other.  An odd number of turns ends with a turn of dummy slots (every list has 64 entries, the dummy's behind the hits).
 // A wave that runs alone issues an instruction every 2.5 ns, waits 24 ns for a row from LDS and 14 ns between a compare and
 // the branch on it; five waves a SIMD cover most of that but not all.  One turn -> two at a time, whole passes: HYBRID K = 16, 3 M
-// Gaussians at 1920x1080 1373 -> 1306 us, FIRST_K 1 M at 1280x720 351 -> 334, OIT 334 k at 1237x821 163.8 -> 159.8.  Cores of 32 have
+// Gaussians at 1920x1080 1373 -> 1306 us, FIRST_K 1 M at 1280x720 351 -> 334, OIT 334 k at 1237x821 163.8 -> 159.8 (3 M at 1920x1080,
+// one wave a tile, is bound by the reads of LDS and gains nothing: blend 800 -> 801).  Cores of 32 have
 // no registers left for a second fragment and keep the walk above, like the walks with three registers a slot.
 template <typename Turns>
 __device__ __forceinline__ void quadrant_list_walk_pairs(const QuadrantLists &ql, uint32_t n_turns, uint32_t lane, Turns &&turns)

@@ -16,7 +16,7 @@ namespace htgs {
 // longer than long_threshold is left to blend_hybrid_long_kernel if the caller provided the list for such tiles.
 // (A core of sixteen with three registers a slot does not fit the 96 registers of five waves per SIMD: 120 bytes a lane in scratch
 // memory, some of it inside the walk.  Four waves without them: training step of 1 M Gaussians at 1920x1080, HYBRID K = 16, 1734 ->
-// 1686 us, FIRST_K 1180 -> 1175.  Where five waves fit, as for the cores of up to eight, four cost 6 %.)
+// 1686 us, FIRST_K 1180 -> 1169, 300 k at 1280x720 481 -> 456.  Where five waves fit, as for the cores of up to eight, four cost 6 %.)
 template <int K>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 8 ? 5 : K <= 16 ? 4 : 3))) blend_hybrid_forward_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,

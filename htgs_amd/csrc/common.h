@@ -156,7 +156,7 @@ struct FrameStart {
 };
 int preprocess_and_start(const htgs_frame *f, const FrameStart &start);                 // preprocess.hip
 // The scan for htgs_run, which also writes tag << 32 | total to host memory.  with_sums: scan_tmp holds FrameStart's sums.
-// Returns in *fused whether the scan was left to create_instances_fused (few Gaussians).
+// Returns in *fused whether the scan was left to create_instances_fused (up to 2^21 Gaussians).
 int scan_offsets_publish(const htgs_frame *f, unsigned long long *host_total, uint32_t tag, bool with_sums, bool *fused);    // instances.hip
 int create_instances_fused(const htgs_frame *f, unsigned long long *host_total, uint32_t tag);
 // (cleared: the ranges, bins and header are zero already; ranged: the sort has written the ranges)

@@ -242,10 +242,11 @@ __global__ void __launch_bounds__(256) create_instances_kernel(
 // where they are written element by element; the large rectangles are the waves' own work, one
 // after the other, the rows in the lanes and then the row's tiles element by element over a search in the rows' ends.
 // Which tile of a Gaussian comes first does not matter: the sort that follows is by tile.
-// SCAN: the offsets are not there yet.  Every block adds up the block sums before its own (few: kFusedScanMost Gaussians)
+// SCAN: the offsets are not there yet.  Every block adds up the block sums before its own (up to kFusedScanMost Gaussians)
 // and scans its counts, which spares the frame the launch of the scan; the last block publishes the total.  A block of 256 counts
-// reads up to 32 KB of sums so: 334 k Gaussians (OIT, 1237x821) 160 -> 158 us, 1 M (FIRST_K, 1280x720) 329.6 -> 326.3, weights of 1 M
-// 606 -> 602.5, 3 M 1296 -> 1294 and 6 M 4806 -> 4812, within the noise: the line is between.
+// reads up to 32 KB of sums so, which grows with the square of the Gaussians.  With a launch of its own -> fused, OIT at 256x256:
+// 200 k Gaussians 110.9 -> 107.1 us, 500 k 160.7 -> 156.7, 1 M 228.7 -> 226.0, 1.5 M 308.3 -> 304.8, 2 M 387.8 -> 384.1; weights of 2 M at
+// 640x400 769.8 -> 763.2.  Frames of 3 M 1296 -> 1294 and of 6 M 4806 -> 4812, within the noise: nothing is gained beyond the line.
 constexpr int kFusedScanMost = 1 << 21;
 struct FusedScan {
     const uint32_t *block_sums;
