@@ -6,8 +6,8 @@
 // the reference's ray / Gaussian expressions in the tile-relative form (TileFrag, blend_common.h), in which |m|^2, |d|^2 and
 // MT3.(d x m) are quadratics of the pixel offset from the tile centre.  log and 2^x are the
 // polynomial routines below, sqrt and division are correctly rounded
-// (-fhip-fp32-correctly-rounded-divide-sqrt; rcp_exact is the same quotient, cheaper).  The CPU
-// checker used by the test-suite follows the same convention, which is what makes tile counts, sort
+// (-fhip-fp32-correctly-rounded-divide-sqrt; rcp_exact is the same quotient, cheaper).  The
+// CPU oracle of the tests follows the same convention, which is what makes tile counts, sort
 // order and every per-fragment accept/reject decision reproducible bit for bit.
 #pragma once
 

@@ -5,7 +5,7 @@ pixels whose accept / reject decisions are not within 1e-4 of a threshold (only 
 gradients of sum(image * grad_image) over those pixels, and the third densification statistic (per Gaussian, the sum
 over those pixels of the 1-norm of the pixel's own position gradient).
 
-The reference ships no test vectors; these are this repository's own, frozen so that a change of the CPU checker and
+The reference ships no test vectors; these are this repository's own, frozen so that a change of the CPU oracle and
 of the kernels in the same direction still has something to answer to.  Run from the repository root:
 
     python tests/golden/make_fixtures.py
