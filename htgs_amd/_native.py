@@ -56,6 +56,7 @@ class Frame(ctypes.Structure):
         ("long_counters", ctypes.c_void_p),
         ("tile_order", ctypes.c_void_p),
         ("depth_order", ctypes.c_void_p),
+        ("depth_bins", ctypes.c_void_p),
         ("n_instances", ctypes.c_uint64),
         ("n_instances_live", ctypes.c_void_p),
         ("keys", ctypes.c_void_p * 2),
@@ -122,6 +123,7 @@ SYMBOLS = {
     "htgs_frame_sort_passes": (ctypes.c_int, [_FRAME_P]),
     "htgs_frame_depth_sort_passes": (ctypes.c_int, [_FRAME_P]),
     "htgs_depth_order_words": (ctypes.c_size_t, [ctypes.c_int]),
+    "htgs_depth_bins_words": (ctypes.c_size_t, [ctypes.c_int]),
     "htgs_depth_order_result_word": (ctypes.c_size_t, [_FRAME_P]),
     "htgs_scan_tmp_words": (ctypes.c_size_t, [ctypes.c_int]),
     "htgs_sort_tmp_words": (ctypes.c_size_t, [ctypes.c_uint64]),

@@ -888,7 +888,7 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
         for (int q = (words & ~3) + threadIdx.x; q < words; q += 256) lds[q] = sh_rest[base_word + q];
     }
     __syncthreads();
-    // Row sums.  The Gaussian's instances are the rows [offsets[i-1], offsets[i]).  Few rows are added up front to back by four
+    // Row sums.  The Gaussian's instances are the n_touched[i] rows before offsets[i].  Few rows are added up front to back by four
     // lanes, a quarter of the row each: a load of the wave then touches sixteen rows, whole lines, where a lane per Gaussian
     // touched a quarter of 64 lines (1 M Gaussians at 1920x1080: 189 -> 174 us, 0.8 GB).  A Gaussian with many rows would keep the other lanes of
     // its wave waiting, so the wave takes those one at a time: 16 rows x 4 quarters per step (1 KB of consecutive memory), a butterfly over the 16
@@ -901,7 +901,7 @@ __global__ void __launch_bounds__(256) preprocess_backward_kernel(
     {
         const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
         uint32_t r0 = 0u, r1 = 0u;
-        if (live) { r0 = i == 0 ? 0u : offsets[i - 1]; r1 = offsets[i]; }
+        if (live) { r1 = offsets[i]; r0 = r1 - n_touched[i]; }
         const uint32_t count = r1 - r0;
         // (lane 4 j + c adds up quarter c of the rows of the sixteen Gaussians' j-th)
 #pragma unroll

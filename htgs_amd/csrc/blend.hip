@@ -187,11 +187,11 @@ static void launch_hybrid(const htgs_frame *f, int selector, uint32_t grid_w, ui
     if (f->long_tiles != nullptr && most_threshold(f) <= kPackedListMost)
         hipLaunchKernelGGL((blend_hybrid_kernel<K, FAST, true>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
-                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
+                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order, binned_spare(f, selector));
     else
         hipLaunchKernelGGL((blend_hybrid_kernel<K, FAST>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
-                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
+                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order, binned_spare(f, selector));
     // (its workgroups find an empty list on ordinary frames)
     launch_hybrid_long<K, FAST, HTGS_PRIM_FLOATS / 4>(f, selector, grid_w, HybridImage{ f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, f->to_chw, f->use_median_depth });
 }
@@ -202,11 +202,11 @@ static void launch_first_k(const htgs_frame *f, int selector, uint32_t grid_w, u
     if (!FAST && f->long_tiles != nullptr && most_threshold(f) <= kPackedListMost)
         hipLaunchKernelGGL((blend_first_k_kernel<K, false, true>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
-                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
+                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order, binned_spare(f, selector));
     else
         hipLaunchKernelGGL((blend_first_k_kernel<K, FAST>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[selector],
                            (const float4 *)f->prim, f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->to_chw,
-                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order);
+                           f->use_median_depth, f->long_tiles, threshold, long_part_floor(f, selector), f->tile_order, binned_spare(f, selector));
     launch_first_k_long<K, FAST, HTGS_PRIM_FLOATS / 4>(f, selector, grid_w, FirstKImage{ f->image, FAST ? nullptr : f->depth, (uint32_t)f->width, (uint32_t)f->height, f->to_chw, f->use_median_depth });
 }
 
@@ -275,6 +275,9 @@ extern "C" int htgs_blend(const htgs_frame *f, int selector)
     const uint32_t n_tiles = grid_w * grid_h;
     // (an entry of the list of long tiles holds the tile in 20 bits; htgs_scan_offsets refuses larger grids as well)
     if ((uint64_t)grid_w * grid_h > (1ull << 20)) return fail(HTGS_ERR_ARGUMENT, "htgs_blend: more than 2^20 tiles");
+    // (the kernels that note where equal depths met)
+    if (frame_depth_binned(f) && !f->fast_math && f->n_instances > 0 && (!f->vals[selector ^ 1] || !f->long_tiles || most_threshold(f) > kPackedListMost))
+        return fail(HTGS_ERR_ARGUMENT, "htgs_blend: depth_bins needs both value buffers and long_tiles with a threshold of no more than %u", kPackedListMost);
     if (blend_waves(f, selector, grid_w, n_tiles)) return check_launch("blend");
     if (f->fast_math) launch_blend<true>(f, selector, grid_w, n_tiles);
     else launch_blend<false>(f, selector, grid_w, n_tiles);

@@ -469,7 +469,7 @@ __device__ __forceinline__ void quadrant_list_walk_pairs(const QuadrantLists &ql
         at = next;
     }
 }
-// The walk over instances [first, last) of a tile's list (whole batches of 64 from `first` on) by one wave, lanes =
+// The walk over instances [first, last) of a tile's list (whole batches of 64 from `first` on, `step` apart) by one wave, lanes =
 // pixels by quadrants: every batch is staged (tile_stage_load with the CULL asked for), its quadrant lists are built and
 // turn(addr) is called for every turn.  SOLO: the wave is the whole workgroup (its barriers are the workgroup's).
 // AHEAD: a lane reads the list entry of the next batch before it walks this one (one register more through the walk; the
@@ -479,16 +479,16 @@ template <int MODE, bool DEPTH, int CULL, bool SOLO, int REC4 = HTGS_PRIM_FLOATS
           typename Turn>
 __device__ __forceinline__ void tile_list_walk(TileStageQ &st, QuadrantLists &ql, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst,
                                                uint32_t first, uint32_t last, uint32_t lane, float cx, float cy, Turn &&turn, uint64_t pixel_lanes = 0,
-                                               float cull_scale = 1.0f)
+                                               float cull_scale = 1.0f, uint32_t step = 64u)
 {
     stage_dummy_init(st, lane);
     uint32_t listed = 0;
     if (AHEAD) listed = first + lane < last ? inst[first + lane] : 0u;
-    for (uint32_t base = first; base < last; base += 64) {
+    for (uint32_t base = first; base < last; base += step) {
         if (SOLO) __syncthreads(); else wave_lds_sync();
         const uint32_t bits = tile_stage_load<MODE, kStageSlots, DEPTH, CULL, true, REC4, UNIT, POS, AHEAD>(st, prim, inst, base + lane, last, lane + 1, cx, cy, pixel_lanes,
                                                                                                            listed, cull_scale);
-        if (AHEAD) listed = base + 64u + lane < last ? inst[base + 64u + lane] : 0u;
+        if (AHEAD) listed = base + step + lane < last ? inst[base + step + lane] : 0u;
         const uint32_t n_turns = quadrant_lists_build(ql, bits, lane, st);
         if (SOLO) __syncthreads(); else wave_lds_sync();
         // lanes outside the image run along (their results are never stored): the loop stays wave-uniform
@@ -750,6 +750,217 @@ __device__ __forceinline__ void subtile_walk(const uint16_t *reach, uint32_t sta
             turns(one != kNoHit ? one + part_base : part_base, one != kNoHit, two != kNoHit ? two + part_base : part_base, two != kNoHit);
         }
     }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Lists in bins of depth (htgs_frame.depth_bins): a tile's list is up to kDepthBins runs, each by Gaussian index.  What the
+// reference's insertion leaves where fragments are exactly equally deep depends on their order by index over the whole list.
+// ---------------------------------------------------------------------------------------------
+// The finished core's entries [i], [i + 1] of equal depth, in the order the reference's insertion leaves them in: an entry that
+// comes nearer than both hops the first over the second, so they are by index if an even number of the nearer entries has a
+// higher index than both, and the other way round if an odd number has.  (All nearer fragments are in the core as long as
+// the two are.)  True where more than two are equally deep: that order takes a walk by index.
+template <int K, typename IndexT>
+__device__ __forceinline__ bool settle_equal_pairs(float (&cd)[K], float (&ca)[K], IndexT (&ci)[K])
+{
+    static_assert(sizeof(IndexT) == 4, "an index or its bit pattern");
+    bool more = false;
+#pragma unroll
+    for (int i = 0; i + 1 < K; ++i) {
+        const bool equal = ca[i + 1] > 0.0f && cd[i] == cd[i + 1];
+        if (!__any(equal)) continue;
+        if (i + 2 < K) more = more || (equal && ca[i + 2 < K ? i + 2 : i] > 0.0f && cd[i + 1] == cd[i + 2 < K ? i + 2 : i]);
+        uint32_t a, b;
+        __builtin_memcpy(&a, &ci[i], 4);
+        __builtin_memcpy(&b, &ci[i + 1], 4);
+        const uint32_t high = a > b ? a : b;
+        bool odd = false;
+#pragma unroll
+        for (int j = 0; j < i; ++j) {
+            uint32_t x;
+            __builtin_memcpy(&x, &ci[j], 4);
+            odd = odd != (x > high);
+        }
+        if (equal && (a > b) != odd) {
+            const float t = ca[i]; ca[i] = ca[i + 1]; ca[i + 1] = t;
+            const IndexT x = ci[i]; ci[i] = ci[i + 1]; ci[i + 1] = x;
+        }
+    }
+    return more;
+}
+
+// What a walk notes of equal depths at the end of a pixel's core: the least depth at which a fragment stayed out of the core, or left it,
+// that is exactly as deep as the entry that is last then (the core's last depth never grows, so the latest such depth is the least); that
+// fragment's index, with kMoreTied if it was not the only one as deep.
+constexpr uint32_t kMoreTied = 1u << 31;
+struct CoreTie {
+    float depth;
+    uint32_t other;
+    __device__ __forceinline__ void init() { depth = __FLT_MAX__; other = 0u; }
+    __device__ __forceinline__ void note(float at, uint32_t index)
+    {
+        asm volatile("");              // (branched over by a wave without one)
+        other = index | (depth == at ? kMoreTied : 0u);
+        depth = at;
+    }
+    // another wave's note of the same pixel
+    __device__ __forceinline__ void join(const CoreTie &t)
+    {
+        other = t.depth < depth ? t.other : t.depth == depth ? other | kMoreTied : other;
+        depth = t.depth < depth ? t.depth : depth;
+    }
+    // (nothing stays out of a core that is not full)
+    __device__ __forceinline__ bool at_end(float last_depth) const { return depth < __FLT_MAX__ && depth <= last_depth; }
+};
+// two entries of the finished core are exactly as deep as each other, or one that is not in it is as deep as its last
+template <int K>
+__device__ __forceinline__ bool core_tied(const float (&cd)[K], const float (&ca)[K], const CoreTie &tie)
+{
+    bool tied = tie.at_end(cd[K - 1]);
+#pragma unroll
+    for (int i = 0; i + 1 < K; ++i) tied = tied || (ca[i + 1] > 0.0f && cd[i] == cd[i + 1]);
+    return tied;
+}
+// The finished core of every pixel of the wave with its entries of equal depth as the reference's insertion leaves them, from the core
+// alone: pairs inside it are put in order (settle_equal_pairs), and where its last entry and one other fragment are equally deep, that
+// fragment is evaluated at the pixel and takes the last entry's place if the order by index says so: of the two, the one
+// with the lower index stays if an even number of the nearer entries has a higher index than both, the other one if an odd number
+// has.  (The last arrival of the K + 1 decides: one of the two is turned away, any other hops the first over the second, which
+// leaves.)  noted: a fragment met the last entry's depth; other: its index, more: it was not the only one (CoreTie).  held(alpha):
+// the alpha that the core would hold; swapped(out, in): the tail has lost a fragment and gained another one of the last entry's
+// depth.  True for the pixels that this does not settle: more than two of a depth, or a tail that cannot give up an opaque fragment.
+// A pixel that is settled so costs the evaluation of one fragment; walking the tile's list for it took as long as a list of a
+// third of its length, at the end of a launch as often as not (6 M Gaussians of the stress scene at 1600x1066: the launch with
+// one wave per tile 1050 -> 730 us).
+template <int MODE, int K, int REC4, typename IndexT, typename Held, typename Swapped>
+__device__ __forceinline__ bool settle_core(TileStageQ &st, const float4 *__restrict__ prim, uint32_t lane, const PixelTerms &pt, float cx, float cy, float (&cd)[K],
+                                            float (&ca)[K], IndexT (&ci)[K], bool noted, uint32_t other, bool more, Held &&held, Swapped &&swapped)
+{
+    bool again = false, pairs = false;
+#pragma unroll
+    for (int i = 0; i + 1 < K; ++i) pairs = pairs || (ca[i + 1] > 0.0f && cd[i] == cd[i + 1]);
+    if (__any(pairs)) again = settle_equal_pairs<K>(cd, ca, ci);
+    if (!__any(noted)) return again;
+    wave_lds_sync();
+    // (a slot for each lane, as in a batch of the walk)
+    tile_stage_load<MODE, kStageSlots, true, kCullNone, true, REC4, false, false, true>(st, prim, nullptr, noted ? 0u : 1u, 1u, (int)lane + 1, cx, cy, 0, other);
+    wave_lds_sync();
+    const uint32_t addr = stage_slot_address(st, lane);
+    TileFrag f;
+    tile_frag_exact<MODE, kStageSlots>(addr, pt, f);
+    const bool meets = noted && tile_frag_depth<kStageSlots>(addr, pt, f) == cd[K - 1];
+    if (meets && (more || (K > 1 && cd[K - 1] == cd[K > 1 ? K - 2 : 0]) || (MODE == HTGS_MODE_HYBRID_BLEND && f.alpha > 0.99f))) again = true;
+    uint32_t last;
+    __builtin_memcpy(&last, &ci[K - 1], 4);
+    const uint32_t high = last > other ? last : other;
+    bool odd = false;
+#pragma unroll
+    for (int j = 0; j + 1 < K; ++j) {
+        uint32_t x;
+        __builtin_memcpy(&x, &ci[j], 4);
+        odd = odd != (x > high);
+    }
+    if (meets && !again && (other > last) == odd) {
+        const float alpha = held(f.alpha);
+        swapped(ca[K - 1], alpha);
+        ca[K - 1] = alpha;
+        __builtin_memcpy(&ci[K - 1], &other, 4);
+    }
+    return again;
+}
+// (the lane and its pixel worked out afresh, so that nothing has to live through the pixels' finish for a rare second walk)
+__device__ __forceinline__ uint32_t fresh_lane()
+{
+    uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
+
+// The tile's list [first, last) of inst by Gaussian index: spare, into whose stretch of the same place the runs are merged, or inst
+// where the list is one run (a frame without bins).  Called by WAVES whole waves (WAVES = 1: by a wave, whatever else its workgroup
+// does) of which each merges a range of the indices; more than one synchronises before it reads what the others wrote.  s_runs:
+// 1 + kDepthBins words of LDS.  A step looks at the next eight entries of every run: what is not above the least of the runs' eighth
+// entries is among the 64, and goes out in its order (28 to 64 entries a step; a list of 500 entries 20 us).
+template <int WAVES>
+__device__ __forceinline__ const uint32_t *list_in_index_order(const uint32_t *inst, uint32_t first, uint32_t last, uint32_t *spare, uint32_t *s_runs, uint32_t wave,
+                                                               uint32_t lane)
+{
+    static_assert(kDepthBins * 8 == kWave, "eight lanes to a run");
+    const auto sync = []() { if (WAVES > 1) __syncthreads(); else wave_lds_sync(); };
+    sync();
+    if (lane == 0 && wave == 0) s_runs[0] = 0u;
+    sync();
+    const uint32_t batches = (last - first + 63u) / 64u;
+    for (uint32_t b = (uint32_t)((uint64_t)batches * wave / WAVES); b < (uint32_t)((uint64_t)batches * (wave + 1u) / WAVES); ++b) {
+        const uint32_t at = first + 64u * b + lane;
+        const bool begins = at < last && at > first && inst[at] < inst[at - 1u];
+        for (uint64_t m = __ballot(begins); m != 0; m &= m - 1) {              // (wave-uniform)
+            if (lane == 0) {
+                const uint32_t k = atomicAdd(s_runs, 1u);
+                if (k < (uint32_t)kDepthBins - 1u) s_runs[1u + k] = first + 64u * b + (uint32_t)__builtin_ctzll(m);
+            }
+        }
+    }
+    sync();
+    const uint32_t more = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_runs[0]);
+    if (more == 0u || more > (uint32_t)kDepthBins - 1u) return inst;
+    // lane r: what is left of run r
+    uint32_t at = last, end = last;
+    if (lane == 0) at = first;
+    uint32_t start = last;
+    if (lane >= 1u && lane <= more) start = s_runs[lane];
+    uint32_t rank = 0;
+    for (uint32_t j = 1; j <= more; ++j) rank += s_runs[j] < start ? 1u : 0u;
+    sync();
+    if (lane >= 1u && lane <= more) s_runs[1u + rank] = start;                  // (every wave the same)
+    sync();
+    if (lane >= 1u && lane <= more) at = s_runs[lane];
+    if (lane < more) end = s_runs[lane + 1u];
+    uint32_t put = first;
+    if (WAVES > 1) {
+        uint32_t top = lane <= more ? inst[end - 1u] : 0u;
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) { const uint32_t v = __shfl_xor(top, d, kWave); top = top > v ? top : v; }
+        const uint64_t values = (uint64_t)top + 1u, bounds[2] = { values * wave / WAVES, values * (wave + 1u) / WAVES };
+        uint32_t cut[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            uint32_t lo = at, hi = end;
+            while (lo < hi) {
+                const uint32_t mid = lo + (hi - lo) / 2u;
+                if ((uint64_t)inst[mid] < bounds[k]) lo = mid + 1u; else hi = mid;
+            }
+            cut[k] = lo;
+        }
+        uint32_t below = cut[0] - at;
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) below += __shfl_xor(below, d, kWave);
+        put += below;
+        at = cut[0]; end = cut[1];
+    }
+    uint32_t left = end - at;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) left += __shfl_xor(left, d, kWave);
+    const uint32_t stop = (uint32_t)__builtin_amdgcn_readfirstlane((int)(put + left));
+    put = (uint32_t)__builtin_amdgcn_readfirstlane((int)put);
+    while (put < stop) {
+        const uint32_t run = lane >> 3, k = lane & 7u;
+        const uint32_t from = __shfl(at, (int)run, kWave) + k, to = __shfl(end, (int)run, kWave);
+        const bool there = from < to;
+        const uint32_t v = there ? inst[from] : 0xffffffffu;
+        uint32_t limit = k == 7u && there ? v : 0xffffffffu;
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) { const uint32_t o = __shfl_xor(limit, d, kWave); limit = limit < o ? limit : o; }
+        const bool goes = there && v <= limit;
+        const uint64_t going = __ballot(goes);
+        uint32_t place = 0;
+        for (uint64_t m = going; m != 0; m &= m - 1) place += (uint32_t)__builtin_amdgcn_readlane((int)v, __builtin_ctzll(m)) < v ? 1u : 0u;
+        if (goes) spare[put + place] = v;
+        if (lane < (uint32_t)kDepthBins) at += (uint32_t)__popcll(going >> (8u * lane) & 0xffull);
+        put += (uint32_t)__popcll(going);
+    }
+    __threadfence_block();
+    return spare;
 }
 
 }  // namespace htgs

@@ -20,7 +20,7 @@ namespace htgs {
 template <int K>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 8 ? 5 : K <= 16 ? 4 : 3))) blend_hybrid_forward_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
-    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, const HybridRecords finish)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const HybridRecords finish)
 {
     __shared__ TileStageQ st;
     __shared__ QuadrantLists ql;
@@ -37,15 +37,28 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 8 
     hybrid_tail_init(tail);
     float cd[K], ca[K], ci[K];                 // ci: the index's bit pattern
     hybrid_core_init<K>(cd, ca, ci);
-    hybrid_walk<K, false, true, false, false, HTGS_PRIM_FLOATS_TRAIN / 4>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, tail);
-    if (!px.inside) return;
-    finish(prim, tile, px, cd, ca, ci, tail);
+    CoreTie tie;
+    tie.init();
+    hybrid_walk<K, false, true, true, false, HTGS_PRIM_FLOATS_TRAIN / 4>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, tail, &tie);
+    // (a list by index is settled: the insertion was the reference's)
+    const bool again = spare != nullptr && settle_exact_core<HTGS_MODE_HYBRID_BLEND, K, HTGS_PRIM_FLOATS_TRAIN / 4>(st, prim, lane, px, cd, ca, ci, tie, tail_swap(tail, cd[K - 1])) && px.inside;
+    const uint64_t again_lanes = __ballot(again);
+    if (px.inside && !again) finish(prim, tile, px, cd, ca, ci, tail);
+    if (again_lanes == 0) return;
+    const uint32_t lane_again = fresh_lane();
+    const TilePixel px_again = quadrant_tile_pixel(tile, grid_w, lane_again, width, height);
+    const uint32_t *const list = list_in_index_order<1>(inst, first, last, spare, ql.a[0], 0u, lane_again);
+    hybrid_tail_init(tail);
+    hybrid_core_init<K>(cd, ca, ci);
+    hybrid_walk<K, false, true, false, true, HTGS_PRIM_FLOATS_TRAIN / 4>(st, ql, list, prim, first, last, lane_again, px_again.pt, px_again.cx, px_again.cy, cd, ca, ci, tail,
+                                                                        nullptr, again_lanes);
+    if ((again_lanes >> lane_again & 1ull) != 0) finish(prim, tile, px_again, cd, ca, ci, tail);
 }
 
 template <int K>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 8 ? 5 : K <= 16 ? 4 : 2))) blend_first_k_forward_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
-    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, const FirstKRecords finish)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const FirstKRecords finish)
 {
     __shared__ TileStageQ st;
     __shared__ QuadrantLists ql;
@@ -61,9 +74,20 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 8 
     float ca[K], cd[K];
     uint32_t ci[K];
     first_k_core_init<K>(cd, ca, ci);
-    first_k_walk<K, false, true, false, HTGS_PRIM_FLOATS_TRAIN / 4>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci);
-    if (!px.inside) return;
-    finish(prim, tile, px, cd, ca, ci);
+    CoreTie tie;
+    tie.init();
+    first_k_walk<K, false, true, true, HTGS_PRIM_FLOATS_TRAIN / 4>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie);
+    const bool again = spare != nullptr && settle_exact_core<HTGS_MODE_ALPHA_BLEND_FIRST_K, K, HTGS_PRIM_FLOATS_TRAIN / 4>(st, prim, lane, px, cd, ca, ci, tie, [](float, float) {}) && px.inside;
+    const uint64_t again_lanes = __ballot(again);
+    if (px.inside && !again) finish(prim, tile, px, cd, ca, ci);
+    if (again_lanes == 0) return;
+    const uint32_t lane_again = fresh_lane();
+    const TilePixel px_again = quadrant_tile_pixel(tile, grid_w, lane_again, width, height);
+    const uint32_t *const list = list_in_index_order<1>(inst, first, last, spare, ql.a[0], 0u, lane_again);
+    first_k_core_init<K>(cd, ca, ci);
+    first_k_walk<K, false, true, false, HTGS_PRIM_FLOATS_TRAIN / 4, true>(st, ql, list, prim, first, last, lane_again, px_again.pt, px_again.cx, px_again.cy, cd, ca, ci,
+                                                                         nullptr, again_lanes);
+    if ((again_lanes >> lane_again & 1ull) != 0) finish(prim, tile, px_again, cd, ca, ci);
 }
 
 __global__ void __launch_bounds__(64) blend_oit_forward_kernel(
@@ -145,7 +169,7 @@ static void launch_hybrid_forward(const htgs_frame *f, int sel, uint32_t grid_w,
     constexpr int REC4 = HTGS_PRIM_FLOATS_TRAIN / 4;
     const HybridRecords finish = { f->image, f->core_idx, (float4 *)f->core_info, f->tail_info, (uint32_t)f->width, (uint32_t)f->height, (size_t)n_tiles * 64u };
     hipLaunchKernelGGL((blend_hybrid_forward_kernel<K>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim,
-                       (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, list_threshold(f), forward_part_floor(f, sel), f->tile_order, finish);
+                       (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, list_threshold(f), forward_part_floor(f, sel), f->tile_order, binned_spare(f, sel), finish);
     launch_hybrid_long<K, false, REC4>(f, sel, grid_w, finish);
 }
 template <int K>
@@ -154,7 +178,7 @@ static void launch_first_k_forward(const htgs_frame *f, int sel, uint32_t grid_w
     constexpr int REC4 = HTGS_PRIM_FLOATS_TRAIN / 4;
     const FirstKRecords finish = { f->image, f->core_idx, (float4 *)f->core_info, (uint32_t)f->width, (uint32_t)f->height, (size_t)n_tiles * 64u };
     hipLaunchKernelGGL((blend_first_k_forward_kernel<K>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim,
-                       (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, list_threshold(f), forward_part_floor(f, sel), f->tile_order, finish);
+                       (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, list_threshold(f), forward_part_floor(f, sel), f->tile_order, binned_spare(f, sel), finish);
     launch_first_k_long<K, false, REC4>(f, sel, grid_w, finish);
 }
 static void launch_oit_forward(const htgs_frame *f, int sel, uint32_t grid_w, uint32_t n_tiles)
@@ -179,7 +203,7 @@ extern "C" int htgs_blend_forward(const htgs_frame *f, int selector)
     if (f->prim_floats != HTGS_PRIM_FLOATS_TRAIN) return fail(HTGS_ERR_ARGUMENT, "htgs_blend_forward: the training kernels read records of HTGS_PRIM_FLOATS_TRAIN floats (prim_floats)");
     const bool needs_core = f->mode == HTGS_MODE_HYBRID_BLEND || f->mode == HTGS_MODE_ALPHA_BLEND_FIRST_K;
     const bool needs_tail = f->mode == HTGS_MODE_HYBRID_BLEND || f->mode == HTGS_MODE_OIT_BLEND;
-    if (!f->ranges || !f->image || (f->n_instances > 0 && (!f->vals[selector] || !f->prim)) ||
+    if (!f->ranges || !f->image || (f->n_instances > 0 && (!f->vals[selector] || !f->prim || (frame_depth_binned(f) && !f->vals[selector ^ 1]))) ||
         (needs_core && (!f->core_idx || !f->core_info)) || (needs_tail && !f->tail_info))
         return fail(HTGS_ERR_ARGUMENT, "htgs_blend_forward: null pointer");
     const int tile = tile_size(f->mode);

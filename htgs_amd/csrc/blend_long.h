@@ -56,9 +56,8 @@ __device__ __forceinline__ void hybrid_core_init(float (&cd)[K], float (&ca)[K],
 // when it is evaluated, and the share of the fragments that end up in the core is taken out again at the end, so an
 // entry pushed out of the core needs no colour: its alpha and depth, which the tail also needs, are in the slot.
 // SOLO: the wave is the whole workgroup (its barriers are the workgroup's).
-// TIES (the walks of blend_hybrid_long_kernel): `tie` receives the least depth at which an entry was pushed out of the core
-// that is exactly as deep as the entry that is now last.  (A candidate as deep as the last slot of a share's own core
-// needs no note: at least K fragments of the share are not farther and came earlier, so it is in nobody's final core.)
+// TIES: `tie` receives what stayed out of the core, or left it, exactly as deep as the entry that is last then.  (A candidate as
+// deep as the last entry counts: another wave's share, or a list in bins of depth, may hold one that came before it by index.)
 // PIXELS: only the pixels of the lanes in pixel_lanes are wanted; instances that do not reach one of them are left out
 // (the other lanes' cores and tails come out incomplete).
 // QUICK: insertion by shifting (core_quick_walk), for a caller that settles every pixel at which depths coincide afterwards, also
@@ -67,7 +66,7 @@ __device__ __forceinline__ void hybrid_core_init(float (&cd)[K], float (&ca)[K],
 template <int K, bool FAST, bool SOLO, bool TIES = false, bool PIXELS = false, int REC4 = HTGS_PRIM_FLOATS / 4, bool QUICK = false>
 __device__ __forceinline__ void hybrid_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                             uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy, float (&cd)[K],
-                                            float (&ca)[K], float (&ci)[K], HybridTail &tail, float *tie = nullptr, uint64_t pixel_lanes = 0)
+                                            float (&ca)[K], float (&ci)[K], HybridTail &tail, CoreTie *tie = nullptr, uint64_t pixel_lanes = 0, uint32_t step = 64u)
 {
     constexpr int MODE = HTGS_MODE_HYBRID_BLEND;
     constexpr int N = kStageSlots;
@@ -86,14 +85,14 @@ __device__ __forceinline__ void hybrid_walk(TileStageQ &st, QuadrantLists &ql, c
         tail.c0 = __builtin_fmaf(p3, col.x, tail.c0);
         tail.c1 = __builtin_fmaf(p3, col.y, tail.c1);
         tail.c2 = __builtin_fmaf(p3, col.z, tail.c2);
-        if (depth < cd[K - 1] && f.alpha >= kMinAlphaCore) {
+        if ((TIES ? depth <= cd[K - 1] : depth < cd[K - 1]) && f.alpha >= kMinAlphaCore) {
             float pi = col.w;
             if constexpr ((FAST && !TIES) || QUICK) core_quick_walk<K>(depth, p3, pi, cd, ca, ci);
             else core_exchange_walk<K>(depth, p3, pi, cd, ca, ci);
-            if (TIES && p3 > 0.0f && depth == cd[K - 1]) *tie = depth < *tie ? depth : *tie;
+            if (TIES && p3 > 0.0f && depth == cd[K - 1]) tie->note(depth, float_to_bits(pi));
         }
         hybrid_tail_add<FAST>(tail, depth, p3);
-    }, pixel_lanes);
+    }, pixel_lanes, 1.0f, step);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -133,6 +132,24 @@ __device__ __forceinline__ CoreKey make_key(float depth, uint32_t low) { return 
 __device__ __forceinline__ uint32_t key_fraction(float alpha, const KeyFormat &f) { return (uint32_t)__builtin_fmaf(alpha, f.one, 0.5f); }      // alpha in [0, 1]
 __device__ __forceinline__ uint32_t key_pack(float alpha, uint32_t place, const KeyFormat &f) { return key_fraction(alpha, f) << f.shift | place; }
 __device__ __forceinline__ float key_alpha(uint32_t low, const KeyFormat &f) { return (float)(low >> f.shift) * f.one_rcp; }
+// What a walk of keys notes of equal depths at the end of a pixel's core (CoreTie), in one register: the fragment's place in the list,
+// the low bits of the depth, whether there is a note, and whether it was not the only one as deep.
+constexpr uint32_t kTieNoted = 1u << 30, kTieMore = 1u << 31, kTieDepthBits = 17, kTieShift = 13;
+static_assert(kPackedListMost <= 1u << kTieShift && kTieShift + kTieDepthBits == 30, "place, depth, two flags");
+__device__ __forceinline__ uint32_t tie_depth(float depth) { return (float_to_bits(depth) & ((1u << kTieDepthBits) - 1u)) << kTieShift | kTieNoted; }
+__device__ __forceinline__ bool tie_is_at(uint32_t tie, float depth) { return ((tie ^ tie_depth(depth)) & ~kTieMore) >> kTieShift == 0u; }
+__device__ __forceinline__ void tie_note(uint32_t &tie, float depth, uint32_t low, const KeyFormat &f)
+{
+    asm volatile("");                  // (branched over by a wave without one, which is nearly every time: not eight instructions for no lane)
+    const bool met = tie_is_at(tie, depth);
+    tie = tie_depth(depth) | (low & f.place_mask) | (met ? kTieMore : 0u);
+}
+// another wave's note of the same pixel; what neither the core's last depth nor its low bits match is of no use any more
+__device__ __forceinline__ void tie_join(uint32_t &tie, uint32_t other, float last_depth)
+{
+    if (!tie_is_at(other, last_depth)) return;
+    tie = tie_is_at(tie, last_depth) ? tie | kTieMore : other;
+}
 __device__ __forceinline__ void key_step(CoreKey &carried, CoreKey &slot)
 {
     CoreKey out;
@@ -150,14 +167,12 @@ __device__ __forceinline__ void core_key_walk(CoreKey &carried, CoreKey (&core)[
         for (int i = g0; i < g1; ++i) key_step(carried, core[i]);
     }
 }
-// FAST or not is the arithmetic of a fragment alone.  Without FAST, `tie` receives the least depth at which the keys may not
-// have kept what the reference's insertion keeps: an entry left the core that is exactly as deep as the entry that is now
-// last (which of the two stays is the insertion's choice; it matters if the finished core still reaches that deep.  Two
-// such entries that both stay are seen in the finished core, key_core_tied).
+// FAST or not is the arithmetic of a fragment alone.  Without FAST, `tie` receives what stayed out of the core, or left it, exactly as
+// deep as the entry that is last then (tie_note).
 template <int K, bool FAST, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, bool AHEAD = false>
 __device__ __forceinline__ void hybrid_key_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                 uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy,
-                                                CoreKey (&core)[K], HybridTail &tail, float &tie, const KeyFormat &fmt, uint32_t list_first)
+                                                CoreKey (&core)[K], HybridTail &tail, uint32_t &tie, const KeyFormat &fmt, uint32_t list_first, uint32_t step = 64u)
 {
     constexpr int MODE = HTGS_MODE_HYBRID_BLEND;
     constexpr int N = kStageSlots;
@@ -165,7 +180,7 @@ __device__ __forceinline__ void hybrid_key_walk(TileStageQ &st, QuadrantLists &q
     // a fragment that passes the tests joins the pixel
     const auto joins = [&](const TileFrag &f, float depth, const float4 &col) {
         float p3 = f.alpha, leaving = p3;
-        if (depth < key_depth(core[K - 1]) && p3 >= kMinAlphaCore) {
+        if ((FAST ? depth < key_depth(core[K - 1]) : depth <= key_depth(core[K - 1])) && p3 >= kMinAlphaCore) {
             // (a fragment that enters the core has the alpha that its key holds from here on: what the colour sums
             // receive now is what is taken out of them again for the entries of the finished core)
             // (the fast path's alpha is opacity * 2^t with the opacity held to 1 and t <= 0 up to the rounding of the staged
@@ -177,8 +192,8 @@ __device__ __forceinline__ void hybrid_key_walk(TileStageQ &st, QuadrantLists &q
             core_key_walk<K>(carried, core);
             depth = key_depth(carried);
             leaving = key_alpha(key_low(carried), fmt);
-            // (the core's last depth never grows, so the latest of these depths is the least; an empty slot's is the largest float)
-            if constexpr (!FAST) tie = depth == key_depth(core[K - 1]) ? depth : tie;
+            if constexpr (!FAST)
+                if (depth == key_depth(core[K - 1]) && leaving > 0.0f) tie_note(tie, depth, key_low(carried), fmt);
         }
         tail.c0 = __builtin_fmaf(p3, col.x, tail.c0);
         tail.c1 = __builtin_fmaf(p3, col.y, tail.c1);
@@ -198,24 +213,15 @@ __device__ __forceinline__ void hybrid_key_walk(TileStageQ &st, QuadrantLists &q
             const float4 col1 = stage_row<N, 5>(one), col2 = stage_row<N, 5>(two);
             if (pass1) joins(f1, depth1, col1);
             if (pass2) joins(f2, depth2, col2);
-        });
+        }, 0, 1.0f, step);
     } else {
         tile_list_walk<MODE, true, kCullAlpha, SOLO, REC4, FAST, true, AHEAD>(st, ql, prim, inst, first, last, lane, cx, cy, [&](uint32_t addr) {
             TileFrag f;
             const bool fragment = FAST ? tile_frag_fast<MODE, N>(addr, pt, f) : tile_frag_exact<MODE, N>(addr, pt, f);
             const float4 col = stage_row<N, 5>(addr);
             if (fragment) joins(f, tile_frag_depth<N>(addr, pt, f), col);
-        });
+        }, 0, 1.0f, step);
     }
-}
-// two entries of the finished core are exactly as deep as each other (their order is the reference's insertion's to choose)
-template <int K>
-__device__ __forceinline__ bool key_core_tied(const CoreKey (&core)[K], const KeyFormat &fmt)
-{
-    bool tied = false;
-#pragma unroll
-    for (int i = 0; i + 1 < K; ++i) tied = tied || (key_low(core[i + 1]) >> fmt.shift != 0u && __double2hiint(core[i]) == __double2hiint(core[i + 1]));
-    return tied;
 }
 // the finished keys as the three arrays the composite takes
 template <int K>
@@ -229,6 +235,34 @@ __device__ __forceinline__ void key_core_unpack(const CoreKey (&core)[K], const 
         ca[i] = key_alpha(low, fmt);
         ci[i] = ca[i] > 0.0f && first + place < last ? bits_to_float(inst[first + place]) : 0.0f;
     }
+}
+
+// settle_core of a core of keys that is unpacked; inside: px.inside, in the kernels that store
+template <int MODE, int K, int REC4, typename IndexT, typename Swapped>
+__device__ __forceinline__ bool settle_key_core(TileStageQ &st, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst, uint32_t first, uint32_t last, uint32_t lane,
+                                                const TilePixel &px, float (&cd)[K], float (&ca)[K], IndexT (&ci)[K], uint32_t tie, const KeyFormat &fmt, Swapped &&swapped)
+{
+    const uint32_t place = first + (tie & ((1u << kTieShift) - 1u));
+    const bool noted = px.inside && tie_is_at(tie, cd[K - 1]) && place < last;
+    return settle_core<MODE, K, REC4>(st, prim, lane, px.pt, px.cx, px.cy, cd, ca, ci, noted, noted ? inst[place] : 0u, (tie & kTieMore) != 0u,
+                                      [&](float alpha) { return (float)key_fraction(alpha, fmt) * fmt.one_rcp; }, swapped);
+}
+// a fragment of the tail's takes the place of another one of the same depth
+__device__ __forceinline__ auto tail_swap(HybridTail &t, float depth)
+{
+    return [&t, depth](float in, float out) {
+        t.alpha += in - out;
+        t.depth = __builtin_fmaf(depth, in - out, t.depth);
+        t.T *= (1.0f - in) / (1.0f - out);
+    };
+}
+// settle_core of the walks by insertion
+template <int MODE, int K, int REC4, typename IndexT, typename Swapped>
+__device__ __forceinline__ bool settle_exact_core(TileStageQ &st, const float4 *__restrict__ prim, uint32_t lane, const TilePixel &px, float (&cd)[K], float (&ca)[K],
+                                                  IndexT (&ci)[K], const CoreTie &tie, Swapped &&swapped)
+{
+    return settle_core<MODE, K, REC4>(st, prim, lane, px.pt, px.cx, px.cy, cd, ca, ci, px.inside && tie.at_end(cd[K - 1]), tie.other & ~kMoreTied,
+                                      (tie.other & kMoreTied) != 0u, [](float alpha) { return alpha; }, swapped);
 }
 
 // core + tail -> pixel (R/include/hybrid_blend/kernels/inference.cuh:172-213)
@@ -298,7 +332,7 @@ struct HybridImage {
 template <int K, bool FAST, int REC4, typename Finish>
 __device__ __forceinline__ void hybrid_tile_by_keys(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                     uint32_t tile, uint32_t first, uint32_t last, uint32_t lane, const TilePixel &px, uint32_t grid_w,
-                                                    uint32_t width, uint32_t height, const Finish &finish)
+                                                    uint32_t width, uint32_t height, uint32_t *__restrict__ spare, const Finish &finish)
 {
     HybridTail tail;
     hybrid_tail_init(tail);
@@ -309,7 +343,7 @@ __device__ __forceinline__ void hybrid_tile_by_keys(TileStageQ &st, QuadrantList
         core[i] = make_key(__FLT_MAX__, 0u);
         asm volatile("" : "+v"(core[i]));      // one register pair per slot, never a wide tuple
     }
-    float tie = __FLT_MAX__;
+    uint32_t tie = 0u;
     const KeyFormat fmt = key_format(last > first ? last - first : 1u);
     hybrid_key_walk<K, FAST, true, REC4, true>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, core, tail, tie, fmt, first);
     if constexpr (FAST) {
@@ -317,9 +351,9 @@ __device__ __forceinline__ void hybrid_tile_by_keys(TileStageQ &st, QuadrantList
         key_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
         finish(prim, tile, px, cd, ca, ci, tail);
     } else {
-        const bool again = px.inside && ((tie < __FLT_MAX__ && tie <= key_depth(core[K - 1])) || key_core_tied<K>(core, fmt));
-        const uint64_t again_lanes = __ballot(again);
         key_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
+        const bool again = settle_key_core<HTGS_MODE_HYBRID_BLEND, K, REC4>(st, prim, inst, first, last, lane, px, cd, ca, ci, tie, fmt, tail_swap(tail, cd[K - 1])) && px.inside;
+        const uint64_t again_lanes = __ballot(again);
         if (px.inside && !again) finish(prim, tile, px, cd, ca, ci, tail);
         if (again_lanes == 0) return;
         // (the lane and its pixel are worked out afresh, so that nothing the first walk keeps in registers has to
@@ -327,9 +361,10 @@ __device__ __forceinline__ void hybrid_tile_by_keys(TileStageQ &st, QuadrantList
         uint32_t lane_again = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
         asm volatile("" : "+v"(lane_again));
         const TilePixel px_again = quadrant_tile_pixel(tile, grid_w, lane_again, width, height);
+        const uint32_t *const list = spare != nullptr ? list_in_index_order<1>(inst, first, last, spare, ql.a[0], 0u, lane_again) : inst;
         hybrid_tail_init(tail);
         hybrid_core_init<K>(cd, ca, ci);
-        hybrid_walk<K, false, true, false, true, REC4>(st, ql, inst, prim, first, last, lane_again, px_again.pt, px_again.cx, px_again.cy, cd, ca, ci, tail, nullptr,
+        hybrid_walk<K, false, true, false, true, REC4>(st, ql, list, prim, first, last, lane_again, px_again.pt, px_again.cx, px_again.cy, cd, ca, ci, tail, nullptr,
                                                        again_lanes);
         if ((again_lanes >> lane_again & 1ull) != 0) finish(prim, tile, px_again, cd, ca, ci, tail);
     }
@@ -374,20 +409,28 @@ __device__ __forceinline__ void sort_bitonic(CoreKey (&core)[K])
 }
 // A core of keys joins the running one; pushed(key) is called with every entry that is in neither's K nearest.  tie: see above.
 template <int K, bool TIES, typename Pushed>
-__device__ __forceinline__ void merge_key_cores(const float *from, CoreKey (&core)[K], float &tie, const KeyFormat &fmt, Pushed &&pushed)
+__device__ __forceinline__ void merge_key_cores(const float *from, CoreKey (&core)[K], uint32_t &tie, const KeyFormat &fmt, Pushed &&pushed)
 {
     float least = __FLT_MAX__;
+    uint32_t least_low = 0u;
+    uint32_t several = 0u;
 #pragma unroll
     for (int i = 0; i < K; ++i) {
         const CoreKey other = __hiloint2double((int)float_to_bits(from[(2 * (K - 1 - i)) * 64]), (int)float_to_bits(from[(2 * (K - 1 - i) + 1) * 64]));
         CoreKey lo, hi;
         asm("v_min_f64 %0, %2, %3\n\tv_max_f64 %1, %2, %3" : "=&v"(lo), "=&v"(hi) : "v"(core[i]), "v"(other));
         core[i] = lo;
-        if (TIES) least = key_low(hi) >> fmt.shift != 0u && key_depth(hi) < least ? key_depth(hi) : least;
+        if (TIES) {                            // (the least of them, without a branch for each)
+            const bool nearer = key_low(hi) >> fmt.shift != 0u && key_depth(hi) <= least;
+            several = nearer ? (key_depth(hi) == least ? kTieMore : 0u) : several;
+            least_low = nearer ? key_low(hi) : least_low;
+            least = nearer ? key_depth(hi) : least;
+            asm volatile("" : "+v"(least), "+v"(least_low), "+v"(several));      // (as in merge_cores)
+        }
         pushed(hi);
     }
     sort_bitonic<K>(core);
-    if (TIES) tie = least == key_depth(core[K - 1]) && least < tie ? least : tie;
+    if (TIES && least == key_depth(core[K - 1])) tie_join(tie, tie_depth(least) | (least_low & fmt.place_mask) | several, least);
 }
 // the same for cores of three registers a slot (an empty slot has alpha 0 and the largest depth)
 template <typename IndexT>
@@ -400,9 +443,10 @@ __device__ __forceinline__ void order_entries(float &d0, float &a0, IndexT &i0, 
     d0 = d; a0 = a; i0 = x;
 }
 template <int K, bool TIES, typename IndexT, typename Pushed>
-__device__ __forceinline__ void merge_cores(const float *from, float (&cd)[K], float (&ca)[K], IndexT (&ci)[K], float &tie, Pushed &&pushed)
+__device__ __forceinline__ void merge_cores(const float *from, float (&cd)[K], float (&ca)[K], IndexT (&ci)[K], CoreTie &tie, Pushed &&pushed)
 {
-    float least = __FLT_MAX__;
+    CoreTie left;
+    left.init();
 #pragma unroll
     for (int i = 0; i < K; ++i) {
         float d = from[(3 * (K - 1 - i)) * 64], a = from[(3 * (K - 1 - i) + 1) * 64];
@@ -410,7 +454,14 @@ __device__ __forceinline__ void merge_cores(const float *from, float (&cd)[K], f
         const float bits = from[(3 * (K - 1 - i) + 2) * 64];
         __builtin_memcpy(&x, &bits, 4);
         order_entries(cd[i], ca[i], ci[i], d, a, x);
-        if (TIES) least = a > 0.0f && d < least ? d : least;
+        if (TIES) {                            // (the least of them, without a branch for each)
+            uint32_t index;
+            __builtin_memcpy(&index, &x, 4);
+            const bool least = a > 0.0f && d <= left.depth;
+            left.other = least ? index | (d == left.depth ? kMoreTied : 0u) : left.other;
+            left.depth = least ? d : left.depth;
+            asm volatile("" : "+v"(left.other), "+v"(left.depth));      // (now, not for all entries at the end: that took a hundred scalar registers)
+        }
         pushed(d, a);
         asm volatile("" : "+v"(cd[i]), "+v"(ca[i]), "+v"(ci[i]));
     }
@@ -420,7 +471,7 @@ __device__ __forceinline__ void merge_cores(const float *from, float (&cd)[K], f
         for (int i = 0; i < K; ++i)
             if ((i & half) == 0) order_entries(cd[i], ca[i], ci[i], cd[i + half], ca[i + half], ci[i + half]);
     }
-    if (TIES) tie = least == cd[K - 1] && least < tie ? least : tie;
+    if (TIES && left.depth == cd[K - 1]) tie.join(left);
 }
 template <int K, typename IndexT>
 __device__ __forceinline__ void give_core(float *to, const float (&cd)[K], const float (&ca)[K], const IndexT (&ci)[K])
@@ -442,19 +493,20 @@ __device__ __forceinline__ void give_key_core(float *to, const CoreKey (&core)[K
     }
 }
 template <int ROW>
-__device__ __forceinline__ void give_tail(float *to, const HybridTail &t, float tie)
+__device__ __forceinline__ void give_tail(float *to, const HybridTail &t)
 {
     to[ROW * 64] = t.T; to[(ROW + 1) * 64] = t.c0; to[(ROW + 2) * 64] = t.c1; to[(ROW + 3) * 64] = t.c2; to[(ROW + 4) * 64] = t.alpha; to[(ROW + 5) * 64] = t.depth;
-    to[(ROW + 6) * 64] = tie;
 }
 template <int ROW>
-__device__ __forceinline__ void take_tail(const float *from, HybridTail &t, float &tie)
+__device__ __forceinline__ void take_tail(const float *from, HybridTail &t)
 {
     t.T *= from[ROW * 64];
     t.c0 += from[(ROW + 1) * 64]; t.c1 += from[(ROW + 2) * 64]; t.c2 += from[(ROW + 3) * 64]; t.alpha += from[(ROW + 4) * 64]; t.depth += from[(ROW + 5) * 64];
-    const float other = from[(ROW + 6) * 64];
-    tie = other < tie ? other : tie;
 }
+template <int ROW>
+__device__ __forceinline__ void give_tie(float *to, const CoreTie &tie) { to[ROW * 64] = tie.depth; to[(ROW + 1) * 64] = bits_to_float(tie.other); }
+template <int ROW>
+__device__ __forceinline__ void take_tie(const float *from, CoreTie &tie) { tie.join(CoreTie{ from[ROW * 64], float_to_bits(from[(ROW + 1) * 64]) }); }
 // ---------------------------------------------------------------------------------------------
 // Tiles with very long lists (HYBRID_BLEND, ALPHA_BLEND_FIRST_K and OIT_BLEND, which walk all of a list): the kernel
 // with one wave per tile puts a tile whose list is longer than long_threshold on a list instead of walking it, if the
@@ -463,7 +515,7 @@ __device__ __forceinline__ void take_tail(const float *from, HybridTail &t, floa
 // launch for 70 ms.
 // long_tiles[0] = entries on the list, [1..3] = work counters, [4] = workgroups done, all zeroed with the
 // ranges and again by the last workgroup of the second launch; [5] = the threshold, if it was chosen on the device
-// (ListThreshold); [6], [7] = tiles with pixels settled by a second look / walked again in one piece (upper half: of these,
+// (ListThreshold); [6], [7] = tiles with pixels settled from their cores or by a second look / walked again in one piece (upper half: of these,
 // after a second look that ran out of room) since the ranges were made (for the tests); then 2 n_tiles words for the entries (tile | part << 20 |
 // (parts - 1) << 25: a tile is on the list once per part, and the parts beyond the first of all tiles together are held
 // to n_tiles, so the list cannot overflow) and n_tiles words that count a tile's finished parts.
@@ -481,8 +533,8 @@ inline void with_long_waves(const htgs_frame *f, Launch &&launch)
 }
 constexpr unsigned long_grid(int waves) { return 256u * (unsigned)(kLongWavesHeld / waves); }
 
-// What a workgroup leaves of its part of a list, in 64-lane rows: HYBRID's core, tail and the depth of a tie.
-template <int K> constexpr uint32_t long_part_words() { return (3u * K + 7u) * 64u; }
+// What a workgroup leaves of its part of a list, in 64-lane rows: HYBRID's core, tail and what met at its end.
+template <int K> constexpr uint32_t long_part_words() { return (3u * K + 8u) * 64u; }
 // The parts a list of this length is walked in by separate workgroups (1: by one).  A part is at least part_least
 // long (least_part), long enough that what the parts leave behind (part_words each) fits into the list's own stretch of
 // the spare value buffer, and at least as long as the frame's average list (part_floor = instances / tiles, rounded
@@ -595,7 +647,7 @@ template <int K, bool FAST, bool KEYS = false>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 5 : KEYS ? 4 : 3))) blend_hybrid_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
     float *__restrict__ image, float *__restrict__ depths, uint32_t width, uint32_t height, uint32_t grid_w, int chw, int median,
-    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare)
 {
     __shared__ TileStageQ st;
     __shared__ QuadrantLists ql;
@@ -609,7 +661,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
     }
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
     if constexpr (KEYS) {
-        hybrid_tile_by_keys<K, FAST, HTGS_PRIM_FLOATS / 4>(st, ql, inst, prim, tile, first, last, lane, px, grid_w, width, height,
+        hybrid_tile_by_keys<K, FAST, HTGS_PRIM_FLOATS / 4>(st, ql, inst, prim, tile, first, last, lane, px, grid_w, width, height, spare,
                                                            HybridImage{ image, depths, width, height, chw, median });
     } else {
         HybridTail tail;
@@ -634,8 +686,43 @@ __device__ __forceinline__ float wave_product(float v)
     for (int o = 32; o > 0; o >>= 1) v *= __shfl_xor(v, o);
     return v;
 }
+// (out of line: the kernels for long lists have no scalar registers left for it)
+template <int WAVES>
+__device__ __attribute__((noinline)) const uint32_t *list_in_index_order_by(const uint32_t *inst, uint32_t first, uint32_t last, uint32_t *spare, uint32_t *s_runs, uint32_t wave,
+                                                                            uint32_t lane)
+{
+    return list_in_index_order<WAVES>(inst, first, last, spare, s_runs, wave, lane);
+}
 constexpr int kAgainPixels = 2;       // pixels a pass of pixels_again takes at once
 constexpr int kAgainMost = 8;         // pixels of a tile beyond which they are walked again in one piece instead
+constexpr uint32_t kAgainEntries = 1024;        // entries of pixels_again, of all waves, beyond which so are they
+// The entries of pixels_again by Gaussian index, or as they are listed (one wave): returns their offsets in `entries`, listed[w] of them
+// from from(w) on, in LDS.
+template <int WAVES, bool BY_INDEX, typename From>
+__device__ __forceinline__ const uint32_t *entries_in_order(const uint32_t *entries, const uint32_t *listed, uint32_t *lds, uint32_t lane, uint32_t &total, From &&from)
+{
+    uint32_t *const index = lds, *const at = lds + kAgainEntries, *const ordered = lds + 2u * kAgainEntries;
+    total = 0;
+#pragma nounroll
+    for (uint32_t w = 0; w < (uint32_t)WAVES; ++w) {
+        const uint32_t n = listed[w], start = from(w);
+        for (uint32_t e = lane; e < n; e += 64u) {
+            at[total + e] = start + 4u * e;
+            index[total + e] = entries[start + 4u * e + 3u];
+        }
+        total += n;
+    }
+    wave_lds_sync();
+    if (!BY_INDEX) return at;
+    for (uint32_t e = lane; e < total; e += 64u) {
+        const uint32_t mine = index[e];
+        uint32_t rank = 0;
+        for (uint32_t j = 0; j < total; ++j) rank += index[j] < mine || (index[j] == mine && j < e) ? 1u : 0u;
+        ordered[rank] = at[e];
+    }
+    wave_lds_sync();
+    return ordered;
+}
 
 // The second look at the pixels of pixel_lanes, whose cores the merge could not settle: lanes = instances.  Every wave
 // goes through its share [first, last) of the tile's list once per kAgainPixels pixels and evaluates each instance at these
@@ -718,20 +805,22 @@ __device__ __forceinline__ uint32_t pixels_again(TileStage<64> &st, const uint32
     return fits ? n_out : ~0u;
 }
 
-// A core, a tail and a tie depth (3K + 7 rows of 64 lanes at from[]) join the running ones: they cover the stretch of the
+// A core, a tail and a tie (3K + 8 rows of 64 lanes at from[]) join the running ones: they cover the stretch of the
 // list that follows.
 template <int K, bool FAST>
 __device__ __forceinline__ void hybrid_merge(const float *from, uint32_t lane, float (&cd)[K], float (&ca)[K], float (&ci)[K], HybridTail &tail,
-                                             float &tie)
+                                             CoreTie &tie)
 {
+    take_tie<3 * K + 6>(from + lane, tie);
     merge_cores<K, !FAST>(from + lane, cd, ca, ci, tie, [&](float depth, float alpha) { hybrid_tail_add<FAST>(tail, depth, alpha); });
-    take_tail<3 * K>(from + lane, tail, tie);
+    take_tail<3 * K>(from + lane, tail);
 }
 template <int K>
-__device__ __forceinline__ void hybrid_put(float *to, uint32_t lane, const float (&cd)[K], const float (&ca)[K], const float (&ci)[K], const HybridTail &tail, float tie)
+__device__ __forceinline__ void hybrid_put(float *to, uint32_t lane, const float (&cd)[K], const float (&ca)[K], const float (&ci)[K], const HybridTail &tail, const CoreTie &tie)
 {
     give_core<K>(to + lane, cd, ca, ci);
-    give_tail<3 * K>(to + lane, tail, tie);
+    give_tail<3 * K>(to + lane, tail);
+    give_tie<3 * K + 6>(to + lane, tie);
 }
 // The waves' shares, merged pairwise into the first wave's: put(buffer) by the wave that hands its share on, merge(buffer) by
 // the one that takes it (all threads of the workgroup call this).
@@ -761,11 +850,12 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ shortlist, ListThreshold threshold, const Finish finish)
 {
     constexpr int kWaves = WAVES;
-    constexpr uint32_t kRows = 3 * K + 7;             // a wave's core, tail and least depth of a tie
+    constexpr uint32_t kRows = 3 * K + 8;             // a wave's core, tail and tie
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<kWaves, kRows>()];
     __shared__ uint32_t s_next;
     __shared__ uint32_t s_redo[2];                    // the pixels (lanes) to walk again
     __shared__ uint32_t s_short[kWaves];          // how many instances of each share reach one of them
+    __shared__ uint32_t s_runs[1 + kDepthBins];
     __shared__ uint32_t s_whole;                      // this workgroup finished the last part of its tile
     __shared__ float s_last_depth[64];                // depth of the merged core's last entry
     __shared__ float s_sums[kWaves][kAgainPixels][6], s_tails[64][6];   // tails of the pixels looked at again: per wave, whole
@@ -790,8 +880,10 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         hybrid_tail_init(tail);
         float cd[K], ca[K], ci[K];
         hybrid_core_init<K>(cd, ca, ci);
-        float tie = __FLT_MAX__;                        // least depth at which two fragments of equal depth met at the end of a core
-        hybrid_walk<K, FAST, false, kTies, false, REC4, true>(wave_stage(lds, wave), wave_lists<kWaves>(lds, wave), inst, prim, seg_first, seg_last, lane, px.pt, px.cx, px.cy, cd, ca, ci, tail, &tie);
+        CoreTie tie;                                    // fragments of equal depth at the end of a core
+        tie.init();
+        hybrid_walk<K, FAST, false, kTies, false, REC4, true>(wave_stage(lds, wave), wave_lists<kWaves>(lds, wave), inst, prim, first + 64u * wave, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, tail, &tie,
+                                                              0, 64u * kWaves);
         merge_all_shares<kWaves, kRows>(lds, wave, [&](float *to) { hybrid_put<K>(to, lane, cd, ca, ci, tail, tie); },
                                         [&](const float *from) { hybrid_merge<K, FAST>(from, lane, cd, ca, ci, tail, tie); });
         if (parts > 1u) {
@@ -808,7 +900,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
                 __threadfence();
                 hybrid_tail_init(tail);
                 hybrid_core_init<K>(cd, ca, ci);
-                tie = __FLT_MAX__;
+                tie.init();
                 for (uint32_t other = 0; other < parts; ++other)
                     hybrid_merge<K, FAST>(left + (size_t)other * long_part_words<K>(), lane, cd, ca, ci, tail, tie);
             }
@@ -820,16 +912,19 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
             // Equal depths matter where they can change the final core: a tie no deeper than its last entry (both
             // fragments of a deeper tie end in the tail either way), or two equal depths next to each other in it.
             // There the merged walk and the single walk can keep different fragments, or keep them in another order: the
-            // reference's insertion lets a displaced entry hop over a stored one of exactly equal depth.  Such pixels (a
-            // handful per frame of very long lists) are walked again in one piece by the first wave, over the instances
-            // that reach one of them; every wave picks those out of its share first (into the tile's own stretch of the
-            // shortlist, in list order), since the walk of one wave alone is bound by the latency of staging.
+            // reference's insertion lets a displaced entry hop over a stored one of exactly equal depth.  Where no more than two are
+            // as deep as each other, what that insertion leaves follows from the core alone (settle_core; the second look cost up to 800 of the
+            // 3400 us of this kernel with 6 M Gaussians of the stress scene at 1600x1066).  The other pixels are looked at again by all
+            // waves, or walked again in one piece by the first one, over the instances that reach one of them; every wave picks those out of
+            // its share first (into the tile's own stretch of the shortlist), since the walk of one wave alone is bound by the
+            // latency of staging.
             bool redo = false;
             if (wave == 0) {
-                // (nothing was pushed out of a core that is not full: no tie there)
-                redo = tie < __FLT_MAX__ && tie <= cd[K - 1];
-#pragma unroll
-                for (int i = 0; i + 1 < K; ++i) redo = redo || (ca[i + 1] > 0.0f && cd[i] == cd[i + 1]);
+                const bool met = core_tied<K>(cd, ca, tie);
+                if (__any(met)) {
+                    redo = settle_exact_core<HTGS_MODE_HYBRID_BLEND, K, REC4>(wave_stage(lds, 0), prim, lane, px, cd, ca, ci, tie, tail_swap(tail, cd[K - 1])) && px.inside;
+                    if (lane == 0 && !__any(redo)) atomicAdd(const_cast<uint32_t *>(long_tiles) + 6, 1u);
+                }
                 const uint64_t lanes = __ballot(redo);
                 if (lane == 0) { s_redo[0] = (uint32_t)lanes; s_redo[1] = (uint32_t)(lanes >> 32); }
             }
@@ -873,23 +968,30 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
                     if (lane == 0) s_short[wave] = listed;
                     __syncthreads();
                     bool settled = true;
-                    for (int w = 0; w < kWaves; ++w) settled = settled && s_short[w] != ~0u;
+                    uint32_t entries = 0;
+#pragma nounroll
+                    for (int w = 0; w < kWaves; ++w) {
+                        settled = settled && s_short[w] != ~0u;
+                        entries += s_short[w];
+                    }
+                    settled = settled && entries <= kAgainEntries;
                     __syncthreads();                            // (s_short is written again below)
                     if (settled) {
                         if (wave == 0) {
-                            // The walk's insertion, on the fragments that decide the cores alone, in list order; every pixel's lane
+                            // The walk's insertion, on the fragments that decide the cores alone, by index; every pixel's lane
                             // takes its own.
                             hybrid_core_init<K>(cd, ca, ci);
                             tail.T = s_tails[lane][0]; tail.c0 = s_tails[lane][1]; tail.c1 = s_tails[lane][2]; tail.c2 = s_tails[lane][3];
                             tail.alpha = s_tails[lane][4]; tail.depth = s_tails[lane][5];
-                            for (uint32_t w = 0; w < (uint32_t)kWaves; ++w) {
-                                const uint32_t *entry = shortlist + first + 64u * (uint32_t)((uint64_t)n_batches * w / kWaves);
-                                for (uint32_t left = s_short[w]; left != 0; --left, entry += 4) {
-                                    float depth = bits_to_float(entry[1]), alpha = bits_to_float(entry[2]), index = bits_to_float(entry[3]);
-                                    if (lane == entry[0]) {
-                                        if (depth < cd[K - 1]) core_exchange_walk<K>(depth, alpha, index, cd, ca, ci);
-                                        hybrid_tail_add<false>(tail, depth, alpha);
-                                    }
+                            uint32_t total;
+                            const uint32_t *const ordered = entries_in_order<kWaves, true>(shortlist, s_short, reinterpret_cast<uint32_t *>(lds), lane, total,
+                                [&](uint32_t w) { return first + 64u * (uint32_t)((uint64_t)n_batches * w / kWaves); });
+                            for (uint32_t e = 0; e < total; ++e) {
+                                const uint32_t *const entry = shortlist + ordered[e];
+                                float depth = bits_to_float(entry[1]), alpha = bits_to_float(entry[2]), index = bits_to_float(entry[3]);
+                                if (lane == entry[0]) {
+                                    if (depth < cd[K - 1]) core_exchange_walk<K>(depth, alpha, index, cd, ca, ci);
+                                    hybrid_tail_add<false>(tail, depth, alpha);
                                 }
                             }
                             if (px.inside && redo) finish(prim, tile, px, cd, ca, ci, tail);
@@ -899,14 +1001,18 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
                     }
                 }
                 if (threadIdx.x == 0) atomicAdd(const_cast<uint32_t *>(long_tiles) + 7, others_done ? 0x10001u : 1u);
+                const uint32_t *const list = shortlist != nullptr ? list_in_index_order_by<kWaves>(inst, first, last, shortlist, s_runs, wave, lane) : inst;
+                __syncthreads();
                 if (shortlist != nullptr) {
                     uint32_t kept = 0;
+                    // (in place where the list by index is in the shortlist: a wave's picks never get ahead of what it has read)
                     for (uint32_t base = seg_first; base < seg_last; base += 64) {
                         const uint32_t fetch = base + lane;
-                        const bool reaches = tile_stage_load<HTGS_MODE_HYBRID_BLEND, 64, true, kCullPixels, true, REC4>(reinterpret_cast<TileStage<64> &>(wave_stage(lds, wave)), prim, inst, fetch, seg_last, lane,
-                                                                                                               px.cx, px.cy, redo_lanes) != 0;
+                        const uint32_t g = fetch < seg_last ? list[fetch] : 0u;
+                        const bool reaches = tile_stage_load<HTGS_MODE_HYBRID_BLEND, 64, true, kCullPixels, true, REC4, false, false, true>(reinterpret_cast<TileStage<64> &>(wave_stage(lds, wave)), prim, list, fetch, seg_last, lane,
+                                                                                                               px.cx, px.cy, redo_lanes, g) != 0;
                         const uint64_t keep = __ballot(reaches);
-                        if (reaches) shortlist[seg_first + kept + (uint32_t)__popcll(keep & ((1ull << lane) - 1ull))] = inst[fetch];
+                        if (reaches) shortlist[seg_first + kept + (uint32_t)__popcll(keep & ((1ull << lane) - 1ull))] = g;
                         kept += (uint32_t)__popcll(keep);
                     }
                     if (lane == 0) s_short[wave] = kept;
@@ -954,7 +1060,7 @@ __device__ __forceinline__ void first_k_core_init(float (&cd)[K], float (&ca)[K]
 template <int K, bool FAST, bool SOLO, bool TIES = false, int REC4 = HTGS_PRIM_FLOATS / 4, bool PIXELS = false>
 __device__ __forceinline__ void first_k_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                              uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy, float (&cd)[K],
-                                             float (&ca)[K], uint32_t (&ci)[K], float *tie = nullptr, uint64_t pixel_lanes = 0)
+                                             float (&ca)[K], uint32_t (&ci)[K], CoreTie *tie = nullptr, uint64_t pixel_lanes = 0, uint32_t step = 64u)
 {
     constexpr int MODE = HTGS_MODE_ALPHA_BLEND_FIRST_K;
     constexpr int N = kStageSlots;
@@ -963,20 +1069,20 @@ __device__ __forceinline__ void first_k_walk(TileStageQ &st, QuadrantLists &ql, 
         const bool in_reach = tile_frag_cutoff<N>(addr, pt, f);
         f.den_rcp = frag_rcp<FAST>(f.den);
         float depth = tile_frag_depth<N>(addr, pt, f);
-        if (!(in_reach && depth < cd[K - 1])) return;          // depth test before the exponential (:151)
+        if (!(in_reach && (TIES ? depth <= cd[K - 1] : depth < cd[K - 1]))) return;          // depth test before the exponential (:151)
         if (!tile_frag_alpha<MODE, FAST>(stage_opacity<N>(addr), f)) return;
         float alpha = f.alpha;
         uint32_t idx = stage_index<N>(addr);
         core_exchange_walk<K>(depth, alpha, idx, cd, ca, ci);
-        if (TIES && alpha > 0.0f && depth == cd[K - 1]) *tie = depth < *tie ? depth : *tie;
-    }, pixel_lanes);
+        if (TIES && alpha > 0.0f && depth == cd[K - 1]) tie->note(depth, idx);
+    }, pixel_lanes, 1.0f, step);
 }
 // The same walk with the core as sorted 64-bit keys (above HYBRID_BLEND's: depth | alpha as a fraction | place in the list),
 // exact arithmetic; `tie` as in hybrid_key_walk.
 template <int K, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4>
 __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                  uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy,
-                                                 CoreKey (&core)[K], float &tie, const KeyFormat &fmt, uint32_t list_first)
+                                                 CoreKey (&core)[K], uint32_t &tie, const KeyFormat &fmt, uint32_t list_first, uint32_t step = 64u)
 {
     constexpr int MODE = HTGS_MODE_ALPHA_BLEND_FIRST_K;
     constexpr int N = kStageSlots;
@@ -994,16 +1100,16 @@ __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &
             depth2 = tile_frag_depth<N>(two, pt, f2);
         }
         const auto joins = [&](uint32_t addr, TileFrag &f, bool in_reach, float depth) {
-            if (!(in_reach && depth < key_depth(core[K - 1]))) return;          // depth test before the exponential (:151)
+            if (!(in_reach && depth <= key_depth(core[K - 1]))) return;         // depth test before the exponential (:151)
             if (!tile_frag_alpha<MODE, false>(stage_opacity<N>(addr), f)) return;
             CoreKey carried = make_key(depth, key_pack(f.alpha, stage_index<N>(addr) - list_first, fmt));      // (the slot's last word is the place in the list)
             core_key_walk<K>(carried, core);
             depth = key_depth(carried);
-            tie = depth == key_depth(core[K - 1]) ? depth : tie;                // (as in hybrid_key_walk)
+            if (depth == key_depth(core[K - 1]) && depth < __FLT_MAX__) tie_note(tie, depth, key_low(carried), fmt);
         };
         joins(one, f1, reach1, depth1);
         joins(two, f2, reach2, depth2);
-    });
+    }, 0, 1.0f, step);
 }
 // the finished keys as the three arrays the composite takes (an empty slot has the index 0xffffffff)
 template <int K>
@@ -1053,8 +1159,8 @@ struct FirstKImage {
         first_k_composite<K>(prim, cd, ca, ci, image, depths, width, height, px.x, px.y, chw, median);
     }
 };
-// what a workgroup leaves of its part of a list: the core and the depth of a tie
-template <int K> constexpr uint32_t first_k_part_words() { return (3u * K + 1u) * 64u; }
+// what a workgroup leaves of its part of a list: the core and what met at its end
+template <int K> constexpr uint32_t first_k_part_words() { return (3u * K + 2u) * 64u; }
 // KEYS (exact arithmetic, with long_tiles and a threshold of no more than kPackedListMost): the core as sorted 64-bit keys;
 // the pixels at which fragments of exactly equal depth met where they decide the core are walked again afterwards, over the
 // instances that reach one of them, with the reference's insertion (as in hybrid_tile_by_keys).
@@ -1062,7 +1168,7 @@ template <int K, bool FAST, bool KEYS = false>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 5 : 2))) blend_first_k_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
     float *__restrict__ image, float *__restrict__ depths, uint32_t width, uint32_t height, uint32_t grid_w, int chw, int median,
-    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare)
 {
     static_assert(!(KEYS && FAST), "the keys of this mode are for the exact path");
     __shared__ TileStageQ st;
@@ -1085,20 +1191,21 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
             core[i] = make_key(__FLT_MAX__, 0u);
             asm volatile("" : "+v"(core[i]));      // one register pair per slot, never a wide tuple
         }
-        float tie = __FLT_MAX__;
+        uint32_t tie = 0u;
         const KeyFormat fmt = key_format(last > first ? last - first : 1u);
         first_k_key_walk<K, true>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, core, tie, fmt, first);
-        const bool again = px.inside && ((tie < __FLT_MAX__ && tie <= key_depth(core[K - 1])) || key_core_tied<K>(core, fmt));
-        const uint64_t again_lanes = __ballot(again);
         first_k_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
+        const bool again = settle_key_core<HTGS_MODE_ALPHA_BLEND_FIRST_K, K, HTGS_PRIM_FLOATS / 4>(st, prim, inst, first, last, lane, px, cd, ca, ci, tie, fmt, [](float, float) {}) && px.inside;
+        const uint64_t again_lanes = __ballot(again);
         if (px.inside && !again) first_k_composite<K>(prim, cd, ca, ci, image, depths, width, height, px.x, px.y, chw, median);
         if (again_lanes == 0) return;
         // (the lane and its pixel are worked out afresh: nothing of the first walk has to live through the composite for this)
         uint32_t lane_again = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
         asm volatile("" : "+v"(lane_again));
         const TilePixel px_again = quadrant_tile_pixel(tile, grid_w, lane_again, width, height);
+        const uint32_t *const list = spare != nullptr ? list_in_index_order<1>(inst, first, last, spare, ql.a[0], 0u, lane_again) : inst;
         first_k_core_init<K>(cd, ca, ci);
-        first_k_walk<K, false, true, false, HTGS_PRIM_FLOATS / 4, true>(st, ql, inst, prim, first, last, lane_again, px_again.pt, px_again.cx, px_again.cy, cd, ca, ci,
+        first_k_walk<K, false, true, false, HTGS_PRIM_FLOATS / 4, true>(st, ql, list, prim, first, last, lane_again, px_again.pt, px_again.cx, px_again.cy, cd, ca, ci,
                                                                          nullptr, again_lanes);
         if ((again_lanes >> lane_again & 1ull) != 0)
             first_k_composite<K>(prim, cd, ca, ci, image, depths, width, height, px_again.x, px_again.y, chw, median);
@@ -1110,20 +1217,19 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
     }
 }
 
-// A core and a tie depth (3K + 1 rows of 64 lanes at from[]) join the running ones: they cover the stretch of the list
+// A core and a tie (3K + 2 rows of 64 lanes at from[]) join the running ones: they cover the stretch of the list
 // that follows.
 template <int K>
-__device__ __forceinline__ void first_k_merge(const float *from, uint32_t lane, float (&cd)[K], float (&ca)[K], uint32_t (&ci)[K], float &tie)
+__device__ __forceinline__ void first_k_merge(const float *from, uint32_t lane, float (&cd)[K], float (&ca)[K], uint32_t (&ci)[K], CoreTie &tie)
 {
+    take_tie<3 * K>(from + lane, tie);
     merge_cores<K, true>(from + lane, cd, ca, ci, tie, [](float, float) {});
-    const float other = from[(3 * K) * 64 + lane];
-    tie = other < tie ? other : tie;
 }
 template <int K>
-__device__ __forceinline__ void first_k_put(float *to, uint32_t lane, const float (&cd)[K], const float (&ca)[K], const uint32_t (&ci)[K], float tie)
+__device__ __forceinline__ void first_k_put(float *to, uint32_t lane, const float (&cd)[K], const float (&ca)[K], const uint32_t (&ci)[K], const CoreTie &tie)
 {
     give_core<K>(to + lane, cd, ca, ci);
-    to[(3 * K) * 64 + lane] = tie;
+    give_tie<3 * K>(to + lane, tie);
 }
 
 // The tiles with very long lists, as in blend_hybrid_long_kernel: every wave of the workgroup walks a share of the list
@@ -1139,9 +1245,9 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ spare, ListThreshold threshold, const Finish finish)
 {
     constexpr int kWaves = WAVES;
-    constexpr uint32_t kRows = 3 * K + 1;
+    constexpr uint32_t kRows = 3 * K + 2;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<kWaves, kRows>()];
-    __shared__ uint32_t s_next, s_whole, s_redo[2], s_listed[kWaves];
+    __shared__ uint32_t s_next, s_whole, s_redo[2], s_listed[kWaves], s_runs[1 + kDepthBins];
     __shared__ float s_last_depth[64];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     if (long_tiles[0] == 0) return;                   // (the ordinary frame)
@@ -1161,8 +1267,10 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         float ca[K], cd[K];
         uint32_t ci[K];
         first_k_core_init<K>(cd, ca, ci);
-        float tie = __FLT_MAX__;
-        first_k_walk<K, FAST, false, kTies, REC4>(wave_stage(lds, wave), wave_lists<kWaves>(lds, wave), inst, prim, share_first, share_last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie);
+        CoreTie tie;
+        tie.init();
+        first_k_walk<K, FAST, false, kTies, REC4>(wave_stage(lds, wave), wave_lists<kWaves>(lds, wave), inst, prim, e.first + 64u * wave, e.last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie,
+                                                0, 64u * kWaves);
         merge_all_shares<kWaves, kRows>(lds, wave, [&](float *to) { first_k_put<K>(to, lane, cd, ca, ci, tie); },
                                         [&](const float *from) { first_k_merge<K>(from, lane, cd, ca, ci, tie); });
         if (e.parts > 1u) {
@@ -1175,7 +1283,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
             if (wave == 0) {
                 __threadfence();
                 first_k_core_init<K>(cd, ca, ci);
-                tie = __FLT_MAX__;
+                tie.init();
                 for (uint32_t other = 0; other < e.parts; ++other)
                     first_k_merge<K>(left + (size_t)other * first_k_part_words<K>(), lane, cd, ca, ci, tie);
             }
@@ -1185,9 +1293,13 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         if (kTies) {
             bool redo = false;
             if (wave == 0) {
-                redo = tie < __FLT_MAX__ && tie <= cd[K - 1];          // (as in blend_hybrid_long_kernel)
-#pragma unroll
-                for (int i = 0; i + 1 < K; ++i) redo = redo || (ca[i + 1] > 0.0f && cd[i] == cd[i + 1]);
+                redo = core_tied<K>(cd, ca, tie);                      // (as in blend_hybrid_long_kernel)
+                if constexpr (!FAST) {
+                    if (__any(redo)) {
+                        redo = settle_exact_core<HTGS_MODE_ALPHA_BLEND_FIRST_K, K, REC4>(wave_stage(lds, 0), prim, lane, px, cd, ca, ci, tie, [](float, float) {}) && px.inside;
+                        if (lane == 0 && !__any(redo)) atomicAdd(const_cast<uint32_t *>(long_tiles) + 6, 1u);
+                    }
+                }
                 const uint64_t lanes = __ballot(redo);
                 if (lane == 0) { s_redo[0] = (uint32_t)lanes; s_redo[1] = (uint32_t)(lanes >> 32); }
                 s_last_depth[lane] = cd[K - 1];
@@ -1205,24 +1317,37 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
                     if (lane == 0) s_listed[wave] = listed;
                     __syncthreads();
                     settled = true;
-                    for (int w = 0; w < kWaves; ++w) settled = settled && s_listed[w] != ~0u;
+                    uint32_t entries = 0;
+#pragma nounroll
+                    for (int w = 0; w < kWaves; ++w) {
+                        settled = settled && s_listed[w] != ~0u;
+                        entries += s_listed[w];
+                    }
+                    settled = settled && entries <= kAgainEntries;
                 }
                 if (threadIdx.x == 0) atomicAdd(const_cast<uint32_t *>(long_tiles) + (settled ? 6 : 7), settled || !looked ? 1u : 0x10001u);
+                const uint32_t *list = inst;
+                if (!FAST && !settled && spare != nullptr) {       // (the fast variant takes the list's own order)
+                    list = list_in_index_order_by<kWaves>(inst, e.tile_first, e.tile_last, spare, s_runs, wave, lane);
+                    __syncthreads();
+                }
                 if (wave == 0) {
                     first_k_core_init<K>(cd, ca, ci);
                     if (settled) {
-                        for (uint32_t w = 0; w < (uint32_t)kWaves; ++w) {
+                        uint32_t total;
+                        const uint32_t *const ordered = entries_in_order<kWaves, !FAST>(spare, s_listed, reinterpret_cast<uint32_t *>(lds), lane, total, [&](uint32_t w) {
                             uint32_t from, to;
                             long_wave_share(e.tile_first, e.tile_last, w, from, to, kWaves);
-                            const uint32_t *candidate = spare + from;
-                            for (uint32_t todo = s_listed[w]; todo != 0; --todo, candidate += 4) {
-                                float depth = bits_to_float(candidate[1]), alpha = bits_to_float(candidate[2]);
-                                uint32_t index = candidate[3];
-                                if (lane == candidate[0] && depth < cd[K - 1]) core_exchange_walk<K>(depth, alpha, index, cd, ca, ci);
-                            }
+                            return from;
+                        });
+                        for (uint32_t k = 0; k < total; ++k) {
+                            const uint32_t *const candidate = spare + ordered[k];
+                            float depth = bits_to_float(candidate[1]), alpha = bits_to_float(candidate[2]);
+                            uint32_t index = candidate[3];
+                            if (lane == candidate[0] && depth < cd[K - 1]) core_exchange_walk<K>(depth, alpha, index, cd, ca, ci);
                         }
                     } else {
-                        first_k_walk<K, FAST, false, false, REC4>(wave_stage(lds, 0), wave_lists<kWaves>(lds, 0), inst, prim, e.tile_first, e.tile_last, lane, px.pt, px.cx, px.cy, cd, ca, ci);
+                        first_k_walk<K, FAST, false, false, REC4>(wave_stage(lds, 0), wave_lists<kWaves>(lds, 0), list, prim, e.tile_first, e.tile_last, lane, px.pt, px.cx, px.cy, cd, ca, ci);
                     }
                     if (px.inside && redo) finish(prim, e.tile, px, cd, ca, ci);
                 }
@@ -1244,7 +1369,7 @@ struct OitSums {
 // DEPTH: the depth sum is wanted (the training pass has no use for it)
 template <bool FAST, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, bool DEPTH = !FAST>
 __device__ __forceinline__ void oit_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t first,
-                                         uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy, OitSums &sum)
+                                         uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy, OitSums &sum, uint32_t step = 64u)
 {
     constexpr int MODE = HTGS_MODE_OIT_BLEND;
     constexpr int N = kStageSlots;
@@ -1267,7 +1392,7 @@ __device__ __forceinline__ void oit_walk(TileStageQ &st, QuadrantLists &ql, cons
         };
         if (pass1) joins(f1, depth1, col1);
         if (pass2) joins(f2, depth2, col2);
-    });
+    }, 0, 1.0f, step);
 }
 __device__ __forceinline__ void oit_composite(const OitSums &sum, float *__restrict__ image, float *__restrict__ depths, uint32_t width, uint32_t height,
                                               uint32_t x, uint32_t y, int chw)
@@ -1336,10 +1461,8 @@ __global__ void __launch_bounds__(64 * WAVES) blend_oit_long_kernel(
     LongEntry entry;
     while (long_tile_take(long_tiles, ranges, long_threshold, threshold.counters, round, &s_next, entry)) {
         const TilePixel px = quadrant_tile_pixel(entry.tile, grid_w, lane, width, height);
-        uint32_t share_first, share_last;
-        long_wave_share(entry.first, entry.last, wave, share_first, share_last, WAVES);
         OitSums sum = { 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 1.0f };
-        oit_walk<FAST, false, REC4, DEPTH>(st[wave], ql[wave], inst, prim, share_first, share_last, lane, px.pt, px.cx, px.cy, sum);
+        oit_walk<FAST, false, REC4, DEPTH>(st[wave], ql[wave], inst, prim, entry.first + 64u * wave, entry.last, lane, px.pt, px.cx, px.cy, sum, 64u * WAVES);
         s_sums[wave][0][lane] = sum.a0; s_sums[wave][1][lane] = sum.a1; s_sums[wave][2][lane] = sum.a2; s_sums[wave][3][lane] = sum.a3;
         s_sums[wave][4][lane] = sum.alpha; s_sums[wave][5][lane] = sum.T;
         __syncthreads();

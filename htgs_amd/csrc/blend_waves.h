@@ -3,8 +3,8 @@
 // The kernels with one wave per tile are bound by the issue rate of their instructions as long as every SIMD has five waves
 // to choose from.  A grid of a few thousand tiles leaves it one or two, and then a launch lasts as long as its longest
 // list: one wave takes 0.25 us for a turn of the walk, whose instructions depend on one another, and most of the device is
-// idle beside it.  Here a workgroup of WAVES waves takes a tile: every wave walks a contiguous share of the list (whole
-// batches) into a core and a tail of its own, and the shares are merged pairwise through LDS, in list order.
+// idle beside it.  Here a workgroup of WAVES waves takes a tile: every wave walks a share of the list (every
+// WAVES-th batch) into a core and a tail of its own, and the shares are merged pairwise through LDS.
 // As in the kernels for very long lists, which entry of exactly equal depth stays is not the reference's choice then, so the
 // walks and the merges note the least depth at which that could matter, and such pixels are walked again in one piece by
 // the reference's insertion.  Sums come out in another order than in a single walk (rounding).
@@ -17,21 +17,13 @@
 
 namespace htgs {
 
-// The share of wave `wave` of a list: whole batches of 64, the same number for each wave as far as they go.  Empty shares
-// are the last ones.
+// The share of wave `wave` of a list: every WAVES-th batch of 64 from its own on.  (In a list in bins of depth the nearer Gaussians, which
+// reach more of a tile, come first: contiguous shares would leave the first wave with the most work.)  Waves without a batch are the last ones.
 struct TileShare {
-    uint32_t first, last, per;             // per: instances to a share
+    uint32_t first, per;                   // per: where the next wave's begins
 };
 template <int WAVES>
-__device__ __forceinline__ TileShare tile_share(uint32_t first, uint32_t last, uint32_t wave)
-{
-    TileShare s;
-    const uint32_t n_batches = (last - first + 63u) / 64u;
-    s.per = 64u * ((n_batches + WAVES - 1) / WAVES);
-    s.first = first + s.per * wave < last ? first + s.per * wave : last;
-    s.last = s.first + s.per < last ? s.first + s.per : last;
-    return s;
-}
+__device__ __forceinline__ TileShare tile_share(uint32_t first, uint32_t wave) { return TileShare{ first + 64u * wave, 64u }; }
 // The pairwise merging: give(buffer) is called by the wave that hands its share over, take(buffer) by the one that receives
 // it (all lanes; buffer: 64-lane rows, one buffer per pair of waves); false: the wave is done.  The buffers lie over the stages,
 // which nobody reads any more.
@@ -51,23 +43,6 @@ __device__ __forceinline__ bool merge_shares(unsigned char *lds, const TileShare
     }
     return wave == 0;
 }
-// two entries of the finished core are exactly as deep as each other, or one that left it is as deep as its last
-template <int K>
-__device__ __forceinline__ bool core_tied(const float (&cd)[K], const float (&ca)[K], float tie)
-{
-    bool tied = tie < __FLT_MAX__ && tie <= cd[K - 1];
-#pragma unroll
-    for (int i = 0; i + 1 < K; ++i) tied = tied || (ca[i + 1] > 0.0f && cd[i] == cd[i + 1]);
-    return tied;
-}
-// (the lane and its pixel worked out afresh, so that nothing has to live through the pixels' finish for a rare second walk)
-__device__ __forceinline__ uint32_t fresh_lane()
-{
-    uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-    asm volatile("" : "+v"(lane));
-    return lane;
-}
-
 // The tile a workgroup takes; false: its list is very long and goes to the kernels for those.
 __device__ __forceinline__ bool tile_of_waves(const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ long_tiles,
                                               const ListThreshold &threshold, const PartFloor &part_floor, uint32_t part_words, uint32_t &tile, uint32_t &first, uint32_t &last)
@@ -85,7 +60,7 @@ __device__ __forceinline__ bool tile_of_waves(const uint32_t *__restrict__ range
 template <int WAVES, int K, bool FAST, typename Finish>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 5 : 4))) blend_hybrid_waves_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
-    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, const Finish finish)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const Finish finish)
 {
     constexpr uint32_t kRows = 2 * K + 7;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<WAVES, kRows>()];
@@ -93,7 +68,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     uint32_t tile, first, last;
     if (!tile_of_waves(ranges, tile_order, long_tiles, threshold, part_floor, long_part_words<K>(), tile, first, last)) return;
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
-    const TileShare share = tile_share<WAVES>(first, last, wave);
+    const TileShare share = tile_share<WAVES>(first, wave);
     HybridTail tail;
     hybrid_tail_init(tail);
     CoreKey core[K];
@@ -102,16 +77,17 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         core[i] = make_key(__FLT_MAX__, 0u);
         asm volatile("" : "+v"(core[i]));
     }
-    float tie = __FLT_MAX__;
+    uint32_t tie = 0u;
     const KeyFormat fmt = key_format(last > first ? last - first : 1u);
     // (places count from the tile's first instance, as in the single walk)
-    hybrid_key_walk<K, FAST, false, HTGS_PRIM_FLOATS / 4, true>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, share.last, lane, px.pt, px.cx, px.cy,
-                                                                core, tail, tie, fmt, first);
+    hybrid_key_walk<K, FAST, false, HTGS_PRIM_FLOATS / 4, true>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy,
+                                                                core, tail, tie, fmt, first, 64u * WAVES);
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
-            [&](float *to) { give_key_core<K>(to + lane, core); give_tail<2 * K>(to + lane, tail, tie); },
+            [&](float *to) { give_key_core<K>(to + lane, core); give_tail<2 * K>(to + lane, tail); to[(2 * K + 6) * 64 + lane] = bits_to_float(tie); },
             [&](const float *from) {
                 merge_key_cores<K, !FAST>(from + lane, core, tie, fmt, [&](CoreKey out) { hybrid_tail_add<FAST>(tail, key_depth(out), key_alpha(key_low(out), fmt)); });
-                take_tail<2 * K>(from + lane, tail, tie);
+                take_tail<2 * K>(from + lane, tail);
+                tie_join(tie, float_to_bits(from[(2 * K + 6) * 64 + lane]), key_depth(core[K - 1]));
             })) return;
     float cd[K], ca[K], ci[K];
     if constexpr (FAST) {
@@ -119,17 +95,19 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         key_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
         finish(prim, tile, px, cd, ca, ci, tail);
     } else {
-        const bool again = px.inside && ((tie < __FLT_MAX__ && tie <= key_depth(core[K - 1])) || key_core_tied<K>(core, fmt));
-        const uint64_t again_lanes = __ballot(again);
         key_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
+        wave_lds_sync();
+        const bool again = settle_key_core<HTGS_MODE_HYBRID_BLEND, K, HTGS_PRIM_FLOATS / 4>(wave_stage(lds, 0), prim, inst, first, last, lane, px, cd, ca, ci, tie, fmt, tail_swap(tail, cd[K - 1])) && px.inside;
+        const uint64_t again_lanes = __ballot(again);
         if (px.inside && !again) finish(prim, tile, px, cd, ca, ci, tail);
         if (again_lanes == 0) return;
         const uint32_t lane_again = fresh_lane();
         const TilePixel px_again = quadrant_tile_pixel(tile, grid_w, lane_again, width, height);
+        const uint32_t *const list = spare != nullptr ? list_in_index_order<1>(inst, first, last, spare, wave_lists<WAVES>(lds, 0).a[0], 0u, lane_again) : inst;
         hybrid_tail_init(tail);
         hybrid_core_init<K>(cd, ca, ci);
         wave_lds_sync();
-        hybrid_walk<K, false, false, false, true>(wave_stage(lds, 0), wave_lists<WAVES>(lds, 0), inst, prim, first, last, lane_again, px_again.pt, px_again.cx, px_again.cy, cd, ca,
+        hybrid_walk<K, false, false, false, true>(wave_stage(lds, 0), wave_lists<WAVES>(lds, 0), list, prim, first, last, lane_again, px_again.pt, px_again.cx, px_again.cy, cd, ca,
                                                   ci, tail, nullptr, again_lanes);
         if ((again_lanes >> lane_again & 1ull) != 0) finish(prim, tile, px_again, cd, ca, ci, tail);
     }
@@ -138,39 +116,40 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
 template <int WAVES, int K, int REC4, typename Finish>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 4 : 3))) blend_hybrid_waves_exact_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
-    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, const Finish finish)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const Finish finish)
 {
-    constexpr uint32_t kRows = 3 * K + 7;
+    constexpr uint32_t kRows = 3 * K + 8;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<WAVES, kRows>()];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     uint32_t tile, first, last;
     if (!tile_of_waves(ranges, tile_order, long_tiles, threshold, part_floor, long_part_words<K>(), tile, first, last)) return;
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
-    const TileShare share = tile_share<WAVES>(first, last, wave);
+    const TileShare share = tile_share<WAVES>(first, wave);
     HybridTail tail;
     hybrid_tail_init(tail);
     float cd[K], ca[K], ci[K];
     hybrid_core_init<K>(cd, ca, ci);
-    float tie = __FLT_MAX__;
-    hybrid_walk<K, false, false, true, false, REC4>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, share.last, lane, px.pt, px.cx, px.cy, cd, ca, ci,
-                                                    tail, &tie);
+    CoreTie tie;
+    tie.init();
+    hybrid_walk<K, false, false, true, false, REC4>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci,
+                                                    tail, &tie, 0, 64u * WAVES);
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
-            [&](float *to) { give_core<K>(to + lane, cd, ca, ci); give_tail<3 * K>(to + lane, tail, tie); },
-            [&](const float *from) {
-                merge_cores<K, true>(from + lane, cd, ca, ci, tie, [&](float depth, float alpha) { hybrid_tail_add<false>(tail, depth, alpha); });
-                take_tail<3 * K>(from + lane, tail, tie);
-            })) return;
-    // (a list that one wave walked is settled: the insertion was the reference's)
-    const bool again = px.inside && first + share.per < last && core_tied<K>(cd, ca, tie);
+            [&](float *to) { hybrid_put<K>(to, lane, cd, ca, ci, tail, tie); },
+            [&](const float *from) { hybrid_merge<K, false>(from, lane, cd, ca, ci, tail, tie); })) return;
+    // (a list by index that one wave walked is settled: the insertion was the reference's)
+    wave_lds_sync();
+    const bool again = (first + share.per < last || spare != nullptr) &&
+                       settle_exact_core<HTGS_MODE_HYBRID_BLEND, K, REC4>(wave_stage(lds, 0), prim, lane, px, cd, ca, ci, tie, tail_swap(tail, cd[K - 1])) && px.inside;
     const uint64_t again_lanes = __ballot(again);
     if (px.inside && !again) finish(prim, tile, px, cd, ca, ci, tail);
     if (again_lanes == 0) return;
     const uint32_t lane_again = fresh_lane();
     const TilePixel px_again = quadrant_tile_pixel(tile, grid_w, lane_again, width, height);
+    const uint32_t *const list = spare != nullptr ? list_in_index_order<1>(inst, first, last, spare, wave_lists<WAVES>(lds, 0).a[0], 0u, lane_again) : inst;
     hybrid_tail_init(tail);
     hybrid_core_init<K>(cd, ca, ci);
     wave_lds_sync();
-    hybrid_walk<K, false, false, false, true, REC4>(wave_stage(lds, 0), wave_lists<WAVES>(lds, 0), inst, prim, first, last, lane_again, px_again.pt, px_again.cx, px_again.cy, cd, ca,
+    hybrid_walk<K, false, false, false, true, REC4>(wave_stage(lds, 0), wave_lists<WAVES>(lds, 0), list, prim, first, last, lane_again, px_again.pt, px_again.cx, px_again.cy, cd, ca,
                                                     ci, tail, nullptr, again_lanes);
     if ((again_lanes >> lane_again & 1ull) != 0) finish(prim, tile, px_again, cd, ca, ci, tail);
 }
@@ -178,7 +157,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
 template <int WAVES, int K, typename Finish>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 5 : 3))) blend_first_k_waves_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
-    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, const Finish finish)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const Finish finish)
 {
     constexpr uint32_t kRows = 2 * K + 1;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<WAVES, kRows>()];
@@ -186,35 +165,36 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     uint32_t tile, first, last;
     if (!tile_of_waves(ranges, tile_order, long_tiles, threshold, part_floor, first_k_part_words<K>(), tile, first, last)) return;
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
-    const TileShare share = tile_share<WAVES>(first, last, wave);
+    const TileShare share = tile_share<WAVES>(first, wave);
     CoreKey core[K];
 #pragma unroll
     for (int i = 0; i < K; ++i) {
         core[i] = make_key(__FLT_MAX__, 0u);
         asm volatile("" : "+v"(core[i]));
     }
-    float tie = __FLT_MAX__;
+    uint32_t tie = 0u;
     const KeyFormat fmt = key_format(last > first ? last - first : 1u);
-    first_k_key_walk<K, false>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, share.last, lane, px.pt, px.cx, px.cy, core, tie, fmt, first);
+    first_k_key_walk<K, false>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, core, tie, fmt, first, 64u * WAVES);
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
-            [&](float *to) { give_key_core<K>(to + lane, core); to[2 * K * 64 + lane] = tie; },
+            [&](float *to) { give_key_core<K>(to + lane, core); to[2 * K * 64 + lane] = bits_to_float(tie); },
             [&](const float *from) {
                 merge_key_cores<K, true>(from + lane, core, tie, fmt, [](CoreKey) {});
-                const float other = from[2 * K * 64 + lane];
-                tie = other < tie ? other : tie;
+                tie_join(tie, float_to_bits(from[2 * K * 64 + lane]), key_depth(core[K - 1]));
             })) return;
-    const bool again = px.inside && ((tie < __FLT_MAX__ && tie <= key_depth(core[K - 1])) || key_core_tied<K>(core, fmt));
-    const uint64_t again_lanes = __ballot(again);
     float cd[K], ca[K];
     uint32_t ci[K];
     first_k_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
+    wave_lds_sync();
+    const bool again = settle_key_core<HTGS_MODE_ALPHA_BLEND_FIRST_K, K, HTGS_PRIM_FLOATS / 4>(wave_stage(lds, 0), prim, inst, first, last, lane, px, cd, ca, ci, tie, fmt, [](float, float) {}) && px.inside;
+    const uint64_t again_lanes = __ballot(again);
     if (px.inside && !again) finish(prim, tile, px, cd, ca, ci);
     if (again_lanes == 0) return;
     const uint32_t lane_again = fresh_lane();
     const TilePixel px_again = quadrant_tile_pixel(tile, grid_w, lane_again, width, height);
+    const uint32_t *const list = spare != nullptr ? list_in_index_order<1>(inst, first, last, spare, wave_lists<WAVES>(lds, 0).a[0], 0u, lane_again) : inst;
     first_k_core_init<K>(cd, ca, ci);
     wave_lds_sync();
-    first_k_walk<K, false, false, false, HTGS_PRIM_FLOATS / 4, true>(wave_stage(lds, 0), wave_lists<WAVES>(lds, 0), inst, prim, first, last, lane_again, px_again.pt, px_again.cx,
+    first_k_walk<K, false, false, false, HTGS_PRIM_FLOATS / 4, true>(wave_stage(lds, 0), wave_lists<WAVES>(lds, 0), list, prim, first, last, lane_again, px_again.pt, px_again.cx,
                                                                      px_again.cy, cd, ca, ci, nullptr, again_lanes);
     if ((again_lanes >> lane_again & 1ull) != 0) finish(prim, tile, px_again, cd, ca, ci);
 }
@@ -222,36 +202,38 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
 template <int WAVES, int K, bool FAST, int REC4, typename Finish>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 4 : 3))) blend_first_k_waves_exact_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
-    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, const Finish finish)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const Finish finish)
 {
-    constexpr uint32_t kRows = 3 * K + 1;
+    constexpr uint32_t kRows = 3 * K + 2;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<WAVES, kRows>()];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     uint32_t tile, first, last;
     if (!tile_of_waves(ranges, tile_order, long_tiles, threshold, part_floor, first_k_part_words<K>(), tile, first, last)) return;
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
-    const TileShare share = tile_share<WAVES>(first, last, wave);
+    const TileShare share = tile_share<WAVES>(first, wave);
     float cd[K], ca[K];
     uint32_t ci[K];
     first_k_core_init<K>(cd, ca, ci);
-    float tie = __FLT_MAX__;
-    first_k_walk<K, FAST, false, true, REC4>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, share.last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie);
+    CoreTie tie;
+    tie.init();
+    first_k_walk<K, FAST, false, true, REC4>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie, 0, 64u * WAVES);
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
-            [&](float *to) { give_core<K>(to + lane, cd, ca, ci); to[3 * K * 64 + lane] = tie; },
-            [&](const float *from) {
-                merge_cores<K, true>(from + lane, cd, ca, ci, tie, [](float, float) {});
-                const float other = from[3 * K * 64 + lane];
-                tie = other < tie ? other : tie;
-            })) return;
-    const bool again = px.inside && first + share.per < last && core_tied<K>(cd, ca, tie);
+            [&](float *to) { first_k_put<K>(to, lane, cd, ca, ci, tie); },
+            [&](const float *from) { first_k_merge<K>(from, lane, cd, ca, ci, tie); })) return;
+    wave_lds_sync();
+    bool again;
+    if constexpr (FAST) again = px.inside && first + share.per < last && core_tied<K>(cd, ca, tie);       // (in the list's own order)
+    else again = (first + share.per < last || spare != nullptr) &&
+                 settle_exact_core<HTGS_MODE_ALPHA_BLEND_FIRST_K, K, REC4>(wave_stage(lds, 0), prim, lane, px, cd, ca, ci, tie, [](float, float) {}) && px.inside;
     const uint64_t again_lanes = __ballot(again);
     if (px.inside && !again) finish(prim, tile, px, cd, ca, ci);
     if (again_lanes == 0) return;
     const uint32_t lane_again = fresh_lane();
     const TilePixel px_again = quadrant_tile_pixel(tile, grid_w, lane_again, width, height);
+    const uint32_t *const list = !FAST && spare != nullptr ? list_in_index_order<1>(inst, first, last, spare, wave_lists<WAVES>(lds, 0).a[0], 0u, lane_again) : inst;
     first_k_core_init<K>(cd, ca, ci);
     wave_lds_sync();
-    first_k_walk<K, FAST, false, false, REC4, true>(wave_stage(lds, 0), wave_lists<WAVES>(lds, 0), inst, prim, first, last, lane_again, px_again.pt, px_again.cx, px_again.cy, cd, ca,
+    first_k_walk<K, FAST, false, false, REC4, true>(wave_stage(lds, 0), wave_lists<WAVES>(lds, 0), list, prim, first, last, lane_again, px_again.pt, px_again.cx, px_again.cy, cd, ca,
                                                     ci, nullptr, again_lanes);
     if ((again_lanes >> lane_again & 1ull) != 0) finish(prim, tile, px_again, cd, ca, ci);
 }
@@ -259,7 +241,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
 template <int WAVES, bool FAST, int REC4, typename Finish, bool DEPTH = !FAST>
 __global__ void __launch_bounds__(64 * WAVES) blend_oit_waves_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
-    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, const Finish finish)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const Finish finish)
 {
     constexpr uint32_t kRows = 6;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<WAVES, kRows>()];
@@ -267,9 +249,9 @@ __global__ void __launch_bounds__(64 * WAVES) blend_oit_waves_kernel(
     uint32_t tile, first, last;
     if (!tile_of_waves(ranges, tile_order, long_tiles, threshold, part_floor, kOitPartWords, tile, first, last)) return;
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
-    const TileShare share = tile_share<WAVES>(first, last, wave);
+    const TileShare share = tile_share<WAVES>(first, wave);
     OitSums sum = { 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 1.0f };
-    oit_walk<FAST, false, REC4, DEPTH>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, share.last, lane, px.pt, px.cx, px.cy, sum);
+    oit_walk<FAST, false, REC4, DEPTH>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, sum, 64u * WAVES);
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
             [&](float *to) {
                 to += lane;
@@ -293,7 +275,7 @@ static void launch_waves(const htgs_frame *f, int sel, uint32_t grid_w, uint32_t
     hipStream_t s = (hipStream_t)f->stream;
     const PartFloor floor = { instance_count(f), f->vals[sel ^ 1] != nullptr ? 1u : 0u };
     hipLaunchKernelGGL(main, dim3(n_tiles), dim3(64 * WAVES), 0, s, f->ranges, f->vals[sel], (const float4 *)f->prim, (uint32_t)f->width, (uint32_t)f->height, grid_w,
-                       f->long_tiles, list_threshold(f), floor, f->tile_order, finish);
+                       f->long_tiles, list_threshold(f), floor, f->tile_order, binned_spare(f, sel), finish);
 }
 // calls launch(std::integral_constant<int, K>{}) for the core size K that f asks for
 template <typename Launch>

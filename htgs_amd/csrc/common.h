@@ -107,6 +107,37 @@ inline DepthKeys depth_key_range(const htgs_frame *f)
     }
     return k;
 }
+// The Gaussians are put into bins of depth, and the instances made bin by bin (htgs_frame.depth_bins).  The parts of
+// depth_bins: the depths at which the bins after the first begin, the instances of each bin, a counter of the scan, the instances
+// of every bin in every block of kCountBlock Gaussians (bin by bin, `stride` words each; the scan makes them the ones before), the
+// bin of every Gaussian.
+constexpr int kDepthBins = 8;
+inline bool frame_depth_binned(const htgs_frame *f)
+{
+    return f->depth_bins != nullptr && f->touch != nullptr && !frame_depth_ordered(f) && (f->mode == HTGS_MODE_HYBRID_BLEND || f->mode == HTGS_MODE_ALPHA_BLEND_FIRST_K);
+}
+struct DepthBins {
+    float *limits;                         // [kDepthBins - 1]
+    unsigned long long *totals;            // [kDepthBins]
+    uint32_t *done, *sums;                 // [1], [kDepthBins][stride]
+    uint8_t *of;                           // [N]
+    uint32_t stride;
+};
+// where the blend stages put a tile's list by index when they need it so; nullptr: every list is
+inline uint32_t *binned_spare(const htgs_frame *f, int selector) { return frame_depth_binned(f) ? f->vals[selector ^ 1] : nullptr; }
+constexpr size_t kDepthBinsHeader = 32;    // words: limits from 0, totals from 8, done at 24
+inline uint32_t depth_bins_stride(int n) { return ((uint32_t)div_up(n > 0 ? n : 1, 256) + 3u) & ~3u; }
+inline DepthBins depth_bin_parts(const htgs_frame *f)
+{
+    DepthBins b;
+    b.stride = depth_bins_stride(f->n_primitives);
+    b.limits = reinterpret_cast<float *>(f->depth_bins);
+    b.totals = reinterpret_cast<unsigned long long *>(f->depth_bins + 8);
+    b.done = f->depth_bins + 24;
+    b.sums = f->depth_bins + kDepthBinsHeader;
+    b.of = reinterpret_cast<uint8_t *>(b.sums + (size_t)kDepthBins * b.stride);
+    return b;
+}
 // stable sort of n (32-bit key, value) pairs by the low end_bit key bits, digit_bits (8 or 9) a pass (radix_sort.hip);
 // the result is in keys / vals[*selector]
 int sort_u32_pairs(void *stream, uint32_t *const keys[2], uint32_t *const vals[2], uint32_t *sort_tmp, uint64_t n, int end_bit, int digit_bits,
@@ -271,6 +302,19 @@ bool blend_forward_waves(const htgs_frame *f, int selector, uint32_t grid_w, uin
 // (launch_scan), so that its rows and columns, each rounded up to a power of two, take 21 bits; unlike the corner's tile
 // number it comes apart without a division.
 __host__ __device__ __forceinline__ uint32_t column_bits(uint32_t grid_w) { return grid_w > 1u ? 32u - (uint32_t)__builtin_clz(grid_w - 1u) : 0u; }
+
+// Workgroups go round the eight XCDs of the device in launch order, and each XCD has an L2 of its own.  Blocks that are
+// neighbours in the input write neighbouring runs of every digit, a run being shorter than a cache line or two; handing
+// every XCD a contiguous eighth of the input lets those partial lines meet in one L2 before they are written back.
+constexpr uint32_t kXcds = 8;
+__device__ __forceinline__ uint32_t xcd_contiguous_block(uint32_t launched, uint32_t n_blocks)
+{
+    // (the launch may be larger than n_blocks asks for: its blocks beyond an XCD's share have nothing to do)
+    const uint32_t per_xcd = (n_blocks + kXcds - 1) / kXcds;
+    return launched / kXcds < per_xcd ? (launched % kXcds) * per_xcd + launched / kXcds : n_blocks;           // >= n_blocks: nothing to do
+}
+__device__ __forceinline__ uint32_t blocks_of(uint32_t n, uint32_t per_block) { return n / per_block + (n % per_block != 0u ? 1u : 0u); }
+inline uint32_t xcd_padded_grid(uint32_t n_blocks) { return (n_blocks + kXcds - 1) / kXcds * kXcds; }
 
 // host side error reporting (api.hip)
 int fail(int code, const char *fmt, ...);

@@ -33,7 +33,7 @@ template <int K, int MODE>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 5 : 2))) max_weights_tile_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
     uint32_t *__restrict__ max_weights, uint32_t width, uint32_t height, uint32_t grid_w, float weight_threshold, const uint32_t *__restrict__ tile_order,
-    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor)
+    uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, uint32_t *__restrict__ spare)
 {
     constexpr bool kCore = MODE != HTGS_MODE_OIT_BLEND;
     constexpr bool kTail = MODE != HTGS_MODE_ALPHA_BLEND_FIRST_K;
@@ -57,47 +57,73 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
     const PixelTerms pt = px.pt;
     const float cx = px.cx, cy = px.cy;
 
-    float alpha_sum = 0.0f, T_tail = 1.0f;
+    float alpha_sum, T_tail;
+    CoreTie tie;
+    tie.init();
     float ca[KS], cd[KS];
     uint32_t ci[KS];
-#pragma unroll
-    for (int i = 0; i < KS; ++i) {
-        ca[i] = 0.0f; cd[i] = __FLT_MAX__; ci[i] = 0xffffffffu;
-        asm volatile("" : "+v"(cd[i]), "+v"(ca[i]), "+v"(ci[i]));      // one register per slot
-    }
-
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
-    tile_list_walk<MODE, kCore, kCullAlpha, true>(st, ql, prim, inst, first, last, lane, cx, cy, [&](uint32_t addr) {
-        TileFrag f;
-        bool in_reach = tile_frag_cutoff<kStageSlots>(addr, pt, f);
-        f.den_rcp = rcp_exact(f.den);
-        float depth = 0.0f;
-        if (MODE == HTGS_MODE_ALPHA_BLEND_FIRST_K) {
-            depth = tile_frag_depth<kStageSlots>(addr, pt, f);
-            in_reach = in_reach && depth < cd[KS - 1];
-        }
-        if (!(tile_frag_alpha<MODE>(stage_opacity<kStageSlots>(addr), f) && in_reach)) return;
-        float alpha = f.alpha;
-        if (MODE == HTGS_MODE_HYBRID_BLEND) depth = tile_frag_depth<kStageSlots>(addr, pt, f);
-        if (kCore && (MODE == HTGS_MODE_ALPHA_BLEND_FIRST_K || (depth < cd[KS - 1] && alpha >= kMinAlphaCore))) {
-            uint32_t idx = stage_index<kStageSlots>(addr);
-            core_exchange_walk<KS>(depth, alpha, idx, cd, ca, ci);
-        }
-        if (kTail) { alpha_sum += alpha; T_tail *= 1.0f - alpha; }
-    });
-    float T_core = 1.0f;
-    if (kCore && inside) {
+    // the walk by the reference's insertion; AGAIN: over a list by index, for the pixels of pixel_lanes
+    const auto walk = [&](auto again, const uint32_t *list, uint64_t pixel_lanes) {
+        constexpr bool AGAIN = decltype(again)::value;
+        alpha_sum = 0.0f; T_tail = 1.0f;
 #pragma unroll
         for (int i = 0; i < KS; ++i) {
-            const float w = T_core * ca[i];
-            T_core *= 1.0f - ca[i];
-            if (T_core < kTransmittanceThreshold) T_core = 0.0f;
-            if (!(w < weight_threshold)) raise_max(max_weights, ci[i], w);
+            ca[i] = 0.0f; cd[i] = __FLT_MAX__; ci[i] = 0xffffffffu;
+            asm volatile("" : "+v"(cd[i]), "+v"(ca[i]), "+v"(ci[i]));      // one register per slot
+        }
+        tile_list_walk<MODE, kCore, AGAIN ? kCullPixels : kCullAlpha, true>(st, ql, prim, list, first, last, lane, cx, cy, [&](uint32_t addr) {
+            // (TIES of hybrid_walk and first_k_walk)
+            const auto enters = [&](float depth) { return AGAIN ? depth < cd[KS - 1] : depth <= cd[KS - 1]; };
+            TileFrag f;
+            bool in_reach = tile_frag_cutoff<kStageSlots>(addr, pt, f);
+            f.den_rcp = rcp_exact(f.den);
+            float depth = 0.0f;
+            if (MODE == HTGS_MODE_ALPHA_BLEND_FIRST_K) {
+                depth = tile_frag_depth<kStageSlots>(addr, pt, f);
+                in_reach = in_reach && enters(depth);
+            }
+            if (!(tile_frag_alpha<MODE>(stage_opacity<kStageSlots>(addr), f) && in_reach)) return;
+            float alpha = f.alpha;
+            if (MODE == HTGS_MODE_HYBRID_BLEND) depth = tile_frag_depth<kStageSlots>(addr, pt, f);
+            if (kCore && (MODE == HTGS_MODE_ALPHA_BLEND_FIRST_K || (enters(depth) && alpha >= kMinAlphaCore))) {
+                uint32_t idx = stage_index<kStageSlots>(addr);
+                core_exchange_walk<KS>(depth, alpha, idx, cd, ca, ci);
+                if (!AGAIN && alpha > 0.0f && depth == cd[KS - 1]) tie.note(depth, idx);
+            }
+            if (kTail) { alpha_sum += alpha; T_tail *= 1.0f - alpha; }
+        }, pixel_lanes);
+    };
+    // the core's weights; returns the weight of a tail fragment per unit of alpha
+    const auto weigh = [&]() {
+        float T_core = 1.0f;
+        if (kCore) {
+#pragma unroll
+            for (int i = 0; i < KS; ++i) {
+                const float w = T_core * ca[i];
+                T_core *= 1.0f - ca[i];
+                if (T_core < kTransmittanceThreshold) T_core = 0.0f;
+                if (!(w < weight_threshold)) raise_max(max_weights, ci[i], w);
+            }
+        }
+        return kTail && alpha_sum >= weight_threshold ? (T_core * (1.0f - T_tail)) * (1.0f / alpha_sum) : 0.0f;
+    };
+    walk(std::false_type{}, inst, 0);
+    float tail_weight = 0.0f;
+    bool again = false;
+    if constexpr (kCore)                       // (a list by index is settled)
+        again = spare != nullptr && settle_exact_core<MODE, KS, HTGS_PRIM_FLOATS / 4>(st, prim, lane, px, cd, ca, ci, tie, [&](float in, float out) {
+            if (kTail) { alpha_sum += in - out; T_tail *= (1.0f - in) / (1.0f - out); }
+        }) && inside;
+    if (inside && !again) tail_weight = weigh();
+    if constexpr (kCore) {
+        const uint64_t again_lanes = __ballot(again);
+        if (again_lanes != 0) {
+            walk(std::true_type{}, list_in_index_order<1>(inst, first, last, spare, ql.a[0], 0u, lane), again_lanes);
+            if (again) tail_weight = weigh();
         }
     }
     if (!kTail) return;
-    float tail_weight = 0.0f;
-    if (inside && alpha_sum >= weight_threshold) tail_weight = (T_core * (1.0f - T_tail)) * (1.0f / alpha_sum);
     const bool active = inside && tail_weight >= weight_threshold;
     if (!__any(active)) return;
     // second walk over the tile's list: alpha * tail weight for every fragment that passes the cut-off (no alpha
@@ -271,7 +297,7 @@ static void launch_tile(const htgs_frame *f, int sel, uint32_t *max_weights, flo
     const bool shared = shares_long_lists<MODE>(f);
     const uint32_t w = (uint32_t)f->width, h = (uint32_t)f->height;
     hipLaunchKernelGGL((max_weights_tile_kernel<K, MODE>), dim3(n_tiles), dim3(64), 0, s, f->ranges, f->vals[sel], (const float4 *)f->prim, max_weights, w, h, grid_w,
-                       thr, f->tile_order, shared ? f->long_tiles : nullptr, threshold, part_floor_of(f, sel, true));
+                       thr, f->tile_order, shared ? f->long_tiles : nullptr, threshold, part_floor_of(f, sel, true), binned_spare(f, sel));
     if (!shared || !may_have_long_lists(f)) return;
     constexpr int REC4 = HTGS_PRIM_FLOATS / 4;
     if constexpr (MODE == HTGS_MODE_HYBRID_BLEND)
@@ -327,7 +353,8 @@ extern "C" int htgs_max_weights_blend(const htgs_frame *f, int selector, float *
     if (selector < 0 || selector > 1 || f->width <= 0 || f->height <= 0) return fail(HTGS_ERR_ARGUMENT, "htgs_max_weights_blend: bad argument");
     if (frame_prim_floats(f) != HTGS_PRIM_FLOATS) return fail(HTGS_ERR_ARGUMENT, "htgs_max_weights_blend: reads records of HTGS_PRIM_FLOATS floats (prim_floats)");
     if (f->n_instances == 0 || f->n_primitives == 0) return HTGS_OK;
-    if (!f->ranges || !f->vals[selector] || !f->prim || !max_weights) return fail(HTGS_ERR_ARGUMENT, "htgs_max_weights_blend: null pointer");
+    if (!f->ranges || !f->vals[selector] || !f->prim || !max_weights || (frame_depth_binned(f) && !f->vals[selector ^ 1]))
+        return fail(HTGS_ERR_ARGUMENT, "htgs_max_weights_blend: null pointer");
     const int tile = tile_size(f->mode);
     const uint32_t grid_w = div_up(f->width, tile), grid_h = div_up(f->height, tile);
     const uint32_t n_tiles = grid_w * grid_h;

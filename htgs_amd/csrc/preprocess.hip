@@ -68,6 +68,64 @@ __device__ __forceinline__ uint32_t wave_sum_last(uint32_t v)
     return v;
 }
 
+// htgs_frame.depth_bins: the depths that part the Gaussians into bins of about as many each, from a sample of them (those
+// in front of the camera and roughly inside the image).  The sample's depths are counted in 2048 classes of the upper bits of
+// their float patterns; a limit is the end of the class that a bin's share of the sample is reached in.  One workgroup: 4 us,
+// most of them the launch and the wait for the sample.
+constexpr int kLimitThreads = 1024, kLimitSample = 2 * kLimitThreads, kLimitClasses = 2 * kLimitThreads;
+__global__ void __launch_bounds__(kLimitThreads) depth_limits_kernel(const float *__restrict__ positions, int n, const float *__restrict__ M, const float *__restrict__ VPM,
+                                                                    float near_plane, float far_plane, float half_w, float half_h, uint32_t base, int shift,
+                                                                    float *__restrict__ limits, uint32_t *__restrict__ done)
+{
+    __shared__ uint32_t s_class[kLimitClasses], s_wave[kLimitThreads / kWave];
+    const uint32_t t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+    s_class[t] = s_class[t + kLimitThreads] = 0u;
+    if (t < (uint32_t)kDepthBins - 1u) limits[t] = __FLT_MAX__;
+    if (t == 0) *done = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kLimitSample / kLimitThreads; ++k) {
+        const size_t i = (size_t)((uint64_t)(t + (uint32_t)k * kLimitThreads) * (uint64_t)n / kLimitSample);
+        const float p[3] = { positions[3 * i], positions[3 * i + 1], positions[3 * i + 2] };
+        const float z = dot3(M + 8, p[0], p[1], p[2]) + M[11];
+        const float x = dot3(VPM, p[0], p[1], p[2]) + VPM[3], y = dot3(VPM + 4, p[0], p[1], p[2]) + VPM[7], w = dot3(VPM + 12, p[0], p[1], p[2]) + VPM[15];
+        const bool seen = z > 0.0f && z >= near_plane && z <= far_plane && __builtin_fabsf(x - half_w * w) <= 1.25f * half_w * w &&
+                          __builtin_fabsf(y - half_h * w) <= 1.25f * half_h * w;
+        if (seen) {
+            const uint32_t c = (float_to_bits(z) - base) >> shift;
+            atomicAdd(&s_class[c < (uint32_t)kLimitClasses ? c : kLimitClasses - 1], 1u);
+        }
+    }
+    __syncthreads();
+    const uint32_t own[2] = { s_class[2 * t], s_class[2 * t + 1] };
+    uint32_t inc = own[0] + own[1];
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+        const uint32_t v = __shfl_up(inc, d, kWave);
+        if ((int)lane >= d) inc += v;
+    }
+    if (lane == kWave - 1) s_wave[wave] = inc;
+    __syncthreads();
+    uint32_t all = 0, before = inc - own[0] - own[1];
+#pragma unroll
+    for (uint32_t w = 0; w < kLimitThreads / kWave; ++w) {
+        before += w < wave ? s_wave[w] : 0u;
+        all += s_wave[w];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k) {
+#pragma unroll
+        for (uint32_t j = 1; j < (uint32_t)kDepthBins; ++j) {
+            const uint32_t share = (all * j + kDepthBins - 1u) / kDepthBins;
+            if (before < share && share <= before + own[k]) {
+                const uint32_t bits = base + ((2u * t + k + 1u) << shift);
+                limits[j - 1u] = bits < 0x7f7fffffu ? bits_to_float(bits) : __FLT_MAX__;
+            }
+        }
+        before += own[k];
+    }
+}
+
 // SH_REGS: 16-byte words of SH coefficients a thread holds while the bounds are computed (ceil(3 total_sh / 4): 12 for degree
 // 3, 16 for the most the kernel takes).  0: no bands beyond the constant one are active, and without those registers twice
 // as many waves fit.
@@ -81,7 +139,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SH_REG
     int n, uint32_t grid_w, uint32_t grid_h, float tile, float min_alpha_rcp,
     int active_sh, int total_sh, float near_plane, float far_plane, float scale_modifier, int rec4,
     uint32_t *__restrict__ depth_keys, uint32_t *__restrict__ depth_vals, uint32_t depth_base, uint32_t depth_culled, int depth_shift,
-    uint4 *__restrict__ touch, float rho_most, int cutoff_only, FrameStart start)
+    uint4 *__restrict__ touch, float rho_most, int cutoff_only, FrameStart start, DepthBins depth_bins)
 {
     // One LDS buffer, used twice: first the block's slice of sh_rest (contiguous in memory, loaded with coalesced
     // 16-byte reads and then read back per Gaussian at a stride of 3 * total_sh words), then the block's records
@@ -90,7 +148,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SH_REG
     extern __shared__ float4 lds4[];
     float *lds = reinterpret_cast<float *>(lds4);
     __shared__ uint8_t s_visible[256];
-    __shared__ uint32_t s_counts[256 / kWave];
+    __shared__ uint32_t s_counts[256 / kWave], s_binned[256 / kWave][kDepthBins];
     const int first = blockIdx.x * 256;
     const int i = first + threadIdx.x;
     const bool in_range = i < n;
@@ -228,6 +286,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SH_REG
         for (int k = 0; k < 5; ++k)
             for (uint32_t w = blockIdx.x * 256u + threadIdx.x; w < start.clear_words[k]; w += gridDim.x * 256u) start.clear[k][w] = 0u;
     }
+    // htgs_frame.depth_bins: the Gaussian's bin, and how many instances each bin gets from this block
+    if (depth_bins.of != nullptr) {
+        uint32_t bin = 0;
+#pragma unroll
+        for (int j = 0; j < kDepthBins - 1; ++j) bin += z >= depth_bins.limits[j] ? 1u : 0u;
+        if (in_range) depth_bins.of[i] = (uint8_t)bin;
+        uint32_t *const mine = s_binned[threadIdx.x / kWave];
+        if ((threadIdx.x & (kWave - 1)) < (uint32_t)kDepthBins) mine[threadIdx.x & (kWave - 1)] = 0u;
+        wave_lds_sync();
+        if (in_range && touched != 0u) atomicAdd(mine + bin, touched);
+    }
     // htgs_frame.depth_order: the pairs that sort the Gaussians by depth (depth_key_range() in common.h)
     if (depth_keys != nullptr && in_range) {
         // (a depth that is not a number passes the cull above, as in the reference, where its bit pattern sorts behind every
@@ -249,6 +318,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SH_REG
     for (int q = (words & ~3) + threadIdx.x; q < words; q += 256) lds[q] = sh_rest[base_word + q];
     __syncthreads();
     if (start.block_sums != nullptr && threadIdx.x == 0) start.block_sums[blockIdx.x] = (s_counts[0] + s_counts[1]) + (s_counts[2] + s_counts[3]);
+    if (depth_bins.of != nullptr && threadIdx.x < (uint32_t)kDepthBins)
+        depth_bins.sums[(size_t)threadIdx.x * depth_bins.stride + blockIdx.x] =
+            (s_binned[0][threadIdx.x] + s_binned[1][threadIdx.x]) + (s_binned[2][threadIdx.x] + s_binned[3][threadIdx.x]);
 
     // view-dependent colour, kernel_utils.cuh:152-187
     float res[3] = { 0.0f, 0.0f, 0.0f };
@@ -352,13 +424,31 @@ int preprocess_and_start(const htgs_frame *f, const FrameStart &start)
     const float cutoff_sq = f->mode == HTGS_MODE_ALPHA_BLEND_FIRST_K ? ModeCfg<HTGS_MODE_ALPHA_BLEND_FIRST_K>::cutoff_sq : ModeCfg<HTGS_MODE_HYBRID_BLEND>::cutoff_sq;
     const DepthOrder order = depth_order_parts(f);
     const DepthKeys order_keys = depth_key_range(f);
+    DepthBins bins = {};
+    if (frame_depth_binned(f)) {
+        if ((uintptr_t)f->depth_bins & 15) return fail(HTGS_ERR_ARGUMENT, "htgs_preprocess: depth_bins must be 16-byte aligned");
+        bins = depth_bin_parts(f);
+        // (the classes: the keys of depth_key_range with as many of the upper bits as there are classes for; without a positive
+        // near plane the patterns of all positive floats)
+        uint32_t base = 0u, range = 0x7f800000u;
+        if (f->near_plane > 0.0f && f->far_plane >= f->near_plane && f->far_plane < __builtin_huge_valf()) {
+            uint32_t hi;
+            __builtin_memcpy(&base, &f->near_plane, 4);
+            __builtin_memcpy(&hi, &f->far_plane, 4);
+            range = hi - base;
+        }
+        int shift = 0;
+        while ((range >> shift) >= (uint32_t)kLimitClasses) ++shift;
+        hipLaunchKernelGGL(depth_limits_kernel, dim3(1), dim3(kLimitThreads), 0, (hipStream_t)f->stream, f->positions, f->n_primitives, f->M, f->VPM, f->near_plane,
+                           f->far_plane, 0.5f * (float)f->width, 0.5f * (float)f->height, base, shift, bins.limits, bins.done);
+    }
     const auto kernel = f->active_sh_bases <= 1 ? preprocess_kernel<0> : f->total_sh_bases <= 15 ? preprocess_kernel<12> : preprocess_kernel<16>;
     hipLaunchKernelGGL(kernel, dim3(div_up(f->n_primitives, 256)), dim3(256), lds_bytes, (hipStream_t)f->stream,
                        f->positions, f->scales, f->rotations, f->opacities, f->sh_0, f->sh_rest, f->M, f->VPM, f->cam_position,
                        f->n_touched, f->bounds, f->prim, f->clamp_info, f->n_primitives, grid_w, grid_h, (float)tile,
                        min_alpha_rcp, f->active_sh_bases, f->total_sh_bases, f->near_plane, f->far_plane, f->scale_modifier, prim_floats / 4,
                        ordered ? order.keys[0] : nullptr, ordered ? order.vals[0] : nullptr, order_keys.base, order_keys.culled, order_keys.shift,
-                       (uint4 *)f->touch, cutoff_sq, f->touch_cutoff_only, start);
+                       (uint4 *)f->touch, cutoff_sq, f->touch_cutoff_only, start, bins);
     return check_launch("preprocess");
 }
 

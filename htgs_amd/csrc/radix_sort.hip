@@ -30,18 +30,6 @@ constexpr int kSortTileMin = 256 * kSortItems;              // sizes the histogr
 template <typename KeyT>
 __device__ __forceinline__ uint32_t digit_of(KeyT k, int shift, uint32_t mask) { return (uint32_t)(k >> shift) & mask; }
 
-// Workgroups go round the eight XCDs of the device in launch order, and each XCD has an L2 of its own.  Blocks that are
-// neighbours in the input write neighbouring runs of every digit, a run being shorter than a cache line or two; handing
-// every XCD a contiguous eighth of the input lets those partial lines meet in one L2 before they are written back.
-constexpr uint32_t kXcds = 8;
-__device__ __forceinline__ uint32_t xcd_contiguous_block(uint32_t launched, uint32_t n_blocks)
-{
-    // (the launch may be larger than n_blocks asks for: its blocks beyond an XCD's share have nothing to do)
-    const uint32_t per_xcd = (n_blocks + kXcds - 1) / kXcds;
-    return launched / kXcds < per_xcd ? (launched % kXcds) * per_xcd + launched / kXcds : n_blocks;           // >= n_blocks: nothing to do
-}
-__device__ __forceinline__ uint32_t blocks_of(uint32_t n, uint32_t per_block) { return n / per_block + (n % per_block != 0u ? 1u : 0u); }
-inline uint32_t xcd_padded_grid(uint32_t n_blocks) { return (n_blocks + kXcds - 1) / kXcds * kXcds; }
 
 template <typename KeyT, int THREADS = SortShape<KeyT>::threads, int BITS = SortDigit<KeyT>::bits, int ITEMS = kSortItems>
 __global__ void __launch_bounds__(THREADS) digit_histogram_kernel(const KeyT *__restrict__ keys, uint32_t *__restrict__ hist,

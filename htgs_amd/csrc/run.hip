@@ -114,6 +114,24 @@ static int waves_of(const htgs_frame *f, int what, uint64_t n_tiles)
     const uint64_t two = train ? (wide ? 8192 : 10240) : wide || f->fast_math ? 13312 : 15360;
     return n_tiles <= 6144 ? 4 : n_tiles <= two ? 2 : 1;
 }
+// From how many Gaussians on the instances are made in bins of depth.  The bins cost 10 us (the sample for their limits, a scan that cannot be
+// left to the duplication, shorter runs of its output) and spare most insertions into a core: the more, the larger the core and
+// the longer the lists.  Whole passes over clusters (and the stress scene, which gains from 100 k on), without / with bins, on both sides
+// of the lines:
+//   images, K = 16    80 k 0.90 to 0.97, 160 k 1.01 to 1.11, 320 k 1.06 to 1.23, 3 M 1.06 (HYBRID_BLEND) and 1.20 (FIRST_K), image alone
+//   images, K = 32    160 k 0.93 to 0.98, 320 k 1.03 to 1.04;   K = 8  400 k 0.93 to 1.0, 1 M 1.02 to 1.04 (1920x1080), 0.97 (640x480), 3 M 1.03 to 1.05
+//   training, K >= 8  80 k 0.98 to 1.02, 160 k 1.04 to 1.06, 1 M 1.04
+//   weights, K >= 8   20 k 0.96 to 0.99, 40 k 0.99 to 1.10, 80 k 1.11 to 1.23, 1 M 1.18
+//   K <= 4            0.92 (320 k) to 1.01 (3 M): never
+static bool takes_depth_bins(const htgs_frame *f, int what, uint64_t n_tiles)
+{
+    if (f->mode != HTGS_MODE_HYBRID_BLEND && f->mode != HTGS_MODE_ALPHA_BLEND_FIRST_K) return false;
+    const int K = htgs_effective_k(f->K);
+    if (K <= 4) return false;
+    if (what == HTGS_RUN_MAX_WEIGHTS) return f->n_primitives >= 60000;
+    if (what == HTGS_RUN_FORWARD) return f->n_primitives >= 120000;
+    return f->n_primitives >= (K == 16 ? 160000 : K == 32 ? 300000 : n_tiles >= 8192 ? 800000 : 2000000);
+}
 constexpr uint64_t kUnorderedTiles = 1280;      // workgroups of four waves
 static uint64_t carve_front(htgs_frame *f, int what, void *base)
 {
@@ -140,10 +158,10 @@ static uint64_t carve_front(htgs_frame *f, int what, void *base)
     f->long_list_threshold = -1;                           // (ListThreshold)
     // (a grid whose workgroups are all on the device at once is taken in any order)
     f->tile_order = n_tiles > kUnorderedTiles ? c.take<uint32_t>(htgs_tile_order_words(f->mode, f->width, f->height)) : nullptr;
-    // GLOBAL_ORDERING without a backward pass, and the image-only fast path of the two modes with a sorted core
-    const bool by_depth = !train && (f->mode == HTGS_MODE_ALPHA_BLEND_GLOBAL_ORDERING ||
-                                     (what == HTGS_RUN_RENDER && f->fast_math && f->mode != HTGS_MODE_OIT_BLEND));
+    // GLOBAL_ORDERING without a backward pass
+    const bool by_depth = !train && f->mode == HTGS_MODE_ALPHA_BLEND_GLOBAL_ORDERING;
     f->depth_order = by_depth ? c.take<uint32_t>(htgs_depth_order_words((int)n)) : nullptr;
+    f->depth_bins = takes_depth_bins(f, what, n_tiles) ? c.take<uint32_t>(htgs_depth_bins_words((int)n)) : nullptr;
     const bool has_core = f->mode == HTGS_MODE_HYBRID_BLEND || f->mode == HTGS_MODE_ALPHA_BLEND_FIRST_K;
     const bool has_tail = f->mode == HTGS_MODE_HYBRID_BLEND || f->mode == HTGS_MODE_OIT_BLEND;
     f->pixel_scratch = what == HTGS_RUN_MAX_WEIGHTS && has_tail ? c.take<float>(64 * n_tiles) : nullptr;

@@ -178,12 +178,14 @@ class FrameBuffers:
     def like(cls, frame: "_native.Frame", *args, **kwargs) -> "FrameBuffers":
         """The stages of a pass that ``_run_pass`` has filled ``frame`` in for: the same lists, order, waves and thresholds."""
         return cls(*args, tight_lists=True, waves_per_tile=frame.waves_per_tile, long_list_threshold=frame.long_list_threshold,
-                   order_tiles=bool(frame.tile_order), long_counters=True, **kwargs)
+                   order_tiles=bool(frame.tile_order), long_counters=True, order_gaussians=bool(frame.depth_order),
+                   depth_bins=bool(frame.depth_bins), **kwargs)
 
     def __init__(self, positions, scales, rotations, opacities, sh_0, sh_rest, settings: RasterizerSettings,
                  to_chw: bool = True, use_median_depth: bool = False, train: bool = False,
                  pool: Optional[ScratchPool] = None, fast: bool = False, long_list_threshold: int = 0, order_tiles: bool = True,
-                 order_gaussians: bool = True, tight_lists: bool = False, waves_per_tile: int = 1, long_counters: bool = False):
+                 order_gaussians: bool = True, tight_lists: bool = False, waves_per_tile: int = 1, long_counters: bool = False,
+                 depth_bins: bool = False):
         mode = _mode_value(settings.mode)
         if mode not in (0, 1, 2, 3):
             raise RuntimeError("unsupported rasterizer mode")
@@ -243,6 +245,8 @@ class FrameBuffers:
         # tile's fragments arrive roughly front to back and few of them have to be inserted in front of others
         self.depth_order = (self._scratch("depth_order", self.lib.htgs_depth_order_words(n), torch.int32)
                             if order_gaussians and not train and (mode == 2 or (fast and mode in (0, 1))) else None)
+        # the instances made bin by bin of depth, nearest first (HYBRID and FIRST_K, what ``rasterize`` and the others do with many Gaussians)
+        self.depth_bins = self._scratch("depth_bins", self.lib.htgs_depth_bins_words(n), torch.int32) if depth_bins and mode in (0, 1) else None
         self.image = torch.empty((3, self.height, self.width) if to_chw else (self.height, self.width, 3),
                                  dtype=torch.float32, device=dev)
         # the image-only fast path (``fast_rasterize``) writes no depth map
@@ -274,6 +278,7 @@ class FrameBuffers:
         f.waves_per_tile = int(waves_per_tile)
         f.tile_order = _ptr(self.tile_order)
         f.depth_order = _ptr(self.depth_order)
+        f.depth_bins = _ptr(self.depth_bins)
         f.long_list_threshold = int(long_list_threshold)      # 0: the library's default
         f.image, f.depth = _ptr(self.image), _ptr(self.depth)
         f.to_chw, f.use_median_depth, f.fast_math = int(bool(to_chw)), int(bool(use_median_depth)), int(bool(fast))

@@ -131,6 +131,16 @@ typedef struct htgs_frame {
                                   instances of the reference's list, roughly front to back instead of by Gaussian
                                   index, which the image-only blend does not mind and which spares it most insertions
                                   into the sorted core.  Ignored in the other cases */
+    uint32_t *depth_bins;      /* htgs_depth_bins_words(N) words or NULL, 16-byte aligned.  HYBRID_BLEND and ALPHA_BLEND_FIRST_K
+                                  with touch (ignored otherwise, and beside depth_order where that is used): htgs_preprocess
+                                  puts every Gaussian into one of eight bins of depth, about as many in each, and
+                                  htgs_create_instances emits the instances bin by bin, nearest first, inside a bin by
+                                  Gaussian index.  Every tile's list then holds the instances of the reference's list roughly
+                                  front to back, which spares most insertions into the sorted core.  offsets[] holds
+                                  the end of each Gaussian's instances (written by htgs_create_instances, training frames only);
+                                  they begin n_touched before it.  Results are those of lists by index: pixels at which
+                                  fragments of exactly equal depth met where they decide the core are settled in index order
+                                  (which takes vals[1 - selector], needed by every blend stage then) */
     /* ---- per-instance scratch (PerInstanceBuffers, buffer_utils.h:56-84) ---- */
     uint64_t n_instances;      /* host copy of *n_instances_dev, needed from htgs_create_instances on */
     const uint32_t *n_instances_live; /* NULL, or n_instances_dev: htgs_create_instances and the stages after it are queued before
@@ -192,6 +202,8 @@ int htgs_key_bytes(int mode, int width, int height);
 int htgs_frame_end_bit(const htgs_frame *f);
 int htgs_frame_key_bytes(const htgs_frame *f);
 int htgs_frame_sort_passes(const htgs_frame *f);
+/* words of htgs_frame.depth_bins for N Gaussians */
+size_t htgs_depth_bins_words(int n_primitives);
 /* words of htgs_frame.depth_order for N Gaussians */
 size_t htgs_depth_order_words(int n_primitives);
 /* digit passes htgs_scan_offsets takes to sort the N (depth key, Gaussian) pairs of a frame with depth_order (three of

@@ -1,0 +1,145 @@
+"""Instances made bin by bin of depth (``htgs_frame.depth_bins``) against lists by Gaussian index: the lists themselves, and what the
+walks make of them where fragments of exactly equal depth meet, whose order by index the reference's insertion depends on
+(R/include/hybrid_blend/kernels/inference.cuh:159-167)."""
+import dataclasses
+
+import pytest
+import torch
+
+from htgs_amd.synthetic import make_scene
+from htgs_amd.torch_bindings import FrameBuffers, RasterizerMode, diff_rasterize, rasterize, update_max_weights
+from htgs_amd.torch_bindings.rasterization import ScratchPool, run_max_weights
+from test_gpu_long_tiles import with_coincident_copies
+
+pytestmark = pytest.mark.gpu
+
+HYBRID, FIRST_K = 0, 1
+
+
+def small_view(scene, width=203, height=149):
+    scene.VPM[0] += (width / 2 - scene.width / 2) * scene.VPM[3]
+    scene.VPM[1] += (height / 2 - scene.height / 2) * scene.VPM[3]
+    scene.width, scene.height = width, height
+    return scene
+
+
+def with_twins(scene, twins):
+    """The first ``twins`` Gaussians once more, among the others by index, with other colours and opacities: pairs of fragments of
+    exactly equal depth wherever they are."""
+    n = scene.positions.shape[0]
+    order = torch.cat([torch.arange(n), torch.arange(twins)])[torch.randperm(n + twins, generator=torch.Generator().manual_seed(5))]
+    pick = lambda t: t[order].contiguous()
+    g = torch.Generator().manual_seed(6)
+    return dataclasses.replace(
+        scene, positions=pick(scene.positions), scales=pick(scene.scales), rotations=pick(scene.rotations), sh_rest=pick(scene.sh_rest),
+        opacities=(pick(scene.opacities) * (0.6 + 0.4 * torch.rand(n + twins, 1, generator=g))).contiguous(),
+        sh_0=(pick(scene.sh_0) + 0.5 * torch.randn(n + twins, *scene.sh_0.shape[1:], generator=g)).contiguous())
+
+
+def build(kind):
+    if kind == "twins":
+        return with_twins(small_view(make_scene(1, 40_000)), 20_000)
+    if kind == "copies":
+        return with_coincident_copies(make_scene(0, 1500), 4)
+    return make_scene(3, 60_000) if kind == "near" else small_view(make_scene(1, 60_000), 640, 400)
+
+
+def frame(sg, mode, K, bins, **kwargs):
+    return FrameBuffers(*sg.gaussians(), sg.settings(RasterizerMode(mode), K), True, kwargs.pop("median", False), tight_lists=True, depth_bins=bins, long_counters=True, **kwargs)
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("n", [1, 63, 257, 70_001])
+def test_lists(cuda, n, train):
+    """Every tile's list holds the same Gaussians as without bins, in up to eight runs by index, of growing depth; a training frame's
+    offsets say where each Gaussian's instances are."""
+    sg = small_view(make_scene(1, n), 640, 400).to(cuda)
+    by_index, binned = (frame(sg, HYBRID, 16, bins, train=train) for bins in (False, True))
+    for fb in (by_index, binned):
+        fb.preprocess()
+        fb.scan()
+        fb.alloc_instances(fb.read_instance_count())
+        fb.create_instances()
+    m = by_index.n_instances
+    assert binned.n_instances == m and torch.equal(binned.n_touched, by_index.n_touched)
+    unsorted = binned.vals[0][:m].clone()
+    for fb in (by_index, binned):
+        fb.selector = fb.sort()
+        fb.extract_ranges()
+    assert torch.equal(binned.ranges, by_index.ranges)
+    pairs = [torch.stack([fb.keys[fb.selector][:m].to(torch.int64), fb.vals[fb.selector][:m].to(torch.int64)]) for fb in (by_index, binned)]
+    assert torch.equal(pairs[0][:, torch.argsort(pairs[0][0] * n + pairs[0][1])], pairs[1][:, torch.argsort(pairs[1][0] * n + pairs[1][1])])
+    if m > 1:
+        same_tile = pairs[1][0][1:] == pairs[1][0][:-1]
+        back = same_tile & (pairs[1][1][1:] < pairs[1][1][:-1])
+        assert int(torch.bincount(pairs[1][0][1:][back], minlength=1).max()) <= 7
+        # a run ends where a nearer bin's depths end: behind a step back by index nothing is nearer than what came before the step's run
+        z = (sg.positions.to(torch.float64) @ sg.M.to(torch.float64)[2, :3] + sg.M.to(torch.float64)[2, 3])[unsorted.to(torch.int64)]
+        steps = torch.nonzero(unsorted[1:] < unsorted[:-1]).flatten() + 1
+        assert len(steps) <= 7
+        for step in steps.tolist():
+            assert float(z[:step].max()) <= float(z[step:].min()) + 1e-5
+    if train:
+        ends, counts = binned.offsets.to(torch.int64), binned.n_touched.to(torch.int64)
+        seen = torch.nonzero(counts).flatten()
+        slots = torch.repeat_interleave(ends[seen] - counts[seen], counts[seen]) + torch.cat([torch.arange(int(c), device=cuda) for c in counts[seen].tolist()] or [counts[:0]])
+        assert torch.equal(unsorted[slots].to(torch.int64), torch.repeat_interleave(seen, counts[seen]))
+
+
+@pytest.mark.parametrize("waves,threshold", [(1, 0), (2, 0), (4, 0), (1, 60)])
+@pytest.mark.parametrize("K", [1, 2, 4, 16, 32])
+@pytest.mark.parametrize("mode", [HYBRID, FIRST_K])
+@pytest.mark.parametrize("kind", ["twins", "copies", "near", "plain"])
+def test_image_and_depth(cuda, kind, mode, K, waves, threshold):
+    """Pairs of equal depth inside a core and at its end, more than two of a depth, near-plane scenes, chance ties: the walk by insertion over
+    the list by index (threshold above 8192) is what both orders have to come to.  Bounds: the keys' rounding of alpha (2^-20 at most)
+    and the tail's sums in another order, as for the walks by index."""
+    print(f"case kind={kind} mode={mode} K={K} waves={waves} threshold={threshold}", flush=True)
+    sg = build(kind).to(cuda)
+    want, want_depth = frame(sg, mode, K, False, long_list_threshold=2 ** 31 - 1).run()
+    got, got_depth = frame(sg, mode, K, True, waves_per_tile=waves, long_list_threshold=threshold).run()
+    assert (got - want).abs().max() < 4e-6
+    assert (got_depth - want_depth).abs().max() < 1e-4
+
+
+@pytest.mark.parametrize("waves,threshold", [(1, 0), (2, 0), (1, 60)])
+@pytest.mark.parametrize("K", [1, 4, 16, 32])
+@pytest.mark.parametrize("mode", [HYBRID, FIRST_K])
+@pytest.mark.parametrize("kind", ["twins", "copies", "plain"])
+def test_training(cuda, kind, mode, K, waves, threshold):
+    """The same core indices, slot by slot; gradients of the rows wherever they are."""
+    print(f"case kind={kind} mode={mode} K={K} waves={waves} threshold={threshold}", flush=True)
+    sg = build(kind).to(cuda)
+    frames = [frame(sg, mode, K, bins, train=True, waves_per_tile=waves if bins else 1, long_list_threshold=threshold if bins else 2 ** 31 - 1) for bins in (False, True)]
+    images = [fb.run_forward() for fb in frames]
+    assert (images[1] - images[0]).abs().max() < 4e-6
+    assert torch.equal(*[fb.records_in_image_order(fb.core_idx) for fb in frames])
+    grad_image = torch.randn(images[0].shape, generator=torch.Generator(device=cuda).manual_seed(3), device=cuda)
+    for a, b in zip(*[fb.run_backward(grad_image, None, False) for fb in frames]):
+        assert a.numel() == 0 or (a - b).abs().max() <= 1e-4 * max(1e-6, float(a.abs().max()))
+
+
+@pytest.mark.parametrize("mode", [HYBRID, FIRST_K])
+def test_operators(cuda, mode):
+    """170 000 Gaussians, a third of them twins: the operators take bins, and come to what the stages by index come to."""
+    print(f"case mode={mode}", flush=True)
+    sg = with_twins(small_view(make_scene(1, 120_000), 400, 304), 50_000).to(cuda)
+    s = sg.settings(RasterizerMode(mode), 16)
+    image, depth = rasterize(*sg.gaussians(), s, True, False)
+    assert ScratchPool.current(cuda).frame.depth_bins
+    want, want_depth = frame(sg, mode, 16, False, long_list_threshold=2 ** 31 - 1).run()
+    assert (image - want).abs().max() < 4e-6 and (depth[0] - want_depth).abs().max() < 1e-4
+    step = diff_rasterize(*[t.requires_grad_() for t in sg.gaussians()], torch.empty(0, device=cuda), s, False)
+    assert step.grad_fn.fb.frame.depth_bins
+    by_index = frame(sg, mode, 16, False, train=True, long_list_threshold=2 ** 31 - 1)
+    assert (step.detach() - by_index.run_forward()).abs().max() < 4e-6
+    weights, by_stages = torch.zeros(170_000, device=cuda), torch.zeros(170_000, device=cuda)
+    with torch.no_grad():
+        update_max_weights(weights, *[t.detach() for t in sg.gaussians()[:4]], s, 0.02)
+        run_max_weights(by_stages, *[t.detach() for t in sg.gaussians()[:4]], s, 0.02, long_list_threshold=2 ** 31 - 1)
+    if mode == FIRST_K:
+        assert torch.equal(weights, by_stages)
+    else:
+        # (a weight within rounding of the threshold may fall on the other side of it)
+        both = (weights > 0) & (by_stages > 0)
+        assert ((weights - by_stages).abs()[both] <= 1e-5 * by_stages[both]).all() and int((both != ((weights > 0) | (by_stages > 0))).sum()) <= 2
