@@ -1,6 +1,8 @@
 // Pieces shared by the inference, training-forward, max-weight and backward blend kernels.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace htgs {
@@ -179,6 +181,21 @@ __device__ __forceinline__ uint32_t tile_quadrant_hits(const float (&n)[6], cons
     return bits;
 }
 
+// A depth that no fragment of an instance is nearer than.  A fragment's point lies within the cut-off, and within the radius at which
+// alpha falls to the mode's least, of the Gaussian's unit space, where depth is MT3.n u + MT3.w: no nearer than MT3.w - radius |MT3.n|.
+// The computed depth is within some 1e-6 times the tile centre's distance in that space of this, so a twentieth of the radius is
+// added and instances whose distance is beyond 100 cut-offs, or anything that is not a number, are not bounded.
+template <int MODE>
+__device__ __forceinline__ float nearest_depth(const float (&n)[6], const float (&d)[6], const float4 &mt3, float opacity)
+{
+    float r = __builtin_fmaf(__builtin_amdgcn_logf(opacity), -1.0f / ModeCfg<MODE>::exp2_scale, 1.0f);
+    r = r < 1.0f ? r : 1.0f;
+    r = r > 0.0f ? r : 0.0f;
+    const float reach = 1.05f * __builtin_amdgcn_sqrtf(ModeCfg<MODE>::cutoff_sq * (r + 1e-3f) * __builtin_fmaf(mt3.z, mt3.z, __builtin_fmaf(mt3.y, mt3.y, mt3.x * mt3.x)));
+    const float depth = mt3.w - __builtin_fmaf(1e-5f, __builtin_fabsf(mt3.w), reach);
+    return n[0] < 1e4f * d[0] ? depth : -__FLT_MAX__;
+}
+
 // Stages instance `fetch` of the sorted list in slot `slot` (the same arithmetic as tile_geometry / tile_quadratics,
 // written out so that every row is stored as soon as it is complete: the kernels that call this hold a K-buffer in
 // registers).  Returns whether the slot holds an instance that can reach a pixel of the tile: always true for a
@@ -230,15 +247,18 @@ enum { kCullNone = 0, kCullAlpha = 1, kCullCutoff = 2, kCullPixels = 3, kCullSca
 // UNIT: the opacity is staged held to at most 1 (the image-only fast path, whose fragments then need no clamp of their own).
 // POS: the last word of the slot holds the instance's place in the list (fetch) instead of the Gaussian's index.
 // GIVEN: the caller has read inst[fetch] already (`given`).
+// nearest: receives a depth that no fragment of the instance is nearer than (nearest_depth).
 template <int MODE, int N, bool DEPTH, int CULL = kCullNone, bool QUADRANTS = false, int REC4 = HTGS_PRIM_FLOATS / 4, bool UNIT = false, bool POS = false,
           bool GIVEN = false>
 __device__ __forceinline__ uint32_t tile_stage_load(TileStage<N> &st, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst,
-                                                    uint32_t fetch, uint32_t last, int slot, float cx, float cy, uint64_t pixel_lanes = 0, uint32_t given = 0, float cull_scale = 1.0f);
+                                                    uint32_t fetch, uint32_t last, int slot, float cx, float cy, uint64_t pixel_lanes = 0, uint32_t given = 0, float cull_scale = 1.0f,
+                                                    float *nearest = nullptr);
 
 // (PixelTerms is complete by the time the template is instantiated)
 template <int MODE, int N, bool DEPTH, int CULL, bool QUADRANTS, int REC4, bool UNIT, bool POS, bool GIVEN>
 __device__ __forceinline__ uint32_t tile_stage_load(TileStage<N> &st, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst,
-                                                    uint32_t fetch, uint32_t last, int slot, float cx, float cy, uint64_t pixel_lanes, uint32_t given, float cull_scale)
+                                                    uint32_t fetch, uint32_t last, int slot, float cx, float cy, uint64_t pixel_lanes, uint32_t given, float cull_scale,
+                                                    float *nearest)
 {
     if (fetch >= last) return 0;
     const uint32_t g = GIVEN ? given : inst[fetch];
@@ -288,6 +308,7 @@ __device__ __forceinline__ uint32_t tile_stage_load(TileStage<N> &st, const floa
         asm volatile("" ::: "memory");
         col = rec[4];
     }
+    if (nearest != nullptr) *nearest = nearest_depth<MODE>(n, d, r3, col.w);
     if (UNIT) col.w = col.w < 1.0f ? col.w : 1.0f;
     st.q[4][slot] = make_float4(zxy, zyy, r3.w, col.w);
     st.q[5][slot] = make_float4(col.x, col.y, col.z, bits_to_float(POS ? fetch : g));
@@ -475,19 +496,44 @@ __device__ __forceinline__ void quadrant_list_walk_pairs(const QuadrantLists &ql
 // AHEAD: a lane reads the list entry of the next batch before it walks this one (one register more through the walk; the
 // entry is then there when the batch is staged, and the records' fetch does not wait for it).
 // PAIRS: two turns at a time, turn(one, two).
+// last_depth(): the depth from which on a fragment is of no use to the lane's pixel any more (AllDepths: none is); an instance that is
+// nowhere nearer than that for all pixels of a quadrant is left out of the quadrant's list.
+struct AllDepths {};
+// the largest of the values of each quadrant's sixteen lanes, the same in all lanes
+struct QuadrantDepths { float q[4]; };
+__device__ __forceinline__ QuadrantDepths quadrant_most(float v)
+{
+    float m = v;
+    const auto step = [&m](float o) { m = m > o ? m : o; };
+    step(bits_to_float((uint32_t)__builtin_amdgcn_update_dpp((int)float_to_bits(m), (int)float_to_bits(m), 0x121, 0xf, 0xf, false)));      // row_ror:1
+    step(bits_to_float((uint32_t)__builtin_amdgcn_update_dpp((int)float_to_bits(m), (int)float_to_bits(m), 0x122, 0xf, 0xf, false)));      // row_ror:2
+    step(bits_to_float((uint32_t)__builtin_amdgcn_update_dpp((int)float_to_bits(m), (int)float_to_bits(m), 0x124, 0xf, 0xf, false)));      // row_ror:4
+    step(bits_to_float((uint32_t)__builtin_amdgcn_update_dpp((int)float_to_bits(m), (int)float_to_bits(m), 0x128, 0xf, 0xf, false)));      // row_ror:8
+    QuadrantDepths most;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) most.q[q] = bits_to_float((uint32_t)__builtin_amdgcn_readlane((int)float_to_bits(m), 16 * q));
+    return most;
+}
 template <int MODE, bool DEPTH, int CULL, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, bool UNIT = false, bool POS = false, bool AHEAD = false, bool PAIRS = false,
-          typename Turn>
+          typename Turn, typename Last = AllDepths>
 __device__ __forceinline__ void tile_list_walk(TileStageQ &st, QuadrantLists &ql, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst,
                                                uint32_t first, uint32_t last, uint32_t lane, float cx, float cy, Turn &&turn, uint64_t pixel_lanes = 0,
-                                               float cull_scale = 1.0f, uint32_t step = 64u)
+                                               float cull_scale = 1.0f, uint32_t step = 64u, Last &&last_depth = Last())
 {
+    constexpr bool kNear = !std::is_same<typename std::decay<Last>::type, AllDepths>::value;
     stage_dummy_init(st, lane);
     uint32_t listed = 0;
     if (AHEAD) listed = first + lane < last ? inst[first + lane] : 0u;
     for (uint32_t base = first; base < last; base += step) {
         if (SOLO) __syncthreads(); else wave_lds_sync();
-        const uint32_t bits = tile_stage_load<MODE, kStageSlots, DEPTH, CULL, true, REC4, UNIT, POS, AHEAD>(st, prim, inst, base + lane, last, lane + 1, cx, cy, pixel_lanes,
-                                                                                                           listed, cull_scale);
+        float nearest = -__FLT_MAX__;
+        uint32_t bits = tile_stage_load<MODE, kStageSlots, DEPTH, CULL, true, REC4, UNIT, POS, AHEAD>(st, prim, inst, base + lane, last, lane + 1, cx, cy, pixel_lanes,
+                                                                                                     listed, cull_scale, kNear ? &nearest : nullptr);
+        if constexpr (kNear) {
+            const QuadrantDepths most = quadrant_most(last_depth());
+#pragma unroll
+            for (int q = 0; q < 4; ++q) bits &= nearest > most.q[q] ? ~(1u << q) : ~0u;
+        }
         if (AHEAD) listed = base + step + lane < last ? inst[base + step + lane] : 0u;
         const uint32_t n_turns = quadrant_lists_build(ql, bits, lane, st);
         if (SOLO) __syncthreads(); else wave_lds_sync();

@@ -1075,7 +1075,7 @@ __device__ __forceinline__ void first_k_walk(TileStageQ &st, QuadrantLists &ql, 
         uint32_t idx = stage_index<N>(addr);
         core_exchange_walk<K>(depth, alpha, idx, cd, ca, ci);
         if (TIES && alpha > 0.0f && depth == cd[K - 1]) tie->note(depth, idx);
-    }, pixel_lanes, 1.0f, step);
+    }, pixel_lanes, 1.0f, step, [&]() { return cd[K - 1]; });
 }
 // The same walk with the core as sorted 64-bit keys (above HYBRID_BLEND's: depth | alpha as a fraction | place in the list),
 // exact arithmetic; `tie` as in hybrid_key_walk.
@@ -1109,7 +1109,7 @@ __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &
         };
         joins(one, f1, reach1, depth1);
         joins(two, f2, reach2, depth2);
-    }, 0, 1.0f, step);
+    }, 0, 1.0f, step, [&]() { return key_depth(core[K - 1]); });
 }
 // the finished keys as the three arrays the composite takes (an empty slot has the index 0xffffffff)
 template <int K>

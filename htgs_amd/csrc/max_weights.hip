@@ -72,7 +72,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
             ca[i] = 0.0f; cd[i] = __FLT_MAX__; ci[i] = 0xffffffffu;
             asm volatile("" : "+v"(cd[i]), "+v"(ca[i]), "+v"(ci[i]));      // one register per slot
         }
-        tile_list_walk<MODE, kCore, AGAIN ? kCullPixels : kCullAlpha, true>(st, ql, prim, list, first, last, lane, cx, cy, [&](uint32_t addr) {
+        const auto turn = [&](uint32_t addr) {
             // (TIES of hybrid_walk and first_k_walk)
             const auto enters = [&](float depth) { return AGAIN ? depth < cd[KS - 1] : depth <= cd[KS - 1]; };
             TileFrag f;
@@ -92,7 +92,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
                 if (!AGAIN && alpha > 0.0f && depth == cd[KS - 1]) tie.note(depth, idx);
             }
             if (kTail) { alpha_sum += alpha; T_tail *= 1.0f - alpha; }
-        }, pixel_lanes);
+        };
+        constexpr int CULL = AGAIN ? kCullPixels : kCullAlpha;
+        if constexpr (kTail) tile_list_walk<MODE, kCore, CULL, true>(st, ql, prim, list, first, last, lane, cx, cy, turn, pixel_lanes);
+        else tile_list_walk<MODE, kCore, CULL, true>(st, ql, prim, list, first, last, lane, cx, cy, turn, pixel_lanes, 1.0f, 64u, [&]() { return cd[KS - 1]; });
     };
     // the core's weights; returns the weight of a tail fragment per unit of alpha
     const auto weigh = [&]() {
