@@ -1053,14 +1053,43 @@ __device__ __forceinline__ void first_k_core_init(float (&cd)[K], float (&ca)[K]
         asm volatile("" : "+v"(cd[i]), "+v"(ca[i]), "+v"(ci[i]));      // one register per slot
     }
 }
+// Waves that share a list know more together than each from its own core: if every wave has k fragments of a pixel with k times WAVES no less than K,
+// the K nearest of all are no deeper than the deepest of those waves' k-th.  Every wave leaves its own in LDS before it stages a batch
+// and takes what the others have left, whatever they have walked until then: a depth that only grows nearer with time, behind
+// which there is nothing to be found for the pixel.
+template <int WAVES, int K>
+struct SharedDepth {
+    static constexpr int kSlot = (K + WAVES - 1) / WAVES - 1;
+    float (*s_depth)[64];                  // LDS, [WAVES][64]
+    uint32_t wave, lane;
+    __device__ __forceinline__ void init() const { s_depth[wave][lane] = __FLT_MAX__; }      // (and a barrier of the workgroup)
+    __device__ __forceinline__ float operator()(float own) const
+    {
+        typedef __attribute__((address_space(3))) volatile float lds_shared;
+        lds_shared *const all = (lds_shared *)&s_depth[0][lane];
+        all[64u * wave] = own;
+        float most = own;
+#pragma unroll
+        for (uint32_t w = 0; w < (uint32_t)WAVES; ++w) {
+            const float v = all[64u * w];
+            most = w != wave && v > most ? v : most;
+        }
+        return most;
+    }
+};
+struct NoSharedDepth {
+    static constexpr int kSlot = 0;
+    __device__ __forceinline__ float operator()(float) const { return __FLT_MAX__; }
+};
 // The walk over instances [first, last) of a tile's list by one wave (SOLO: the wave is the whole workgroup).  TIES (the
 // walks of blend_first_k_long_kernel): `tie` receives the least depth at which an entry was pushed out of the core that is
 // exactly as deep as the entry that is now last.
 // PIXELS: only the pixels of the lanes in pixel_lanes are wanted; instances that do not reach one of them are left out.
-template <int K, bool FAST, bool SOLO, bool TIES = false, int REC4 = HTGS_PRIM_FLOATS / 4, bool PIXELS = false>
+template <int K, bool FAST, bool SOLO, bool TIES = false, int REC4 = HTGS_PRIM_FLOATS / 4, bool PIXELS = false, typename Shared = NoSharedDepth>
 __device__ __forceinline__ void first_k_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                              uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy, float (&cd)[K],
-                                             float (&ca)[K], uint32_t (&ci)[K], CoreTie *tie = nullptr, uint64_t pixel_lanes = 0, uint32_t step = 64u)
+                                             float (&ca)[K], uint32_t (&ci)[K], CoreTie *tie = nullptr, uint64_t pixel_lanes = 0, uint32_t step = 64u,
+                                             const Shared &shared = Shared())
 {
     constexpr int MODE = HTGS_MODE_ALPHA_BLEND_FIRST_K;
     constexpr int N = kStageSlots;
@@ -1075,14 +1104,18 @@ __device__ __forceinline__ void first_k_walk(TileStageQ &st, QuadrantLists &ql, 
         uint32_t idx = stage_index<N>(addr);
         core_exchange_walk<K>(depth, alpha, idx, cd, ca, ci);
         if (TIES && alpha > 0.0f && depth == cd[K - 1]) tie->note(depth, idx);
-    }, pixel_lanes, 1.0f, step, [&]() { return cd[K - 1]; });
+    }, pixel_lanes, 1.0f, step, [&]() {
+        const float of_all = shared(cd[Shared::kSlot]);
+        return cd[K - 1] < of_all ? cd[K - 1] : of_all;
+    });
 }
 // The same walk with the core as sorted 64-bit keys (above HYBRID_BLEND's: depth | alpha as a fraction | place in the list),
 // exact arithmetic; `tie` as in hybrid_key_walk.
-template <int K, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4>
+template <int K, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, typename Shared = NoSharedDepth>
 __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                  uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy,
-                                                 CoreKey (&core)[K], uint32_t &tie, const KeyFormat &fmt, uint32_t list_first, uint32_t step = 64u)
+                                                 CoreKey (&core)[K], uint32_t &tie, const KeyFormat &fmt, uint32_t list_first, uint32_t step = 64u,
+                                                 const Shared &shared = Shared())
 {
     constexpr int MODE = HTGS_MODE_ALPHA_BLEND_FIRST_K;
     constexpr int N = kStageSlots;
@@ -1109,7 +1142,10 @@ __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &
         };
         joins(one, f1, reach1, depth1);
         joins(two, f2, reach2, depth2);
-    }, 0, 1.0f, step, [&]() { return key_depth(core[K - 1]); });
+    }, 0, 1.0f, step, [&]() {
+        const float of_all = shared(key_depth(core[Shared::kSlot])), own = key_depth(core[K - 1]);
+        return own < of_all ? own : of_all;
+    });
 }
 // the finished keys as the three arrays the composite takes (an empty slot has the index 0xffffffff)
 template <int K>
@@ -1248,6 +1284,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     constexpr uint32_t kRows = 3 * K + 2;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<kWaves, kRows>()];
     __shared__ uint32_t s_next, s_whole, s_redo[2], s_listed[kWaves], s_runs[1 + kDepthBins];
+    __shared__ float s_depth[kWaves][64];
     __shared__ float s_last_depth[64];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     if (long_tiles[0] == 0) return;                   // (the ordinary frame)
@@ -1269,8 +1306,11 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         first_k_core_init<K>(cd, ca, ci);
         CoreTie tie;
         tie.init();
-        first_k_walk<K, FAST, false, kTies, REC4>(wave_stage(lds, wave), wave_lists<kWaves>(lds, wave), inst, prim, e.first + 64u * wave, e.last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie,
-                                                0, 64u * kWaves);
+        const SharedDepth<kWaves, K> shared = { s_depth, wave, lane };
+        shared.init();
+        __syncthreads();
+        first_k_walk<K, FAST, false, kTies, REC4, false>(wave_stage(lds, wave), wave_lists<kWaves>(lds, wave), inst, prim, e.first + 64u * wave, e.last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie,
+                                                       0, 64u * kWaves, shared);
         merge_all_shares<kWaves, kRows>(lds, wave, [&](float *to) { first_k_put<K>(to, lane, cd, ca, ci, tie); },
                                         [&](const float *from) { first_k_merge<K>(from, lane, cd, ca, ci, tie); });
         if (e.parts > 1u) {

@@ -174,7 +174,11 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     }
     uint32_t tie = 0u;
     const KeyFormat fmt = key_format(last > first ? last - first : 1u);
-    first_k_key_walk<K, false>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, core, tie, fmt, first, 64u * WAVES);
+    __shared__ float s_depth[WAVES][64];
+    const SharedDepth<WAVES, K> shared = { s_depth, wave, lane };
+    shared.init();
+    __syncthreads();
+    first_k_key_walk<K, false>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, core, tie, fmt, first, 64u * WAVES, shared);
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
             [&](float *to) { give_key_core<K>(to + lane, core); to[2 * K * 64 + lane] = bits_to_float(tie); },
             [&](const float *from) {
@@ -216,7 +220,11 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     first_k_core_init<K>(cd, ca, ci);
     CoreTie tie;
     tie.init();
-    first_k_walk<K, FAST, false, true, REC4>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie, 0, 64u * WAVES);
+    __shared__ float s_depth[WAVES][64];
+    const SharedDepth<WAVES, K> shared = { s_depth, wave, lane };
+    shared.init();
+    __syncthreads();
+    first_k_walk<K, FAST, false, true, REC4, false>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie, 0, 64u * WAVES, shared);
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
             [&](float *to) { first_k_put<K>(to, lane, cd, ca, ci, tie); },
             [&](const float *from) { first_k_merge<K>(from, lane, cd, ca, ci, tie); })) return;
