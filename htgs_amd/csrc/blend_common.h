@@ -498,7 +498,13 @@ __device__ __forceinline__ void quadrant_list_walk_pairs(const QuadrantLists &ql
 // PAIRS: two turns at a time, turn(one, two).
 // last_depth(): the depth from which on a fragment is of no use to the lane's pixel any more (AllDepths: none is); an instance that is
 // nowhere nearer than that for all pixels of a quadrant is left out of the quadrant's list.
+// step: from one batch of the wave's to the next, and how many instances each has (waves that share a list: blend_waves.h).
 struct AllDepths {};
+struct ListStep {
+    uint32_t step, batch;
+    __device__ __forceinline__ ListStep(uint32_t s, uint32_t b = 64u) : step(s), batch(b) {}
+    __device__ __forceinline__ uint32_t at(uint32_t base, uint32_t last, uint32_t lane) const { return batch >= 64u || lane < batch ? base + lane : last; }
+};
 // the largest of the values of each quadrant's sixteen lanes, the same in all lanes
 struct QuadrantDepths { float q[4]; };
 __device__ __forceinline__ QuadrantDepths quadrant_most(float v)
@@ -518,23 +524,24 @@ template <int MODE, bool DEPTH, int CULL, bool SOLO, int REC4 = HTGS_PRIM_FLOATS
           typename Turn, typename Last = AllDepths>
 __device__ __forceinline__ void tile_list_walk(TileStageQ &st, QuadrantLists &ql, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst,
                                                uint32_t first, uint32_t last, uint32_t lane, float cx, float cy, Turn &&turn, uint64_t pixel_lanes = 0,
-                                               float cull_scale = 1.0f, uint32_t step = 64u, Last &&last_depth = Last())
+                                               float cull_scale = 1.0f, ListStep step = 64u, Last &&last_depth = Last())
 {
     constexpr bool kNear = !std::is_same<typename std::decay<Last>::type, AllDepths>::value;
     stage_dummy_init(st, lane);
     uint32_t listed = 0;
-    if (AHEAD) listed = first + lane < last ? inst[first + lane] : 0u;
-    for (uint32_t base = first; base < last; base += step) {
+    const auto list_entry = [&](uint32_t base) { const uint32_t at = step.at(base, last, lane); return at < last ? inst[at] : 0u; };
+    if (AHEAD) listed = list_entry(first);
+    for (uint32_t base = first; base < last; base += step.step) {
         if (SOLO) __syncthreads(); else wave_lds_sync();
         float nearest = -__FLT_MAX__;
-        uint32_t bits = tile_stage_load<MODE, kStageSlots, DEPTH, CULL, true, REC4, UNIT, POS, AHEAD>(st, prim, inst, base + lane, last, lane + 1, cx, cy, pixel_lanes,
+        uint32_t bits = tile_stage_load<MODE, kStageSlots, DEPTH, CULL, true, REC4, UNIT, POS, AHEAD>(st, prim, inst, step.at(base, last, lane), last, lane + 1, cx, cy, pixel_lanes,
                                                                                                      listed, cull_scale, kNear ? &nearest : nullptr);
         if constexpr (kNear) {
             const QuadrantDepths most = quadrant_most(last_depth());
 #pragma unroll
             for (int q = 0; q < 4; ++q) bits &= nearest > most.q[q] ? ~(1u << q) : ~0u;
         }
-        if (AHEAD) listed = base + step + lane < last ? inst[base + step + lane] : 0u;
+        if (AHEAD) listed = list_entry(base + step.step);
         const uint32_t n_turns = quadrant_lists_build(ql, bits, lane, st);
         if (SOLO) __syncthreads(); else wave_lds_sync();
         // lanes outside the image run along (their results are never stored): the loop stays wave-uniform

@@ -66,7 +66,7 @@ __device__ __forceinline__ void hybrid_core_init(float (&cd)[K], float (&ca)[K],
 template <int K, bool FAST, bool SOLO, bool TIES = false, bool PIXELS = false, int REC4 = HTGS_PRIM_FLOATS / 4, bool QUICK = false>
 __device__ __forceinline__ void hybrid_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                             uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy, float (&cd)[K],
-                                            float (&ca)[K], float (&ci)[K], HybridTail &tail, CoreTie *tie = nullptr, uint64_t pixel_lanes = 0, uint32_t step = 64u)
+                                            float (&ca)[K], float (&ci)[K], HybridTail &tail, CoreTie *tie = nullptr, uint64_t pixel_lanes = 0, ListStep step = 64u)
 {
     constexpr int MODE = HTGS_MODE_HYBRID_BLEND;
     constexpr int N = kStageSlots;
@@ -172,7 +172,7 @@ __device__ __forceinline__ void core_key_walk(CoreKey &carried, CoreKey (&core)[
 template <int K, bool FAST, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, bool AHEAD = false>
 __device__ __forceinline__ void hybrid_key_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                 uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy,
-                                                CoreKey (&core)[K], HybridTail &tail, uint32_t &tie, const KeyFormat &fmt, uint32_t list_first, uint32_t step = 64u)
+                                                CoreKey (&core)[K], HybridTail &tail, uint32_t &tie, const KeyFormat &fmt, uint32_t list_first, ListStep step = 64u)
 {
     constexpr int MODE = HTGS_MODE_HYBRID_BLEND;
     constexpr int N = kStageSlots;
@@ -1088,7 +1088,7 @@ struct NoSharedDepth {
 template <int K, bool FAST, bool SOLO, bool TIES = false, int REC4 = HTGS_PRIM_FLOATS / 4, bool PIXELS = false, typename Shared = NoSharedDepth>
 __device__ __forceinline__ void first_k_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                              uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy, float (&cd)[K],
-                                             float (&ca)[K], uint32_t (&ci)[K], CoreTie *tie = nullptr, uint64_t pixel_lanes = 0, uint32_t step = 64u,
+                                             float (&ca)[K], uint32_t (&ci)[K], CoreTie *tie = nullptr, uint64_t pixel_lanes = 0, ListStep step = 64u,
                                              const Shared &shared = Shared())
 {
     constexpr int MODE = HTGS_MODE_ALPHA_BLEND_FIRST_K;
@@ -1114,7 +1114,7 @@ __device__ __forceinline__ void first_k_walk(TileStageQ &st, QuadrantLists &ql, 
 template <int K, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, typename Shared = NoSharedDepth>
 __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                  uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy,
-                                                 CoreKey (&core)[K], uint32_t &tie, const KeyFormat &fmt, uint32_t list_first, uint32_t step = 64u,
+                                                 CoreKey (&core)[K], uint32_t &tie, const KeyFormat &fmt, uint32_t list_first, ListStep step = 64u,
                                                  const Shared &shared = Shared())
 {
     constexpr int MODE = HTGS_MODE_ALPHA_BLEND_FIRST_K;
@@ -1409,7 +1409,7 @@ struct OitSums {
 // DEPTH: the depth sum is wanted (the training pass has no use for it)
 template <bool FAST, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, bool DEPTH = !FAST>
 __device__ __forceinline__ void oit_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t first,
-                                         uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy, OitSums &sum, uint32_t step = 64u)
+                                         uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy, OitSums &sum, ListStep step = 64u)
 {
     constexpr int MODE = HTGS_MODE_OIT_BLEND;
     constexpr int N = kStageSlots;

@@ -17,13 +17,26 @@
 
 namespace htgs {
 
-// The share of wave `wave` of a list: every WAVES-th batch of 64 from its own on.  (In a list in bins of depth the nearer Gaussians, which
-// reach more of a tile, come first: contiguous shares would leave the first wave with the most work.)  Waves without a batch are the last ones.
+// The share of wave `wave` of a list: every WAVES-th batch from its own on.  (In a list in bins of depth the nearer Gaussians, which
+// reach more of a tile, come first: contiguous shares would leave the first wave with the most work.)  The batches are as large as
+// they come out if every wave has the same number of them, 64 at most.  Waves without a batch are the last ones.
+// Small frames have lists of less than a batch, which one wave walked alone, and a list of 70 was 64 and 6.  Below the least share another
+// wave's core costs more to merge than its turns take.  Whole passes, batches of 64 -> shares of 32 and more -> of 8 and 16 as here: HYBRID
+// K = 4 10 k at 256x256 46.1 -> 43.9 -> 42.5 us, OIT 334 k at 1237x821 151.0 -> 148.7 -> 148.3, training of
+// 20 k at 660x834, HYBRID K = 4, 232 -> 222 -> 219, of 244 k at 1694x265, K = 16, 317 -> 311.6 -> 310.
+// FIRST_K's waves know from one another how deep they have to look (SharedDepth), and merge more than they
+// spare below twice that (K = 4, 108 k at 451x862: 86.3 -> 85.4 -> 85.9).
+constexpr uint32_t least_share(int K, bool tail) { return (K <= 4 ? 8u : 16u) * (tail ? 1u : 2u); }
 struct TileShare {
     uint32_t first, per;                   // per: where the next wave's begins
 };
-template <int WAVES>
-__device__ __forceinline__ TileShare tile_share(uint32_t first, uint32_t wave) { return TileShare{ first + 64u * wave, 64u }; }
+template <int WAVES, uint32_t LEAST>
+__device__ __forceinline__ TileShare tile_share(uint32_t first, uint32_t last, uint32_t wave)
+{
+    const uint32_t n = last - first, rounds = n > 64u * WAVES ? (n + 64u * WAVES - 1u) / (64u * WAVES) : 1u;
+    const uint32_t batch = (n + rounds * WAVES - 1u) / (rounds * WAVES), per = batch > LEAST ? batch : LEAST;
+    return TileShare{ first + per * wave, per };
+}
 // The pairwise merging: give(buffer) is called by the wave that hands its share over, take(buffer) by the one that receives
 // it (all lanes; buffer: 64-lane rows, one buffer per pair of waves); false: the wave is done.  The buffers lie over the stages,
 // which nobody reads any more.
@@ -68,7 +81,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     uint32_t tile, first, last;
     if (!tile_of_waves(ranges, tile_order, long_tiles, threshold, part_floor, long_part_words<K>(), tile, first, last)) return;
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
-    const TileShare share = tile_share<WAVES>(first, wave);
+    const TileShare share = tile_share<WAVES, least_share(K, true)>(first, last, wave);
     HybridTail tail;
     hybrid_tail_init(tail);
     CoreKey core[K];
@@ -81,7 +94,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     const KeyFormat fmt = key_format(last > first ? last - first : 1u);
     // (places count from the tile's first instance, as in the single walk)
     hybrid_key_walk<K, FAST, false, HTGS_PRIM_FLOATS / 4, true>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy,
-                                                                core, tail, tie, fmt, first, 64u * WAVES);
+                                                                core, tail, tie, fmt, first, ListStep(share.per * WAVES, share.per));
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
             [&](float *to) { give_key_core<K>(to + lane, core); give_tail<2 * K>(to + lane, tail); to[(2 * K + 6) * 64 + lane] = bits_to_float(tie); },
             [&](const float *from) {
@@ -124,7 +137,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     uint32_t tile, first, last;
     if (!tile_of_waves(ranges, tile_order, long_tiles, threshold, part_floor, long_part_words<K>(), tile, first, last)) return;
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
-    const TileShare share = tile_share<WAVES>(first, wave);
+    const TileShare share = tile_share<WAVES, least_share(K, true)>(first, last, wave);
     HybridTail tail;
     hybrid_tail_init(tail);
     float cd[K], ca[K], ci[K];
@@ -132,7 +145,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     CoreTie tie;
     tie.init();
     hybrid_walk<K, false, false, true, false, REC4>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci,
-                                                    tail, &tie, 0, 64u * WAVES);
+                                                    tail, &tie, 0, ListStep(share.per * WAVES, share.per));
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
             [&](float *to) { hybrid_put<K>(to, lane, cd, ca, ci, tail, tie); },
             [&](const float *from) { hybrid_merge<K, false>(from, lane, cd, ca, ci, tail, tie); })) return;
@@ -165,7 +178,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     uint32_t tile, first, last;
     if (!tile_of_waves(ranges, tile_order, long_tiles, threshold, part_floor, first_k_part_words<K>(), tile, first, last)) return;
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
-    const TileShare share = tile_share<WAVES>(first, wave);
+    const TileShare share = tile_share<WAVES, least_share(K, false)>(first, last, wave);
     CoreKey core[K];
 #pragma unroll
     for (int i = 0; i < K; ++i) {
@@ -178,7 +191,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     const SharedDepth<WAVES, K> shared = { s_depth, wave, lane };
     shared.init();
     __syncthreads();
-    first_k_key_walk<K, false>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, core, tie, fmt, first, 64u * WAVES, shared);
+    first_k_key_walk<K, false>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, core, tie, fmt, first, ListStep(share.per * WAVES, share.per), shared);
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
             [&](float *to) { give_key_core<K>(to + lane, core); to[2 * K * 64 + lane] = bits_to_float(tie); },
             [&](const float *from) {
@@ -214,7 +227,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     uint32_t tile, first, last;
     if (!tile_of_waves(ranges, tile_order, long_tiles, threshold, part_floor, first_k_part_words<K>(), tile, first, last)) return;
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
-    const TileShare share = tile_share<WAVES>(first, wave);
+    const TileShare share = tile_share<WAVES, least_share(K, false)>(first, last, wave);
     float cd[K], ca[K];
     uint32_t ci[K];
     first_k_core_init<K>(cd, ca, ci);
@@ -224,7 +237,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     const SharedDepth<WAVES, K> shared = { s_depth, wave, lane };
     shared.init();
     __syncthreads();
-    first_k_walk<K, FAST, false, true, REC4, false>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie, 0, 64u * WAVES, shared);
+    first_k_walk<K, FAST, false, true, REC4, false>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie, 0, ListStep(share.per * WAVES, share.per), shared);
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
             [&](float *to) { first_k_put<K>(to, lane, cd, ca, ci, tie); },
             [&](const float *from) { first_k_merge<K>(from, lane, cd, ca, ci, tie); })) return;
@@ -257,9 +270,9 @@ __global__ void __launch_bounds__(64 * WAVES) blend_oit_waves_kernel(
     uint32_t tile, first, last;
     if (!tile_of_waves(ranges, tile_order, long_tiles, threshold, part_floor, kOitPartWords, tile, first, last)) return;
     const TilePixel px = quadrant_tile_pixel(tile, grid_w, lane, width, height);
-    const TileShare share = tile_share<WAVES>(first, wave);
+    const TileShare share = tile_share<WAVES, least_share(1, true)>(first, last, wave);
     OitSums sum = { 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 1.0f };
-    oit_walk<FAST, false, REC4, DEPTH>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, sum, 64u * WAVES);
+    oit_walk<FAST, false, REC4, DEPTH>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, sum, ListStep(share.per * WAVES, share.per));
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
             [&](float *to) {
                 to += lane;

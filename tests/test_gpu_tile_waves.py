@@ -5,6 +5,7 @@ import torch
 
 from htgs_amd.synthetic import make_scene
 from htgs_amd.torch_bindings import FrameBuffers, RasterizerMode
+from util import tie_scene
 
 pytestmark = pytest.mark.gpu
 
@@ -70,3 +71,23 @@ def test_training_records(cuda, kind, mode, K, waves):
     if mode in (0, 3):
         x, y = one.records_in_image_order(one.tail_info), four.records_in_image_order(four.tail_info)
         assert ((x - y).abs() <= 1e-5 * (1.0 + x.abs())).all()
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 64, 65, 127, 128, 129, 256, 257, 300, 513])
+@pytest.mark.parametrize("mode", [0, 1, 3])
+def test_shares(cuda, mode, n):
+    """Lists of exactly n instances, around the lengths at which a wave more gets a batch, the batches grow or there is a round more:
+    every instance is walked once.  Bounds as in test_image_and_depth."""
+    g = torch.Generator().manual_seed(n)
+    scene = tie_scene((2.0 + 30.0 * torch.rand(n, generator=g)).tolist(), (0.06 + 0.3 * torch.rand(n, generator=g)).tolist(), torch.rand(n, 3, generator=g).tolist()).to(cuda)
+    for K in (4, 16) if mode != 3 else (1,):
+        s = scene.settings(RasterizerMode(mode), K)
+        one = FrameBuffers(*scene.gaussians(), s, True, False)
+        image, depth = one.run()
+        assert int((one.ranges[:, 1] - one.ranges[:, 0]).max()) == n
+        trained = FrameBuffers(*scene.gaussians(), s, True, False, train=True).run_forward()
+        for waves in (2, 4):
+            print(f"case mode={mode} n={n} K={K} waves={waves}", flush=True)
+            image4, depth4 = FrameBuffers(*scene.gaussians(), s, True, False, waves_per_tile=waves).run()
+            assert (image4 - image).abs().max() < 2e-6 and (depth4 - depth).abs().max() < 5e-5
+            assert (FrameBuffers(*scene.gaussians(), s, True, False, train=True, waves_per_tile=waves).run_forward() - trained).abs().max() < 2e-6
