@@ -3,6 +3,7 @@
 import torch
 
 from .. import _native
+from .rasterization import current_stream_handle
 
 
 def update_3d_filter(
@@ -30,4 +31,4 @@ def update_3d_filter(
     _native.check(_native.lib().htgs_update_3d_filter(
         positions.data_ptr(), w2c.data_ptr(), filter_3d.data_ptr(), visibility_mask.data_ptr(), n, int(width), int(height),
         float(focal_x), float(focal_y), float(center_x), float(center_y), float(near_plane), float(clipping_tolerance),
-        float(distance2filter), torch.cuda.current_stream(positions.device).cuda_stream))
+        float(distance2filter), current_stream_handle(positions.device)))

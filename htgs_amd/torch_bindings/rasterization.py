@@ -63,6 +63,12 @@ def _ptr(t: Optional[torch.Tensor]) -> int:
     return 0 if t is None or t.numel() == 0 else t.data_ptr()
 
 
+def current_stream_handle(device: torch.device) -> int:
+    """``torch.cuda.current_stream(device).cuda_stream`` without the Python object around it, which is 8 us of a call (three of them in a
+    training step of 200 us that the host decides)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
+
+
 MAX_INSTANCES = 0xfffffffe
 
 
@@ -122,7 +128,7 @@ class ScratchPool:
 
     @staticmethod
     def _stream_id(device: torch.device) -> int:
-        return torch.cuda.current_stream(device).cuda_stream if device.type == "cuda" else 0
+        return current_stream_handle(device) if device.type == "cuda" else 0
 
     @classmethod
     def current(cls, device: torch.device) -> "ScratchPool":
@@ -409,6 +415,18 @@ class FrameBuffers:
         _native.check(self.lib.htgs_preprocess_backward(self._ref))
 
 
+# grad_image ... densification_info, densification_rows, use_distance_scaling: what a backward pass adds
+_FRAME_BACKWARD = struct.Struct("=10Q2i")
+_FRAME_BACKWARD_AT = _native.Frame.grad_image.offset
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _gradient_of(t: Optional[torch.Tensor], shape: tuple, f32: dict) -> torch.Tensor:
+    """An uninitialised gradient of that shape (like its input, which is there already, at half the cost: 2 us each)."""
+    alike = type(t) in _PLAIN and t.shape == shape and t.dtype is f32["dtype"] and t.device == f32["device"] and t.is_contiguous()
+    return torch.empty_like(t) if alike else torch.empty(shape, **f32)
+
+
 # positions ... cam_position, n_primitives ... height, near_plane, far_plane, scale_modifier: the head of ``htgs_frame``
 _FRAME_HEAD = struct.Struct("=9Q7i3f")
 _UINT8 = torch.uint8
@@ -530,12 +548,13 @@ class _TrainingFrame:
     def backward(self, grad_image, densification_info, use_distance_scaling):
         if self.fallback is not None:
             return self.fallback.run_backward(grad_image, densification_info, use_distance_scaling)
-        return _run_backward(self.frame, self.selector, self.device, grad_image, densification_info, use_distance_scaling)[0]
+        return _run_backward(self.frame, self.selector, self.device, grad_image, densification_info, use_distance_scaling, self.keep)[0]
 
 
 def _run_backward(f: "_native.Frame", selector: int, dev: torch.device, grad_image: torch.Tensor, densification_info: Optional[torch.Tensor],
-                  use_distance_scaling: bool):
-    """The six gradients of the training frame ``f``, and the other buffers its pointers lead to afterwards."""
+                  use_distance_scaling: bool, inputs=(None,) * 6):
+    """The six gradients of the training frame ``f``, and the other buffers its pointers lead to afterwards.  ``inputs``: its six Gaussian
+    tensors first, if at hand."""
     n, total_sh, n_instances = f.n_primitives, f.total_sh_bases, f.n_instances
     grad_image = _dev_f32(grad_image, "grad_image", dev)
     if tuple(grad_image.shape) != (3, f.height, f.width):
@@ -543,11 +562,8 @@ def _run_backward(f: "_native.Frame", selector: int, dev: torch.device, grad_ima
     f32 = dict(dtype=torch.float32, device=dev)
     # one row per instance, every one written by the blend kernels: no initialisation needed
     grad_rows = torch.empty((max(n_instances, 1), 16), **f32)
-    grads = [torch.empty((n, 3), **f32), torch.empty((n, 3), **f32), torch.empty((n, 4), **f32), torch.empty((n, 1), **f32),
-             torch.empty((n, 1, 3), **f32), torch.empty((n, total_sh, 3), **f32)]
+    grads = [_gradient_of(t, shape, f32) for t, shape in zip(inputs, ((n, 3), (n, 3), (n, 4), (n, 1), (n, 1, 3), (n, total_sh, 3)))]
     f.stream = ScratchPool._stream_id(dev)
-    f.grad_image, f.grad_rows = _ptr(grad_image), grad_rows.data_ptr()
-    (f.grad_positions, f.grad_scales, f.grad_rotations, f.grad_opacities, f.grad_sh_0, f.grad_sh_rest) = [_ptr(g) for g in grads]
     rows, helper = 0, None
     if densification_info is not None and densification_info.numel() > 0:
         rows = int(densification_info.shape[0])
@@ -556,10 +572,8 @@ def _run_backward(f: "_native.Frame", selector: int, dev: torch.device, grad_ima
             raise RuntimeError("densification_info must be a contiguous float32 [2,N] or [3,N] tensor on the GPU")
         if rows == 3:
             helper = torch.empty(max(n_instances, 1), **f32)
-    f.densification_info = densification_info.data_ptr() if rows else 0
-    f.densification_rows = rows
-    f.dens_helper = _ptr(helper)
-    f.use_distance_scaling = int(bool(use_distance_scaling))
+    _FRAME_BACKWARD.pack_into(f, _FRAME_BACKWARD_AT, _ptr(grad_image), grad_rows.data_ptr(), _ptr(helper), *[_ptr(g) for g in grads],
+                              densification_info.data_ptr() if rows else 0, rows, bool(use_distance_scaling))
     _native.check(_native.lib().htgs_backward(ctypes.byref(f), selector))
     return grads, (grad_image, grad_rows, helper)
 

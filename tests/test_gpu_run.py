@@ -11,7 +11,7 @@ import torch
 from htgs_amd import _native
 from htgs_amd.synthetic import make_scene
 from htgs_amd.torch_bindings import FrameBuffers, RasterizerMode, diff_rasterize, fast_rasterize, rasterize, update_max_weights
-from htgs_amd.torch_bindings.rasterization import ScratchPool, run_max_weights
+from htgs_amd.torch_bindings.rasterization import ScratchPool, current_stream_handle, run_max_weights
 
 pytestmark = pytest.mark.gpu
 
@@ -282,3 +282,28 @@ def test_stages_like_a_pass(cuda, mode, fast):
     n, waves = frame.n_instances, frame.waves_per_tile
     fb = FrameBuffers.like(frame, *scene.gaussians(), s, True, False, fast=fast)
     assert torch.equal(fb.run()[0], image) and fb.n_instances == n and fb.frame.waves_per_tile == waves
+
+
+def test_current_stream_handle(cuda):
+    """The stream that a pass is queued on: torch's current one, of the device asked for, with or without an index."""
+    for device in (cuda, torch.device("cuda")):
+        assert current_stream_handle(device) == torch.cuda.current_stream(device).cuda_stream
+        side = torch.cuda.Stream(device)
+        with torch.cuda.stream(side):
+            assert current_stream_handle(device) == side.cuda_stream != 0
+        assert current_stream_handle(device) == torch.cuda.current_stream(device).cuda_stream
+
+
+@pytest.mark.parametrize("parameters", [False, True])
+def test_gradients_are_plain_contiguous_tensors(cuda, parameters):
+    """Gradients laid out as documented whatever the inputs are: parameters, tensors, views with odd strides of dimensions of one."""
+    scene = make_scene(1, 300).to(cuda)
+    given = [t.requires_grad_() for t in scene.gaussians()]
+    if parameters:
+        given = [torch.nn.Parameter(t.detach()) for t in given]
+    else:
+        given[3] = torch.as_strided(given[3].detach(), (300, 1), (1, 7)).requires_grad_()
+        given[4] = torch.as_strided(given[4].detach(), (300, 1, 3), (3, 11, 1)).requires_grad_()
+    image = diff_rasterize(*given, torch.empty(0, device=cuda), scene.settings(RasterizerMode(0), 4), False)
+    for t, grad in zip(given, torch.autograd.grad(image, given, torch.ones_like(image))):
+        assert type(grad) is torch.Tensor and grad.shape == t.shape and grad.is_contiguous() and not grad.requires_grad
