@@ -51,7 +51,7 @@ __device__ __forceinline__ int find_core_slot(const uint32_t *__restrict__ keys,
 // (R/include/alpha_blend_first_k/kernels/backward.cuh:60-206); walking the tile's list and looking each
 // (Gaussian, pixel) up in the stored core visits the same fragments.
 // ---------------------------------------------------------------------------------------------
-// A workgroup is four waves sharing one tile's per-pixel terms and a chunk of 256 instances in LDS (25 KB for K = 16); the
+// A workgroup is four waves sharing one tile's per-pixel terms and a chunk of 256 instances in LDS (17 KB for K = 16); the
 // waves take the turns of the chunk one after the other.
 constexpr int kBackwardWaves = 4;
 
@@ -202,15 +202,19 @@ constexpr uint32_t kTurnPairs = 61;
 // densification row (HELPER) is a sum of absolute values per fragment and cannot go through the moments: it takes
 // the fourth components of the fragment's dL/dVPMT rows, which need m and the two plane normals at the pixel.
 // ---------------------------------------------------------------------------------------------
-// LDS of a workgroup of the kernels below
+// LDS of a workgroup of the kernels below.  A slot of a core is its weight and dL/dalpha alone, and the pixel's gradient is read beside it:
+// 17 KB for K = 16 and 29 for K = 32, where the products of the two took 25 and 46, with which a compute unit held three
+// workgroups.  Where the registers allow no more of them at a time, room in LDS still counts: two of a workgroup's waves are
+// often done before the others, and the next one then starts in their place.  Training steps: K = 32, 1 M Gaussians at 1920x1080, HYBRID
+// 2682 -> 2288 us, FIRST_K 1933 -> 1659; K = 16 HYBRID 1598 -> 1577, 100 k at 1280x720 FIRST_K 300 -> 295.
 template <int K, bool HELPER>
 struct BackwardTileTerms {
     static constexpr int KS = K > 0 ? K : 1;
     // per-pixel terms, pixels in the order and with the skew of pixel_slot (one 16-byte word per quadrant)
     __attribute__((aligned(16))) uint32_t s_idx[64 * KS + 16];      // [pixel][slot]: Gaussian << 5 | slot
-    float4 s_core[64 * KS + 4];   // (weight * g, dC/dalpha . g)
-    float4 s_tail[64 + 4];        // (full weight * g, common)
-    float s_tail_a[64 + 4];
+    float4 s_grad[64 + 4];        // upstream gradient, the tail's full weight
+    float2 s_core[64 * KS + 4];   // (weight, dC/dalpha . g)
+    float2 s_tail[64 + 4];        // what is added to dL/dalpha in the tail: (common, the part that is divided by 1 - alpha)
     float s_pos[HELPER ? 64 : 1][6];   // per pixel: (dL/dpx.w, dL/dpy.w) of a fragment -> its dL/dposition
     uint32_t s_g[64 * kBackwardWaves];         // the Gaussians of the chunk
     uint16_t s_pairs[kBackwardWaves][256];     // by the wave that staged them: (thread << 4 | quadrant << 2 | number among the Gaussian's pairs)
@@ -229,8 +233,8 @@ __device__ __forceinline__ void backward_tile(BackwardTileTerms<K, HELPER> &lds,
     constexpr bool kHasTail = MODE != HTGS_MODE_ALPHA_BLEND_FIRST_K;
     constexpr int KS = K > 0 ? K : 1;
     uint32_t *const s_idx = lds.s_idx;
-    float4 *const s_core = lds.s_core, *const s_tail = lds.s_tail;
-    float *const s_tail_a = lds.s_tail_a;
+    float4 *const s_grad = lds.s_grad;
+    float2 *const s_core = lds.s_core, *const s_tail = lds.s_tail;
     float (*const s_pos)[6] = lds.s_pos;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t x0 = (tile % grid_w) * 8, y0 = (tile / grid_w) * 8;
@@ -287,19 +291,18 @@ __device__ __forceinline__ void backward_tile(BackwardTileTerms<K, HELPER> &lds,
         float g0 = 0.0f, g1 = 0.0f, g2 = 0.0f;
         if (inside) { g0 = grad_image[pix]; g1 = grad_image[np + pix]; g2 = grad_image[2 * np + pix]; }
         if (wave == 0) {
-            float4 tail = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            float tail_a = 0.0f;
+            float full = 0.0f;
+            float2 tail = make_float2(0.0f, 0.0f);
             if (inside && kHasTail) {
                 const float r0 = tail_info[rp], r1 = tail_info[rnp + rp], r2 = tail_info[2 * rnp + rp];
                 const float asr = tail_info[3 * rnp + rp], T_tail = tail_info[4 * rnp + rp], T_core = tail_info[5 * rnp + rp];
                 const float w_tail = T_core * asr;                                   // backward.cuh:166
-                const float full = w_tail * (1.0f - T_tail);                         // :168
+                full = w_tail * (1.0f - T_tail);                                     // :168
                 const float rdg = r0 * g0 + r1 * g1 + r2 * g2;
-                tail = make_float4(full * g0, full * g1, full * g2, -full * asr * rdg);   // :170-172
-                tail_a = w_tail * T_tail * rdg;                                      // :173
+                tail = make_float2(-full * asr * rdg, w_tail * T_tail * rdg);        // :170-173
             }
+            s_grad[ps + pq] = make_float4(g0, g1, g2, full);
             s_tail[ps + pq] = tail;
-            s_tail_a[ps + pq] = tail_a;
             if (HELPER) {
                 // dL/dVPMT4.w = -x dL/dpx.w - y dL/dpy.w (:288), and dL/dposition = VPM[:, :3]^T of the three w components (:292-305)
                 const float fx = (float)x, fy = (float)y;
@@ -316,11 +319,11 @@ __device__ __forceinline__ void backward_tile(BackwardTileTerms<K, HELPER> &lds,
                 const int i = i0 + (int)wave;
                 if (i < KS) {
                     uint32_t idx = 0xffffffffu;
-                    float4 c = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    float2 c = make_float2(0.0f, 0.0f);
                     if (inside) {
                         idx = core_idx[(size_t)i * rnp + rp];
                         const float4 info = core_info[(size_t)i * rnp + rp];
-                        c = make_float4(info.w * g0, info.w * g1, info.w * g2, info.x * g0 + info.y * g1 + info.z * g2);   // :154-155
+                        c = make_float2(info.w, info.x * g0 + info.y * g1 + info.z * g2);   // :154-155
                     }
                     s_idx[ps * KS + 4 * pq + i] = idx == 0xffffffffu ? idx : (idx << kSlotBits) | (uint32_t)i;
                     s_core[ps * KS + pq + i] = c;
@@ -419,18 +422,20 @@ __device__ __forceinline__ void backward_tile(BackwardTileTerms<K, HELPER> &lds,
                         slot = find_core_slot<KS>(s_idx + p * KS + 4u * quadrant, g);                   // :231-235
                     }
                     if (!kHasTail && slot < 0) continue;                                   // FIRST_K: only stored fragments carry gradient
-                    float dL_dalpha;
+                    const float4 grad = s_grad[p + quadrant];
+                    float weight, dL_dalpha;
                     if (slot >= 0) {
-                        const float4 t = s_core[p * KS + slot + quadrant];
-                        a0 += t.x; a1 += t.y; a2 += t.z;                                 // :241
-                        dL_dalpha = t.w;                                                 // :250
+                        const float2 t = s_core[p * KS + slot + quadrant];
+                        weight = t.x;                                                    // :241
+                        dL_dalpha = t.y;                                                 // :250
                     } else {
-                        const float4 t = s_tail[p + quadrant];
-                        a0 += t.x * alpha; a1 += t.y * alpha; a2 += t.z * alpha;         // :244
+                        const float2 t = s_tail[p + quadrant];
+                        weight = grad.w * alpha;                                         // :244
                         const float oma = 1.0f - alpha;
-                        dL_dalpha = t.w + (col.x * t.x + col.y * t.y + col.z * t.z)
-                                  + s_tail_a[p + quadrant] * rcp_refined(oma > kOneMinusAlphaEps ? oma : kOneMinusAlphaEps);   // :253-255; [1e-8, 1] is inside the refined reciprocal's exact range
+                        dL_dalpha = t.x + grad.w * (col.x * grad.x + col.y * grad.y + col.z * grad.z)
+                                  + t.y * rcp_refined(oma > kOneMinusAlphaEps ? oma : kOneMinusAlphaEps);   // :253-255; [1e-8, 1] is inside the refined reciprocal's exact range
                     }
+                    a0 = __builtin_fmaf(weight, grad.x, a0); a1 = __builtin_fmaf(weight, grad.y, a1); a2 = __builtin_fmaf(weight, grad.z, a2);
                     if (dL_dalpha == 0.0f) continue;                                     // :258
                     a_op += dL_dalpha * G;                                               // :262
                     // rho^2 = num / (kc den) with num = kc |m|^2:  dL/dnum and dL/dden  (:263-266)
@@ -489,8 +494,10 @@ __device__ __forceinline__ void backward_tile(BackwardTileTerms<K, HELPER> &lds,
     }
 }
 
+// (Four waves per SIMD with the third row, which takes 128 registers for up to four that spill: 1 M at 1920x1080, HYBRID K = 16, 2044 -> 1844 us with
+// the LDS above, 500 k at 1280x720, K = 32, 1102 -> 976.)
 template <int K, int MODE, bool HELPER>
-__global__ void __launch_bounds__(64 * kBackwardWaves) __attribute__((amdgpu_waves_per_eu(HELPER ? 3 : 5))) blend_tail_backward_moments_kernel(
+__global__ void __launch_bounds__(64 * kBackwardWaves) __attribute__((amdgpu_waves_per_eu(HELPER ? 4 : 5))) blend_tail_backward_moments_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
     const uint32_t *__restrict__ core_idx, const float4 *__restrict__ core_info, const float *__restrict__ tail_info,
     const float *__restrict__ grad_image, const float *__restrict__ VPM, float4 *__restrict__ grad_rows, float *__restrict__ helper_rows,
