@@ -202,21 +202,81 @@ constexpr uint32_t kTurnPairs = 61;
 // densification row (HELPER) is a sum of absolute values per fragment and cannot go through the moments: it takes
 // the fourth components of the fragment's dL/dVPMT rows, which need m and the two plane normals at the pixel.
 // ---------------------------------------------------------------------------------------------
+// ALPHA_BLEND_FIRST_K: the quadrants of the tile in whose cores a Gaussian of the chunk is at all.  The others' pixels have nothing for it,
+// however much of them it covers, and what is behind every core, most of a long list, has a row of zeros without being
+// evaluated.  The chunk's Gaussians are entered into a hash table of chains, and every entry of the cores is looked up in it.
+// Training steps: 1 M Gaussians at 1920x1080 K = 16 1068 -> 1010 us, K = 4 816 -> 735, three rows 500 k at 1280x720 K = 4 417 -> 381, 600 k of the
+// stress scene at 1600x1066 1500 -> 1416.
+struct CoreMembers {
+    static constexpr uint32_t kEnd = 256;
+    uint32_t head[256];                    // of the chain of a hash: thread, kEnd: none
+    uint32_t quadrants[256];
+    uint16_t next[256 + 2];                // (of kEnd: kEnd)
+    uint32_t full;                         // pixels whose cores are full
+    static __device__ __forceinline__ uint32_t hash(uint32_t g) { return (g * 0x9e3779b1u) >> 24; }
+    // all threads, a barrier between one step and the next
+    __device__ __forceinline__ void clear(uint32_t thread)
+    {
+        head[thread] = kEnd;
+        quadrants[thread] = 0u;
+        if (thread == 0u) next[kEnd] = (uint16_t)kEnd;
+    }
+    __device__ __forceinline__ void enter(uint32_t thread, uint32_t g) { next[thread] = (uint16_t)atomicExch(&head[hash(g)], thread); }
+    // chunk[thread]: its Gaussian (a word more may be read); keys: the cores, Gaussian << kSlotBits | slot, in the order of s_idx
+    template <int KS>
+    __device__ __forceinline__ void mark(const uint32_t *__restrict__ chunk, const uint32_t *__restrict__ keys, uint32_t thread)
+    {
+        constexpr int kAtOnce = KS >= 16 ? 4 : KS >= 8 ? 2 : 1;         // entries of a thread that are looked up side by side
+#pragma unroll
+        for (uint32_t e = 0; e < 64u * KS; e += 256u * kAtOnce) {
+            if (64u * KS < 256u && thread >= 64u * KS) break;
+            uint32_t g[kAtOnce], t[kAtOnce];
+            bool more = false;
+#pragma unroll
+            for (int k = 0; k < kAtOnce; ++k) {
+                const uint32_t at = e + 256u * k + thread, key = keys[at + 4u * (at / (16u * KS))];
+                g[k] = key == 0xffffffffu ? 0xffffffffu : key >> kSlotBits;
+                t[k] = key == 0xffffffffu ? kEnd : head[hash(g[k])];
+                more = more || t[k] != kEnd;
+            }
+            while (more) {
+                more = false;
+#pragma unroll
+                for (int k = 0; k < kAtOnce; ++k) {
+                    const uint32_t held = chunk[t[k]], after = next[t[k]];
+                    const bool found = t[k] != kEnd && held == g[k];
+                    if (found) atomicOr(&quadrants[t[k]], 1u << ((e + 256u * k + thread) / (16u * KS)));
+                    t[k] = found ? kEnd : after;
+                    more = more || t[k] != kEnd;
+                }
+            }
+        }
+    }
+};
+struct NoCoreMembers {};
+template <bool YES> struct CoreMembersIf { using type = CoreMembers; };
+template <> struct CoreMembersIf<false> { using type = NoCoreMembers; };
+// The members are looked for in lists of this many instances and more, if this many of the tile's 64 cores are full: what is not full holds all that
+// its pixel has, and nothing would be left out.  (300 k at 800x600, K = 16, lists of 88 with half-empty cores: 306 -> 305 us; K = 32 at
+// 1920x1080, where lists are hardly longer than that: 1660 -> 1666.)
+template <int K> constexpr uint32_t kMembersList = 4u * K;
+constexpr uint32_t kMembersFull = 32u;
 // LDS of a workgroup of the kernels below.  A slot of a core is its weight and dL/dalpha alone, and the pixel's gradient is read beside it:
 // 17 KB for K = 16 and 29 for K = 32, where the products of the two took 25 and 46, with which a compute unit held three
 // workgroups.  Where the registers allow no more of them at a time, room in LDS still counts: two of a workgroup's waves are
 // often done before the others, and the next one then starts in their place.  Training steps: K = 32, 1 M Gaussians at 1920x1080, HYBRID
 // 2682 -> 2288 us, FIRST_K 1933 -> 1659; K = 16 HYBRID 1598 -> 1577, 100 k at 1280x720 FIRST_K 300 -> 295.
-template <int K, bool HELPER>
+template <int K, int MODE, bool HELPER>
 struct BackwardTileTerms {
     static constexpr int KS = K > 0 ? K : 1;
+    typename CoreMembersIf<MODE == HTGS_MODE_ALPHA_BLEND_FIRST_K>::type members;
     // per-pixel terms, pixels in the order and with the skew of pixel_slot (one 16-byte word per quadrant)
     __attribute__((aligned(16))) uint32_t s_idx[64 * KS + 16];      // [pixel][slot]: Gaussian << 5 | slot
     float4 s_grad[64 + 4];        // upstream gradient, the tail's full weight
     float2 s_core[64 * KS + 4];   // (weight, dC/dalpha . g)
     float2 s_tail[64 + 4];        // what is added to dL/dalpha in the tail: (common, the part that is divided by 1 - alpha)
     float s_pos[HELPER ? 64 : 1][6];   // per pixel: (dL/dpx.w, dL/dpy.w) of a fragment -> its dL/dposition
-    uint32_t s_g[64 * kBackwardWaves];         // the Gaussians of the chunk
+    uint32_t s_g[64 * kBackwardWaves + 1];     // the Gaussians of the chunk
     uint16_t s_pairs[kBackwardWaves][256];     // by the wave that staged them: (thread << 4 | quadrant << 2 | number among the Gaussian's pairs)
     uint32_t s_count[kBackwardWaves];          // and their numbers
 };
@@ -224,7 +284,7 @@ struct BackwardTileTerms {
 // taken in chunks of 256.  Every instance writes a gradient row of its own, so a list may be cut anywhere
 // and its pieces given to different workgroups.  (All threads; the caller synchronises before the LDS is used again.)
 template <int K, int MODE, bool HELPER>
-__device__ __forceinline__ void backward_tile(BackwardTileTerms<K, HELPER> &lds, uint32_t tile, uint32_t first, uint32_t last, uint32_t n_tiles,
+__device__ __forceinline__ void backward_tile(BackwardTileTerms<K, MODE, HELPER> &lds, uint32_t tile, uint32_t first, uint32_t last, uint32_t n_tiles,
     const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
     const uint32_t *__restrict__ core_idx, const float4 *__restrict__ core_info, const float *__restrict__ tail_info,
     const float *__restrict__ grad_image, const float *__restrict__ VPM, float4 *__restrict__ grad_rows, float *__restrict__ helper_rows,
@@ -242,18 +302,43 @@ __device__ __forceinline__ void backward_tile(BackwardTileTerms<K, HELPER> &lds,
     const float cx = tile_centre(x0, 8), cy = tile_centre(y0, 8);
     const TilePlace place = tile_place(tile, grid_w);
     const auto inst_at = [&](uint32_t base) { return base + threadIdx.x < last ? inst[base + threadIdx.x] : 0u; };
+    bool members = !kHasTail && last - first >= kMembersList<KS>;        // (the same in all threads)
+    if constexpr (!kHasTail)
+        if (members) {
+            lds.members.clear(threadIdx.x);
+            __syncthreads();
+        }
     // ---- staging: thread = Gaussian (g, the list's entry at base + thread) ----
     const auto stage = [&](uint32_t base, uint32_t g) {
-        uint32_t reach = 0;
-        if (base + threadIdx.x < last) {
-            const float4 *rec = prim + (size_t)g * kTrainRec4;
-            TileGeometry t;
-            float qn[6], qd[6];
-            tile_geometry(rec[0], rec[1], rec[2], cx, cy, t);
-            tile_quadratics<MODE>(t, qn, qd);
-            reach = tile_quadrant_hits<MODE>(qn, qd, rec[HTGS_PRIM_FLOATS / 4 - 1].w);
-            lds.s_g[threadIdx.x] = g;
-            if (reach == 0) {                            // reaches no pixel of the tile: its row is zeros
+        uint32_t reach = 0, wanted = 0xfu;
+        const bool listed = base + threadIdx.x < last;
+        if (listed) lds.s_g[threadIdx.x] = g;
+        // (on their way while the members are looked for)
+        const float4 *const rec = prim + (size_t)g * kTrainRec4;
+        float4 V1, V2, V4;
+        float opacity = 0.0f;
+        V1 = V2 = V4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (listed) { V1 = rec[0]; V2 = rec[1]; V4 = rec[2]; opacity = rec[HTGS_PRIM_FLOATS / 4 - 1].w; }
+        if constexpr (!kHasTail)
+            if (members) {
+                if (listed) lds.members.enter(threadIdx.x, g);
+                __syncthreads();                         // (in the first chunk the cores are there, too)
+                members = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.members.full) >= kMembersFull;
+                if (members) {
+                    lds.members.template mark<KS>(lds.s_g, s_idx, threadIdx.x);
+                    __syncthreads();
+                    wanted = lds.members.quadrants[threadIdx.x];
+                }
+            }
+        if (listed) {
+            if (wanted != 0u) {
+                TileGeometry t;
+                float qn[6], qd[6];
+                tile_geometry(V1, V2, V4, cx, cy, t);
+                tile_quadratics<MODE>(t, qn, qd);
+                reach = tile_quadrant_hits<MODE>(qn, qd, opacity) & wanted;
+            }
+            if (reach == 0) {                            // adds to no pixel of the tile: its row is zeros
                 const uint32_t slot = instance_slot(prim, g, place);
                 float4 *row = grad_rows + 4 * (size_t)slot;
                 const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -327,6 +412,11 @@ __device__ __forceinline__ void backward_tile(BackwardTileTerms<K, HELPER> &lds,
                     }
                     s_idx[ps * KS + 4 * pq + i] = idx == 0xffffffffu ? idx : (idx << kSlotBits) | (uint32_t)i;
                     s_core[ps * KS + pq + i] = c;
+                    if constexpr (!kHasTail)
+                        if (i == KS - 1) {
+                            const uint64_t full = __ballot(idx != 0xffffffffu);
+                            if (lane == 0) lds.members.full = (uint32_t)__popcll(full);
+                        }
                 }
             }
         }
@@ -337,6 +427,11 @@ __device__ __forceinline__ void backward_tile(BackwardTileTerms<K, HELPER> &lds,
     for (uint32_t base = first; base < last; base += 64u * kBackwardWaves) {
         if (base != first) {
             __syncthreads();                             // (the chunk before is read)
+            if constexpr (!kHasTail)
+                if (members) {
+                    lds.members.clear(threadIdx.x);
+                    __syncthreads();
+                }
             stage(base, inst_at(base));
             __syncthreads();
         }
@@ -504,7 +599,7 @@ __global__ void __launch_bounds__(64 * kBackwardWaves) __attribute__((amdgpu_wav
     uint32_t width, uint32_t height, uint32_t grid_w, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ long_tiles, ListThreshold threshold,
     uint32_t part_floor)
 {
-    __shared__ BackwardTileTerms<K, HELPER> lds;
+    __shared__ BackwardTileTerms<K, MODE, HELPER> lds;
     const uint32_t tile = block_tile(tile_order);
     const uint32_t first = ranges[2 * tile], last = ranges[2 * tile + 1];
     if (first == last) return;               // nothing was drawn into this tile (whole workgroup)
@@ -530,7 +625,7 @@ __global__ void __launch_bounds__(64 * kBackwardWaves) __attribute__((amdgpu_wav
     const float *__restrict__ grad_image, const float *__restrict__ VPM, float4 *__restrict__ grad_rows, float *__restrict__ helper_rows,
     uint32_t width, uint32_t height, uint32_t grid_w, const uint32_t *long_tiles, ListThreshold threshold)
 {
-    __shared__ BackwardTileTerms<K, HELPER> lds;
+    __shared__ BackwardTileTerms<K, MODE, HELPER> lds;
     __shared__ uint32_t s_next;
     if (long_tiles[0] == 0) return;                   // (the ordinary frame)
     const uint32_t long_threshold = threshold.get(long_tiles);

@@ -92,3 +92,11 @@ def test_rows_of_a_gaussian_are_added_up(cuda, n):
     drawn = torch.from_numpy(counts > 0)
     start = torch.from_numpy(ends - counts)[drawn]
     assert torch.equal(results[0][3].reshape(-1).cpu()[drawn], sums[start, 3]) and torch.equal(results[0][6][2].cpu()[drawn], total[start])
+
+
+@pytest.mark.parametrize("K", [1, 2, 8, 16, 32])
+@pytest.mark.parametrize("kind,times,more", [("wide", 4, -1), ("wide", 4, 0), ("mixed", 8, 0), ("wide", 0, 256), ("mixed", 0, 257), ("wide", 0, 770)])
+def test_gradients_of_core_members(cuda, kind, times, more, K):
+    """ALPHA_BLEND_FIRST_K leaves out what is in no core of a quadrant, in lists from 4 K on, a chunk of 256 at a time."""
+    for rows in (2, 3):
+        test_gradients_around_turns_and_chunks(cuda, kind, times * K + more, 1, K, rows)
