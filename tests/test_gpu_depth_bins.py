@@ -121,9 +121,9 @@ def test_training(cuda, kind, mode, K, waves, threshold):
 
 @pytest.mark.parametrize("mode", [HYBRID, FIRST_K])
 def test_operators(cuda, mode):
-    """170 000 Gaussians, a third of them twins: the operators take bins, and come to what the stages by index come to."""
+    """340 000 Gaussians, a third of them twins, on a grid of one wave a tile: the operators take bins, and come to what the stages by index come to."""
     print(f"case mode={mode}", flush=True)
-    sg = with_twins(small_view(make_scene(1, 120_000), 400, 304), 50_000).to(cuda)
+    sg = with_twins(small_view(make_scene(1, 240_000), 1300, 1000), 100_000).to(cuda)
     s = sg.settings(RasterizerMode(mode), 16)
     image, depth = rasterize(*sg.gaussians(), s, True, False)
     assert ScratchPool.current(cuda).frame.depth_bins
@@ -133,7 +133,7 @@ def test_operators(cuda, mode):
     assert step.grad_fn.fb.frame.depth_bins
     by_index = frame(sg, mode, 16, False, train=True, long_list_threshold=2 ** 31 - 1)
     assert (step.detach() - by_index.run_forward()).abs().max() < 4e-6
-    weights, by_stages = torch.zeros(170_000, device=cuda), torch.zeros(170_000, device=cuda)
+    weights, by_stages = torch.zeros(340_000, device=cuda), torch.zeros(340_000, device=cuda)
     with torch.no_grad():
         update_max_weights(weights, *[t.detach() for t in sg.gaussians()[:4]], s, 0.02)
         run_max_weights(by_stages, *[t.detach() for t in sg.gaussians()[:4]], s, 0.02, long_list_threshold=2 ** 31 - 1)
@@ -143,3 +143,14 @@ def test_operators(cuda, mode):
         # (a weight within rounding of the threshold may fall on the other side of it)
         both = (weights > 0) & (by_stages > 0)
         assert ((weights - by_stages).abs()[both] <= 1e-5 * by_stages[both]).all() and int((both != ((weights > 0) | (by_stages > 0))).sum()) <= 2
+
+
+@pytest.mark.parametrize("width,height,n,bins", [(640, 480, 340_000, False), (1300, 1000, 199_999, False), (1300, 1000, 340_000, True)])
+def test_lines(cuda, width, height, n, bins):
+    """Grids that four waves share a tile of take no bins at these sizes; what the operators return does not depend on it."""
+    sg = small_view(make_scene(1, n), width, height).to(cuda)
+    s = sg.settings(RasterizerMode(HYBRID), 16)
+    image, depth = rasterize(*sg.gaussians(), s, True, False)
+    assert bool(ScratchPool.current(cuda).frame.depth_bins) == bins
+    want, want_depth = frame(sg, HYBRID, 16, False, long_list_threshold=2 ** 31 - 1).run()
+    assert (image - want).abs().max() < 4e-6 and (depth[0] - want_depth).abs().max() < 1e-4
