@@ -695,7 +695,14 @@ __device__ __forceinline__ void quadrant_sum_16(float (&v)[16])
     }
 }
 
-constexpr int kGlobalBatch = 32;              // Gaussians per staged batch (a bit each in a quadrant's hit mask); sized by the LDS the quadrants' sums take
+// Gaussians per staged batch, and (Gaussian, quadrant) pairs that there is room for: a batch is the Gaussians whose pairs fit, 27 of them at
+// least (sixteen quadrants each) and most often all 64.  The longer a batch, the fewer of a wave's turns serve less than four quadrants and
+// the fewer barriers a list takes; with room for every quadrant of every Gaussian 32 were the most that leave a compute unit four
+// workgroups (24: 6 to 10 % slower, 16: 13 to 26).  Training steps, 32 -> the pairs that fit: 411 k Gaussians at
+// 1297x839 708 -> 675 us, 1 M at 1920x1080 1460 -> 1404, 50 k at 269x922 558 -> 509, 200 k at 800x600 476 -> 445.
+constexpr int kGlobalBatch = 64;
+constexpr uint32_t kGlobalPairs = 432;
+static_assert(kGlobalPairs >= 16, "a Gaussian fits");
 // A wave holds one 8x8 sub-tile of the 16x16 tile and walks the hits of its own four 4x4 quadrants (subtile_walk): a turn
 // serves up to four Gaussians, one per quadrant, whose sixteen sums are taken over the quadrant's sixteen lanes and parked
 // in LDS per (quadrant, Gaussian); the thread that finishes a Gaussian adds the parts of the quadrants it can reach, in
@@ -710,9 +717,10 @@ __global__ void __launch_bounds__(256) blend_global_backward_kernel(
     __shared__ TileStage<kGlobalBatch> st;
     __shared__ float4 s_rows[4][kGlobalBatch];                // VPMT1, VPMT2, VPMT4 and the word that places the gradient row:
                                                               // fetched by the waves that do not stage, for the threads that finish the Gaussians
-    __shared__ float4 s_part[16][kGlobalBatch][4];            // per quadrant of the tile: the 16 sums of one Gaussian
-    __shared__ float s_help[HELPER ? 16 : 1][kGlobalBatch];
-    __shared__ uint16_t s_reach[kGlobalBatch];                // per staged Gaussian: the quadrants it can reach
+    __shared__ float4 s_part[kGlobalPairs + 1][4];            // per (Gaussian, quadrant it can reach): the 16 sums (one more is read, for nothing)
+    __shared__ float s_help[HELPER ? kGlobalPairs + 1 : 1];
+    __shared__ uint32_t s_pairs[kGlobalBatch];                // per staged Gaussian: its first pair << 16 | the quadrants it can reach
+    __shared__ uint32_t s_taken;                              // how many of the staged Gaussians are this batch
     __shared__ uint32_t s_walked;                             // bit w: wave w walked this batch (its pixels were not all opaque)
     const uint32_t tile = block_tile(tile_order);
     const uint32_t t = threadIdx.x;
@@ -756,24 +764,33 @@ __global__ void __launch_bounds__(256) blend_global_backward_kernel(
     };
     uint32_t base = first;
     fetch(base);
-    for (; base < last; base += kGlobalBatch) {
+    for (int nb = 0; base < last; base += (uint32_t)nb) {
         // (the barrier also separates the previous batch's reads of the rows and sums from the writes below)
         if (__syncthreads_count(done) == 256) break;
-        if (lane < (uint32_t)kGlobalBatch) {
-            if (wave == 0) {
-                s_reach[lane] = (uint16_t)reach_next;
-                if (lane == 0) s_walked = 0u;
-            } else {
-                s_rows[wave - 1][lane] = row_next;
-                if (wave == 3) s_rows[3][lane] = slot_next;
+        if (wave == 0) {
+            const uint32_t own = (uint32_t)__builtin_popcount(reach_next);
+            uint32_t upto = own;
+#pragma unroll
+            for (int d = 1; d < kWave; d <<= 1) {
+                const uint32_t v = (uint32_t)__shfl_up((int)upto, d, kWave);
+                if ((int)lane >= d) upto += v;
             }
+            const uint64_t fits = __ballot(upto <= kGlobalPairs);                // (the first of them)
+            s_pairs[lane] = upto <= kGlobalPairs ? (upto - own) << 16 | reach_next : 0u;
+            if (lane == 0) { s_walked = 0u; s_taken = (uint32_t)__popcll(fits); }
+        } else {
+            s_rows[wave - 1][lane] = row_next;
+            if (wave == 3) s_rows[3][lane] = slot_next;
         }
         __syncthreads();
-        const int nb = last - base < (uint32_t)kGlobalBatch ? (int)(last - base) : kGlobalBatch;
+        {
+            const uint32_t taken = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_taken);
+            nb = (int)(last - base < taken ? last - base : taken);
+        }
         const uint32_t stage_base = __builtin_amdgcn_readfirstlane(stage_address(st));
         if (__ballot(!done) != 0) {                                              // wave-uniform
             if (lane == 0) atomicOr(&s_walked, 1u << wave);
-            QuadrantHits hits = quadrant_ballot(lane < (uint32_t)kGlobalBatch ? ((uint32_t)s_reach[lane] >> (4u * wave)) & 0xfu : 0u);
+            QuadrantHits hits = quadrant_ballot((s_pairs[lane] >> (4u * wave)) & 0xfu);
             // Two turns at a time: what a fragment is without the transmittance, its alpha, is worked out for both together, two
             // chains of some forty dependent instructions side by side (training step of 411 k Gaussians at 1297x839: 810 -> 774 us,
             // of 51 k at 269x922: 826 -> 763).
@@ -863,8 +880,9 @@ __global__ void __launch_bounds__(256) blend_global_backward_kernel(
                     }
                 }
                 if ((lane & 3u) == 0u) {                                         // row r of the wave holds sums 4 r .. 4 r + 3
-                    s_part[quadrant][j][lane >> 4] = make_float4(acc[0], acc[1], acc[2], acc[3]);
-                    if (HELPER && lane < 16u) s_help[quadrant][j] = help;
+                    const uint32_t held = s_pairs[j], pair = (held >> 16) + (uint32_t)__builtin_popcount(held & ((1u << quadrant) - 1u));
+                    s_part[pair][lane >> 4] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+                    if (HELPER && lane < 16u) s_help[pair] = help;
                 }
             };
             while (quadrant_pending(hits)) {
@@ -875,22 +893,25 @@ __global__ void __launch_bounds__(256) blend_global_backward_kernel(
             }
         }
         __syncthreads();
-        if (base + kGlobalBatch < last) fetch(base + kGlobalBatch);
-        // Four lanes per Gaussian of the batch, of the last two waves: each adds up its four of the sixteen sums over the
+        if (base + (uint32_t)nb < last) fetch(base + (uint32_t)nb);
+        // Four lanes per Gaussian of the batch, from the last wave on: each adds up its four of the sixteen sums over the
         // quadrants, in their order (neighbouring lanes read neighbouring words of LDS, all of them at once), the four share
         // them, and each writes a quarter of the row.
-        if (t >= 128u && t - 128u < 4u * (uint32_t)nb) {
-            const uint32_t g = (t - 128u) >> 2, c = t & 3u;
-            const uint32_t reach = s_reach[g], walked = s_walked;
+        const uint32_t idle = 256u - 4u * (uint32_t)nb;
+        if (t >= idle) {
+            const uint32_t g = (t - idle) >> 2, c = t & 3u;
+            const uint32_t held = s_pairs[g], walked = s_walked;
             float own[4] = { 0.0f, 0.0f, 0.0f, 0.0f }, help = 0.0f;
             bool any = false;
+            uint32_t pair = held >> 16;
 #pragma unroll
             for (uint32_t qd = 0; qd < 16; ++qd) {
-                const bool counts = ((reach >> qd) & 1u) && ((walked >> (qd >> 2)) & 1u);
-                const float4 p = s_part[qd][g][c];
+                const bool reached = (held >> qd) & 1u, counts = reached && ((walked >> (qd >> 2)) & 1u);
+                const float4 p = s_part[pair][c];
                 own[0] += counts ? p.x : 0.0f; own[1] += counts ? p.y : 0.0f; own[2] += counts ? p.z : 0.0f; own[3] += counts ? p.w : 0.0f;
-                if (HELPER) { const float h = s_help[qd][g]; help += counts ? h : 0.0f; }
+                if (HELPER) { const float h = s_help[pair]; help += counts ? h : 0.0f; }
                 any = any || counts;
+                pair += reached ? 1u : 0u;
             }
             // (quad_perm: sums 4 r .. 4 r + 3 from lane r of the four)
             float m[16];

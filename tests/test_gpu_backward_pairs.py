@@ -100,3 +100,10 @@ def test_gradients_of_core_members(cuda, kind, times, more, K):
     """ALPHA_BLEND_FIRST_K leaves out what is in no core of a quadrant, in lists from 4 K on, a chunk of 256 at a time."""
     for rows in (2, 3):
         test_gradients_around_turns_and_chunks(cuda, kind, times * K + more, 1, K, rows)
+
+
+@pytest.mark.parametrize("rows", [2, 3])
+@pytest.mark.parametrize("kind,n", [("wide", 1), ("wide", 26), ("wide", 27), ("wide", 28), ("narrow", 63), ("narrow", 64), ("narrow", 65), ("mixed", 130), ("mixed", 400), ("wide", 200)])
+def test_gradients_around_batches_of_pairs(cuda, kind, n, rows):
+    """ALPHA_BLEND_GLOBAL_ORDERING takes 64 Gaussians at a time, or as many as have 432 (Gaussian, quadrant) pairs: 27 that reach all sixteen."""
+    test_gradients_around_turns_and_chunks(cuda, kind, n, 2, 1, rows)
