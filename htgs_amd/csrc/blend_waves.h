@@ -26,7 +26,7 @@ namespace htgs {
 // 20 k at 660x834, HYBRID K = 4, 232 -> 222 -> 219, of 244 k at 1694x265, K = 16, 317 -> 311.6 -> 310.
 // FIRST_K's waves know from one another how deep they have to look (SharedDepth), and merge more than they
 // spare below twice that (K = 4, 108 k at 451x862: 86.3 -> 85.4 -> 85.9).
-constexpr uint32_t least_share(int K, bool tail) { return (K <= 4 ? 8u : 16u) * (tail ? 1u : 2u); }
+constexpr uint32_t least_share(int K, bool tail) { return K > 16 ? 64u : (K <= 4 ? 8u : 16u) * (tail ? 1u : 2u); }
 struct TileShare {
     uint32_t first, per;                   // per: where the next wave's begins
 };
@@ -71,7 +71,7 @@ __device__ __forceinline__ bool tile_of_waves(const uint32_t *__restrict__ range
 
 // HYBRID_BLEND, the core as keys (inference)
 template <int WAVES, int K, bool FAST, typename Finish>
-__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 5 : 4))) blend_hybrid_waves_kernel(
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(K > 16 && !FAST ? 3 : K > 16 || (K == 16 && !FAST && WAVES == 4) ? 4 : 5))) blend_hybrid_waves_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
     uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const Finish finish)
 {
