@@ -126,13 +126,15 @@ static int waves_of(const htgs_frame *f, int what, uint64_t n_tiles)
 //     150 k 0.99, 400 k 1.01 to 1.03;  image alone  200 k 0.98, 500 k 1.03
 //   K = 8  400 k 0.93 to 1.0, 1 M 1.02 to 1.04 (1920x1080), 0.97 (640x480), 3 M 1.03 to 1.05;   K <= 4  0.92 (320 k) to 1.01 (3 M): never
 //   weights (one wave)  70 k 0.88 to 0.98 on all, 150 k 1.02 to 1.12 (400x400, 900x700), 0.94 to 0.98 (1920x1080), 400 k 0.99 to 1.33, 1.07 to 1.08
+//     on the smallest grids the lists are long and walked in shares, the first of which then has the near Gaussians: stress scene 600 k at 309x378
+//     K = 16 0.87, K = 32 0.84, 250 k at 400x400 0.92; clusters 400 k at 400x400 1.01 to 1.03, 150 k at 640x480 (4800 tiles) 1.08
 static bool takes_depth_bins(const htgs_frame *f, int what, uint64_t n_tiles)
 {
     if (f->mode != HTGS_MODE_HYBRID_BLEND && f->mode != HTGS_MODE_ALPHA_BLEND_FIRST_K) return false;
     const int K = htgs_effective_k(f->K), n = f->n_primitives;
     const bool wide = n_tiles > 16384;
     if (K <= 4) return false;
-    if (what == HTGS_RUN_MAX_WEIGHTS) return n >= (wide ? 250000 : 120000);
+    if (what == HTGS_RUN_MAX_WEIGHTS) return n_tiles > 4096 && n >= (wide ? 250000 : 120000);
     if (n_tiles <= 6144) return n >= 2000000;
     if (what == HTGS_RUN_FORWARD) return n >= 200000;
     if (K == 8) return n >= (n_tiles >= 8192 ? 800000 : 2000000);
