@@ -132,24 +132,6 @@ __device__ __forceinline__ CoreKey make_key(float depth, uint32_t low) { return 
 __device__ __forceinline__ uint32_t key_fraction(float alpha, const KeyFormat &f) { return (uint32_t)__builtin_fmaf(alpha, f.one, 0.5f); }      // alpha in [0, 1]
 __device__ __forceinline__ uint32_t key_pack(float alpha, uint32_t place, const KeyFormat &f) { return key_fraction(alpha, f) << f.shift | place; }
 __device__ __forceinline__ float key_alpha(uint32_t low, const KeyFormat &f) { return (float)(low >> f.shift) * f.one_rcp; }
-// What a walk of keys notes of equal depths at the end of a pixel's core (CoreTie), in one register: the fragment's place in the list,
-// the low bits of the depth, whether there is a note, and whether it was not the only one as deep.
-constexpr uint32_t kTieNoted = 1u << 30, kTieMore = 1u << 31, kTieDepthBits = 17, kTieShift = 13;
-static_assert(kPackedListMost <= 1u << kTieShift && kTieShift + kTieDepthBits == 30, "place, depth, two flags");
-__device__ __forceinline__ uint32_t tie_depth(float depth) { return (float_to_bits(depth) & ((1u << kTieDepthBits) - 1u)) << kTieShift | kTieNoted; }
-__device__ __forceinline__ bool tie_is_at(uint32_t tie, float depth) { return ((tie ^ tie_depth(depth)) & ~kTieMore) >> kTieShift == 0u; }
-__device__ __forceinline__ void tie_note(uint32_t &tie, float depth, uint32_t low, const KeyFormat &f)
-{
-    asm volatile("");                  // (branched over by a wave without one, which is nearly every time: not eight instructions for no lane)
-    const bool met = tie_is_at(tie, depth);
-    tie = tie_depth(depth) | (low & f.place_mask) | (met ? kTieMore : 0u);
-}
-// another wave's note of the same pixel; what neither the core's last depth nor its low bits match is of no use any more
-__device__ __forceinline__ void tie_join(uint32_t &tie, uint32_t other, float last_depth)
-{
-    if (!tie_is_at(other, last_depth)) return;
-    tie = tie_is_at(tie, last_depth) ? tie | kTieMore : other;
-}
 __device__ __forceinline__ void key_step(CoreKey &carried, CoreKey &slot)
 {
     CoreKey out;
@@ -168,11 +150,12 @@ __device__ __forceinline__ void core_key_walk(CoreKey &carried, CoreKey (&core)[
     }
 }
 // FAST or not is the arithmetic of a fragment alone.  Without FAST, `tie` receives what stayed out of the core, or left it, exactly as
-// deep as the entry that is last then (tie_note).
+// deep as the entry that is last then; `other` of the note is the place in the tile's list.  (The whole depth: a note that another wave's last
+// depth was taken for by some of its bits would stand in the way of the real one.)
 template <int K, bool FAST, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, bool AHEAD = false>
 __device__ __forceinline__ void hybrid_key_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                 uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy,
-                                                CoreKey (&core)[K], HybridTail &tail, uint32_t &tie, const KeyFormat &fmt, uint32_t list_first, ListStep step = 64u)
+                                                CoreKey (&core)[K], HybridTail &tail, CoreTie &tie, const KeyFormat &fmt, uint32_t list_first, ListStep step = 64u)
 {
     constexpr int MODE = HTGS_MODE_HYBRID_BLEND;
     constexpr int N = kStageSlots;
@@ -193,7 +176,7 @@ __device__ __forceinline__ void hybrid_key_walk(TileStageQ &st, QuadrantLists &q
             depth = key_depth(carried);
             leaving = key_alpha(key_low(carried), fmt);
             if constexpr (!FAST)
-                if (depth == key_depth(core[K - 1]) && leaving > 0.0f) tie_note(tie, depth, key_low(carried), fmt);
+                if (depth == key_depth(core[K - 1]) && leaving > 0.0f) tie.note(depth, key_low(carried) & fmt.place_mask);
         }
         tail.c0 = __builtin_fmaf(p3, col.x, tail.c0);
         tail.c1 = __builtin_fmaf(p3, col.y, tail.c1);
@@ -240,11 +223,11 @@ __device__ __forceinline__ void key_core_unpack(const CoreKey (&core)[K], const 
 // settle_core of a core of keys that is unpacked; inside: px.inside, in the kernels that store
 template <int MODE, int K, int REC4, typename IndexT, typename Swapped>
 __device__ __forceinline__ bool settle_key_core(TileStageQ &st, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst, uint32_t first, uint32_t last, uint32_t lane,
-                                                const TilePixel &px, float (&cd)[K], float (&ca)[K], IndexT (&ci)[K], uint32_t tie, const KeyFormat &fmt, Swapped &&swapped)
+                                                const TilePixel &px, float (&cd)[K], float (&ca)[K], IndexT (&ci)[K], const CoreTie &tie, const KeyFormat &fmt, Swapped &&swapped)
 {
-    const uint32_t place = first + (tie & ((1u << kTieShift) - 1u));
-    const bool noted = px.inside && tie_is_at(tie, cd[K - 1]) && place < last;
-    return settle_core<MODE, K, REC4>(st, prim, lane, px.pt, px.cx, px.cy, cd, ca, ci, noted, noted ? inst[place] : 0u, (tie & kTieMore) != 0u,
+    const uint32_t place = first + (tie.other & ~kMoreTied);
+    const bool noted = px.inside && tie.at_end(cd[K - 1]) && place < last;
+    return settle_core<MODE, K, REC4>(st, prim, lane, px.pt, px.cx, px.cy, cd, ca, ci, noted, noted ? inst[place] : 0u, (tie.other & kMoreTied) != 0u,
                                       [&](float alpha) { return (float)key_fraction(alpha, fmt) * fmt.one_rcp; }, swapped);
 }
 // a fragment of the tail's takes the place of another one of the same depth
@@ -343,7 +326,8 @@ __device__ __forceinline__ void hybrid_tile_by_keys(TileStageQ &st, QuadrantList
         core[i] = make_key(__FLT_MAX__, 0u);
         asm volatile("" : "+v"(core[i]));      // one register pair per slot, never a wide tuple
     }
-    uint32_t tie = 0u;
+    CoreTie tie;
+    tie.init();
     const KeyFormat fmt = key_format(last > first ? last - first : 1u);
     hybrid_key_walk<K, FAST, true, REC4, true>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, core, tail, tie, fmt, first);
     if constexpr (FAST) {
@@ -409,11 +393,10 @@ __device__ __forceinline__ void sort_bitonic(CoreKey (&core)[K])
 }
 // A core of keys joins the running one; pushed(key) is called with every entry that is in neither's K nearest.  tie: see above.
 template <int K, bool TIES, typename Pushed>
-__device__ __forceinline__ void merge_key_cores(const float *from, CoreKey (&core)[K], uint32_t &tie, const KeyFormat &fmt, Pushed &&pushed)
+__device__ __forceinline__ void merge_key_cores(const float *from, CoreKey (&core)[K], CoreTie &tie, const KeyFormat &fmt, Pushed &&pushed)
 {
-    float least = __FLT_MAX__;
-    uint32_t least_low = 0u;
-    uint32_t several = 0u;
+    CoreTie left;
+    left.init();
 #pragma unroll
     for (int i = 0; i < K; ++i) {
         const CoreKey other = __hiloint2double((int)float_to_bits(from[(2 * (K - 1 - i)) * 64]), (int)float_to_bits(from[(2 * (K - 1 - i) + 1) * 64]));
@@ -421,16 +404,15 @@ __device__ __forceinline__ void merge_key_cores(const float *from, CoreKey (&cor
         asm("v_min_f64 %0, %2, %3\n\tv_max_f64 %1, %2, %3" : "=&v"(lo), "=&v"(hi) : "v"(core[i]), "v"(other));
         core[i] = lo;
         if (TIES) {                            // (the least of them, without a branch for each)
-            const bool nearer = key_low(hi) >> fmt.shift != 0u && key_depth(hi) <= least;
-            several = nearer ? (key_depth(hi) == least ? kTieMore : 0u) : several;
-            least_low = nearer ? key_low(hi) : least_low;
-            least = nearer ? key_depth(hi) : least;
-            asm volatile("" : "+v"(least), "+v"(least_low), "+v"(several));      // (as in merge_cores)
+            const bool least = key_low(hi) >> fmt.shift != 0u && key_depth(hi) <= left.depth;
+            left.other = least ? (key_low(hi) & fmt.place_mask) | (key_depth(hi) == left.depth ? kMoreTied : 0u) : left.other;
+            left.depth = least ? key_depth(hi) : left.depth;
+            asm volatile("" : "+v"(left.other), "+v"(left.depth));      // (as in merge_cores)
         }
         pushed(hi);
     }
     sort_bitonic<K>(core);
-    if (TIES && least == key_depth(core[K - 1])) tie_join(tie, tie_depth(least) | (least_low & fmt.place_mask) | several, least);
+    if (TIES && left.depth == key_depth(core[K - 1])) tie.join(left);
 }
 // the same for cores of three registers a slot (an empty slot has alpha 0 and the largest depth)
 template <typename IndexT>
@@ -1114,7 +1096,7 @@ __device__ __forceinline__ void first_k_walk(TileStageQ &st, QuadrantLists &ql, 
 template <int K, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, typename Shared = NoSharedDepth>
 __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                  uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy,
-                                                 CoreKey (&core)[K], uint32_t &tie, const KeyFormat &fmt, uint32_t list_first, ListStep step = 64u,
+                                                 CoreKey (&core)[K], CoreTie &tie, const KeyFormat &fmt, uint32_t list_first, ListStep step = 64u,
                                                  const Shared &shared = Shared())
 {
     constexpr int MODE = HTGS_MODE_ALPHA_BLEND_FIRST_K;
@@ -1138,7 +1120,7 @@ __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &
             CoreKey carried = make_key(depth, key_pack(f.alpha, stage_index<N>(addr) - list_first, fmt));      // (the slot's last word is the place in the list)
             core_key_walk<K>(carried, core);
             depth = key_depth(carried);
-            if (depth == key_depth(core[K - 1]) && depth < __FLT_MAX__) tie_note(tie, depth, key_low(carried), fmt);
+            if (depth == key_depth(core[K - 1]) && depth < __FLT_MAX__) tie.note(depth, key_low(carried) & fmt.place_mask);
         };
         joins(one, f1, reach1, depth1);
         joins(two, f2, reach2, depth2);
@@ -1227,7 +1209,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
             core[i] = make_key(__FLT_MAX__, 0u);
             asm volatile("" : "+v"(core[i]));      // one register pair per slot, never a wide tuple
         }
-        uint32_t tie = 0u;
+        CoreTie tie;
+        tie.init();
         const KeyFormat fmt = key_format(last > first ? last - first : 1u);
         first_k_key_walk<K, true>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, core, tie, fmt, first);
         first_k_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);

@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
     uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const Finish finish)
 {
-    constexpr uint32_t kRows = 2 * K + 7;
+    constexpr uint32_t kRows = 2 * K + 8;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<WAVES, kRows>()];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     uint32_t tile, first, last;
@@ -90,17 +90,18 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         core[i] = make_key(__FLT_MAX__, 0u);
         asm volatile("" : "+v"(core[i]));
     }
-    uint32_t tie = 0u;
+    CoreTie tie;
+    tie.init();
     const KeyFormat fmt = key_format(last > first ? last - first : 1u);
     // (places count from the tile's first instance, as in the single walk)
     hybrid_key_walk<K, FAST, false, HTGS_PRIM_FLOATS / 4, true>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy,
                                                                 core, tail, tie, fmt, first, ListStep(share.per * WAVES, share.per));
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
-            [&](float *to) { give_key_core<K>(to + lane, core); give_tail<2 * K>(to + lane, tail); to[(2 * K + 6) * 64 + lane] = bits_to_float(tie); },
+            [&](float *to) { give_key_core<K>(to + lane, core); give_tail<2 * K>(to + lane, tail); if (!FAST) give_tie<2 * K + 6>(to + lane, tie); },
             [&](const float *from) {
+                if (!FAST) take_tie<2 * K + 6>(from + lane, tie);
                 merge_key_cores<K, !FAST>(from + lane, core, tie, fmt, [&](CoreKey out) { hybrid_tail_add<FAST>(tail, key_depth(out), key_alpha(key_low(out), fmt)); });
                 take_tail<2 * K>(from + lane, tail);
-                tie_join(tie, float_to_bits(from[(2 * K + 6) * 64 + lane]), key_depth(core[K - 1]));
             })) return;
     float cd[K], ca[K], ci[K];
     if constexpr (FAST) {
@@ -172,7 +173,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
     uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const Finish finish)
 {
-    constexpr uint32_t kRows = 2 * K + 1;
+    constexpr uint32_t kRows = 2 * K + 2;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<WAVES, kRows>()];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     uint32_t tile, first, last;
@@ -185,7 +186,8 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         core[i] = make_key(__FLT_MAX__, 0u);
         asm volatile("" : "+v"(core[i]));
     }
-    uint32_t tie = 0u;
+    CoreTie tie;
+    tie.init();
     const KeyFormat fmt = key_format(last > first ? last - first : 1u);
     __shared__ float s_depth[WAVES][64];
     const SharedDepth<WAVES, K> shared = { s_depth, wave, lane };
@@ -193,10 +195,10 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     __syncthreads();
     first_k_key_walk<K, false>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, core, tie, fmt, first, ListStep(share.per * WAVES, share.per), shared);
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
-            [&](float *to) { give_key_core<K>(to + lane, core); to[2 * K * 64 + lane] = bits_to_float(tie); },
+            [&](float *to) { give_key_core<K>(to + lane, core); give_tie<2 * K>(to + lane, tie); },
             [&](const float *from) {
+                take_tie<2 * K>(from + lane, tie);
                 merge_key_cores<K, true>(from + lane, core, tie, fmt, [](CoreKey) {});
-                tie_join(tie, float_to_bits(from[2 * K * 64 + lane]), key_depth(core[K - 1]));
             })) return;
     float cd[K], ca[K];
     uint32_t ci[K];
