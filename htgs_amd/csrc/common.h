@@ -109,8 +109,8 @@ inline DepthKeys depth_key_range(const htgs_frame *f)
 }
 // The Gaussians are put into bins of depth, and the instances made bin by bin (htgs_frame.depth_bins).  The parts of
 // depth_bins: the depths at which the bins after the first begin, the instances of each bin, a counter of the scan, the instances
-// of every bin in every block of kCountBlock Gaussians (bin by bin, `stride` words each; the scan makes them the ones before), the
-// bin of every Gaussian.
+// of every bin in every block of kCountBlock Gaussians (bin by bin, `stride` words each), the ones before each of these (the scan's
+// result, apart from what it reads: it may be called again), the bin of every Gaussian.
 constexpr int kDepthBins = 8;
 inline bool frame_depth_binned(const htgs_frame *f)
 {
@@ -119,7 +119,7 @@ inline bool frame_depth_binned(const htgs_frame *f)
 struct DepthBins {
     float *limits;                         // [kDepthBins - 1]
     unsigned long long *totals;            // [kDepthBins]
-    uint32_t *done, *sums;                 // [1], [kDepthBins][stride]
+    uint32_t *done, *sums, *before;        // [1], [kDepthBins][stride] twice
     uint8_t *of;                           // [N]
     uint32_t stride;
 };
@@ -135,7 +135,8 @@ inline DepthBins depth_bin_parts(const htgs_frame *f)
     b.totals = reinterpret_cast<unsigned long long *>(f->depth_bins + 8);
     b.done = f->depth_bins + 24;
     b.sums = f->depth_bins + kDepthBinsHeader;
-    b.of = reinterpret_cast<uint8_t *>(b.sums + (size_t)kDepthBins * b.stride);
+    b.before = b.sums + (size_t)kDepthBins * b.stride;
+    b.of = reinterpret_cast<uint8_t *>(b.before + (size_t)kDepthBins * b.stride);
     return b;
 }
 // stable sort of n (32-bit key, value) pairs by the low end_bit key bits, digit_bits (8 or 9) a pass (radix_sort.hip);

@@ -165,8 +165,8 @@ __global__ void __launch_bounds__(kScanBlock) scan_apply_kernel(const uint32_t *
     if (sums_per_tile != 0u && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) publish_total(before + total, total_out, host_total, tag);
 }
 
-// The scan of a frame with htgs_frame.depth_bins: a workgroup per bin makes its blocks' sums, which the per-Gaussian stage has
-// left, the sums before each block, in place, and the last workgroup to be done adds up the bins.  (3 M Gaussians: 8 x 12 k words,
+// The scan of a frame with htgs_frame.depth_bins: a workgroup per bin turns its blocks' sums, which the per-Gaussian stage has
+// left, into the sums before each block, and the last workgroup to be done adds up the bins.  (3 M Gaussians: 8 x 12 k words,
 // 5 us; the scan of all counts that it stands for takes 17.)
 __global__ void __launch_bounds__(1024) scan_bins_kernel(DepthBins bins, uint32_t n_blocks, uint32_t *__restrict__ total_out, unsigned long long *__restrict__ host_total,
                                                          uint32_t tag)
@@ -174,7 +174,8 @@ __global__ void __launch_bounds__(1024) scan_bins_kernel(DepthBins bins, uint32_
     __shared__ unsigned long long s_wave[1024 / kWave];
     constexpr uint32_t kWords = 4;                         // of four sums each, per thread and round (4.2 M Gaussians in one round)
     const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    uint4 *const words = reinterpret_cast<uint4 *>(bins.sums + (size_t)blockIdx.x * bins.stride);
+    const uint4 *const words = reinterpret_cast<const uint4 *>(bins.sums + (size_t)blockIdx.x * bins.stride);
+    uint4 *const before_words = reinterpret_cast<uint4 *>(bins.before + (size_t)blockIdx.x * bins.stride);
     unsigned long long carry = 0;
     for (uint32_t first = 0; 4u * first < n_blocks; first += 1024u * kWords) {
         uint4 v[kWords];
@@ -210,7 +211,7 @@ __global__ void __launch_bounds__(1024) scan_bins_kernel(DepthBins bins, uint32_
         for (uint32_t k = 0; k < kWords; ++k) {
             const uint32_t q = first + kWords * threadIdx.x + k;
             const uint32_t b1 = run + v[k].x, b2 = b1 + v[k].y, b3 = b2 + v[k].z;
-            if (4u * q < n_blocks) words[q] = make_uint4(run, b1, b2, b3);
+            if (4u * q < n_blocks) before_words[q] = make_uint4(run, b1, b2, b3);
             run = b3 + v[k].w;
         }
         carry += all;
@@ -372,7 +373,7 @@ __global__ void __launch_bounds__(256) create_listed_kernel(
         for (int b = 0; b < kDepthBins; ++b) all += bins.totals[b];
         if (n_instances == 0u || all > (unsigned long long)n_instances) return;
         if (threadIdx.x < (uint32_t)kDepthBins) {
-            uint32_t start = bins.sums[(size_t)threadIdx.x * bins.stride + block];
+            uint32_t start = bins.before[(size_t)threadIdx.x * bins.stride + block];
 #pragma unroll
             for (int b = 0; b < kDepthBins - 1; ++b) start += b < (int)threadIdx.x ? (uint32_t)bins.totals[b] : 0u;
             s_place[threadIdx.x] = start;
@@ -935,7 +936,7 @@ extern "C" size_t htgs_depth_order_words(int n_primitives)
 extern "C" size_t htgs_depth_bins_words(int n_primitives)
 {
     const size_t n = n_primitives > 0 ? (size_t)n_primitives : 0;
-    return kDepthBinsHeader + (size_t)kDepthBins * depth_bins_stride(n_primitives) + (n + 3) / 4;
+    return kDepthBinsHeader + 2 * (size_t)kDepthBins * depth_bins_stride(n_primitives) + (n + 3) / 4;
 }
 
 extern "C" size_t htgs_depth_order_result_word(const htgs_frame *f)

@@ -86,6 +86,30 @@ def test_lists(cuda, n, train):
         assert torch.equal(unsorted[slots].to(torch.int64), torch.repeat_interleave(seen, counts[seen]))
 
 
+@pytest.mark.parametrize("n,scans", [(1, 2), (257, 2), (70_001, 3), (4_194_304, 1), (4_194_305, 1), (4_300_001, 2)])
+def test_scan(cuda, n, scans):
+    """The scan of the bins may be called again, and takes more than one round of 4 194 304 Gaussians: as many instances as by index, each in
+    the same tile."""
+    print(f"case n={n} scans={scans}", flush=True)
+    sg = small_view(make_scene(1, min(n, 70_001)), 640, 400).to(cuda)
+    if n > 70_001:
+        more = lambda t: t.repeat(n // 70_001 + 1, *[1] * (t.ndim - 1))[:n].contiguous()
+        g = torch.Generator(device=cuda).manual_seed(1)
+        sg = dataclasses.replace(sg, positions=more(sg.positions) + 0.05 * torch.randn(n, 3, generator=g, device=cuda), scales=more(sg.scales), rotations=more(sg.rotations),
+                                 opacities=more(sg.opacities), sh_0=more(sg.sh_0), sh_rest=torch.zeros(n, 0, 3, device=cuda), active_sh_bases=1)
+    pairs = []
+    for bins in (False, True):
+        fb = frame(sg, HYBRID, 16, bins)
+        fb.preprocess()
+        for _ in range(scans):
+            fb.scan()
+        fb.alloc_instances(fb.read_instance_count())
+        fb.create_instances()
+        m = fb.n_instances
+        pairs.append(torch.sort((fb.keys[0][:m].to(torch.int64) & 0xffff) * n + fb.vals[0][:m].to(torch.int64)).values)
+    assert torch.equal(*pairs)
+
+
 @pytest.mark.parametrize("waves,threshold", [(1, 0), (2, 0), (4, 0), (1, 60)])
 @pytest.mark.parametrize("K", [1, 2, 4, 16, 32])
 @pytest.mark.parametrize("mode", [HYBRID, FIRST_K])
