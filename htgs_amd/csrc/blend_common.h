@@ -859,11 +859,13 @@ struct CoreTie {
     float depth;
     uint32_t other;
     __device__ __forceinline__ void init() { depth = __FLT_MAX__; other = 0u; }
-    __device__ __forceinline__ void note(float at, uint32_t index)
+    // the lanes with `met` note it; a wave without one branches over it, on the compare's own result
+    __device__ __forceinline__ void note(bool met, float at, uint32_t index)
     {
-        asm volatile("");              // (branched over by a wave without one)
-        other = index | (depth == at ? kMoreTied : 0u);
-        depth = at;
+        if (__ballot(met) == 0ull) return;
+        asm volatile("");
+        other = met ? index | (depth == at ? kMoreTied : 0u) : other;
+        depth = met ? at : depth;
     }
     // another wave's note of the same pixel
     __device__ __forceinline__ void join(const CoreTie &t)
@@ -874,6 +876,14 @@ struct CoreTie {
     // (nothing stays out of a core that is not full)
     __device__ __forceinline__ bool at_end(float last_depth) const { return depth < __FLT_MAX__ && depth <= last_depth; }
 };
+// Whether what stayed out of a core, or left it, is as deep as the entry that is last now.  (An empty slot, whose depth is the largest float, is not:
+// the last entry's depth is held below it, which takes one instruction where a second test takes three.)
+__device__ __forceinline__ bool meets_core_end(float depth, float last_depth)
+{
+    float last;
+    asm("v_min_f32 %0, 0x7f7ffffe, %1" : "=v"(last) : "v"(last_depth));
+    return depth == last;
+}
 // two entries of the finished core are exactly as deep as each other, or one that is not in it is as deep as its last
 template <int K>
 __device__ __forceinline__ bool core_tied(const float (&cd)[K], const float (&ca)[K], const CoreTie &tie)
@@ -883,26 +893,12 @@ __device__ __forceinline__ bool core_tied(const float (&cd)[K], const float (&ca
     for (int i = 0; i + 1 < K; ++i) tied = tied || (ca[i + 1] > 0.0f && cd[i] == cd[i + 1]);
     return tied;
 }
-// The finished core of every pixel of the wave with its entries of equal depth as the reference's insertion leaves them, from the core
-// alone: pairs inside it are put in order (settle_equal_pairs), and where its last entry and one other fragment are equally deep, that
-// fragment is evaluated at the pixel and takes the last entry's place if the order by index says so: of the two, the one
-// with the lower index stays if an even number of the nearer entries has a higher index than both, the other one if an odd number
-// has.  (The last arrival of the K + 1 decides: one of the two is turned away, any other hops the first over the second, which
-// leaves.)  noted: a fragment met the last entry's depth; other: its index, more: it was not the only one (CoreTie).  held(alpha):
-// the alpha that the core would hold; swapped(out, in): the tail has lost a fragment and gained another one of the last entry's
-// depth.  True for the pixels that this does not settle: more than two of a depth, or a tail that cannot give up an opaque fragment.
-// A pixel that is settled so costs the evaluation of one fragment; walking the tile's list for it took as long as a list of a
-// third of its length, at the end of a launch as often as not (6 M Gaussians of the stress scene at 1600x1066: the launch with
-// one wave per tile 1050 -> 730 us).
-template <int MODE, int K, int REC4, typename IndexT, typename Held, typename Swapped>
-__device__ __forceinline__ bool settle_core(TileStageQ &st, const float4 *__restrict__ prim, uint32_t lane, const PixelTerms &pt, float cx, float cy, float (&cd)[K],
-                                            float (&ca)[K], IndexT (&ci)[K], bool noted, uint32_t other, bool more, Held &&held, Swapped &&swapped)
+// Depth and alpha of Gaussian `other` at the pixels of the lanes that have noted one, by the walk's own arithmetic.
+struct TieFragment { float depth, alpha; };
+template <int MODE, int REC4>
+__device__ __forceinline__ TieFragment tie_fragment(TileStageQ &st, const float4 *__restrict__ prim, uint32_t lane, const PixelTerms &pt, float cx, float cy, bool noted,
+                                                    uint32_t other)
 {
-    bool again = false, pairs = false;
-#pragma unroll
-    for (int i = 0; i + 1 < K; ++i) pairs = pairs || (ca[i + 1] > 0.0f && cd[i] == cd[i + 1]);
-    if (__any(pairs)) again = settle_equal_pairs<K>(cd, ca, ci);
-    if (!__any(noted)) return again;
     wave_lds_sync();
     // (a slot for each lane, as in a batch of the walk)
     tile_stage_load<MODE, kStageSlots, true, kCullNone, true, REC4, false, false, true>(st, prim, nullptr, noted ? 0u : 1u, 1u, (int)lane + 1, cx, cy, 0, other);
@@ -910,7 +906,29 @@ __device__ __forceinline__ bool settle_core(TileStageQ &st, const float4 *__rest
     const uint32_t addr = stage_slot_address(st, lane);
     TileFrag f;
     tile_frag_exact<MODE, kStageSlots>(addr, pt, f);
-    const bool meets = noted && tile_frag_depth<kStageSlots>(addr, pt, f) == cd[K - 1];
+    return TieFragment{ tile_frag_depth<kStageSlots>(addr, pt, f), f.alpha };
+}
+// The finished core of every pixel of the wave with its entries of equal depth as the reference's insertion leaves them, from the core
+// alone: pairs inside it are put in order (settle_equal_pairs), and where its last entry and one other fragment are equally deep, that
+// fragment is evaluated at the pixel and takes the last entry's place if the order by index says so: of the two, the one
+// with the lower index stays if an even number of the nearer entries has a higher index than both, the other one if an odd number
+// has.  (The last arrival of the K + 1 decides: one of the two is turned away, any other hops the first over the second, which
+// leaves.)  noted: a fragment met the last entry's depth; other: its index, more: it was not the only one (CoreTie).
+// swapped(in, out): the tail has gained a fragment of the last entry's depth and lost another one.  True for the pixels that this does not settle: more than two of a depth, or a tail that cannot give up an opaque fragment.
+// A pixel that is settled so costs the evaluation of one fragment; walking the tile's list for it took as long as a list of a
+// third of its length, at the end of a launch as often as not (6 M Gaussians of the stress scene at 1600x1066: the launch with
+// one wave per tile 1050 -> 730 us).
+template <int MODE, int K, int REC4, typename IndexT, typename Swapped>
+__device__ __forceinline__ bool settle_core(TileStageQ &st, const float4 *__restrict__ prim, uint32_t lane, const PixelTerms &pt, float cx, float cy, float (&cd)[K],
+                                            float (&ca)[K], IndexT (&ci)[K], bool noted, uint32_t other, bool more, Swapped &&swapped)
+{
+    bool again = false, pairs = false;
+#pragma unroll
+    for (int i = 0; i + 1 < K; ++i) pairs = pairs || (ca[i + 1] > 0.0f && cd[i] == cd[i + 1]);
+    if (__any(pairs)) again = settle_equal_pairs<K>(cd, ca, ci);
+    if (!__any(noted)) return again;
+    const TieFragment f = tie_fragment<MODE, REC4>(st, prim, lane, pt, cx, cy, noted, other);
+    const bool meets = noted && f.depth == cd[K - 1];
     if (meets && (more || (K > 1 && cd[K - 1] == cd[K > 1 ? K - 2 : 0]) || (MODE == HTGS_MODE_HYBRID_BLEND && f.alpha > 0.99f))) again = true;
     uint32_t last;
     __builtin_memcpy(&last, &ci[K - 1], 4);
@@ -923,9 +941,8 @@ __device__ __forceinline__ bool settle_core(TileStageQ &st, const float4 *__rest
         odd = odd != (x > high);
     }
     if (meets && !again && (other > last) == odd) {
-        const float alpha = held(f.alpha);
-        swapped(ca[K - 1], alpha);
-        ca[K - 1] = alpha;
+        swapped(ca[K - 1], f.alpha);
+        ca[K - 1] = f.alpha;
         __builtin_memcpy(&ci[K - 1], &other, 4);
     }
     return again;

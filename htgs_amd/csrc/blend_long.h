@@ -89,7 +89,7 @@ __device__ __forceinline__ void hybrid_walk(TileStageQ &st, QuadrantLists &ql, c
             float pi = col.w;
             if constexpr ((FAST && !TIES) || QUICK) core_quick_walk<K>(depth, p3, pi, cd, ca, ci);
             else core_exchange_walk<K>(depth, p3, pi, cd, ca, ci);
-            if (TIES && p3 > 0.0f && depth == cd[K - 1]) tie->note(depth, float_to_bits(pi));
+            if (TIES) tie->note(meets_core_end(depth, cd[K - 1]), depth, float_to_bits(pi));
         }
         hybrid_tail_add<FAST>(tail, depth, p3);
     }, pixel_lanes, 1.0f, step);
@@ -132,6 +132,19 @@ __device__ __forceinline__ CoreKey make_key(float depth, uint32_t low) { return 
 __device__ __forceinline__ uint32_t key_fraction(float alpha, const KeyFormat &f) { return (uint32_t)__builtin_fmaf(alpha, f.one, 0.5f); }      // alpha in [0, 1]
 __device__ __forceinline__ uint32_t key_pack(float alpha, uint32_t place, const KeyFormat &f) { return key_fraction(alpha, f) << f.shift | place; }
 __device__ __forceinline__ float key_alpha(uint32_t low, const KeyFormat &f) { return (float)(low >> f.shift) * f.one_rcp; }
+// What a walk of keys notes of equal depths at the end of a pixel's core: the low words of the last two entries that stayed out of it, or left it,
+// exactly as deep as the entry that was last then (0: an empty slot, or none).  Three vector instructions a fragment and no branch; how deep they
+// are, and whether they are equally deep, is evaluated after the walk where there is one (noted_ties).  (With the depth and a flag noted behind
+// a branch -> so, the launch alone: HYBRID 250 k Gaussians at 1280x720 120.1 -> 112.4 us, 200 k at 1920x1080 214.7 -> 210.1, FIRST_K 137.9 -> 134.9.)
+struct KeyNotes {
+    uint32_t latest, before;
+    __device__ __forceinline__ void init() { latest = before = 0u; }
+    __device__ __forceinline__ void note(bool met, uint32_t low)
+    {
+        before = met ? latest : before;
+        latest = met ? low : latest;
+    }
+};
 __device__ __forceinline__ void key_step(CoreKey &carried, CoreKey &slot)
 {
     CoreKey out;
@@ -150,12 +163,11 @@ __device__ __forceinline__ void core_key_walk(CoreKey &carried, CoreKey (&core)[
     }
 }
 // FAST or not is the arithmetic of a fragment alone.  Without FAST, `tie` receives what stayed out of the core, or left it, exactly as
-// deep as the entry that is last then; `other` of the note is the place in the tile's list.  (The whole depth: a note that another wave's last
-// depth was taken for by some of its bits would stand in the way of the real one.)
+// deep as the entry that is last then.
 template <int K, bool FAST, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, bool AHEAD = false>
 __device__ __forceinline__ void hybrid_key_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                 uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy,
-                                                CoreKey (&core)[K], HybridTail &tail, CoreTie &tie, const KeyFormat &fmt, uint32_t list_first, ListStep step = 64u)
+                                                CoreKey (&core)[K], HybridTail &tail, KeyNotes &notes, const KeyFormat &fmt, uint32_t list_first, ListStep step = 64u)
 {
     constexpr int MODE = HTGS_MODE_HYBRID_BLEND;
     constexpr int N = kStageSlots;
@@ -175,8 +187,7 @@ __device__ __forceinline__ void hybrid_key_walk(TileStageQ &st, QuadrantLists &q
             core_key_walk<K>(carried, core);
             depth = key_depth(carried);
             leaving = key_alpha(key_low(carried), fmt);
-            if constexpr (!FAST)
-                if (depth == key_depth(core[K - 1]) && leaving > 0.0f) tie.note(depth, key_low(carried) & fmt.place_mask);
+            if constexpr (!FAST) notes.note(depth == key_depth(core[K - 1]), key_low(carried));
         }
         tail.c0 = __builtin_fmaf(p3, col.x, tail.c0);
         tail.c1 = __builtin_fmaf(p3, col.y, tail.c1);
@@ -220,15 +231,82 @@ __device__ __forceinline__ void key_core_unpack(const CoreKey (&core)[K], const 
     }
 }
 
-// settle_core of a core of keys that is unpacked; inside: px.inside, in the kernels that store
-template <int MODE, int K, int REC4, typename IndexT, typename Swapped>
-__device__ __forceinline__ bool settle_key_core(TileStageQ &st, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst, uint32_t first, uint32_t last, uint32_t lane,
-                                                const TilePixel &px, float (&cd)[K], float (&ca)[K], IndexT (&ci)[K], const CoreTie &tie, const KeyFormat &fmt, Swapped &&swapped)
+// The notes of a walk with the depth they are at; `other` is the place in the tile's list.  (The walk's last depth never grows: the latest note is the
+// least deep.)
+template <int MODE, int REC4>
+__device__ __forceinline__ CoreTie noted_ties(TileStageQ &st, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst, uint32_t first, uint32_t last, uint32_t lane,
+                                              const TilePixel &px, const KeyNotes &notes, const KeyFormat &fmt)
 {
-    const uint32_t place = first + (tie.other & ~kMoreTied);
-    const bool noted = px.inside && tie.at_end(cd[K - 1]) && place < last;
-    return settle_core<MODE, K, REC4>(st, prim, lane, px.pt, px.cx, px.cy, cd, ca, ci, noted, noted ? inst[place] : 0u, (tie.other & kMoreTied) != 0u,
-                                      [&](float alpha) { return (float)key_fraction(alpha, fmt) * fmt.one_rcp; }, swapped);
+    CoreTie tie;
+    tie.init();
+    const uint32_t place = notes.latest & fmt.place_mask, place_before = notes.before & fmt.place_mask;
+    const bool noted = px.inside && notes.latest >> fmt.shift != 0u && first + place < last;
+    if (!__any(noted)) return tie;
+    const float depth = tie_fragment<MODE, REC4>(st, prim, lane, px.pt, px.cx, px.cy, noted, noted ? inst[first + place] : 0u).depth;
+    const bool twice = noted && notes.before >> fmt.shift != 0u && first + place_before < last;
+    bool more = false;
+    if (__any(twice))
+        more = tie_fragment<MODE, REC4>(st, prim, lane, px.pt, px.cx, px.cy, twice, twice ? inst[first + place_before] : 0u).depth == depth && twice;
+    if (noted) {
+        tie.depth = depth;
+        tie.other = place | (more ? kMoreTied : 0u);
+    }
+    return tie;
+}
+// settle_core of a core of keys, before it is unpacked: nearly every wave has no two equal depths that matter and is through after a compare for each
+// slot, and where one has, the keys, the indices that the pairs and the parity take and then the staged record are not all held at once.
+// (From the unpacked core, with the tail and the record beside it, the kernels with K = 16 spilled 43 and 57 registers instead of 30 and
+// 31, also for the waves without a tie, and K = 32 took 291 us for 300 k Gaussians at 1280x720 instead of 274.)
+template <int MODE, int K, int REC4, typename Swapped>
+__device__ __forceinline__ bool settle_keys(TileStageQ &st, const float4 *__restrict__ prim, const uint32_t *__restrict__ inst, uint32_t first, uint32_t last, uint32_t lane,
+                                            const TilePixel &px, CoreKey (&core)[K], const CoreTie &tie, const KeyFormat &fmt, Swapped &&swapped)
+{
+    const auto equal = [&](int i) { return key_low(core[i + 1]) >> fmt.shift != 0u && key_depth(core[i]) == key_depth(core[i + 1]); };
+    const auto held = [&](uint32_t place, bool is) { return is && first + place < last ? inst[first + place] : 0u; };
+    const uint32_t place = tie.other & ~kMoreTied;
+    const bool noted = px.inside && tie.at_end(key_depth(core[K - 1])) && first + place < last;
+    bool pairs = false;
+#pragma unroll
+    for (int i = 0; i + 1 < K; ++i) pairs = pairs || equal(i);
+    pairs = pairs && px.inside;
+    if (!__any(pairs || noted)) return false;
+    bool again = false, stays;
+    const uint32_t other = held(place, noted);
+    {
+        uint32_t x[K];
+#pragma unroll
+        for (int i = 0; i < K; ++i) x[i] = held(key_low(core[i]) & fmt.place_mask, key_low(core[i]) >> fmt.shift != 0u);
+        const auto odd_above = [&](int n, uint32_t high) {
+            bool odd = false;
+#pragma unroll
+            for (int j = 0; j < K; ++j)
+                if (j < n) odd = odd != (x[j] > high);
+            return odd;
+        };
+#pragma unroll
+        for (int i = 0; i + 1 < K; ++i) {
+            const bool here = pairs && equal(i);
+            if (!__any(here)) continue;
+            if (i + 2 < K) again = again || (here && equal(i + 2 < K ? i + 1 : i));
+            if (here && (x[i] > x[i + 1]) != odd_above(i, x[i] > x[i + 1] ? x[i] : x[i + 1])) {
+                const uint32_t low = key_low(core[i]), y = x[i];
+                core[i] = make_key(key_depth(core[i]), key_low(core[i + 1])); x[i] = x[i + 1];
+                core[i + 1] = make_key(key_depth(core[i + 1]), low); x[i + 1] = y;
+            }
+        }
+        stays = (other > x[K - 1]) != odd_above(K - 1, other > x[K - 1] ? other : x[K - 1]);
+    }
+    if (!__any(noted)) return again;
+    const TieFragment f = tie_fragment<MODE, REC4>(st, prim, lane, px.pt, px.cx, px.cy, noted, other);
+    const bool meets = noted && f.depth == key_depth(core[K - 1]);
+    if (meets && ((tie.other & kMoreTied) != 0u || (K > 1 && key_depth(core[K - 1]) == key_depth(core[K > 1 ? K - 2 : 0])) || (MODE == HTGS_MODE_HYBRID_BLEND && f.alpha > 0.99f)))
+        again = true;
+    if (meets && !again && !stays) {
+        const uint32_t fraction = key_fraction(f.alpha, fmt);
+        swapped(key_alpha(key_low(core[K - 1]), fmt), (float)fraction * fmt.one_rcp);
+        core[K - 1] = make_key(key_depth(core[K - 1]), fraction << fmt.shift | place);
+    }
+    return again;
 }
 // a fragment of the tail's takes the place of another one of the same depth
 __device__ __forceinline__ auto tail_swap(HybridTail &t, float depth)
@@ -245,7 +323,7 @@ __device__ __forceinline__ bool settle_exact_core(TileStageQ &st, const float4 *
                                                   IndexT (&ci)[K], const CoreTie &tie, Swapped &&swapped)
 {
     return settle_core<MODE, K, REC4>(st, prim, lane, px.pt, px.cx, px.cy, cd, ca, ci, px.inside && tie.at_end(cd[K - 1]), tie.other & ~kMoreTied,
-                                      (tie.other & kMoreTied) != 0u, [](float alpha) { return alpha; }, swapped);
+                                      (tie.other & kMoreTied) != 0u, swapped);
 }
 
 // core + tail -> pixel (R/include/hybrid_blend/kernels/inference.cuh:172-213)
@@ -326,18 +404,19 @@ __device__ __forceinline__ void hybrid_tile_by_keys(TileStageQ &st, QuadrantList
         core[i] = make_key(__FLT_MAX__, 0u);
         asm volatile("" : "+v"(core[i]));      // one register pair per slot, never a wide tuple
     }
-    CoreTie tie;
-    tie.init();
+    KeyNotes notes;
+    notes.init();
     const KeyFormat fmt = key_format(last > first ? last - first : 1u);
-    hybrid_key_walk<K, FAST, true, REC4, true>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, core, tail, tie, fmt, first);
+    hybrid_key_walk<K, FAST, true, REC4, true>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, core, tail, notes, fmt, first);
     if constexpr (FAST) {
         if (!px.inside) return;
         key_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
         finish(prim, tile, px, cd, ca, ci, tail);
     } else {
-        key_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
-        const bool again = settle_key_core<HTGS_MODE_HYBRID_BLEND, K, REC4>(st, prim, inst, first, last, lane, px, cd, ca, ci, tie, fmt, tail_swap(tail, cd[K - 1])) && px.inside;
+        const CoreTie tie = noted_ties<HTGS_MODE_HYBRID_BLEND, REC4>(st, prim, inst, first, last, lane, px, notes, fmt);
+        const bool again = settle_keys<HTGS_MODE_HYBRID_BLEND, K, REC4>(st, prim, inst, first, last, lane, px, core, tie, fmt, tail_swap(tail, key_depth(core[K - 1])));
         const uint64_t again_lanes = __ballot(again);
+        key_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
         if (px.inside && !again) finish(prim, tile, px, cd, ca, ci, tail);
         if (again_lanes == 0) return;
         // (the lane and its pixel are worked out afresh, so that nothing the first walk keeps in registers has to
@@ -391,28 +470,40 @@ __device__ __forceinline__ void sort_bitonic(CoreKey (&core)[K])
             }
     }
 }
+// The least deep of the entries that a merge of two cores pushes out, and the next (an empty slot has the largest depth): four instructions for
+// each.  (With the flag worked out on the way, eight, and a row more of what
+// a part of a list leaves: long lists of the weights of 600 k Gaussians of the stress scene at 309x378, FIRST_K K = 32 467 -> 451 us, HYBRID K = 16 313 -> 309.)
+struct LeastPushed {
+    float least = __FLT_MAX__, next = __FLT_MAX__;
+    uint32_t index = 0u;
+    __device__ __forceinline__ void add(float depth, uint32_t x)
+    {
+        index = depth < least ? x : index;
+        next = __builtin_amdgcn_fmed3f(depth, least, next);
+        least = depth < least ? depth : least;
+        asm volatile("" : "+v"(index), "+v"(next), "+v"(least));      // (now, not for all entries at the end: that took a hundred scalar registers)
+    }
+    __device__ __forceinline__ void join(CoreTie &tie, float last_depth) const
+    {
+        if (least == last_depth) tie.join(CoreTie{ least, index | (next == least ? kMoreTied : 0u) });
+    }
+};
 // A core of keys joins the running one; pushed(key) is called with every entry that is in neither's K nearest.  tie: see above.
 template <int K, bool TIES, typename Pushed>
 __device__ __forceinline__ void merge_key_cores(const float *from, CoreKey (&core)[K], CoreTie &tie, const KeyFormat &fmt, Pushed &&pushed)
 {
-    CoreTie left;
-    left.init();
+    LeastPushed left;
 #pragma unroll
     for (int i = 0; i < K; ++i) {
         const CoreKey other = __hiloint2double((int)float_to_bits(from[(2 * (K - 1 - i)) * 64]), (int)float_to_bits(from[(2 * (K - 1 - i) + 1) * 64]));
         CoreKey lo, hi;
         asm("v_min_f64 %0, %2, %3\n\tv_max_f64 %1, %2, %3" : "=&v"(lo), "=&v"(hi) : "v"(core[i]), "v"(other));
         core[i] = lo;
-        if (TIES) {                            // (the least of them, without a branch for each)
-            const bool least = key_low(hi) >> fmt.shift != 0u && key_depth(hi) <= left.depth;
-            left.other = least ? (key_low(hi) & fmt.place_mask) | (key_depth(hi) == left.depth ? kMoreTied : 0u) : left.other;
-            left.depth = least ? key_depth(hi) : left.depth;
-            asm volatile("" : "+v"(left.other), "+v"(left.depth));      // (as in merge_cores)
-        }
+        if (TIES) left.add(key_depth(hi), key_low(hi) & fmt.place_mask);
         pushed(hi);
     }
     sort_bitonic<K>(core);
-    if (TIES && left.depth == key_depth(core[K - 1])) tie.join(left);
+    if (TIES) left.join(tie, key_depth(core[K - 1]));
 }
 // the same for cores of three registers a slot (an empty slot has alpha 0 and the largest depth)
 template <typename IndexT>
@@ -427,8 +518,7 @@ __device__ __forceinline__ void order_entries(float &d0, float &a0, IndexT &i0, 
 template <int K, bool TIES, typename IndexT, typename Pushed>
 __device__ __forceinline__ void merge_cores(const float *from, float (&cd)[K], float (&ca)[K], IndexT (&ci)[K], CoreTie &tie, Pushed &&pushed)
 {
-    CoreTie left;
-    left.init();
+    LeastPushed left;
 #pragma unroll
     for (int i = 0; i < K; ++i) {
         float d = from[(3 * (K - 1 - i)) * 64], a = from[(3 * (K - 1 - i) + 1) * 64];
@@ -436,13 +526,10 @@ __device__ __forceinline__ void merge_cores(const float *from, float (&cd)[K], f
         const float bits = from[(3 * (K - 1 - i) + 2) * 64];
         __builtin_memcpy(&x, &bits, 4);
         order_entries(cd[i], ca[i], ci[i], d, a, x);
-        if (TIES) {                            // (the least of them, without a branch for each)
+        if (TIES) {
             uint32_t index;
             __builtin_memcpy(&index, &x, 4);
-            const bool least = a > 0.0f && d <= left.depth;
-            left.other = least ? index | (d == left.depth ? kMoreTied : 0u) : left.other;
-            left.depth = least ? d : left.depth;
-            asm volatile("" : "+v"(left.other), "+v"(left.depth));      // (now, not for all entries at the end: that took a hundred scalar registers)
+            left.add(d, index);
         }
         pushed(d, a);
         asm volatile("" : "+v"(cd[i]), "+v"(ca[i]), "+v"(ci[i]));
@@ -453,7 +540,7 @@ __device__ __forceinline__ void merge_cores(const float *from, float (&cd)[K], f
         for (int i = 0; i < K; ++i)
             if ((i & half) == 0) order_entries(cd[i], ca[i], ci[i], cd[i + half], ca[i + half], ci[i + half]);
     }
-    if (TIES && left.depth == cd[K - 1]) tie.join(left);
+    if (TIES) left.join(tie, cd[K - 1]);
 }
 template <int K, typename IndexT>
 __device__ __forceinline__ void give_core(float *to, const float (&cd)[K], const float (&ca)[K], const IndexT (&ci)[K])
@@ -485,10 +572,16 @@ __device__ __forceinline__ void take_tail(const float *from, HybridTail &t)
     t.T *= from[ROW * 64];
     t.c0 += from[(ROW + 1) * 64]; t.c1 += from[(ROW + 2) * 64]; t.c2 += from[(ROW + 3) * 64]; t.alpha += from[(ROW + 4) * 64]; t.depth += from[(ROW + 5) * 64];
 }
+// A note in one row: it is of use if it is as deep as the core's last entry, whose depth is in the core (from row LAST on).
+constexpr uint32_t kNoTie = ~0u;
 template <int ROW>
-__device__ __forceinline__ void give_tie(float *to, const CoreTie &tie) { to[ROW * 64] = tie.depth; to[(ROW + 1) * 64] = bits_to_float(tie.other); }
-template <int ROW>
-__device__ __forceinline__ void take_tie(const float *from, CoreTie &tie) { tie.join(CoreTie{ from[ROW * 64], float_to_bits(from[(ROW + 1) * 64]) }); }
+__device__ __forceinline__ void give_tie(float *to, const CoreTie &tie, float last_depth) { to[ROW * 64] = bits_to_float(tie.at_end(last_depth) ? tie.other : kNoTie); }
+template <int ROW, int LAST>
+__device__ __forceinline__ void take_tie(const float *from, CoreTie &tie)
+{
+    const uint32_t other = float_to_bits(from[ROW * 64]);
+    tie.join(CoreTie{ other != kNoTie ? from[LAST * 64] : __FLT_MAX__, other });
+}
 // ---------------------------------------------------------------------------------------------
 // Tiles with very long lists (HYBRID_BLEND, ALPHA_BLEND_FIRST_K and OIT_BLEND, which walk all of a list): the kernel
 // with one wave per tile puts a tile whose list is longer than long_threshold on a list instead of walking it, if the
@@ -516,7 +609,7 @@ inline void with_long_waves(const htgs_frame *f, Launch &&launch)
 constexpr unsigned long_grid(int waves) { return 256u * (unsigned)(kLongWavesHeld / waves); }
 
 // What a workgroup leaves of its part of a list, in 64-lane rows: HYBRID's core, tail and what met at its end.
-template <int K> constexpr uint32_t long_part_words() { return (3u * K + 8u) * 64u; }
+template <int K> constexpr uint32_t long_part_words() { return (3u * K + 7u) * 64u; }
 // The parts a list of this length is walked in by separate workgroups (1: by one).  A part is at least part_least
 // long (least_part), long enough that what the parts leave behind (part_words each) fits into the list's own stretch of
 // the spare value buffer, and at least as long as the frame's average list (part_floor = instances / tiles, rounded
@@ -787,13 +880,13 @@ __device__ __forceinline__ uint32_t pixels_again(TileStage<64> &st, const uint32
     return fits ? n_out : ~0u;
 }
 
-// A core, a tail and a tie (3K + 8 rows of 64 lanes at from[]) join the running ones: they cover the stretch of the
+// A core, a tail and a tie (3K + 7 rows of 64 lanes at from[]) join the running ones: they cover the stretch of the
 // list that follows.
 template <int K, bool FAST>
 __device__ __forceinline__ void hybrid_merge(const float *from, uint32_t lane, float (&cd)[K], float (&ca)[K], float (&ci)[K], HybridTail &tail,
                                              CoreTie &tie)
 {
-    take_tie<3 * K + 6>(from + lane, tie);
+    take_tie<3 * K + 6, 3 * (K - 1)>(from + lane, tie);
     merge_cores<K, !FAST>(from + lane, cd, ca, ci, tie, [&](float depth, float alpha) { hybrid_tail_add<FAST>(tail, depth, alpha); });
     take_tail<3 * K>(from + lane, tail);
 }
@@ -802,7 +895,7 @@ __device__ __forceinline__ void hybrid_put(float *to, uint32_t lane, const float
 {
     give_core<K>(to + lane, cd, ca, ci);
     give_tail<3 * K>(to + lane, tail);
-    give_tie<3 * K + 6>(to + lane, tie);
+    give_tie<3 * K + 6>(to + lane, tie, cd[K - 1]);
 }
 // The waves' shares, merged pairwise into the first wave's: put(buffer) by the wave that hands its share on, merge(buffer) by
 // the one that takes it (all threads of the workgroup call this).
@@ -832,7 +925,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ shortlist, ListThreshold threshold, const Finish finish)
 {
     constexpr int kWaves = WAVES;
-    constexpr uint32_t kRows = 3 * K + 8;             // a wave's core, tail and tie
+    constexpr uint32_t kRows = 3 * K + 7;             // a wave's core, tail and tie
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<kWaves, kRows>()];
     __shared__ uint32_t s_next;
     __shared__ uint32_t s_redo[2];                    // the pixels (lanes) to walk again
@@ -1085,7 +1178,7 @@ __device__ __forceinline__ void first_k_walk(TileStageQ &st, QuadrantLists &ql, 
         float alpha = f.alpha;
         uint32_t idx = stage_index<N>(addr);
         core_exchange_walk<K>(depth, alpha, idx, cd, ca, ci);
-        if (TIES && alpha > 0.0f && depth == cd[K - 1]) tie->note(depth, idx);
+        if (TIES) tie->note(meets_core_end(depth, cd[K - 1]), depth, idx);
     }, pixel_lanes, 1.0f, step, [&]() {
         const float of_all = shared(cd[Shared::kSlot]);
         return cd[K - 1] < of_all ? cd[K - 1] : of_all;
@@ -1096,7 +1189,7 @@ __device__ __forceinline__ void first_k_walk(TileStageQ &st, QuadrantLists &ql, 
 template <int K, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, typename Shared = NoSharedDepth>
 __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                  uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy,
-                                                 CoreKey (&core)[K], CoreTie &tie, const KeyFormat &fmt, uint32_t list_first, ListStep step = 64u,
+                                                 CoreKey (&core)[K], KeyNotes &notes, const KeyFormat &fmt, uint32_t list_first, ListStep step = 64u,
                                                  const Shared &shared = Shared())
 {
     constexpr int MODE = HTGS_MODE_ALPHA_BLEND_FIRST_K;
@@ -1120,7 +1213,7 @@ __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &
             CoreKey carried = make_key(depth, key_pack(f.alpha, stage_index<N>(addr) - list_first, fmt));      // (the slot's last word is the place in the list)
             core_key_walk<K>(carried, core);
             depth = key_depth(carried);
-            if (depth == key_depth(core[K - 1]) && depth < __FLT_MAX__) tie.note(depth, key_low(carried) & fmt.place_mask);
+            notes.note(depth == key_depth(core[K - 1]), key_low(carried));
         };
         joins(one, f1, reach1, depth1);
         joins(two, f2, reach2, depth2);
@@ -1178,7 +1271,7 @@ struct FirstKImage {
     }
 };
 // what a workgroup leaves of its part of a list: the core and what met at its end
-template <int K> constexpr uint32_t first_k_part_words() { return (3u * K + 2u) * 64u; }
+template <int K> constexpr uint32_t first_k_part_words() { return (3u * K + 1u) * 64u; }
 // KEYS (exact arithmetic, with long_tiles and a threshold of no more than kPackedListMost): the core as sorted 64-bit keys;
 // the pixels at which fragments of exactly equal depth met where they decide the core are walked again afterwards, over the
 // instances that reach one of them, with the reference's insertion (as in hybrid_tile_by_keys).
@@ -1209,13 +1302,14 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
             core[i] = make_key(__FLT_MAX__, 0u);
             asm volatile("" : "+v"(core[i]));      // one register pair per slot, never a wide tuple
         }
-        CoreTie tie;
-        tie.init();
+        KeyNotes notes;
+        notes.init();
         const KeyFormat fmt = key_format(last > first ? last - first : 1u);
-        first_k_key_walk<K, true>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, core, tie, fmt, first);
-        first_k_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
-        const bool again = settle_key_core<HTGS_MODE_ALPHA_BLEND_FIRST_K, K, HTGS_PRIM_FLOATS / 4>(st, prim, inst, first, last, lane, px, cd, ca, ci, tie, fmt, [](float, float) {}) && px.inside;
+        first_k_key_walk<K, true>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, core, notes, fmt, first);
+        const CoreTie tie = noted_ties<HTGS_MODE_ALPHA_BLEND_FIRST_K, HTGS_PRIM_FLOATS / 4>(st, prim, inst, first, last, lane, px, notes, fmt);
+        const bool again = settle_keys<HTGS_MODE_ALPHA_BLEND_FIRST_K, K, HTGS_PRIM_FLOATS / 4>(st, prim, inst, first, last, lane, px, core, tie, fmt, [](float, float) {});
         const uint64_t again_lanes = __ballot(again);
+        first_k_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
         if (px.inside && !again) first_k_composite<K>(prim, cd, ca, ci, image, depths, width, height, px.x, px.y, chw, median);
         if (again_lanes == 0) return;
         // (the lane and its pixel are worked out afresh: nothing of the first walk has to live through the composite for this)
@@ -1236,19 +1330,19 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
     }
 }
 
-// A core and a tie (3K + 2 rows of 64 lanes at from[]) join the running ones: they cover the stretch of the list
+// A core and a tie (3K + 1 rows of 64 lanes at from[]) join the running ones: they cover the stretch of the list
 // that follows.
 template <int K>
 __device__ __forceinline__ void first_k_merge(const float *from, uint32_t lane, float (&cd)[K], float (&ca)[K], uint32_t (&ci)[K], CoreTie &tie)
 {
-    take_tie<3 * K>(from + lane, tie);
+    take_tie<3 * K, 3 * (K - 1)>(from + lane, tie);
     merge_cores<K, true>(from + lane, cd, ca, ci, tie, [](float, float) {});
 }
 template <int K>
 __device__ __forceinline__ void first_k_put(float *to, uint32_t lane, const float (&cd)[K], const float (&ca)[K], const uint32_t (&ci)[K], const CoreTie &tie)
 {
     give_core<K>(to + lane, cd, ca, ci);
-    give_tie<3 * K>(to + lane, tie);
+    give_tie<3 * K>(to + lane, tie, cd[K - 1]);
 }
 
 // The tiles with very long lists, as in blend_hybrid_long_kernel: every wave of the workgroup walks a share of the list
@@ -1264,7 +1358,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ spare, ListThreshold threshold, const Finish finish)
 {
     constexpr int kWaves = WAVES;
-    constexpr uint32_t kRows = 3 * K + 2;
+    constexpr uint32_t kRows = 3 * K + 1;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<kWaves, kRows>()];
     __shared__ uint32_t s_next, s_whole, s_redo[2], s_listed[kWaves], s_runs[1 + kDepthBins];
     __shared__ float s_depth[kWaves][64];

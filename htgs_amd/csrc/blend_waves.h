@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
     uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const Finish finish)
 {
-    constexpr uint32_t kRows = 2 * K + 8;
+    constexpr uint32_t kRows = 2 * K + 7;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<WAVES, kRows>()];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     uint32_t tile, first, last;
@@ -90,16 +90,19 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         core[i] = make_key(__FLT_MAX__, 0u);
         asm volatile("" : "+v"(core[i]));
     }
-    CoreTie tie;
-    tie.init();
+    KeyNotes notes;
+    notes.init();
     const KeyFormat fmt = key_format(last > first ? last - first : 1u);
     // (places count from the tile's first instance, as in the single walk)
     hybrid_key_walk<K, FAST, false, HTGS_PRIM_FLOATS / 4, true>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy,
-                                                                core, tail, tie, fmt, first, ListStep(share.per * WAVES, share.per));
+                                                                core, tail, notes, fmt, first, ListStep(share.per * WAVES, share.per));
+    CoreTie tie;
+    if constexpr (FAST) tie.init();
+    else tie = noted_ties<HTGS_MODE_HYBRID_BLEND, HTGS_PRIM_FLOATS / 4>(wave_stage(lds, wave), prim, inst, first, last, lane, px, notes, fmt);
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
-            [&](float *to) { give_key_core<K>(to + lane, core); give_tail<2 * K>(to + lane, tail); if (!FAST) give_tie<2 * K + 6>(to + lane, tie); },
+            [&](float *to) { give_key_core<K>(to + lane, core); give_tail<2 * K>(to + lane, tail); if (!FAST) give_tie<2 * K + 6>(to + lane, tie, key_depth(core[K - 1])); },
             [&](const float *from) {
-                if (!FAST) take_tie<2 * K + 6>(from + lane, tie);
+                if (!FAST) take_tie<2 * K + 6, 2 * (K - 1)>(from + lane, tie);
                 merge_key_cores<K, !FAST>(from + lane, core, tie, fmt, [&](CoreKey out) { hybrid_tail_add<FAST>(tail, key_depth(out), key_alpha(key_low(out), fmt)); });
                 take_tail<2 * K>(from + lane, tail);
             })) return;
@@ -109,10 +112,10 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         key_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
         finish(prim, tile, px, cd, ca, ci, tail);
     } else {
-        key_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
         wave_lds_sync();
-        const bool again = settle_key_core<HTGS_MODE_HYBRID_BLEND, K, HTGS_PRIM_FLOATS / 4>(wave_stage(lds, 0), prim, inst, first, last, lane, px, cd, ca, ci, tie, fmt, tail_swap(tail, cd[K - 1])) && px.inside;
+        const bool again = settle_keys<HTGS_MODE_HYBRID_BLEND, K, HTGS_PRIM_FLOATS / 4>(wave_stage(lds, 0), prim, inst, first, last, lane, px, core, tie, fmt, tail_swap(tail, key_depth(core[K - 1])));
         const uint64_t again_lanes = __ballot(again);
+        key_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
         if (px.inside && !again) finish(prim, tile, px, cd, ca, ci, tail);
         if (again_lanes == 0) return;
         const uint32_t lane_again = fresh_lane();
@@ -132,7 +135,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
     uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const Finish finish)
 {
-    constexpr uint32_t kRows = 3 * K + 8;
+    constexpr uint32_t kRows = 3 * K + 7;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<WAVES, kRows>()];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     uint32_t tile, first, last;
@@ -173,7 +176,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
     uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const Finish finish)
 {
-    constexpr uint32_t kRows = 2 * K + 2;
+    constexpr uint32_t kRows = 2 * K + 1;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<WAVES, kRows>()];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     uint32_t tile, first, last;
@@ -186,26 +189,27 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         core[i] = make_key(__FLT_MAX__, 0u);
         asm volatile("" : "+v"(core[i]));
     }
-    CoreTie tie;
-    tie.init();
+    KeyNotes notes;
+    notes.init();
     const KeyFormat fmt = key_format(last > first ? last - first : 1u);
     __shared__ float s_depth[WAVES][64];
     const SharedDepth<WAVES, K> shared = { s_depth, wave, lane };
     shared.init();
     __syncthreads();
-    first_k_key_walk<K, false>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, core, tie, fmt, first, ListStep(share.per * WAVES, share.per), shared);
+    first_k_key_walk<K, false>(wave_stage(lds, wave), wave_lists<WAVES>(lds, wave), inst, prim, share.first, last, lane, px.pt, px.cx, px.cy, core, notes, fmt, first, ListStep(share.per * WAVES, share.per), shared);
+    CoreTie tie = noted_ties<HTGS_MODE_ALPHA_BLEND_FIRST_K, HTGS_PRIM_FLOATS / 4>(wave_stage(lds, wave), prim, inst, first, last, lane, px, notes, fmt);
     if (!merge_shares<WAVES, kRows>(lds, share, first, last, wave,
-            [&](float *to) { give_key_core<K>(to + lane, core); give_tie<2 * K>(to + lane, tie); },
+            [&](float *to) { give_key_core<K>(to + lane, core); give_tie<2 * K>(to + lane, tie, key_depth(core[K - 1])); },
             [&](const float *from) {
-                take_tie<2 * K>(from + lane, tie);
+                take_tie<2 * K, 2 * (K - 1)>(from + lane, tie);
                 merge_key_cores<K, true>(from + lane, core, tie, fmt, [](CoreKey) {});
             })) return;
     float cd[K], ca[K];
     uint32_t ci[K];
-    first_k_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
     wave_lds_sync();
-    const bool again = settle_key_core<HTGS_MODE_ALPHA_BLEND_FIRST_K, K, HTGS_PRIM_FLOATS / 4>(wave_stage(lds, 0), prim, inst, first, last, lane, px, cd, ca, ci, tie, fmt, [](float, float) {}) && px.inside;
+    const bool again = settle_keys<HTGS_MODE_ALPHA_BLEND_FIRST_K, K, HTGS_PRIM_FLOATS / 4>(wave_stage(lds, 0), prim, inst, first, last, lane, px, core, tie, fmt, [](float, float) {});
     const uint64_t again_lanes = __ballot(again);
+    first_k_core_unpack<K>(core, inst, first, last, cd, ca, ci, fmt);
     if (px.inside && !again) finish(prim, tile, px, cd, ca, ci);
     if (again_lanes == 0) return;
     const uint32_t lane_again = fresh_lane();
@@ -223,7 +227,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
     uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const Finish finish)
 {
-    constexpr uint32_t kRows = 3 * K + 2;
+    constexpr uint32_t kRows = 3 * K + 1;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<WAVES, kRows>()];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     uint32_t tile, first, last;

@@ -89,7 +89,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16
             if (kCore && (MODE == HTGS_MODE_ALPHA_BLEND_FIRST_K || (enters(depth) && alpha >= kMinAlphaCore))) {
                 uint32_t idx = stage_index<kStageSlots>(addr);
                 core_exchange_walk<KS>(depth, alpha, idx, cd, ca, ci);
-                if (!AGAIN && alpha > 0.0f && depth == cd[KS - 1]) tie.note(depth, idx);
+                if (!AGAIN) tie.note(meets_core_end(depth, cd[KS - 1]), depth, idx);
             }
             if (kTail) { alpha_sum += alpha; T_tail *= 1.0f - alpha; }
         };
