@@ -17,7 +17,8 @@ namespace htgs {
 // (A core of sixteen with three registers a slot does not fit the 96 registers of five waves per SIMD: 120 bytes a lane in scratch
 // memory, some of it inside the walk.  Four waves without them: training step of 1 M Gaussians at 1920x1080, HYBRID K = 16, 1734 ->
 // 1686 us, FIRST_K 1180 -> 1169, 300 k at 1280x720 481 -> 456.  Where five waves fit, as for the cores of up to eight, four cost 6 %.)
-template <int K>
+// BINNED: the lists are in bins of depth (a list by index is settled by the insertion itself, and nothing is looked for: max_weights_tile_kernel).
+template <int K, bool BINNED>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 8 ? 5 : K <= 16 ? 4 : 3))) blend_hybrid_forward_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
     uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const HybridRecords finish)
@@ -39,9 +40,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 8 
     hybrid_core_init<K>(cd, ca, ci);
     CoreTie tie;
     tie.init();
-    hybrid_walk<K, false, true, true, false, HTGS_PRIM_FLOATS_TRAIN / 4>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, tail, &tie);
-    // (a list by index is settled: the insertion was the reference's)
-    const bool again = spare != nullptr && settle_exact_core<HTGS_MODE_HYBRID_BLEND, K, HTGS_PRIM_FLOATS_TRAIN / 4>(st, prim, lane, px, cd, ca, ci, tie, tail_swap(tail, cd[K - 1])) && px.inside;
+    hybrid_walk<K, false, true, BINNED, false, HTGS_PRIM_FLOATS_TRAIN / 4>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, tail, &tie);
+    const bool again = BINNED && settle_exact_core<HTGS_MODE_HYBRID_BLEND, K, HTGS_PRIM_FLOATS_TRAIN / 4>(st, prim, lane, px, cd, ca, ci, tie, tail_swap(tail, cd[K - 1])) && px.inside;
     const uint64_t again_lanes = __ballot(again);
     if (px.inside && !again) finish(prim, tile, px, cd, ca, ci, tail);
     if (again_lanes == 0) return;
@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 8 
     if ((again_lanes >> lane_again & 1ull) != 0) finish(prim, tile, px_again, cd, ca, ci, tail);
 }
 
-template <int K>
+template <int K, bool BINNED>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 8 ? 5 : K <= 16 ? 4 : 2))) blend_first_k_forward_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, uint32_t width, uint32_t height, uint32_t grid_w,
     uint32_t *__restrict__ long_tiles, ListThreshold threshold, PartFloor part_floor, const uint32_t *__restrict__ tile_order, uint32_t *__restrict__ spare, const FirstKRecords finish)
@@ -76,8 +76,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 8 
     first_k_core_init<K>(cd, ca, ci);
     CoreTie tie;
     tie.init();
-    first_k_walk<K, false, true, true, HTGS_PRIM_FLOATS_TRAIN / 4>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie);
-    const bool again = spare != nullptr && settle_exact_core<HTGS_MODE_ALPHA_BLEND_FIRST_K, K, HTGS_PRIM_FLOATS_TRAIN / 4>(st, prim, lane, px, cd, ca, ci, tie, [](float, float) {}) && px.inside;
+    first_k_walk<K, false, true, BINNED, HTGS_PRIM_FLOATS_TRAIN / 4>(st, ql, inst, prim, first, last, lane, px.pt, px.cx, px.cy, cd, ca, ci, &tie);
+    const bool again = BINNED && settle_exact_core<HTGS_MODE_ALPHA_BLEND_FIRST_K, K, HTGS_PRIM_FLOATS_TRAIN / 4>(st, prim, lane, px, cd, ca, ci, tie, [](float, float) {}) && px.inside;
     const uint64_t again_lanes = __ballot(again);
     if (px.inside && !again) finish(prim, tile, px, cd, ca, ci);
     if (again_lanes == 0) return;
@@ -168,7 +168,8 @@ static void launch_hybrid_forward(const htgs_frame *f, int sel, uint32_t grid_w,
 {
     constexpr int REC4 = HTGS_PRIM_FLOATS_TRAIN / 4;
     const HybridRecords finish = { f->image, f->core_idx, (float4 *)f->core_info, f->tail_info, (uint32_t)f->width, (uint32_t)f->height, (size_t)n_tiles * 64u };
-    hipLaunchKernelGGL((blend_hybrid_forward_kernel<K>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim,
+    const auto kernel = frame_depth_binned(f) ? blend_hybrid_forward_kernel<K, true> : blend_hybrid_forward_kernel<K, false>;
+    hipLaunchKernelGGL(kernel, dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim,
                        (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, list_threshold(f), forward_part_floor(f, sel), f->tile_order, binned_spare(f, sel), finish);
     launch_hybrid_long<K, false, REC4>(f, sel, grid_w, finish);
 }
@@ -177,7 +178,8 @@ static void launch_first_k_forward(const htgs_frame *f, int sel, uint32_t grid_w
 {
     constexpr int REC4 = HTGS_PRIM_FLOATS_TRAIN / 4;
     const FirstKRecords finish = { f->image, f->core_idx, (float4 *)f->core_info, (uint32_t)f->width, (uint32_t)f->height, (size_t)n_tiles * 64u };
-    hipLaunchKernelGGL((blend_first_k_forward_kernel<K>), dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim,
+    const auto kernel = frame_depth_binned(f) ? blend_first_k_forward_kernel<K, true> : blend_first_k_forward_kernel<K, false>;
+    hipLaunchKernelGGL(kernel, dim3(n_tiles), dim3(64), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel], (const float4 *)f->prim,
                        (uint32_t)f->width, (uint32_t)f->height, grid_w, f->long_tiles, list_threshold(f), forward_part_floor(f, sel), f->tile_order, binned_spare(f, sel), finish);
     launch_first_k_long<K, false, REC4>(f, sel, grid_w, finish);
 }
