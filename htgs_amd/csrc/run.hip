@@ -116,29 +116,33 @@ static int waves_of(const htgs_frame *f, int what, uint64_t n_tiles)
 }
 // From how many Gaussians on the instances are made in bins of depth.  The bins cost 10 us (the sample for their limits, a scan that cannot be
 // left to the duplication, shorter runs of its output) and spare most insertions into a core: the more, the larger the core and
-// the longer the lists.  Four waves that share a list gain nothing: the near batches come first, and each wave still fills a core of its
+// the longer the lists.  Four waves that share a list gain little: the near batches come first, and each wave still fills a core of its
 // own.  Whole passes, without / with bins, over clusters (and the stress scene) on both sides of the lines:
-//   grids of four waves (374x512 to 640x480)   images, K = 16  200 k 0.89 to 0.93, 800 k 0.98 to 1.03, 1.5 M 1.00 (250 k 0.82 to 0.89, 500 k
-//     0.86 to 0.89);  K = 32  800 k 0.98, 1.5 M 1.00;  training  150 k 0.86 to 0.95, 400 k 0.97 (250 k 0.84 to 0.86, 500 k 0.82 to 0.88)
+//   grids of four waves (374x512 to 640x480)   images, K = 16  200 k 0.89 to 0.93, 800 k 0.98 to 1.03, 1.5 M 1.00, 2 M 1.02 (640x480) and 0.99 (374x512),
+//     3 M 1.05, 6 M 1.07 (250 k 0.82 to 0.89, 500 k 0.86 to 0.89);  K = 32  800 k 0.98, 1.5 M 1.00, 2 M 1.04;  K = 8  1 M 0.97, 2 M 0.99;  image alone  2 M 1.01;
+//     FIRST_K  1 M 0.98, 2 M 1.00;  training  150 k 0.86 to 0.95, 400 k 0.97 (250 k 0.84 to 0.86, 500 k 0.82 to 0.88), 2 M 1.04, FIRST_K 2 M 1.10
 //   up to 16384 tiles (900x700 to 1280x720)    images, K = 16  400 k 0.96 to 0.97, 800 k 1.02 (250 k 1.05 to 1.08, 500 k 1.01 to 1.02);  image alone
 //     500 k 0.97, 1 M 1.01;  K = 32  400 k 0.99, 800 k 1.04;  training  150 k 0.98, 400 k 1.01 to 1.03 (130 k 1.03, 250 k 1.04 to 1.06)
+//     FIRST_K, which looks at no instance behind its cores with or without bins:  K = 16  200 k 0.91, 400 k 0.94, 600 k 0.98, 800 k 1.01;  training 250 k 0.97
 //   beyond (1920x1080)                         images, K = 16  200 k 0.97 to 0.98, 400 k 1.02, 800 k 1.06;  K = 32  400 k 1.01, 800 k 1.05;  training
-//     150 k 0.99, 400 k 1.01 to 1.03;  image alone  200 k 0.98, 500 k 1.03
-//   K = 8  400 k 0.93 to 1.0, 1 M 1.02 to 1.04 (1920x1080), 0.97 (640x480), 3 M 1.03 to 1.05;   K <= 4  0.92 (320 k) to 1.01 (3 M): never
-//   weights (one wave)  70 k 0.88 to 0.98 on all, 150 k 1.02 to 1.12 (400x400, 900x700), 0.94 to 0.98 (1920x1080), 400 k 0.99 to 1.33, 1.07 to 1.08
+//     150 k 0.99, 400 k 1.01 to 1.03;  image alone  200 k 0.98, 500 k 1.03;  FIRST_K  K = 16  400 k 0.99, 600 k 1.04;  K = 32  300 k 0.97;  training  300 k 0.99, 500 k 1.02
+//   K = 8  400 k 0.93 to 1.0, 1 M 1.02 to 1.04 (1920x1080), 3 M 1.03 to 1.05, 2 M 1.00 (800x600);  FIRST_K 400 k 1.00, 800 k 1.03 (1920x1080);   K <= 4
+//     0.92 (320 k) to 1.01 (3 M): never
+//   weights (one wave)  HYBRID 1280x720 120 k 1.00, 200 k 0.97, 400 k 1.04;  1920x1080 250 k 0.96, 400 k 1.02;  640x480 150 k 0.96;  K = 32 200 k 0.93, K = 8 0.97
+//     (150 k 1.05, 400 k 1.05);  FIRST_K 1280x720 120 k 0.96, 250 k 0.99, 500 k 1.05, 1 M 1.11;  1920x1080 250 k 0.94, 500 k 1.06, 1 M 1.18;  640x480 300 k 1.12 (250 k 0.96)
 //     on the smallest grids the lists are long and walked in shares, the first of which then has the near Gaussians: stress scene 600 k at 309x378
-//     K = 16 0.87, K = 32 0.84, 250 k at 400x400 0.92; clusters 400 k at 400x400 1.01 to 1.03, 150 k at 640x480 (4800 tiles) 1.08
+//     K = 16 0.87, K = 32 0.84, 250 k at 400x400 0.92; clusters 400 k at 400x400 1.01 to 1.03
 static bool takes_depth_bins(const htgs_frame *f, int what, uint64_t n_tiles)
 {
     if (f->mode != HTGS_MODE_HYBRID_BLEND && f->mode != HTGS_MODE_ALPHA_BLEND_FIRST_K) return false;
     const int K = htgs_effective_k(f->K), n = f->n_primitives;
-    const bool wide = n_tiles > 16384;
+    const bool wide = n_tiles > 16384, first_k = f->mode == HTGS_MODE_ALPHA_BLEND_FIRST_K;
     if (K <= 4) return false;
-    if (what == HTGS_RUN_MAX_WEIGHTS) return n_tiles > 4096 && n >= (wide ? 250000 : 120000);
+    if (what == HTGS_RUN_MAX_WEIGHTS) return n_tiles > 4096 && n >= (wide ? 320000 : 300000);
     if (n_tiles <= 6144) return n >= 2000000;
-    if (what == HTGS_RUN_FORWARD) return n >= 200000;
+    if (what == HTGS_RUN_FORWARD) return n >= (first_k ? (wide ? 300000 : 400000) : 200000);
     if (K == 8) return n >= (n_tiles >= 8192 ? 800000 : 2000000);
-    return n >= (K == 16 ? (wide ? 300000 : 500000) : wide ? 400000 : 600000);
+    return n >= (K == 16 ? (wide ? 300000 : first_k ? 700000 : 500000) : wide ? 400000 : first_k ? 700000 : 600000);
 }
 constexpr uint64_t kUnorderedTiles = 1280;      // workgroups of four waves
 static uint64_t carve_front(htgs_frame *f, int what, void *base)
