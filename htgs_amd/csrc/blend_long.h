@@ -917,12 +917,14 @@ __device__ __forceinline__ void merge_all_shares(unsigned char *lds, uint32_t wa
 // the core, of either, joins the tail), the tails add up.  The pixel gets the K nearest fragments of the whole list and
 // everything else in its tail, as in a single walk; what differs from the single walk is the order in which the tail's
 // sums are added (rounding) and which of two stored fragments of exactly equal depth is kept when a nearer one arrives.
+// binned: the lists are in bins of depth (htgs_frame.depth_bins) and are put in order by index before one is walked again; the others
+// are as they are and not searched for runs.
 // finish(prim, tile, px, cd, ca, ci, tail) is called by the lanes of the first wave whose pixels lie inside the image, once
 // per pixel, with the pixel's finished core and tail.
 template <int K, int WAVES, bool FAST, int REC4, typename Finish>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(K > 16 ? 2 : kLongWavesHeld / 4))) blend_hybrid_long_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, const uint32_t *long_tiles,
-    uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ shortlist, ListThreshold threshold, const Finish finish)
+    uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ shortlist, int binned, ListThreshold threshold, const Finish finish)
 {
     constexpr int kWaves = WAVES;
     constexpr uint32_t kRows = 3 * K + 7;             // a wave's core, tail and tie
@@ -1076,7 +1078,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
                     }
                 }
                 if (threadIdx.x == 0) atomicAdd(const_cast<uint32_t *>(long_tiles) + 7, others_done ? 0x10001u : 1u);
-                const uint32_t *const list = shortlist != nullptr ? list_in_index_order_by<kWaves>(inst, first, last, shortlist, s_runs, wave, lane) : inst;
+                const uint32_t *const list = binned && shortlist != nullptr ? list_in_index_order_by<kWaves>(inst, first, last, shortlist, s_runs, wave, lane) : inst;
                 __syncthreads();
                 if (shortlist != nullptr) {
                     uint32_t kept = 0;
@@ -1355,7 +1357,7 @@ __device__ __forceinline__ void first_k_put(float *to, uint32_t lane, const floa
 template <int K, int WAVES, bool FAST, int REC4, typename Finish>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(K > 16 ? 2 : kLongWavesHeld / 4))) blend_first_k_long_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, const uint32_t *long_tiles,
-    uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ spare, ListThreshold threshold, const Finish finish)
+    uint32_t width, uint32_t height, uint32_t grid_w, uint32_t *__restrict__ spare, int binned, ListThreshold threshold, const Finish finish)
 {
     constexpr int kWaves = WAVES;
     constexpr uint32_t kRows = 3 * K + 1;
@@ -1444,7 +1446,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
                 }
                 if (threadIdx.x == 0) atomicAdd(const_cast<uint32_t *>(long_tiles) + (settled ? 6 : 7), settled || !looked ? 1u : 0x10001u);
                 const uint32_t *list = inst;
-                if (!FAST && !settled && spare != nullptr) {       // (the fast variant takes the list's own order)
+                if (!FAST && !settled && binned && spare != nullptr) {       // (the fast variant takes the list's own order)
                     list = list_in_index_order_by<kWaves>(inst, e.tile_first, e.tile_last, spare, s_runs, wave, lane);
                     __syncthreads();
                 }
@@ -1619,7 +1621,7 @@ static void launch_hybrid_long(const htgs_frame *f, int sel, uint32_t grid_w, co
     with_long_waves<K>(f, [&](auto waves) {
         constexpr int WAVES = decltype(waves)::value;
         hipLaunchKernelGGL((blend_hybrid_long_kernel<K, WAVES, FAST, REC4, Finish>), dim3(long_grid(WAVES)), dim3(64 * WAVES), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel],
-                           (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->vals[sel ^ 1], list_threshold(f), finish);
+                           (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->vals[sel ^ 1], frame_depth_binned(f) ? 1 : 0, list_threshold(f), finish);
     });
 }
 template <int K, bool FAST, int REC4, typename Finish>
@@ -1629,7 +1631,7 @@ static void launch_first_k_long(const htgs_frame *f, int sel, uint32_t grid_w, c
     with_long_waves<K>(f, [&](auto waves) {
         constexpr int WAVES = decltype(waves)::value;
         hipLaunchKernelGGL((blend_first_k_long_kernel<K, WAVES, FAST, REC4, Finish>), dim3(long_grid(WAVES)), dim3(64 * WAVES), 0, (hipStream_t)f->stream, f->ranges, f->vals[sel],
-                           (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->vals[sel ^ 1], list_threshold(f), finish);
+                           (const float4 *)f->prim, f->long_tiles, (uint32_t)f->width, (uint32_t)f->height, grid_w, f->vals[sel ^ 1], frame_depth_binned(f) ? 1 : 0, list_threshold(f), finish);
     });
 }
 template <bool FAST, int REC4, bool DEPTH, typename Finish>
