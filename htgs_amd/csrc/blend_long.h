@@ -929,6 +929,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     constexpr int kWaves = WAVES;
     constexpr uint32_t kRows = 3 * K + 7;             // a wave's core, tail and tie
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<kWaves, kRows>()];
+    static_assert(shared_walk_lds<kWaves, kRows>() >= 3u * kAgainEntries * sizeof(uint32_t), "entries_in_order lies over it");
     __shared__ uint32_t s_next;
     __shared__ uint32_t s_redo[2];                    // the pixels (lanes) to walk again
     __shared__ uint32_t s_short[kWaves];          // how many instances of each share reach one of them
@@ -1362,6 +1363,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     constexpr int kWaves = WAVES;
     constexpr uint32_t kRows = 3 * K + 1;
     __shared__ __attribute__((aligned(16))) unsigned char lds[shared_walk_lds<kWaves, kRows>()];
+    static_assert(shared_walk_lds<kWaves, kRows>() >= 3u * kAgainEntries * sizeof(uint32_t), "entries_in_order lies over it");
     __shared__ uint32_t s_next, s_whole, s_redo[2], s_listed[kWaves], s_runs[1 + kDepthBins];
     __shared__ float s_depth[kWaves][64];
     __shared__ float s_last_depth[64];
