@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from htgs_amd.synthetic import make_scene
-from htgs_amd.torch_bindings import FrameBuffers, RasterizerMode, diff_rasterize, rasterize, update_max_weights
+from htgs_amd.torch_bindings import FrameBuffers, RasterizerMode, diff_rasterize, fast_rasterize, rasterize, update_max_weights
 from htgs_amd.torch_bindings.rasterization import ScratchPool, run_max_weights
 from test_gpu_long_tiles import with_coincident_copies
 
@@ -167,6 +167,40 @@ def test_operators(cuda, mode):
         # (a weight within rounding of the threshold may fall on the other side of it)
         both = (weights > 0) & (by_stages > 0)
         assert ((weights - by_stages).abs()[both] <= 1e-5 * by_stages[both]).all() and int((both != ((weights > 0) | (by_stages > 0))).sum()) <= 2
+
+
+def within_fast_bounds(fast, exact):
+    """What the image-only path may differ by (tests/test_gpu_parity.py): a fragment within an ulp of an alpha threshold is decided differently,
+    1/20 of a colour at most, in fewer than a pixel of a thousand."""
+    diff = (fast - exact).abs()
+    return float((diff > 1e-5).float().mean()) < 1e-3 and float(diff.max()) <= 5e-2
+
+
+@pytest.mark.parametrize("waves,threshold", [(1, 0), (2, 0), (4, 0), (1, 60)])
+@pytest.mark.parametrize("K", [1, 8, 16, 32])
+@pytest.mark.parametrize("mode", [HYBRID, FIRST_K])
+@pytest.mark.parametrize("kind", ["plain", "near"])
+def test_image_alone(cuda, kind, mode, K, waves, threshold):
+    """The image-only kernels over lists in bins, against the exact walk by insertion over the list by index."""
+    print(f"case kind={kind} mode={mode} K={K} waves={waves} threshold={threshold}", flush=True)
+    sg = build(kind).to(cuda)
+    want, _ = frame(sg, mode, K, False, long_list_threshold=2 ** 31 - 1).run()
+    fb = frame(sg, mode, K, True, fast=True, order_gaussians=False, waves_per_tile=waves, long_list_threshold=threshold)
+    got, _ = fb.run()
+    assert fb.frame.depth_bins and not fb.frame.depth_order
+    assert within_fast_bounds(got, want)
+
+
+@pytest.mark.parametrize("K", [8, 16, 32])
+@pytest.mark.parametrize("mode", [HYBRID, FIRST_K])
+def test_fast_operator(cuda, mode, K):
+    """``fast_rasterize`` takes bins for 810 000 Gaussians on a grid of one wave a tile."""
+    print(f"case mode={mode} K={K}", flush=True)
+    sg = small_view(make_scene(1, 810_000), 1300, 1000).to(cuda)
+    s = sg.settings(RasterizerMode(mode), K)
+    got = fast_rasterize(*sg.gaussians(), s, True)
+    assert ScratchPool.current(cuda).frame.depth_bins
+    assert within_fast_bounds(got, frame(sg, mode, K, False, long_list_threshold=2 ** 31 - 1).run()[0])
 
 
 @pytest.mark.parametrize("width,height,n,bins", [(640, 480, 340_000, False), (1300, 1000, 199_999, False), (1300, 1000, 340_000, True)])
