@@ -51,7 +51,7 @@ __device__ __forceinline__ int find_core_slot(const uint32_t *__restrict__ keys,
 // (R/include/alpha_blend_first_k/kernels/backward.cuh:60-206); walking the tile's list and looking each
 // (Gaussian, pixel) up in the stored core visits the same fragments.
 // ---------------------------------------------------------------------------------------------
-// A workgroup is four waves sharing one tile's per-pixel terms and a chunk of 256 instances in LDS (17 KB for K = 16); the
+// A workgroup is four waves sharing one tile's per-pixel terms and a chunk of 256 instances in LDS (17 KB for K = 16, FIRST_K 2.5 more); the
 // waves take the turns of the chunk one after the other.
 constexpr int kBackwardWaves = 4;
 

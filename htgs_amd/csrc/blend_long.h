@@ -106,7 +106,8 @@ __device__ __forceinline__ void hybrid_walk(TileStageQ &st, QuadrantLists &ql, c
 // is pushed out carries the alpha that the tail needs.  The Gaussian's index, which only the final core needs, is looked
 // up from the place in the list when the pixel is composited.  Which of two fragments of equal depth comes first is
 // decided by the low word here, not by the reference's insertion: the image-only fast path leaves it at that; with exact
-// arithmetic the walk notes where it can matter (hybrid_key_walk) and such pixels are walked again.
+// arithmetic the walk notes where it can matter (hybrid_key_walk), such pixels are settled from their cores (settle_core), and those
+// with more than two fragments of a depth are walked again.
 // ---------------------------------------------------------------------------------------------
 typedef double CoreKey;
 constexpr uint32_t kPackedListMost = 8192;
@@ -388,8 +389,8 @@ struct HybridImage {
 
 // One tile by one wave with the core as keys; finish(prim, tile, px, cd, ca, ci, tail) is called once per pixel inside the
 // image.  Without FAST, the pixels at which fragments of exactly equal depth met where they decide the core (a pixel or
-// two in a tile in a hundred) are walked again afterwards, over the instances that reach one of them, with the
-// reference's insertion.
+// two in a tile in a hundred) are settled from it, and where more than two are as deep as each other walked again afterwards, over
+// the instances that reach one of them, with the reference's insertion.
 template <int K, bool FAST, int REC4, typename Finish>
 __device__ __forceinline__ void hybrid_tile_by_keys(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                     uint32_t tile, uint32_t first, uint32_t last, uint32_t lane, const TilePixel &px, uint32_t grid_w,
@@ -434,11 +435,11 @@ __device__ __forceinline__ void hybrid_tile_by_keys(TileStageQ &st, QuadrantList
 }
 
 // ---------------------------------------------------------------------------------------------
-// Several waves share a list: what each has walked is merged pairwise, in list order.  Two sorted cores are merged without
+// Several waves share a list, every WAVES-th batch of it each: what each has walked is merged pairwise.  Two sorted cores are merged without
 // insertions: the nearer of entry i of one and entry K - 1 - i of the other are the K nearest of both (what is farther
 // joins the tail), in an order that log2 K rounds of compare and exchange sort -- K = 16: 48 exchanges of 28 cycles (8 for
 // keys), where inserting sixteen entries one by one takes 9000 cycles.  Which entry of exactly equal depth stays is not the
-// reference's choice then: tie receives the least depth at which that can matter, as in the walks.
+// reference's choice then: the merges note what was left out exactly as deep as the last entry that stays, as the walks do.
 // ---------------------------------------------------------------------------------------------
 // LDS of a workgroup whose waves walk shares and then hand them on, ROWS rows of 64 lanes a share: the merge buffers, one
 // per pair of waves, lie over the stages.
@@ -911,10 +912,9 @@ __device__ __forceinline__ void merge_all_shares(unsigned char *lds, uint32_t wa
     }
     __syncthreads();                                       // (the stages are free again)
 }
-// The long tiles: a workgroup of WAVES waves takes a tile, every wave walks a contiguous share of the list (whole
-// batches of 64) into a core and a tail of its own, and the shares are then merged into the first wave's, in list
-// order, through LDS: the entries of the incoming core enter the running core like fragments (what does not stay in
-// the core, of either, joins the tail), the tails add up.  The pixel gets the K nearest fragments of the whole list and
+// The long tiles: a workgroup of WAVES waves takes a tile, every wave walks a share of the list (every WAVES-th batch of 64)
+// into a core and a tail of its own, and the shares are then merged pairwise into the first wave's, through LDS: the nearer
+// entries of both cores stay (what does not, of either, joins the tail), the tails add up.  Nothing of this is in list order.  The pixel gets the K nearest fragments of the whole list and
 // everything else in its tail, as in a single walk; what differs from the single walk is the order in which the tail's
 // sums are added (rounding) and which of two stored fragments of exactly equal depth is kept when a nearer one arrives.
 // binned: the lists are in bins of depth (htgs_frame.depth_bins) and are put in order by index before one is walked again; the others
@@ -967,7 +967,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         if (parts > 1u) {
             // One of several parts: what it came to goes to the tile's stretch of the spare value buffer (which is as long as the
             // list and unused until pixels are walked again), and the workgroup that finds the other parts there already
-            // merges them all, in list order, and goes on with the whole tile.
+            // merges them all, one after the other, and goes on with the whole tile.
             float *const left = reinterpret_cast<float *>(shortlist + tile_first);
             if (wave == 0) {
                 hybrid_put<K>(left + (size_t)part * long_part_words<K>(), lane, cd, ca, ci, tail, tie);
@@ -1025,7 +1025,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
                         reinterpret_cast<TileStage<64> &>(wave_stage(lds, wave)), inst, prim, seg_first, seg_last, lane, px.cx, px.cy, redo_lanes, s_last_depth, s_sums[wave], shortlist + seg_first,
                         (seg_last - seg_first) / 4u, [&](const uint32_t (&pixel)[kAgainPixels]) {
                             __syncthreads();
-                            if (wave == 0 && lane < (uint32_t)kAgainPixels) {      // the waves' sums of a pixel, in list order
+                            if (wave == 0 && lane < (uint32_t)kAgainPixels) {      // the waves' sums of a pixel, wave after wave (contiguous shares here)
                                 uint32_t mine = pixel[0];
 #pragma unroll
                                 for (int j = 1; j < kAgainPixels; ++j) mine = lane == (uint32_t)j ? pixel[j] : mine;
@@ -1160,8 +1160,8 @@ struct NoSharedDepth {
     __device__ __forceinline__ float operator()(float) const { return __FLT_MAX__; }
 };
 // The walk over instances [first, last) of a tile's list by one wave (SOLO: the wave is the whole workgroup).  TIES (the
-// walks of blend_first_k_long_kernel): `tie` receives the least depth at which an entry was pushed out of the core that is
-// exactly as deep as the entry that is now last.
+// walks whose pixels are settled afterwards): `tie` notes the entries that stayed out of the core, or left it, exactly as deep as the
+// entry that is now last (CoreTie).
 // PIXELS: only the pixels of the lanes in pixel_lanes are wanted; instances that do not reach one of them are left out.
 template <int K, bool FAST, bool SOLO, bool TIES = false, int REC4 = HTGS_PRIM_FLOATS / 4, bool PIXELS = false, typename Shared = NoSharedDepth>
 __device__ __forceinline__ void first_k_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
@@ -1188,7 +1188,7 @@ __device__ __forceinline__ void first_k_walk(TileStageQ &st, QuadrantLists &ql, 
     });
 }
 // The same walk with the core as sorted 64-bit keys (above HYBRID_BLEND's: depth | alpha as a fraction | place in the list),
-// exact arithmetic; `tie` as in hybrid_key_walk.
+// exact arithmetic; `notes` as in hybrid_key_walk.
 template <int K, bool SOLO, int REC4 = HTGS_PRIM_FLOATS / 4, typename Shared = NoSharedDepth>
 __device__ __forceinline__ void first_k_key_walk(TileStageQ &st, QuadrantLists &ql, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
                                                  uint32_t first, uint32_t last, uint32_t lane, const PixelTerms &pt, float cx, float cy,
@@ -1276,8 +1276,8 @@ struct FirstKImage {
 // what a workgroup leaves of its part of a list: the core and what met at its end
 template <int K> constexpr uint32_t first_k_part_words() { return (3u * K + 1u) * 64u; }
 // KEYS (exact arithmetic, with long_tiles and a threshold of no more than kPackedListMost): the core as sorted 64-bit keys;
-// the pixels at which fragments of exactly equal depth met where they decide the core are walked again afterwards, over the
-// instances that reach one of them, with the reference's insertion (as in hybrid_tile_by_keys).
+// the pixels at which fragments of exactly equal depth met where they decide the core are settled as in hybrid_tile_by_keys: from the
+// core, or by another walk with the reference's insertion over the instances that reach one of them.
 template <int K, bool FAST, bool KEYS = false>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(K <= 16 ? 5 : 2))) blend_first_k_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim,
@@ -1349,12 +1349,12 @@ __device__ __forceinline__ void first_k_put(float *to, uint32_t lane, const floa
 }
 
 // The tiles with very long lists, as in blend_hybrid_long_kernel: every wave of the workgroup walks a share of the list
-// into a core of its own, the cores are merged in list order (and so are those of the parts of a list that several
+// into a core of its own, the cores are merged (and so are those of the parts of a list that several
 // workgroups walked, through the tile's stretch of the spare value buffer `spare`), and the pixels at which fragments of
-// exactly equal depth met where they can change the final core get a second look (pixels_again) with the insertion
-// replayed on the fragments that are not farther than the merged core's last entry -- or, when they are many or the room
+// exactly equal depth met where they can change the final core are settled from it where no more than two are of a depth (exact
+// arithmetic); the others get a second look (pixels_again) with the insertion replayed by index on the fragments that are not farther than the merged core's last entry -- or, when they are many or the room
 // for those fragments does not do, the first wave walks the whole list again for them.
-// finish(prim, tile, px, cd, ca, ci): as for blend_hybrid_long_kernel, with the pixel's finished core.
+// binned, finish(prim, tile, px, cd, ca, ci): as for blend_hybrid_long_kernel, with the pixel's finished core.
 template <int K, int WAVES, bool FAST, int REC4, typename Finish>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(K > 16 ? 2 : kLongWavesHeld / 4))) blend_first_k_long_kernel(
     const uint32_t *__restrict__ ranges, const uint32_t *__restrict__ inst, const float4 *__restrict__ prim, const uint32_t *long_tiles,

@@ -6,8 +6,8 @@
 // idle beside it.  Here a workgroup of WAVES waves takes a tile: every wave walks a share of the list (every
 // WAVES-th batch) into a core and a tail of its own, and the shares are merged pairwise through LDS.
 // As in the kernels for very long lists, which entry of exactly equal depth stays is not the reference's choice then, so the
-// walks and the merges note the least depth at which that could matter, and such pixels are walked again in one piece by
-// the reference's insertion.  Sums come out in another order than in a single walk (rounding).
+// walks and the merges note the entries as deep as the last one of the core, such pixels are settled from their cores (settle_core), and
+// those with more than two fragments of a depth are walked again in one piece by the reference's insertion.  Sums come out in another order than in a single walk (rounding).
 // Tiles x waves, one -> four waves: 10 k Gaussians at 256x256, K = 4: 38 -> 25 us; training pass of 20 k at 400x304, K = 16: 81 -> 36 us.
 // From some number of tiles on, the workgroup's LDS, which is held until its first wave has finished the pixels, and the merging
 // cost more than the shorter lists give (1920x1080 HYBRID 965 -> 1137 us); htgs_run's lines are in run.hip (waves_of).

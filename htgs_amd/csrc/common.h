@@ -45,8 +45,8 @@ inline int frame_prim_floats(const htgs_frame *f)
 }
 
 // The Gaussians are sorted by depth before the instances are made (htgs_frame.depth_order): ALPHA_BLEND_GLOBAL_ORDERING,
-// whose lists must be in depth order, and the image-only fast path of the two modes with a sorted core, whose lists may
-// be in any order and whose insertions become rare when the fragments arrive roughly front to back (coarse keys, one pass)
+// whose lists must be in depth order, and, for callers of the stages that ask for it, the image-only fast path of the two modes with a
+// sorted core, whose lists may be in any order (coarse keys, one pass; htgs_run has bins of depth there instead)
 inline bool frame_coarse_depth_ordered(const htgs_frame *f)
 {
     return f->depth_order != nullptr && f->fast_math && (f->mode == HTGS_MODE_HYBRID_BLEND || f->mode == HTGS_MODE_ALPHA_BLEND_FIRST_K);

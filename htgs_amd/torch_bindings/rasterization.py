@@ -247,8 +247,8 @@ class FrameBuffers:
                            if order_tiles else None)
         # GLOBAL_ORDERING inference: the Gaussians sorted by depth before the instances are made, whose keys then hold the
         # tile alone (two sort passes over 2-byte keys instead of five over 8-byte keys, the same sorted list).  The
-        # image-only fast path of the two modes with a sorted core: the same with coarse depth keys (one pass), so that a
-        # tile's fragments arrive roughly front to back and few of them have to be inserted in front of others
+        # image-only fast path of the two modes with a sorted core, by these stages (``fast_rasterize`` takes bins of depth instead): the same
+        # with coarse depth keys (one pass), so that a tile's fragments arrive roughly front to back
         self.depth_order = (self._scratch("depth_order", self.lib.htgs_depth_order_words(n), torch.int32)
                             if order_gaussians and not train and (mode == 2 or (fast and mode in (0, 1))) else None)
         # the instances made bin by bin of depth, nearest first (HYBRID and FIRST_K, what ``rasterize`` and the others do with many Gaussians)

@@ -242,9 +242,9 @@ int htgs_extract_ranges(const htgs_frame *f, int selector);
 /* blend_cu of the frame's mode (R/include/<mode>/kernels/inference.cuh:78-216).
  * HYBRID_BLEND, ALPHA_BLEND_FIRST_K and OIT_BLEND with f->long_tiles: a second launch walks the tiles whose lists exceed
  * long_list_threshold with sixteen waves each (the longest in parts, by several such workgroups) and merges their
- * K-buffers and sums in list order; a pixel's result is that of the single walk up to the rounding of the sums of
- * HYBRID's tail and of OIT (pixels at which fragments of exactly equal depth met get the reference's insertion replayed in
- * list order on the fragments that decide the K-buffer; FIRST_K comes out bit for bit).  That launch uses the spare
+ * K-buffers and sums; a pixel's result is that of the single walk up to the rounding of the sums of
+ * HYBRID's tail and of OIT (pixels at which fragments of exactly equal depth met are settled from the K-buffer, or get the reference's
+ * insertion replayed by index on the fragments that decide it; FIRST_K comes out bit for bit).  That launch uses the spare
  * value buffer vals[1 - selector] as scratch (its content is lost; NULL: a slower path without it, one workgroup per
  * tile).  Without long_tiles the stage reads vals[selector] only.  How a long list is split over workgroups depends on its
  * length and on n_instances alone: results do not depend on the order in which workgroups run.

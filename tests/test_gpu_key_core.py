@@ -1,6 +1,6 @@
 """The kernels of HYBRID_BLEND and ALPHA_BLEND_FIRST_K with one wave per tile keep the K nearest fragments as sorted 64-bit keys (depth above alpha as a
 fraction of 19 to 23 bits above the place in the list) when the frame has the list for long tiles and no list of the launch
-is longer than 8192; pixels at which fragments of exactly equal depth met where they decide the core are walked again with the
+is longer than 8192; pixels at which fragments of exactly equal depth met where they decide the core are settled from it, or walked again with the
 reference's exchange insertion (R/include/hybrid_blend/kernels/inference.cuh:159-167,
 R/include/alpha_blend_first_k/kernels/inference.cuh:155-163).  Without that list -- or with a
 threshold above 8192 -- the same kernel keeps (depth, alpha, index) triples and inserts by exchange throughout.  The two
